@@ -220,6 +220,37 @@ def test_ipa_prove_vs_oracle(zkh, ctx, n):
     assert bytes(st_g) == bytes(st_o)
 
 
+@pytest.mark.parametrize("ns", [(16,), (128, 2, 512), (256, 1, 256, 256)])
+def test_ipa_special_points_vs_oracle(zkh, ctx, ns):
+    """Batches whose generators hold the point at infinity, equal points and opposite ones, with
+    zero, one and r - 1 among the scalars: the doubling, infinity and cancelling branches of the
+    row-form point operations, trees of one block and of two launches, jobs that drop out."""
+    rng = np.random.default_rng(350 + len(ns))
+    jobs, want = [], []
+    for t, n in enumerate(ns):
+        gens = gens_for(90 + t, n + 1)
+        if n > 2:
+            gens[1] = G.g1_zero()
+            gens[n // 2] = gens[0]
+            gens[n // 2 + 1] = C.g1_mul(gens[2], np.array(P.to_limbs(P.R - 1), np.uint32))
+        a = [int.from_bytes(rng.bytes(32), "little") % P.R for _ in range(n)]
+        a[0], a[n // 2], a[n - 1] = 1, 0, P.R - 1
+        if n > 4:
+            a[n // 2 + 2] = a[n // 2 + 3] = 1
+        b = C.ints_to_fr([int.from_bytes(rng.bytes(32), "little") % P.R for _ in range(n)])
+        a = C.ints_to_fr(a)
+        st_o = C.tr_init("ipas-%d" % t)
+        rc, L, R, af = C.ipa_prove(st_o, a, b, gens[:n], gens[n], n)
+        assert rc == 0
+        want.append((L, R, af, bytes(st_o)))
+        jobs.append((zkh.transcript("ipas-%d" % t), ctx.from_fr(a), ctx.from_fr(b), ctx.g1_from_host(gens[:n]), gens[n]))
+    got = ctx.ipa_prove_batch(jobs)
+    for (st, *_), g, (L, R, af, st_o) in zip(jobs, got, want):
+        assert np.array_equal(g["L"], L) and np.array_equal(g["R"], R)
+        assert np.array_equal(g["a_final"], af)
+        assert bytes(st) == st_o
+
+
 def test_ipa_prove_int_witness_and_errors(zkh, ctx):
     """a from an int32 tensor (a folded weight row is small until it is folded); sizes that
     are not a power of two or disagree are ZKH_EARG."""

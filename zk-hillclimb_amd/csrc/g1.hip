@@ -1,5 +1,6 @@
 // g1.hip -- G1 Pedersen commitment kernels (bucket method, commitment.cu:47-103).
 #include "fp_dev.hpp"
+#include "fp_row.hpp"
 #include "fr_dev.hpp"
 #include "g1.hpp"
 
@@ -233,43 +234,39 @@ __device__ __forceinline__ g1_t g1_mul_quad(g1_t a, const uint32_t s[8], int q) 
     return acc;
 }
 
-// G1Jacobian_mul as g1_mul_quad, split over the two waves of a 128-thread block: wave 0 runs
-// the doubling chain a, 2a, 4a, ... and hands each 2^i a to wave 1 through LDS, G1P_B
-// doublings per block barrier; wave 1 adds the ones whose bit is set into acc one barrier
-// later.  The additions and doublings are those of g1_mul_quad in the same order (the same
-// Jacobian representative); the two chains run side by side instead of one after the
-// other.  Both waves call it with the same scalar for lane slot threadIdx.x & 63 and the
-// same `active` (wave 1 does not read `a`); the product is in wave 1's lanes.  Every thread
-// of the block takes the same 256 / G1P_B + 1 barriers.
-#define G1P_B 8
-typedef uint32_t g1_pipe_buf[2][G1P_B][16][36];
-__device__ __forceinline__ g1_t g1_mul_quad_pipe(g1_t a, const uint32_t s[8], int q, bool active,
-                                                 g1_pipe_buf& buf) {
+// G1Jacobian_mul (g1-tensor.cu:445-454) on two waves of the row form (fp_row.hpp): wave 0 of
+// the pair runs the doubling chain a, 2a, 4a, ... and hands each 2^i a to wave 1 through LDS,
+// G1P_B doublings per block barrier; wave 1 adds the ones whose bit is set into acc one barrier
+// later.  The additions and doublings are those of the one-chain form in the same order (the
+// same Jacobian representative), and the doublings after the highest set bit are skipped.  The
+// chain is latency-bound: 0.77 us per doubling and 1.28 us per addition on an idle SIMD (a
+// lane quad per point took 6.9 and 13.5 us), so 255 doublings and 127 additions side by side
+// take 0.2 ms.  At 16 doublings per barrier the additions of a chunk (10 +- 2.6 us) rarely
+// outlast its doublings (12.3 us).  Every wave of the block calls it (dbl: its part), with one
+// scalar per pair; the product is in the adding wave, which does not read `a`.
+#define G1P_B 16
+typedef uint32_t g1_pipe_buf[2][G1P_B][G1R_WORDS];
+__device__ __forceinline__ g1r_t g1r_mul_pipe(g1r_t a, const uint32_t s[8], bool dbl, g1_pipe_buf& buf,
+                                              const fpr_k& c) {
     static_assert(32 % G1P_B == 0, "a chunk's bits lie in one scalar limb");
-    const bool dbl_wave = threadIdx.x < 64;
-    const uint32_t slot = (threadIdx.x & 63) >> 2;
     int top = -1;
-    if (active)
-        for (int l = 7; l >= 0 && top < 0; l--)
-            if (s[l]) top = 32 * l + 31 - __builtin_clz(s[l]);
-    g1_t acc = g1_zero();
+    for (int l = 7; l >= 0 && top < 0; l--)
+        if (s[l]) top = 32 * l + 31 - __builtin_clz(s[l]);
+    g1r_t acc = g1r_zero(c);
     constexpr int NC = 256 / G1P_B;
     for (int k = 0; k <= NC; k++) {
-        if (dbl_wave) {
-            if (k < NC) {
-                for (int j = 0; j < G1P_B; j++) {
-                    const int i = k * G1P_B + j;
-                    if (i <= top) {
-                        if (q == 0) g1_store(buf[k & 1][j][slot], a);
-                        if (i < top) a = g1_dbl_quad(a, q);
-                    }
-                }
+        if (dbl) {
+            for (int j = 0; j < G1P_B; j++) {
+                const int i = k * G1P_B + j;
+                if (i > top) break;
+                g1r_put(buf[k & 1][j], a, c);
+                if (i < top) a = g1r_dbl(a, c);
             }
         } else if (k > 0) {
             const uint32_t w = limb8(s, (uint32_t)((k - 1) * G1P_B) >> 5);
             for (int j = 0; j < G1P_B; j++) {
                 const int i = (k - 1) * G1P_B + j;
-                if (i <= top && ((w >> (i & 31)) & 1u)) acc = g1_add_quad(acc, g1_load(buf[(k - 1) & 1][j][slot]), q);
+                if (i <= top && ((w >> (i & 31)) & 1u)) acc = g1r_add(acc, g1r_get(buf[(k - 1) & 1][j], c), c);
             }
         }
         __syncthreads();
@@ -305,122 +302,163 @@ __global__ __launch_bounds__(64) void k_g1_addmul(const uint32_t* __restrict__ a
 }
 
 // ---- inner-product argument rounds (ipa_prove, vrf_common.cuh:302-336) ----
-// a, b: plain Fr, 8 words per entry; g, P: points.  Round of size 2h:
-//   ip = (<a_lo, b_hi>, <a_hi, b_lo>)                       (dev_ip, one block)
+// a, b: plain Fr, 8 words per entry; g, Q, P: points in row form (G1R_WORDS each).  Round of
+// size 2h:
+//   ip = (<a_lo, b_hi>, <a_hi, b_lo>)
 //   P[j] = g_hi[j] a_lo[j], P[h + j] = g_lo[j] a_hi[j], P[2h] = Q ip_L, P[2h+1] = Q ip_R
 //   pairwise trees over P[0, h) and P[h, 2h)                  (dev_msm's order)
 //   L = P[0] + P[2h], R = P[h] + P[2h+1]
 //   fold: a' = x a_lo + x^-1 a_hi, b' = x^-1 b_lo + x b_hi, g' = x^-1 g_lo + x g_hi
-__global__ __launch_bounds__(256) void k_ipa_ip(IpaBatchDev B, fr_t r2) {
+// A round of few points is the latency of its two scalar-multiply chains (scale and fold) and
+// one of many points the instruction rate; both are taken on two waves per product.
+
+// the working copies of g and Q in row form, one wave per point (point n of a job is Q)
+__global__ __launch_bounds__(256) void k_ipa_points(IpaBatchDev B) {
     const IpaJobDev& J = B.j[blockIdx.y];
-    const uint32_t h = J.h;
-    if (!h) return;  // the job has finished its rounds (whole block)
-    const uint32_t *a = J.a, *b = J.b;
-    __shared__ fr_t red[2][256];
-    fr_t sl = fr_zero(), sr = fr_zero();
-    for (uint32_t i = threadIdx.x; i < h; i += 256) {
-        sl = fr_add(sl, mont_mul(ld_aos(a, i), ld_aos(b, h + i)));
-        sr = fr_add(sr, mont_mul(ld_aos(a, h + i), ld_aos(b, i)));
-    }
-    red[0][threadIdx.x] = sl;
-    red[1][threadIdx.x] = sr;
+    const uint32_t n = 2 * J.h, i = blockIdx.x * 4 + threadIdx.x / 64;
+    if (i > n) return;
+    const fpr_k c = fpr_consts();
+    g1r_put(J.g0 + G1R_WORDS * (size_t)i, g1r_load(i < n ? J.g_in + 36 * (size_t)i : J.Q, c), c);
+}
+// Scale and fold launches hold exactly the blocks of the jobs still folding (job j's from
+// scale0 / fold0 on), and ask for so much LDS that a CU takes no more than its share of them:
+// the dispatcher otherwise stacks blocks on some CUs while others idle, and a chain sharing
+// its SIMD runs at the SIMD's rate, not at its own latency.
+__device__ __forceinline__ uint32_t ipa_job(const IpaBatchDev& B, uint32_t nj, uint32_t blk, bool scale) {
+    uint32_t job = 0;
+    for (uint32_t j = 1; j < nj; j++)
+        if (B.j[j].h && blk >= (scale ? B.j[j].scale0 : B.j[j].fold0)) job = j;
+    return job;
+}
+// dynamic LDS per block beside `used` static bytes; `least` blocks give every SIMD of a CU one wave
+static uint32_t lds_share(uint32_t blocks, uint32_t least, uint32_t used) {
+    const uint32_t per_cu = blocks <= 256 * least ? least : (blocks + 255) / 256;
+    if (per_cu > 8) return 0;
+    const uint32_t want = 160 * 1024 / (per_cu + 1) + 512;  // per_cu + 1 blocks do not fit
+    return want > used ? want - used : 0;
+}
+// <a_lo, b_hi> (side 0) or <a_hi, b_lo> (side 1) by the block's threads, plain, to `out` (LDS)
+__device__ __forceinline__ void ipa_inner(const IpaJobDev& J, uint32_t side, const fr_t& r2, fr_t* red,
+                                          uint32_t* out) {
+    const uint32_t h = J.h, nt = blockDim.x;
+    fr_t s = fr_zero();
+    for (uint32_t i = threadIdx.x; i < h; i += nt)
+        s = fr_add(s, mont_mul(ld_aos(J.a, side ? h + i : i), ld_aos(J.b, side ? i : h + i)));
+    red[threadIdx.x] = s;
     __syncthreads();
-    for (uint32_t o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) {
-            red[0][threadIdx.x] = fr_add(red[0][threadIdx.x], red[0][threadIdx.x + o]);
-            red[1][threadIdx.x] = fr_add(red[1][threadIdx.x], red[1][threadIdx.x + o]);
-        }
+    for (uint32_t o = nt / 2; o > 0; o >>= 1) {
+        if (threadIdx.x < o) red[threadIdx.x] = fr_add(red[threadIdx.x], red[threadIdx.x + o]);
         __syncthreads();
     }
-    // sums of a b 2^-256; times R^2 2^-256 gives the plain sums
-    if (threadIdx.x < 2) st_aos(J.ip, threadIdx.x, mont_mul(red[threadIdx.x][0], r2));
+    // a sum of a b 2^-256; times R^2 2^-256 gives the plain sum
+    if (threadIdx.x == 0) st_aos(out, 0, mont_mul(red[0], r2));
+    __syncthreads();
 }
 // L and R terms (vrf_common.cuh:316-319): P[j] = g[h + j] a[j], P[h + j] = g[j] a[h + j],
-// P[2h], P[2h + 1] = Q <a_lo, b_hi>, Q <a_hi, b_lo>; 16 products per 128-thread block, each
-// on a quad of both waves (g1_mul_quad_pipe); blockIdx.y is the job
-__global__ __launch_bounds__(128) void k_ipa_scale(IpaBatchDev B) {
-    const IpaJobDev& J = B.j[blockIdx.y];
-    const uint32_t h = J.h;
-    if (blockIdx.x * 16 >= 2 * h + 2 || !h) return;  // whole block: past the job's products
+// P[2h], P[2h + 1] = Q <a_lo, b_hi>, Q <a_hi, b_lo>; one product per block.  Blocks 0 and 1
+// take the Q products and their inner products (first, since they are the longest).
+__global__ __launch_bounds__(128) void k_ipa_scale(IpaBatchDev B, uint32_t nj, fr_t r2) {
+    const IpaJobDev& J = B.j[ipa_job(B, nj, blockIdx.x, true)];
+    const uint32_t h = J.h, blk = blockIdx.x - J.scale0;
+    if (blk >= 2 * h + 2) return;  // whole block
     __shared__ g1_pipe_buf buf;
-    const uint32_t j = blockIdx.x * 16 + (threadIdx.x & 63) / 4;
-    const int q = threadIdx.x & 3;
-    const bool active = j < 2 * h + 2;
-    uint32_t sc[8] = {};
-    g1_t base = g1_zero();
-    if (active) {
-        const uint32_t* bp = j < h ? J.g + 36 * (size_t)(h + j) : j < 2 * h ? J.g + 36 * (size_t)(j - h) : J.Q;
-        const uint32_t* sp = j < 2 * h ? J.a + 8 * (size_t)j : J.ip + 8 * (j - 2 * h);
+    __shared__ fr_t red[128];
+    __shared__ uint32_t ip[8];
+    const fpr_k c = fpr_consts();
+    const uint32_t j = blk < 2 ? 2 * h + blk : blk - 2;
+    const bool dbl = __builtin_amdgcn_readfirstlane(threadIdx.x / 64) == 0;
+    if (blk < 2) ipa_inner(J, blk, r2, red, ip);
+    const uint32_t* sp = blk < 2 ? ip : J.a + 8 * (size_t)j;
+    uint32_t sc[8];
 #pragma unroll
-        for (int k = 0; k < 8; k++) sc[k] = sp[k];
-        if (threadIdx.x < 64) base = g1_load(bp);
+    for (int k = 0; k < 8; k++) sc[k] = __builtin_amdgcn_readfirstlane(sp[k]);
+    const uint32_t* bp = j < h ? J.g + G1R_WORDS * (size_t)(h + j) : j < 2 * h ? J.g + G1R_WORDS * (size_t)(j - h) : J.Qr;
+    g1r_t base = g1r_zero(c);
+    if (dbl) base = g1r_get(bp, c);
+    const g1r_t r = g1r_mul_pipe(base, sc, dbl, buf, c);
+    if (!dbl) g1r_put(J.P + G1R_WORDS * (size_t)j, r, c);
+}
+// pairwise trees over P[0, h) and P[h, 2h): of a side's m = h >> shift remaining points a block
+// takes the K = min(m, 64) at distance m / K (six levels of the tree: level by level the halves
+// are added, as dev_msm does) and leaves their sum in the first; the block that takes the last
+// ones adds the side's Q term and writes L or R, canonical, to the host.  Sixteen waves, one
+// addition each per level; partial sums stay in LDS.
+static_assert(ZKH_ROW_WORDS == G1R_WORDS, "point size");
+__global__ __launch_bounds__(1024) void k_ipa_tree(IpaBatchDev B, uint32_t shift) {
+    const IpaJobDev& J = B.j[blockIdx.y];
+    const uint32_t h = J.h, side = blockIdx.z, m = h >> shift;
+    if (!m || (shift >= 6 && (h >> (shift - 6)) <= 64)) return;  // no such job, or done before
+    const uint32_t K = m < 64 ? m : 64, dist = m / K;
+    if (blockIdx.x >= dist) return;
+    __shared__ uint32_t sum[32][G1R_WORDS];
+    const fpr_k c = fpr_consts();
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    uint32_t* P = J.P + G1R_WORDS * (size_t)(side * h + blockIdx.x);
+    auto at = [&](uint32_t i) { return g1r_get(P + G1R_WORDS * (size_t)(i * dist), c); };
+    if (K == 1) {
+        if (w == 0) g1r_put(sum[0], at(0), c);
+    } else {
+        for (uint32_t i = w; i < K / 2; i += 16) g1r_put(sum[i], g1r_add(at(i), at(i + K / 2), c), c);
     }
-    const g1_t r = g1_mul_quad_pipe(base, sc, q, active, buf);
-    if (active && threadIdx.x >= 64 && q == 0) g1_store(J.P + 36 * (size_t)j, r);
-}
-// one level of the pairwise trees over P[0, h) and P[h, 2h): half = h >> shift per job
-__global__ __launch_bounds__(64) void k_ipa_tree(IpaBatchDev B, uint32_t shift) {
-    const IpaJobDev& J = B.j[blockIdx.y];
-    const uint32_t h = J.h, half = h >> shift;
-    const uint32_t i = blockIdx.x * 16 + threadIdx.x / 4;
-    const int q = threadIdx.x & 3;
-    if (i >= 2 * half) return;
-    const size_t k = (size_t)(i / half) * h + i % half;
-    const g1_t r = g1_add_quad(g1_load(J.P + 36 * k), g1_load(J.P + 36 * (k + half)), q);
-    if (q == 0) g1_store(J.P + 36 * k, r);
-}
-__global__ __launch_bounds__(64) void k_ipa_lr(IpaBatchDev B) {
-    const IpaJobDev& J = B.j[blockIdx.y];
-    const uint32_t side = threadIdx.x / 4, h = J.h;
-    const int q = threadIdx.x & 3;
-    if (side >= 2 || !h) return;
-    const g1_t r = g1_add_quad(g1_load(J.P + 36 * (size_t)(side * h)), g1_load(J.P + 36 * (size_t)(2 * h + side)), q);
-    if (q == 0) g1_store(J.LR + 36 * side, r);
-}
-// eight lanes per element: quad 0 computes x^-1 g_lo[i], quad 1 x g_hi[i] (k_g1_fold2's
-// two products, vrf_common.cuh:71-76), then quad 0 adds them in that order
-__global__ __launch_bounds__(128) void k_ipa_fold(IpaBatchDev B) {
-    const IpaJobDev& J = B.j[blockIdx.y];
-    const uint32_t h = J.h;
-    if (blockIdx.x * 8 >= h) return;  // whole block: past the job's pairs (or a finished job)
-    __shared__ g1_pipe_buf buf;
-    __shared__ uint32_t hi_pt[8][36];
-    const uint32_t e = (threadIdx.x & 63) / 8, i = blockIdx.x * 8 + e;
-    const int q = threadIdx.x & 3, half_sel = (threadIdx.x >> 2) & 1;
-    const bool active = i < h, add_wave = threadIdx.x >= 64;
-    g1_t base = g1_zero();
-    if (active && !add_wave) base = g1_load(J.g + 36 * (size_t)(i + half_sel * h));
-    g1_t r = g1_mul_quad_pipe(base, half_sel ? J.x : J.xi, q, active, buf);
-    if (add_wave && active && half_sel && q == 0) g1_store(hi_pt[e], r);
     __syncthreads();
-    if (add_wave && active && !half_sel) {
-        r = g1_add_quad(r, g1_load(hi_pt[e]), q);
-        if (q == 0) {
-            fr_t xm, xim;
-#pragma unroll
-            for (int k = 0; k < 8; k++) xm.v[k] = J.xm[k], xim.v[k] = J.xim[k];
-            g1_store(J.g2 + 36 * (size_t)i, r);
-            st_aos(J.a2, i, fr_add(mont_mul(xm, ld_aos(J.a, i)), mont_mul(xim, ld_aos(J.a, i + h))));
-            st_aos(J.b2, i, fr_add(mont_mul(xim, ld_aos(J.b, i)), mont_mul(xm, ld_aos(J.b, i + h))));
-        }
+    for (uint32_t half = K / 4; half >= 1; half >>= 1) {
+        if (w < half) g1r_put(sum[w], g1r_add(g1r_get(sum[w], c), g1r_get(sum[w + half], c), c), c);
+        __syncthreads();
     }
+    if (w) return;
+    const g1r_t r = g1r_get(sum[0], c);
+    if (dist > 1) g1r_put(P, r, c);
+    else g1r_store(J.LR + 36 * side, g1r_add(r, g1r_get(J.P + G1R_WORDS * (size_t)(2 * h + side), c), c), c);
 }
-void launch_ipa_ip(hipStream_t s, const IpaBatchDev& B, uint32_t nj, const uint32_t r2[8]) {
+// one folded generator per block: waves 0 and 1 compute x^-1 g_lo[i], waves 2 and 3 x g_hi[i]
+// (k_g1_fold2's two products, vrf_common.cuh:71-76), then wave 1 adds them in that order; two
+// lanes of wave 1 fold a and b while its first doublings are under way
+__global__ __launch_bounds__(256) void k_ipa_fold(IpaBatchDev B, uint32_t nj) {
+    const IpaJobDev& J = B.j[ipa_job(B, nj, blockIdx.x, false)];
+    const uint32_t h = J.h, i = blockIdx.x - J.fold0;
+    if (i >= h) return;  // whole block
+    __shared__ g1_pipe_buf buf[2];
+    const fpr_k c = fpr_consts();
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), hi = wave >> 1;
+    const bool dbl = !(wave & 1);
+    uint32_t sc[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) sc[k] = hi ? J.x[k] : J.xi[k];
+    g1r_t base = g1r_zero(c);
+    if (dbl) base = g1r_get(J.g + G1R_WORDS * (size_t)(i + hi * h), c);
+    if (wave == 1 && c.lane == 0 && c.row < 2) {
+        fr_t xm, xim;
+#pragma unroll
+        for (int k = 0; k < 8; k++) xm.v[k] = J.xm[k], xim.v[k] = J.xim[k];
+        const uint32_t* src = c.row ? J.b : J.a;
+        uint32_t* dst = c.row ? J.b2 : J.a2;
+        st_aos(dst, i, fr_add(mont_mul(c.row ? xim : xm, ld_aos(src, i)), mont_mul(c.row ? xm : xim, ld_aos(src, i + h))));
+    }
+    g1r_t r = g1r_mul_pipe(base, sc, dbl, buf[hi], c);
+    if (wave == 3) g1r_put(buf[0][0][0], r, c);
+    __syncthreads();
+    if (wave == 1) g1r_put(J.g2 + G1R_WORDS * (size_t)i, g1r_add(r, g1r_get(buf[0][0][0], c), c), c);
+}
+void launch_ipa_points(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax) {
+    hipLaunchKernelGGL(k_ipa_points, dim3((2 * hmax + 1 + 3) / 4, nj), dim3(256), 0, s, B);
+}
+void launch_ipa_scale(hipStream_t s, const IpaBatchDev& B, uint32_t nj, const uint32_t r2[8]) {
     fr_t R2;
     for (int k = 0; k < 8; k++) R2.v[k] = r2[k];
-    hipLaunchKernelGGL(k_ipa_ip, dim3(1, nj), dim3(256), 0, s, B, R2);
+    uint32_t blocks = 0;
+    for (uint32_t j = 0; j < nj; j++) blocks += B.j[j].h ? 2 * B.j[j].h + 2 : 0;
+    hipLaunchKernelGGL(k_ipa_scale, dim3(blocks), dim3(128), lds_share(blocks, 2, sizeof(g1_pipe_buf) + 129 * 32), s, B, nj, R2);
 }
-void launch_ipa_scale(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax) {
-    hipLaunchKernelGGL(k_ipa_scale, dim3((2 * hmax + 2 + 15) / 16, nj), dim3(128), 0, s, B);
+void launch_ipa_tree(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax) {
+    for (uint32_t shift = 0; shift == 0 || (hmax >> (shift - 6)) > 64; shift += 6) {
+        const uint32_t m = hmax >> shift;
+        hipLaunchKernelGGL(k_ipa_tree, dim3(m > 64 ? m / 64 : 1, nj, 2), dim3(1024), 0, s, B, shift);
+    }
 }
-void launch_ipa_tree(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax, uint32_t shift) {
-    hipLaunchKernelGGL(k_ipa_tree, dim3((2 * (hmax >> shift) + 15) / 16, nj), dim3(64), 0, s, B, shift);
-}
-void launch_ipa_lr(hipStream_t s, const IpaBatchDev& B, uint32_t nj) {
-    hipLaunchKernelGGL(k_ipa_lr, dim3(1, nj), dim3(64), 0, s, B);
-}
-void launch_ipa_fold(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax) {
-    hipLaunchKernelGGL(k_ipa_fold, dim3((hmax + 7) / 8, nj), dim3(128), 0, s, B);
+void launch_ipa_fold(hipStream_t s, const IpaBatchDev& B, uint32_t nj) {
+    uint32_t blocks = 0;
+    for (uint32_t j = 0; j < nj; j++) blocks += B.j[j].h;
+    hipLaunchKernelGGL(k_ipa_fold, dim3(blocks), dim3(256), lds_share(blocks, 1, sizeof(g1_pipe_buf) * 2), s, B, nj);
 }
 // planes -> 8-word entries
 __global__ __launch_bounds__(256) void k_planes_to_aos(const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,

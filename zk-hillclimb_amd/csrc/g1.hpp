@@ -40,24 +40,27 @@ void launch_pip_window(hipStream_t s, const uint32_t* buckets, const uint32_t* o
                        uint32_t m, uint32_t* partials);
 void launch_pip_combine(hipStream_t s, const uint32_t* partials, uint32_t m, uint32_t* out);
 // inner-product argument rounds (ipa_prove) of up to ZKH_IPA_MAX_JOBS openings per launch
-// (blockIdx.y = job); a, b plain Fr 8 words per entry, g/P points.  A job with h = 0 has
-// finished its rounds and is skipped.  x, xi plain; xm, xim in Montgomery form.
+// (blockIdx.y = job); a, b plain Fr 8 words per entry.  g, g2, Qr, P: points in row form
+// (fp_row.hpp, ZKH_ROW_WORDS each); g_in, Q: 144-byte points; LR: two 144-byte points (host).
+// A job with h = 0 has finished its rounds and is skipped.  x, xi plain; xm, xim in
+// Montgomery form.
 #define ZKH_IPA_MAX_JOBS 8
+#define ZKH_ROW_WORDS 64
 struct IpaJobDev {
-    const uint32_t *g, *a, *b, *Q;
-    uint32_t *ip, *P, *LR, *g2, *a2, *b2;
-    uint32_t h, pad;
+    const uint32_t *g_in, *Q, *g, *a, *b, *Qr;
+    uint32_t *g0, *P, *LR, *g2, *a2, *b2;
+    uint32_t h, scale0, fold0, pad;  // scale0, fold0: the job's first block of the launch
     uint32_t x[8], xi[8], xm[8], xim[8];
 };
 struct IpaBatchDev {
     IpaJobDev j[ZKH_IPA_MAX_JOBS];
 };
-void launch_ipa_ip(hipStream_t s, const IpaBatchDev& B, uint32_t nj, const uint32_t r2[8]);
-void launch_ipa_scale(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax);
-// one tree level: half = h >> shift per job (hmax the largest h)
-void launch_ipa_tree(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax, uint32_t shift);
-void launch_ipa_lr(hipStream_t s, const IpaBatchDev& B, uint32_t nj);
-void launch_ipa_fold(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax);
+// g0[0, 2h] = row forms of g_in[0, 2h) and Q
+void launch_ipa_points(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax);
+void launch_ipa_scale(hipStream_t s, const IpaBatchDev& B, uint32_t nj, const uint32_t r2[8]);
+// every tree level and L, R (hmax the largest h)
+void launch_ipa_tree(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax);
+void launch_ipa_fold(hipStream_t s, const IpaBatchDev& B, uint32_t nj);
 void launch_planes_to_aos(hipStream_t s, const uint32_t* lo, const uint32_t* hi, uint32_t n, uint32_t* out);
 // out[i] = base[i % nb] * s[i] (G1Jacobian_mul, raw scalar bits)
 // a scalar passed by value to a kernel: 8 plain little-endian words

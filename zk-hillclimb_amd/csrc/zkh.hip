@@ -3883,19 +3883,21 @@ extern "C" int zkh_ipa_prove_batch(zkh_ctx* c, uint32_t nj, uint8_t* const* tran
         if (a[j]->n != n || b[j]->n != n) return fail(c, ZKH_EARG, "ipa_prove: a, b and g sizes differ");
         if (n > 1 && (!L_out[j] || !R_out[j])) return fail(c, ZKH_EARG, "null argument");
         fr_words += (size_t)n * 32;
-        g_words += (size_t)n * 72;
-        p_words += (size_t)(n + 2) * 36 + 256;
+        g_words += (size_t)(n + n / 2 + 1) * ZKH_ROW_WORDS;
+        p_words += (size_t)(n + 2) * ZKH_ROW_WORDS;
         nmax = std::max(nmax, n);
     }
     HIPCHK(c, hipSetDevice(c->device));
     int rc = 0;
-    // per job: a, b, g working copies (two of each, the fold writes the other), round
-    // products P, inner products, Q; one L, R area for all jobs (one copy to the host per round)
+    // per job: a, b working copies (two of each, the fold writes the other) and the row-form
+    // points: g with Q behind it, the first fold's g, the round's products; Q as given; L, R
+    // of all jobs in the pinned area of published sums, written by the round's last tree launch
     uint32_t* fr_w = (uint32_t*)scratch_slot(c, SL_TMP1, fr_words * 4, &rc);
     uint32_t* g_w = rc ? nullptr : (uint32_t*)scratch_slot(c, SL_TMP2, g_words * 4, &rc);
-    uint32_t* p_w = rc ? nullptr : (uint32_t*)scratch_slot(c, SL_TMP3, (p_words + 72 * (size_t)nj) * 4, &rc);
+    uint32_t* p_w = rc ? nullptr : (uint32_t*)scratch_slot(c, SL_TMP3, (p_words + 36 * (size_t)nj) * 4, &rc);
     if (rc) return rc;
-    uint32_t* LR = p_w + p_words;
+    static_assert(72 * ZKH_IPA_MAX_JOBS <= ZKH_MAX_BATCH * 11 * 8, "L and R of a round fit the published sums");
+    uint32_t* lr = c->pub_host;
     IpaBatchDev B{};
     uint32_t sz[ZKH_IPA_MAX_JOBS];
     uint32_t *A0[ZKH_IPA_MAX_JOBS], *B0[ZKH_IPA_MAX_JOBS], *G0[ZKH_IPA_MAX_JOBS];
@@ -3910,48 +3912,51 @@ extern "C" int zkh_ipa_prove_batch(zkh_ctx* c, uint32_t nj, uint8_t* const* tran
         B1[j] = b0 + 8 * (size_t)n;
         of += 32 * (size_t)n;
         uint32_t* g0 = g_w + og;
-        G1[j] = g0 + 36 * (size_t)n;
-        og += 72 * (size_t)n;
+        J.Qr = g0 + ZKH_ROW_WORDS * (size_t)n;
+        G1[j] = g0 + ZKH_ROW_WORDS * (size_t)(n + 1);
+        og += ZKH_ROW_WORDS * (size_t)(n + n / 2 + 1);
         J.P = p_w + op;
-        J.ip = J.P + 36 * (size_t)(n + 2);
-        uint32_t* Qd = J.ip + 16;
-        op += (size_t)(n + 2) * 36 + 256;
-        J.LR = LR + 72 * (size_t)j;
+        op += (size_t)(n + 2) * ZKH_ROW_WORDS;
+        J.LR = lr + 72 * (size_t)j;
+        uint32_t* Qd = p_w + p_words + 36 * (size_t)j;
         DevPlanes pa, pb;
         if ((rc = as_planes(c, a[j], SL_TMP0, &pa))) return rc;
         launch_planes_to_aos(c->stream, pa.lo(), pa.hi(), n, a0);
         if ((rc = as_planes(c, b[j], SL_TMP0, &pb))) return rc;
         launch_planes_to_aos(c->stream, pb.lo(), pb.hi(), n, b0);
-        HIPCHK(c, hipMemcpyAsync(g0, g[j]->d, (size_t)n * 144, hipMemcpyDeviceToDevice, c->stream));
-        HIPCHK(c, hipMemcpyAsync(Qd, Q[j], 144, hipMemcpyHostToDevice, c->stream));
+        if ((rc = upload(c, Qd, Q[j], 144))) return rc;
+        J.g_in = (const uint32_t*)g[j]->d;
+        J.Q = Qd;
         J.a = A0[j] = a0;
         J.b = B0[j] = b0;
-        J.g = G0[j] = g0;
-        J.Q = Qd;
+        J.g = J.g0 = G0[j] = g0;
+        J.h = n / 2;
         sz[j] = n;
     }
+    if (nmax > 1) launch_ipa_points(c->stream, B, nj, nmax / 2);
     uint32_t r2[8];
     fr_store(kR2, r2);
-    std::vector<uint32_t> lr(72 * (size_t)nj);
     for (uint32_t round = 0; (nmax >> round) > 1; round++) {
-        uint32_t hmax = 0;
+        uint32_t hmax = 0, scale0 = 0, fold0 = 0;
         for (uint32_t j = 0; j < nj; j++) {
-            B.j[j].h = sz[j] > 1 ? sz[j] / 2 : 0;
-            hmax = std::max(hmax, B.j[j].h);
+            const uint32_t h = B.j[j].h = sz[j] > 1 ? sz[j] / 2 : 0;
+            B.j[j].scale0 = scale0;
+            B.j[j].fold0 = fold0;
+            scale0 += h ? 2 * h + 2 : 0;
+            fold0 += h;
+            hmax = std::max(hmax, h);
         }
         {
             ProfScope ps(c, "ipa_msm", 0);
-            launch_ipa_ip(c->stream, B, nj, r2);
-            launch_ipa_scale(c->stream, B, nj, hmax);
-            for (uint32_t shift = 1; (hmax >> shift) >= 1; shift++) launch_ipa_tree(c->stream, B, nj, hmax, shift);
-            launch_ipa_lr(c->stream, B, nj);
+            launch_ipa_scale(c->stream, B, nj, r2);
+            launch_ipa_tree(c->stream, B, nj, hmax);
         }
-        HIPCHK(c, hipMemcpyAsync(lr.data(), LR, lr.size() * 4, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        HIPCHK(c, hipGetLastError());
+        if ((rc = settle(c))) return rc;
         for (uint32_t j = 0; j < nj; j++) {
             IpaJobDev& J = B.j[j];
             if (!J.h) continue;
-            const uint32_t* l = lr.data() + 72 * (size_t)j;
+            const uint32_t* l = lr + 72 * (size_t)j;
             tr_absorb(transcripts[j], "L", 1, l, 144);
             tr_absorb(transcripts[j], "R", 1, l + 36, 144);
             const Fr x = tr_challenge(transcripts[j]), xi = fr_inv(x);
@@ -3967,7 +3972,7 @@ extern "C" int zkh_ipa_prove_batch(zkh_ctx* c, uint32_t nj, uint8_t* const* tran
         }
         {
             ProfScope ps(c, "ipa_fold", 0);
-            launch_ipa_fold(c->stream, B, nj, hmax);
+            launch_ipa_fold(c->stream, B, nj);
         }
         for (uint32_t j = 0; j < nj; j++) {
             IpaJobDev& J = B.j[j];
