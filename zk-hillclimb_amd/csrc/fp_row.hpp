@@ -177,17 +177,19 @@ FDEV uint32_t fpr_unpack(const uint32_t* w, const fpr_k& c) {
     if (off > 4 && i < 11) v |= w[i + 1] << (32 - off);
     return v & FPR_MASK;
 }
-// a point in memory or LDS in row form: 16 limbs each of x, y, z, then 16 copies of the flag
-#define G1R_WORDS 64
+// a point in memory or LDS in row form: 16 words each for x, y, z (14 limbs), word 14 the flag
+#define G1R_WORDS 48
 FDEV void g1r_put(uint32_t* p, const g1r_t& a, const fpr_k& c) {
-    p[threadIdx.x & 63] = row_sel(c, a.x, a.y, a.z, a.inf ? 1u : 0u);
+    const uint32_t v = c.row == 0 && c.lane == 14 ? (a.inf ? 1u : 0u) : row_sel(c, a.x, a.y, a.z, a.z);
+    if (c.row < 3) p[threadIdx.x & 63] = v;
 }
 FDEV g1r_t g1r_get(const uint32_t* p, const fpr_k& c) {
     g1r_t o;
-    o.x = p[c.lane];
+    const uint32_t x = p[c.lane];
+    o.x = c.lane < 14 ? x : 0;
     o.y = p[16 + c.lane];
     o.z = p[32 + c.lane];
-    o.inf = __builtin_amdgcn_readfirstlane((int)p[48]) != 0;
+    o.inf = __builtin_amdgcn_readfirstlane((int)row_bcast<14>(x)) != 0;
     return o;
 }
 // 144-byte point (fp_dev.hpp form): row r converts coordinate r

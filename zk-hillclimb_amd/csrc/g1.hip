@@ -4,34 +4,47 @@
 #include "fr_dev.hpp"
 #include "g1.hpp"
 
-// Lane w of the row's wave owns window w (bits 4w..4w+3 of the raw scalar, commitment.cu:
-// 50-55): it reads limb w/8 of every element, counts the digits in its LDS row, turns the
-// counts into offsets, then lists every element with a nonzero digit under that digit.
-// Lists hold at most n entries per (row, window); offs[.][0] is the total, offs[.][d] the
-// start of digit d.
-__global__ __launch_bounds__(64) void k_pip_sort(const uint32_t* __restrict__ lo,
-                                                 const uint32_t* __restrict__ hi, uint32_t n,
-                                                 uint16_t* __restrict__ lists, uint32_t* __restrict__ offs) {
-    __shared__ uint32_t cnt[64 * 17];
-    const uint32_t row = blockIdx.x, w = threadIdx.x;
+// A block per row, lane w of every wave owning window w (bits 4w..4w+3 of the raw scalar,
+// commitment.cu:50-55): a wave reads limb w/8 of its eighth of the elements and counts the
+// digits in its LDS row; one wave turns the counts into offsets, per digit and eighth; then
+// every wave lists its elements with a nonzero digit under that digit (ascending: eighths in
+// order).  Lists hold at most n entries per (row, window); offs[.][0] is the total, offs[.][d]
+// the start of digit d.  One wave per row walked the elements through one chain of LDS updates:
+// 0.61 ms at 512 x 2048 against 0.38 (the 2-byte stores into 64 lists are most of that).
+#define PIP_SEG 8
+__global__ __launch_bounds__(64 * PIP_SEG) void k_pip_sort(const uint32_t* __restrict__ lo,
+                                                           const uint32_t* __restrict__ hi, uint32_t n,
+                                                           uint16_t* __restrict__ lists,
+                                                           uint32_t* __restrict__ offs) {
+    __shared__ uint32_t cnt[PIP_SEG][64][17];
+    const uint32_t row = blockIdx.x, w = threadIdx.x & 63, seg = threadIdx.x >> 6;
     const uint32_t limb = w >> 3, sh = 4 * (w & 7);
     const uint32_t* src = (limb < 4 ? lo : hi) + (limb & 3) + 4 * (size_t)row * n;
-    uint32_t* my = cnt + 17 * w;
+    const uint32_t i0 = (uint32_t)((uint64_t)n * seg / PIP_SEG), i1 = (uint32_t)((uint64_t)n * (seg + 1) / PIP_SEG);
+    uint32_t* my = cnt[seg][w];
 #pragma unroll
     for (int d = 0; d < 16; d++) my[d] = 0;
-    for (uint32_t i = 0; i < n; i++) my[(src[4 * (size_t)i] >> sh) & 15u] += 1;
+#pragma unroll 8
+    for (uint32_t i = i0; i < i1; i++) my[(src[4 * (size_t)i] >> sh) & 15u] += 1;
+    __syncthreads();
     const size_t rw = (size_t)row * 64 + w;
-    uint32_t* o = offs + rw * 16;
-    uint32_t run = 0;
-    for (int d = 1; d < 16; d++) {
-        const uint32_t c = my[d];
-        my[d] = run;
-        o[d] = run;
-        run += c;
+    if (seg == 0) {
+        uint32_t* o = offs + rw * 16;
+        uint32_t run = 0;
+        for (int d = 1; d < 16; d++) {
+            o[d] = run;
+            for (int s = 0; s < PIP_SEG; s++) {
+                const uint32_t k = cnt[s][w][d];
+                cnt[s][w][d] = run;
+                run += k;
+            }
+        }
+        o[0] = run;
     }
-    o[0] = run;
+    __syncthreads();
     uint16_t* L = lists + rw * n;
-    for (uint32_t i = 0; i < n; i++) {
+#pragma unroll 8
+    for (uint32_t i = i0; i < i1; i++) {
         const uint32_t d = (src[4 * (size_t)i] >> sh) & 15u;
         if (d) {
             const uint32_t pos = my[d];
@@ -54,36 +67,35 @@ __device__ __forceinline__ uint64_t pip_mix(uint64_t z) {
 // (window, digit) chains of a row with the same list produce the same bytes.  For small
 // signed scalars this is the common case: a negative v is r - |v|, whose digits above
 // |v|'s top window are those of r - 2^k for every such element, so the windows above
-// the witness width all hold the list of negative entries under one digit each.  One
-// wave per row works through the row's chains together (coalesced list reads): it
-// fingerprints each nonempty list (count, sum of mixed indices), then, in window order,
-// looks for the first earlier chain with an equal fingerprint and confirms the match
-// entry by entry.  alias holds the (window * 16 + digit) whose bucket stands in, itself
-// when there is none; representatives are always first occurrences.
+// the witness width all hold the list of negative entries under one digit each.  A block
+// per row, its sixteen waves taking the chains in turn: each nonempty list is fingerprinted
+// (count, sum of mixed indices; coalesced reads), then looked up among the earlier windows'
+// chains, and the first one with an equal fingerprint confirmed entry by entry.  alias holds
+// the (window * 16 + digit) whose bucket stands in, itself when there is none;
+// representatives are always first occurrences.  One wave per row took 1.9 ms at 512 rows of
+// 1024 field elements, sixteen 0.26.
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
     return v;
 }
-__global__ __launch_bounds__(64) void k_pip_alias(const uint16_t* __restrict__ lists,
-                                                  const uint32_t* __restrict__ offs, uint32_t n,
-                                                  uint16_t* __restrict__ alias) {
+__global__ __launch_bounds__(1024) void k_pip_alias(const uint16_t* __restrict__ lists,
+                                                    const uint32_t* __restrict__ offs, uint32_t n,
+                                                    uint16_t* __restrict__ alias) {
     __shared__ uint32_t beg_s[1024], cnt_s[1024];
     __shared__ uint64_t fp_s[1024];
-    __shared__ uint16_t tgt_s[1024];
-    const uint32_t row = blockIdx.x, lane = threadIdx.x;
+    const uint32_t row = blockIdx.x, lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint16_t* Lrow = lists + (size_t)row * 64 * n;
     {
-        const uint32_t* o = offs + ((size_t)row * 64 + lane) * 16;
-        for (int d = 1; d < 16; d++) {
-            const uint32_t b = o[d], e = d == 15 ? o[0] : o[d + 1];
-            beg_s[lane * 16 + d] = b;
-            cnt_s[lane * 16 + d] = e - b;
-        }
+        const uint32_t c = threadIdx.x, d = c & 15;
+        const uint32_t* o = offs + (size_t)row * 1024 + (c & ~15u);
+        const uint32_t b = d ? o[d] : 0, e = d == 15 ? o[0] : d ? o[d + 1] : 0;
+        beg_s[c] = b;
+        cnt_s[c] = e - b;
     }
     __syncthreads();
-    for (uint32_t c = 0; c < 1024; c++) {
-        if ((c & 15) == 0) continue;
+    for (uint32_t c = wave; c < 1024; c += 16) {
         const uint32_t cnt = cnt_s[c];
         uint64_t h = 0;
         if (cnt) {
@@ -94,17 +106,17 @@ __global__ __launch_bounds__(64) void k_pip_alias(const uint16_t* __restrict__ l
         if (lane == 0) fp_s[c] = h;
     }
     __syncthreads();
-    for (uint32_t c = 0; c < 1024; c++) {
-        if ((c & 15) == 0) continue;
+    uint16_t* out = alias + (size_t)row * 1024;
+    for (uint32_t c = wave; c < 1024; c += 16) {
         const uint32_t cnt = cnt_s[c];
         uint32_t target = c;
         if (cnt && c >= 16) {
             const uint64_t h = fp_s[c];
             const uint16_t* A = Lrow + (size_t)(c >> 4) * n + beg_s[c];
-            // candidates in earlier windows, 64 at a time, lowest first
+            // candidates in earlier windows, 64 at a time, lowest first (digit 0 has no list)
             for (uint32_t base = 0; base < (c & ~15u) && target == c; base += 64) {
                 const uint32_t cc = base + lane;
-                const bool hit = cc < (c & ~15u) && (cc & 15) && cnt_s[cc] == cnt && fp_s[cc] == h;
+                const bool hit = cc < (c & ~15u) && cnt_s[cc] == cnt && fp_s[cc] == h;
                 uint64_t hits = __ballot(hit);
                 while (hits && target == c) {
                     const uint32_t cand = base + __builtin_ctzll(hits);
@@ -116,11 +128,8 @@ __global__ __launch_bounds__(64) void k_pip_alias(const uint16_t* __restrict__ l
                 }
             }
         }
-        if (lane == 0) tgt_s[c] = (uint16_t)target;
+        if (lane == 0) out[c] = (uint16_t)target;
     }
-    __syncthreads();
-    uint16_t* out = alias + (size_t)row * 1024;
-    for (uint32_t c = lane; c < 1024; c += 64) out[c] = tgt_s[c];
 }
 
 // Bucket chains, two ways in one launch.  A long chain (at least long_min additions: with
@@ -179,38 +188,36 @@ __global__ __launch_bounds__(64) void k_pip_bucket(const uint32_t* __restrict__ 
 }
 
 // sum_b b * bucket[b] by the running sum acc += bucket[b]; run += acc, b = 15..1
-// (commitment.cu:73-77); one quad per (row, window) shares each addition
+// (commitment.cu:73-77), a chain of up to 30 additions; one wave per (row, window) in row form
 __global__ __launch_bounds__(64) void k_pip_window(const uint32_t* __restrict__ buckets,
                                                    const uint32_t* __restrict__ offs,
-                                                   const uint16_t* __restrict__ alias, uint32_t m,
+                                                   const uint16_t* __restrict__ alias,
                                                    uint32_t* __restrict__ partials) {
-    const size_t t = (size_t)blockIdx.x * 16 + threadIdx.x / 4;
-    const int q = threadIdx.x & 3;
-    if (t >= (size_t)m * 64) return;
+    const size_t t = blockIdx.x;
+    const fpr_k c = fpr_consts();
     const uint32_t* o = offs + t * 16;
     const size_t row0 = t / 64 * 64;
-    g1_t acc = g1_zero(), run = g1_zero();
+    g1r_t acc = g1r_zero(c), run = acc;
     for (int b = 15; b >= 1; b--) {
         const uint32_t e = b == 15 ? o[0] : o[b + 1];
-        const g1_t bk = e == o[b] ? g1_zero() : g1_load(buckets + ((row0 * 16 + alias[t * 16 + b])) * 36);
-        acc = g1_add_quad(acc, bk, q);
-        run = g1_add_quad(run, acc, q);
+        if (e != o[b]) acc = g1r_add(acc, g1r_load(buckets + ((row0 * 16 + alias[t * 16 + b])) * 36, c), c);
+        run = g1r_add(run, acc, c);
     }
-    if (q == 0) g1_store(partials + t * 36, run);
+    g1r_put(partials + t * G1R_WORDS, run, c);
 }
 
-// Horner over the windows, most significant first (commitment.cu:81-89); one quad per row
-__global__ __launch_bounds__(64) void k_pip_combine(const uint32_t* __restrict__ partials, uint32_t m,
+// Horner over the windows, most significant first (commitment.cu:81-89): 252 doublings and 64
+// additions in sequence, one wave per row in row form (0.33 ms; 2.5 ms on a lane quad)
+__global__ __launch_bounds__(64) void k_pip_combine(const uint32_t* __restrict__ partials,
                                                     uint32_t* __restrict__ out) {
-    const uint32_t row = blockIdx.x * 16 + threadIdx.x / 4;
-    const int q = threadIdx.x & 3;
-    if (row >= m) return;
-    g1_t acc = g1_zero();
+    const uint32_t row = blockIdx.x;
+    const fpr_k c = fpr_consts();
+    g1r_t acc = g1r_zero(c);
     for (int w = 63; w >= 0; w--) {
-        for (int k = 0; k < 4; k++) acc = g1_dbl_quad(acc, q);
-        acc = g1_add_quad(acc, g1_load(partials + ((size_t)row * 64 + w) * 36), q);
+        for (int k = 0; k < 4; k++) acc = g1r_dbl(acc, c);
+        acc = g1r_add(acc, g1r_get(partials + ((size_t)row * 64 + w) * G1R_WORDS, c), c);
     }
-    if (q == 0) g1_store(out + (size_t)row * 36, acc);
+    g1r_store(out + (size_t)row * 36, acc, c);
 }
 
 // G1Jacobian_mul (g1-tensor.cu:445-454) on a quad: double-and-add over the scalar's raw
@@ -480,11 +487,11 @@ void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint3
 }
 void launch_pip_sort(hipStream_t s, const uint32_t* lo, const uint32_t* hi, uint32_t m, uint32_t n,
                      uint16_t* lists, uint32_t* offs) {
-    hipLaunchKernelGGL(k_pip_sort, dim3(m), dim3(64), 0, s, lo, hi, n, lists, offs);
+    hipLaunchKernelGGL(k_pip_sort, dim3(m), dim3(64 * PIP_SEG), 0, s, lo, hi, n, lists, offs);
 }
 void launch_pip_alias(hipStream_t s, const uint16_t* lists, const uint32_t* offs, uint32_t m, uint32_t n,
                       uint16_t* alias) {
-    hipLaunchKernelGGL(k_pip_alias, dim3(m), dim3(64), 0, s, lists, offs, n, alias);
+    hipLaunchKernelGGL(k_pip_alias, dim3(m), dim3(1024), 0, s, lists, offs, n, alias);
 }
 void launch_pip_bucket(hipStream_t s, const uint32_t* gens, const uint16_t* lists, const uint32_t* offs,
                        const uint16_t* alias, uint32_t m, uint32_t n, uint32_t* buckets) {
@@ -497,8 +504,8 @@ void launch_pip_bucket(hipStream_t s, const uint32_t* gens, const uint16_t* list
 }
 void launch_pip_window(hipStream_t s, const uint32_t* buckets, const uint32_t* offs, const uint16_t* alias,
                        uint32_t m, uint32_t* partials) {
-    hipLaunchKernelGGL(k_pip_window, dim3(4 * m), dim3(64), 0, s, buckets, offs, alias, m, partials);
+    hipLaunchKernelGGL(k_pip_window, dim3(64 * m), dim3(64), 0, s, buckets, offs, alias, partials);
 }
 void launch_pip_combine(hipStream_t s, const uint32_t* partials, uint32_t m, uint32_t* out) {
-    hipLaunchKernelGGL(k_pip_combine, dim3((m + 15) / 16), dim3(64), 0, s, partials, m, out);
+    hipLaunchKernelGGL(k_pip_combine, dim3(m), dim3(64), 0, s, partials, out);
 }

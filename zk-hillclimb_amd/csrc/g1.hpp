@@ -45,7 +45,7 @@ void launch_pip_combine(hipStream_t s, const uint32_t* partials, uint32_t m, uin
 // A job with h = 0 has finished its rounds and is skipped.  x, xi plain; xm, xim in
 // Montgomery form.
 #define ZKH_IPA_MAX_JOBS 8
-#define ZKH_ROW_WORDS 64
+#define ZKH_ROW_WORDS 48
 struct IpaJobDev {
     const uint32_t *g_in, *Q, *g, *a, *b, *Qr;
     uint32_t *g0, *P, *LR, *g2, *a2, *b2;

@@ -3827,7 +3827,7 @@ extern "C" int zkh_commit(zkh_ctx* c, const zkh_g1* gens, const zkh_tensor* t, z
         if (!(rc = as_planes(c, t, SL_TMP0, &p))) lists = (uint16_t*)scratch_slot(c, SL_TMP1, (size_t)m * 64 * n * 2, &rc);
         if (!rc) offs = (uint32_t*)scratch_slot(c, SL_TMP2, (size_t)m * 64 * 16 * 4, &rc);
         if (!rc) buckets = (uint32_t*)scratch_slot(c, SL_TMP3, (size_t)m * 64 * 16 * 144, &rc);
-        if (!rc) partials = (uint32_t*)scratch_slot(c, SL_TMP6, (size_t)m * 64 * 144, &rc);
+        if (!rc) partials = (uint32_t*)scratch_slot(c, SL_TMP6, (size_t)m * 64 * ZKH_ROW_WORDS * 4, &rc);
         uint16_t* alias = nullptr;
         if (!rc) alias = (uint16_t*)scratch_slot(c, SL_TMP4, (size_t)m * 64 * 16 * 2, &rc);
         if (rc) {
