@@ -101,6 +101,29 @@ def test_commit_special_generators(ctx):
     check(ctx, gens, ctx.from_i32(v.reshape(-1)), C.ints_to_fr(v.reshape(-1)), n)
 
 
+@pytest.mark.parametrize("m,n", [(260, 24), (230, 150)])
+def test_commit_lane_chains_special_generators(ctx, m, n):
+    """Enough full-size rows that the short chains and the window sums run on one lane each
+    (more than 13000 windows): equal and opposite generators and one at infinity meet there in
+    the same bucket; sampled rows against the oracle, the last of a partial lane group too."""
+    gens = gens_for(9, n)
+    gens[1] = gens[0]
+    gens[2] = gens[0]
+    y = G.from_limbs12(gens[0][12:24])
+    gens[2][12:24] = G.limbs12((G.P - y) % G.P)
+    gens[4] = G.jac_point(0, 1, 0)
+    rng = np.random.default_rng(m)
+    sc = np.frombuffer(rng.bytes(32 * m * n), np.uint32).reshape(m, n, 8).copy()
+    sc[:, :, 7] %= 0x73EDA753
+    sc[::3, 1] = sc[::3, 0]           # doubling in every bucket that holds generator 0
+    sc[1::3, 2] = sc[1::3, 0]         # P + (-P)
+    sc[::2, 4] = sc[::2, 3]           # infinity behind and before other points
+    sc[1::2, 4, :] = sc[1::2, 5, :]
+    sc[5, 5:] = 0
+    sc = sc.reshape(-1, 8)
+    check(ctx, gens, ctx.from_fr(sc), sc, n, rows=[0, 1, 2, 3, 4, 5, 6, 7, m // 2, m - 2, m - 1])
+
+
 def test_commit_dimension_errors(zkh, ctx):
     gens = ctx.g1_from_host(gens_for(6, 4))
     with pytest.raises(zkh.ZkhError) as e:

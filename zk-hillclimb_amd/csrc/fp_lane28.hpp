@@ -18,6 +18,7 @@ struct f28_t {
 };
 __device__ constexpr int32_t k_f28_p[16] = {FPR_P_LIMBS};
 __device__ constexpr int32_t k_f28_m[16] = {FPR_M_LIMBS};
+__device__ constexpr int32_t k_f28_kb[16] = {FPR_KB_LIMBS};  // 32 p, limbs raised by 2^30
 
 FDEV f28_t f28_add(const f28_t& a, const f28_t& b) {
     f28_t r;
@@ -95,32 +96,130 @@ FDEV f28_t f28_dot(const f28_t& a0, const f28_t& b0, const f28_t& a1, const f28_
 FDEV f28_t f28_mul(const f28_t& a, const f28_t& b) { return f28_dot<1, false>(a, b, a, b); }
 FDEV f28_t f28_sqr(const f28_t& a) { return f28_dot<1, true>(a, a, a, a); }
 
+// whether x (within 32 p of zero) is a multiple of p: a multiple j p has limb 0 = j p_0 mod 2^28,
+// so all but 2^-22 of the other values stop at the first test
+FDEV bool f28_zero(const f28_t& x) {
+    if ((((uint32_t)x.v[0] * FPR_PINV + 32) & FPR_MASK) > 64) return false;
+    f28_t t = x;
+#pragma unroll
+    for (int i = 0; i < 14; i++) t.v[i] += k_f28_kb[i];
+#pragma unroll 1
+    for (int j = 0; j <= 64; j++) {
+        t = f28_carry(t);
+        int32_t o = 0;
+#pragma unroll
+        for (int i = 0; i < 14; i++) o |= t.v[i];
+        if (o == 0) return true;
+#pragma unroll
+        for (int i = 0; i < 14; i++) t.v[i] -= k_f28_p[i];
+    }
+    return false;
+}
+
 struct g28_t {
     f28_t x, y, z;
 };
-// a second operand with its Z^2 and Z^3, taken once for all the additions it enters
-struct g28b_t {
-    f28_t x, y, z, zz, zzz;
-};
-
-// add-2007-bl of a and b, neither at infinity, without the equal-point branch: h and r are left
-// to the caller's test.  Coordinates: limbs [0, 1], values within 3.
-FDEV g28_t g28_add_core(const g28_t& a, const g28b_t& b, f28_t& h, f28_t& r) {
-    const f28_t z1z1 = f28_sqr(a.z);
-    const f28_t u1 = f28_mul(a.x, b.zz);
-    h = f28_sub(f28_mul(b.x, z1z1), u1);
-    const f28_t s1 = f28_mul(a.y, b.zzz);
-    r = f28_sub(f28_mul(b.y, f28_mul(a.z, z1z1)), s1);
+FDEV g28_t g28_zero() {
+    constexpr int32_t one[16] = {FPR_ONE_LIMBS};
     g28_t o;
+#pragma unroll
+    for (int i = 0; i < 14; i++) o.x.v[i] = o.z.v[i] = 0, o.y.v[i] = one[i];
+    return o;
+}
+// limbs of a row-form point's coordinate (16 words, 14 limbs)
+FDEV f28_t f28_load(const uint32_t* p) {
+    const uint4* q = (const uint4*)p;
+    f28_t r;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const uint4 t = q[k];
+        r.v[4 * k] = (int32_t)t.x, r.v[4 * k + 1] = (int32_t)t.y;
+        r.v[4 * k + 2] = (int32_t)t.z, r.v[4 * k + 3] = (int32_t)t.w;
+    }
+    const uint2 t = ((const uint2*)p)[6];
+    r.v[12] = (int32_t)t.x, r.v[13] = (int32_t)t.y;
+    return r;
+}
+// as a nonnegative value with carried limbs (x within 32 p of zero, stored plus 32 p); word 14
+// = extra
+FDEV void f28_store(uint32_t* p, const f28_t& x, uint32_t extra) {
+    f28_t t;
+#pragma unroll
+    for (int i = 0; i < 14; i++) t.v[i] = x.v[i] + k_f28_kb[i];
+    t = f28_carry(t);
+    uint4* q = (uint4*)p;
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        q[k] = make_uint4((uint32_t)t.v[4 * k], (uint32_t)t.v[4 * k + 1], (uint32_t)t.v[4 * k + 2], (uint32_t)t.v[4 * k + 3]);
+    q[3] = make_uint4((uint32_t)t.v[12], (uint32_t)t.v[13], extra, 0);
+}
+// a row-form point (fp_row.hpp; G1R_WORDS) from and to a lane; inf: its flag
+FDEV g28_t g28_load(const uint32_t* p, bool& inf) {
+    g28_t o;
+    o.x = f28_load(p);
+    o.y = f28_load(p + 16);
+    o.z = f28_load(p + 32);
+    inf = p[14] != 0;
+    return o;
+}
+FDEV void g28_store(uint32_t* p, const g28_t& a, bool inf) {
+    f28_store(p, a.x, inf ? 1u : 0u);
+    f28_store(p + 16, a.y, 0);
+    f28_store(p + 32, a.z, 0);
+}
+
+// dbl-2009-l as g1r_dbl, for a point not at infinity.  Coordinates between operations: limbs
+// [0, 1] (z from the row form: [0, 2]) with a signed top limb, x and y in (-17, 36), z in
+// (-1, 36).
+FDEV g28_t g28_dbl(const g28_t& a) {
+    const f28_t A = f28_sqr(a.x), B = f28_sqr(a.y), C = f28_sqr(B), XB = f28_mul(a.x, B);
+    g28_t o;
+    o.z = f28_mul(a.y, f28_twice(a.z));
+    f28_t E, t;
+#pragma unroll
+    for (int i = 0; i < 14; i++) E.v[i] = 3 * A.v[i];
+    const f28_t F = f28_sqr(f28_carry(E));
+#pragma unroll
+    for (int i = 0; i < 14; i++) t.v[i] = F.v[i] - 8 * XB.v[i];
+    o.x = f28_carry(t);
+    // E (D - X3): limbs 3 x 1
+#pragma unroll
+    for (int i = 0; i < 14; i++) t.v[i] = 4 * XB.v[i] - o.x.v[i];
+    const f28_t y = f28_mul(E, f28_carry(t));
+#pragma unroll
+    for (int i = 0; i < 14; i++) t.v[i] = y.v[i] - 8 * C.v[i];
+    o.y = f28_carry(t);
+    return o;
+}
+
+// add-2007-bl as g1r_add, of a (inf: its flag, updated) and a point b not at infinity with its
+// Z^2 and Z^3: the equal-point branch doubles a, U1 = U2 with S1 != S2 leaves Z3 = 0.
+FDEV void g28_add(g28_t& a, bool& inf, const g28_t& b, const f28_t& zz2, const f28_t& zzz2) {
+    if (inf) {
+        a = b;
+        inf = false;
+        return;
+    }
+    const f28_t z1z1 = f28_sqr(a.z);
+    const f28_t u1 = f28_mul(a.x, zz2);
+    const f28_t h = f28_sub(f28_mul(b.x, z1z1), u1);
+    const f28_t s1 = f28_mul(a.y, zzz2);
+    const f28_t r = f28_sub(f28_mul(b.y, f28_mul(a.z, z1z1)), s1);
+    const bool h0 = f28_zero(h);
+    if (h0 && f28_zero(r)) {
+        inf = f28_zero(a.y);  // Z3 = 2 Y Z
+        a = g28_dbl(a);
+        return;
+    }
+    inf = h0;
     const f28_t h2 = f28_twice(h), r2 = f28_twice(r);
-    o.z = f28_mul(f28_mul(a.z, b.z), h2);
-    const f28_t i = f28_sqr(h2);  // limbs 2 x 2 = 4
+    a.z = f28_mul(f28_mul(a.z, b.z), h2);
+    const f28_t i = f28_sqr(h2);  // limbs 2 x 2
     const f28_t j = f28_mul(h, i), v = f28_mul(u1, i);
-    o.x = f28_carry(f28_sub(f28_sub(f28_sqr(r2), j), f28_twice(v)));
-    // r (V - X3) - 2 S1 J: limbs 2 x 1 + 2 x 1 = 4
+    a.x = f28_carry(f28_sub(f28_sub(f28_sqr(r2), j), f28_twice(v)));
+    // r (V - X3) - 2 S1 J: limbs 2 x 1 + 1 x 2
     f28_t nj;
 #pragma unroll
     for (int k = 0; k < 14; k++) nj.v[k] = -2 * j.v[k];
-    o.y = f28_dot<2, false>(r2, f28_sub(v, o.x), s1, nj);
-    return o;
+    a.y = f28_dot<2, false>(r2, f28_sub(v, a.x), s1, nj);
 }

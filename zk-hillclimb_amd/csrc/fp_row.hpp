@@ -217,8 +217,9 @@ FDEV void g1r_store(uint32_t* p, const g1r_t& a, const fpr_k& c) {
     if (c.lane < 12 && c.row < 3) p[12 * c.row + c.lane] = w;
 }
 
-// Coordinates between operations: x, y below 29 p with limbs below 2^28 + 16, z below 6 p with
-// limbs below 2^29 + 32.
+// Coordinates between operations: x, y below 36 p with limbs below 2^28 + 16, z below 36 p with
+// limbs below 2^29 + 32 (x, y below 28 p and z below 6 p from the operations here, up to 36 p
+// from fp_lane28.hpp's stores).
 //
 // dbl-2009-l with D = 4 X B for 2 ((X + B)^2 - A - C): A = X^2, B = Y^2, C = B^2, E = 3 A,
 // F = E^2, X3 = F - 2 D, Y3 = E (D - X3) - 8 C, Z3 = 2 Y Z; Z = 0 returns the point unchanged

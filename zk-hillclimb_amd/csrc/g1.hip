@@ -1,5 +1,6 @@
 // g1.hip -- G1 Pedersen commitment kernels (bucket method, commitment.cu:47-103).
 #include "fp_dev.hpp"
+#include "fp_lane28.hpp"
 #include "fp_row.hpp"
 #include "fr_dev.hpp"
 #include "g1.hpp"
@@ -79,11 +80,27 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
     for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
     return v;
 }
+// length class: exact below 128, then 16 per factor of two (n <= 65536)
+__device__ __forceinline__ uint32_t pip_bin(uint32_t len) {
+    if (len < 128) return len;
+    const uint32_t l2 = 31 - __builtin_clz(len);
+    return 128 + 16 * (l2 - 7) + ((len >> (l2 - 4)) & 15);
+}
+// the longest length of a class
+__device__ __forceinline__ uint32_t pip_bin_len(uint32_t b) {
+    if (b < 128) return b;
+    const uint32_t l2 = 7 + (b - 128) / 16;
+    return (1u << l2) + (((b - 128) % 16 + 1) << (l2 - 4)) - 1;
+}
+
 __global__ __launch_bounds__(1024) void k_pip_alias(const uint16_t* __restrict__ lists,
                                                     const uint32_t* __restrict__ offs, uint32_t n,
-                                                    uint16_t* __restrict__ alias) {
-    __shared__ uint32_t beg_s[1024], cnt_s[1024];
+                                                    uint16_t* __restrict__ alias, uint16_t* __restrict__ walias,
+                                                    PipPlan* __restrict__ plan, uint32_t* __restrict__ wins) {
+    __shared__ uint32_t beg_s[1024], cnt_s[1024], hist[PIP_BINS];
     __shared__ uint64_t fp_s[1024];
+    __shared__ uint16_t sig[1024];
+    __shared__ uint32_t nwin, wbase;
     const uint32_t row = blockIdx.x, lane = threadIdx.x & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint16_t* Lrow = lists + (size_t)row * 64 * n;
@@ -93,6 +110,8 @@ __global__ __launch_bounds__(1024) void k_pip_alias(const uint16_t* __restrict__
         const uint32_t b = d ? o[d] : 0, e = d == 15 ? o[0] : d ? o[d + 1] : 0;
         beg_s[c] = b;
         cnt_s[c] = e - b;
+        if (c < PIP_BINS) hist[c] = 0;
+        if (c == 0) nwin = 0;
     }
     __syncthreads();
     for (uint32_t c = wave; c < 1024; c += 16) {
@@ -128,94 +147,258 @@ __global__ __launch_bounds__(1024) void k_pip_alias(const uint16_t* __restrict__
                 }
             }
         }
-        if (lane == 0) out[c] = (uint16_t)target;
+        if (lane == 0) {
+            out[c] = (uint16_t)target;
+            sig[c] = cnt ? (uint16_t)target : 0xffff;  // the digit's bucket; none
+            if (cnt && target == c) atomicAdd(&hist[pip_bin(cnt)], 1u);
+        }
     }
+    __syncthreads();
+    // windows whose digits share their buckets share their sum: the first of them stands in
+    // (small signed scalars: the windows above the witness width have r's digits, 15 at most)
+    uint32_t first = 64, slot = 0;
+    if (threadIdx.x < 64) {
+        first = lane;
+        for (uint32_t v = 0; v < lane && first == lane; v++) {
+            bool same = true;
+            for (uint32_t d = 15; d >= 1 && same; d--) same = sig[v * 16 + d] == sig[lane * 16 + d];
+            if (same) first = v;
+        }
+        walias[(size_t)row * 64 + lane] = (uint16_t)first;
+        if (first == lane) slot = atomicAdd(&nwin, 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) wbase = atomicAdd(&plan->nwin, nwin);
+    for (uint32_t b = threadIdx.x; b < PIP_BINS; b += 1024)
+        if (hist[b]) atomicAdd(&plan->total[b], hist[b]);
+    __syncthreads();
+    if (first == lane && threadIdx.x < 64) wins[wbase + slot] = row * 64 + lane;
 }
 
-// Bucket chains, two ways in one launch.  A long chain (at least long_min additions: with
-// small signed scalars, the shared list of negative entries) is latency-bound, so one
-// quad (4 lanes) shares each addition (g1_add_quad: 5 multiply rounds instead of 16); a
-// short chain runs on one lane (g1_add), which costs fewer instructions in total.  Blocks
-// [0, nq) are quad blocks: a wave holds 16 rows of one (window, digit); the rest are lane
-// blocks of 64 rows.  In both, block b -> row block b % RB, digit (b / RB) % 15 + 1,
-// window b / (15 RB): the row block varies fastest because blocks go round-robin to the 8
-// XCDs and nearly all of a window's work sits in one digit, so any other order puts a
-// window's long chains on one XCD.  A chain starts from the point at infinity, so its
-// first addition returns the generator itself (bls12-381.cu:1432), as the reference's
-// bucket does; the next generator is loaded one addition ahead.
-template <bool QUAD>
-__device__ __forceinline__ void pip_chain(const uint32_t* __restrict__ gens, const uint16_t* __restrict__ L,
-                                          uint32_t beg, uint32_t end, int q, uint32_t* out) {
-    g1_t acc = g1_load(gens + 36 * (size_t)L[beg]);
-    g1_t nxt = acc;
-    uint32_t idx = beg + 1 < end ? L[beg + 1] : 0;
-    if (beg + 1 < end) nxt = g1_load(gens + 36 * (size_t)idx);
-    if (beg + 2 < end) idx = L[beg + 2];
-    for (uint32_t k = beg + 1; k < end; k++) {
-        const g1_t g = nxt;
-        if (k + 1 < end) nxt = g1_load(gens + 36 * (size_t)idx);
-        if (k + 2 < end) idx = L[k + 2];
-        acc = QUAD ? g1_add_quad(acc, g, q) : g1_add(acc, g);
-    }
-    if (!QUAD || q == 0) g1_store(out, acc);
+// ---- bucket chains.  A chain starts from the point at infinity, so its first addition returns
+// the generator itself (bls12-381.cu:1432), as the reference's bucket does.  Two ways to run
+// one: in row form a wave takes one chain, 1.3 us per addition and 1.06 us of a SIMD's time; a
+// lane takes one chain (fp_lane28.hpp), 13 us per addition and 0.2 us of a SIMD's time.  With
+// small signed scalars the row's shared list of negative entries is a chain of n/2 additions,
+// with full-size scalars every chain has about n/16: so the chains are sorted by length, the
+// ones from a length on go to waves and the others, 64 of about one length together, to lanes.
+// 512 rows of 2048 int16: 17.7 ms with long chains on lane quads and short ones on lanes of
+// 32-bit limbs, 2.7 so; 512 rows of 1000 field elements 15.3 and 6.7 (0.2 us x 31M additions
+// over 1024 SIMDs = 6.0).
+
+// the generators in row form with Z^2 and Z^3 behind them (they enter every addition), one
+// wave per point; the plan's counters start at zero
+__global__ __launch_bounds__(256) void k_pip_gens(const uint32_t* __restrict__ gens, uint32_t n,
+                                                  uint32_t* __restrict__ tab, PipPlan* __restrict__ plan) {
+    const uint32_t i = blockIdx.x * 4 + threadIdx.x / 64;
+    if (blockIdx.x == 0)
+        for (uint32_t k = threadIdx.x; k < sizeof(PipPlan) / 4; k += 256) ((uint32_t*)plan)[k] = 0;
+    if (i >= n) return;
+    const fpr_k c = fpr_consts();
+    const g1r_t g = g1r_load(gens + 36 * (size_t)i, c);
+    uint32_t* o = tab + PIP_GEN_WORDS * (size_t)i;
+    g1r_put(o, g, c);
+    const uint32_t zz = fpr_mul(g.z, g.z, c), zzz = fpr_mul(zz, g.z, c);
+    if (c.row < 2) o[G1R_WORDS + 16 * c.row + c.lane] = c.row ? zzz : zz;
 }
-__global__ __launch_bounds__(64) void k_pip_bucket(const uint32_t* __restrict__ gens,
-                                                   const uint16_t* __restrict__ lists,
-                                                   const uint32_t* __restrict__ offs,
-                                                   const uint16_t* __restrict__ alias, uint32_t m, uint32_t n,
-                                                   uint32_t long_min, uint32_t nq,
-                                                   uint32_t* __restrict__ buckets) {
-    const bool quad = blockIdx.x < nq;
-    const uint32_t b = quad ? blockIdx.x : blockIdx.x - nq;
-    const uint32_t RB = quad ? (m + 15) / 16 : (m + 63) / 64;
-    const uint32_t d = (b / RB) % 15 + 1, w = b / (15 * RB);
-    const uint32_t row = (b % RB) * (quad ? 16 : 64) + (quad ? threadIdx.x / 4 : threadIdx.x);
-    if (row >= m) return;
-    const size_t rw = (size_t)row * 64 + w;
-    const uint32_t* o = offs + rw * 16;
-    const uint32_t beg = o[d], end = d == 15 ? o[0] : o[d + 1];
-    // empty chains are the point at infinity and aliased ones are another chain's bucket:
-    // k_pip_window reads neither from here
-    if (beg == end || alias[rw * 16 + d] != w * 16 + d || (end - beg >= long_min) != quad) return;
-    const uint16_t* L = lists + rw * n;
-    uint32_t* out = buckets + (rw * 16 + d) * 36;
-    if (quad) {
-        // the long chains set the kernel's length: their waves issue first on a shared SIMD
-        __builtin_amdgcn_s_setprio(3);
-        pip_chain<true>(gens, L, beg, end, threadIdx.x & 3, out);
+// Where each length class starts in the sorted list (longest first) and from which class on
+// chains go to waves.  The cost of a choice, in us: the busiest of (the SIMDs' total work, the
+// longest lane chain, the longest wave chain), with the total again at a tenth to break ties.
+__global__ __launch_bounds__(512) void k_pip_plan(PipPlan* __restrict__ plan) {
+    static_assert(PIP_BINS <= 512, "one thread per class");
+    __shared__ uint32_t cnt[512], lmax[512];
+    __shared__ float work[512], best[512];
+    __shared__ uint32_t arg[512];
+    const uint32_t b = threadIdx.x;
+    const uint32_t t = b < PIP_BINS ? plan->total[b] : 0;
+    const float len = (float)pip_bin_len(b);
+    cnt[b] = t;
+    work[b] = t * len;
+    lmax[b] = t ? pip_bin_len(b) : 0;
+    __syncthreads();
+    // inclusive sums over the classes from b on; the longest length up to b
+    for (uint32_t o = 1; o < 512; o <<= 1) {
+        const uint32_t ca = b + o < 512 ? cnt[b + o] : 0, la = b >= o ? lmax[b - o] : 0;
+        const float wa = b + o < 512 ? work[b + o] : 0;
+        __syncthreads();
+        cnt[b] += ca;
+        work[b] += wa;
+        lmax[b] = lmax[b] > la ? lmax[b] : la;
+        __syncthreads();
     }
-    else pip_chain<false>(gens, L, beg, end, 0, out);
+    // the choice b: classes from b on to waves
+    const float rows = work[b], lanes = work[0] - rows, sum = (rows * 1.06f + lanes * 0.2f) / 1024;
+    const float lane_t = b ? 13.0f * lmax[b - 1] : 0, wave_t = rows > 0 ? 1.3f * lmax[511] : 0;
+    best[b] = fmaxf(sum, fmaxf(lane_t, wave_t)) + 0.1f * sum;
+    arg[b] = b;
+    __syncthreads();
+    for (uint32_t o = 256; o > 0; o >>= 1) {
+        if (b < o && best[b + o] < best[b]) best[b] = best[b + o], arg[b] = arg[b + o];
+        __syncthreads();
+    }
+    if (b < PIP_BINS) plan->cursor[b] = cnt[b] - t;
+    if (b == 0) {
+        plan->items = cnt[0];
+        plan->waves = arg[0] < 512 ? cnt[arg[0]] : 0;
+    }
+}
+// the representative chains (row * 1024 + window * 16 + digit) into their classes' places
+__global__ __launch_bounds__(1024) void k_pip_scatter(const uint32_t* __restrict__ offs,
+                                                      const uint16_t* __restrict__ alias,
+                                                      PipPlan* __restrict__ plan, uint32_t* __restrict__ items) {
+    __shared__ uint32_t hist[PIP_BINS], base[PIP_BINS];
+    const uint32_t row = blockIdx.x, c = threadIdx.x, d = c & 15;
+    for (uint32_t b = c; b < PIP_BINS; b += 1024) hist[b] = 0;
+    __syncthreads();
+    const uint32_t* o = offs + (size_t)row * 1024 + (c & ~15u);
+    const uint32_t len = d ? (d == 15 ? o[0] : o[d + 1]) - o[d] : 0;
+    const bool mine = len && alias[(size_t)row * 1024 + c] == c;
+    const uint32_t bin = pip_bin(len);
+    uint32_t at = 0;
+    if (mine) at = atomicAdd(&hist[bin], 1u);
+    __syncthreads();
+    for (uint32_t b = c; b < PIP_BINS; b += 1024)
+        if (hist[b]) base[b] = atomicAdd(&plan->cursor[b], hist[b]);
+    __syncthreads();
+    if (mine) items[base[bin] + at] = row * 1024 + c;
+}
+// the lists of a chain
+__device__ __forceinline__ const uint16_t* pip_list(uint32_t item, const uint16_t* lists, const uint32_t* offs,
+                                                    uint32_t n, uint32_t& len) {
+    const uint32_t d = item & 15;
+    const uint32_t* o = offs + (item & ~15u);
+    const uint32_t beg = o[d];
+    len = (d == 15 ? o[0] : o[d + 1]) - beg;
+    return lists + (size_t)(item >> 4) * n + beg;
+}
+// Persistent waves, two per SIMD: odd blocks take wave chains while there are any and then lane
+// groups, even blocks the other way round, so both kinds start with their longest at once.
+// A wave ends when both queues are empty.
+__global__ __launch_bounds__(64, 2) void k_pip_bucket(const uint32_t* __restrict__ tab,
+                                                      const uint16_t* __restrict__ lists,
+                                                      const uint32_t* __restrict__ offs,
+                                                      const uint32_t* __restrict__ items, uint32_t n,
+                                                      PipPlan* __restrict__ plan, uint32_t* __restrict__ buckets) {
+    const uint32_t nrow = plan->waves, nall = plan->items, ngrp = (nall - nrow + 63) / 64;
+    const fpr_k c = fpr_consts();
+    for (uint32_t turn = 0; turn < 2; turn++) {
+        const bool rows = (blockIdx.x & 1) != turn;
+        const uint32_t tasks = rows ? nrow : ngrp;
+        for (;;) {
+            uint32_t task = 0;
+            if (threadIdx.x == 0) task = atomicAdd(&plan->taken[rows ? 0 : 1], 1u);
+            task = __builtin_amdgcn_readfirstlane(task);
+            if (task >= tasks) break;
+            if (rows) {
+                const uint32_t item = items[task];
+                uint32_t len;
+                const uint16_t* L = pip_list(item, lists, offs, n, len);
+                g1r_t acc = g1r_get(tab + PIP_GEN_WORDS * (size_t)L[0], c), nxt = acc;
+                // the next generator is loaded one addition ahead, its index two
+                uint32_t idx = len > 1 ? L[1] : 0;
+                if (len > 1) nxt = g1r_get(tab + PIP_GEN_WORDS * (size_t)idx, c);
+                if (len > 2) idx = L[2];
+                for (uint32_t k = 1; k < len; k++) {
+                    const g1r_t g = nxt;
+                    if (k + 1 < len) nxt = g1r_get(tab + PIP_GEN_WORDS * (size_t)idx, c);
+                    if (k + 2 < len) idx = L[k + 2];
+                    acc = g1r_add(acc, g, c);
+                }
+                g1r_put(buckets + (size_t)item * G1R_WORDS, acc, c);
+            } else {
+                const uint32_t at = nrow + task * 64 + threadIdx.x;
+                const bool mine = at < nall;
+                const uint32_t item = items[mine ? at : nall - 1];
+                uint32_t len;
+                const uint16_t* L = pip_list(item, lists, offs, n, len);
+                bool inf;
+                g28_t acc = g28_load(tab + PIP_GEN_WORDS * (size_t)L[0], inf);
+                uint32_t idx = len > 1 ? L[1] : 0;
+                for (uint32_t k = 1; k < len; k++) {
+                    const uint32_t* p = tab + PIP_GEN_WORDS * (size_t)idx;
+                    if (k + 1 < len) idx = L[k + 1];
+                    bool binf;
+                    const g28_t b = g28_load(p, binf);
+                    if (!binf) g28_add(acc, inf, b, f28_load(p + G1R_WORDS), f28_load(p + G1R_WORDS + 16));
+                }
+                if (mine) g28_store(buckets + (size_t)item * G1R_WORDS, acc, inf);
+            }
+        }
+    }
 }
 
 // sum_b b * bucket[b] by the running sum acc += bucket[b]; run += acc, b = 15..1
-// (commitment.cu:73-77), a chain of up to 30 additions; one wave per (row, window) in row form
-__global__ __launch_bounds__(64) void k_pip_window(const uint32_t* __restrict__ buckets,
-                                                   const uint32_t* __restrict__ offs,
-                                                   const uint16_t* __restrict__ alias,
-                                                   uint32_t* __restrict__ partials) {
-    const size_t t = blockIdx.x;
+// (commitment.cu:73-77), a chain of up to 30 additions, for the windows that stand in for
+// themselves: on one wave each in row form (40 us a chain) or, where there are more than the
+// SIMDs take that way in a lane chain's 0.42 ms, on one lane each
+#define PIP_WIN_LANES 13000u
+__global__ __launch_bounds__(64) void k_pip_window_rows(const uint32_t* __restrict__ buckets,
+                                                        const uint32_t* __restrict__ offs,
+                                                        const uint16_t* __restrict__ alias,
+                                                        const PipPlan* __restrict__ plan,
+                                                        const uint32_t* __restrict__ wins,
+                                                        uint32_t* __restrict__ partials) {
+    const uint32_t nw = plan->nwin;
+    if (nw > PIP_WIN_LANES) return;
     const fpr_k c = fpr_consts();
-    const uint32_t* o = offs + t * 16;
-    const size_t row0 = t / 64 * 64;
-    g1r_t acc = g1r_zero(c), run = acc;
-    for (int b = 15; b >= 1; b--) {
-        const uint32_t e = b == 15 ? o[0] : o[b + 1];
-        if (e != o[b]) acc = g1r_add(acc, g1r_load(buckets + ((row0 * 16 + alias[t * 16 + b])) * 36, c), c);
-        run = g1r_add(run, acc, c);
+    for (uint32_t k = blockIdx.x; k < nw; k += gridDim.x) {
+        const size_t t = wins[k], row0 = t / 64 * 64;
+        const uint32_t* o = offs + t * 16;
+        g1r_t acc = g1r_zero(c), run = acc;
+        for (int b = 15; b >= 1; b--) {
+            const uint32_t e = b == 15 ? o[0] : o[b + 1];
+            if (e != o[b]) acc = g1r_add(acc, g1r_get(buckets + (row0 * 16 + alias[t * 16 + b]) * G1R_WORDS, c), c);
+            run = g1r_add(run, acc, c);
+        }
+        g1r_put(partials + t * G1R_WORDS, run, c);
     }
-    g1r_put(partials + t * G1R_WORDS, run, c);
+}
+__global__ __launch_bounds__(64) void k_pip_window_lanes(const uint32_t* __restrict__ buckets,
+                                                         const uint32_t* __restrict__ offs,
+                                                         const uint16_t* __restrict__ alias,
+                                                         const PipPlan* __restrict__ plan,
+                                                         const uint32_t* __restrict__ wins,
+                                                         uint32_t* __restrict__ partials) {
+    const uint32_t nw = plan->nwin;
+    if (nw <= PIP_WIN_LANES) return;
+    for (uint32_t k = blockIdx.x * 64 + threadIdx.x; k < nw; k += gridDim.x * 64) {
+        const size_t t = wins[k], row0 = t / 64 * 64;
+        const uint32_t* o = offs + t * 16;
+        bool ainf = true, rinf = true;
+        g28_t acc = g28_zero(), run = acc;
+#pragma unroll 1
+        for (int step = 29; step >= 0; step--) {  // odd: acc += bucket, even: run += acc
+            const int b = step / 2 + 1;
+            g28_t x = acc;
+            bool xinf = ainf;
+            if (step & 1) {
+                const uint32_t e = b == 15 ? o[0] : o[b + 1];
+                xinf = e == o[b];
+                if (!xinf) x = g28_load(buckets + (row0 * 16 + alias[t * 16 + b]) * G1R_WORDS, xinf);
+            }
+            if (xinf) continue;
+            const f28_t zz = f28_sqr(x.z), zzz = f28_mul(zz, x.z);
+            g28_t y = step & 1 ? acc : run;
+            bool yinf = step & 1 ? ainf : rinf;
+            g28_add(y, yinf, x, zz, zzz);
+            if (step & 1) acc = y, ainf = yinf;
+            else run = y, rinf = yinf;
+        }
+        g28_store(partials + t * G1R_WORDS, run, rinf);
+    }
 }
 
 // Horner over the windows, most significant first (commitment.cu:81-89): 252 doublings and 64
 // additions in sequence, one wave per row in row form (0.33 ms; 2.5 ms on a lane quad)
 __global__ __launch_bounds__(64) void k_pip_combine(const uint32_t* __restrict__ partials,
+                                                    const uint16_t* __restrict__ walias,
                                                     uint32_t* __restrict__ out) {
     const uint32_t row = blockIdx.x;
     const fpr_k c = fpr_consts();
     g1r_t acc = g1r_zero(c);
     for (int w = 63; w >= 0; w--) {
         for (int k = 0; k < 4; k++) acc = g1r_dbl(acc, c);
-        acc = g1r_add(acc, g1r_get(partials + ((size_t)row * 64 + w) * G1R_WORDS, c), c);
+        acc = g1r_add(acc, g1r_get(partials + ((size_t)row * 64 + walias[(size_t)row * 64 + w]) * G1R_WORDS, c), c);
     }
     g1r_store(out + (size_t)row * 36, acc, c);
 }
@@ -489,23 +672,28 @@ void launch_pip_sort(hipStream_t s, const uint32_t* lo, const uint32_t* hi, uint
                      uint16_t* lists, uint32_t* offs) {
     hipLaunchKernelGGL(k_pip_sort, dim3(m), dim3(64 * PIP_SEG), 0, s, lo, hi, n, lists, offs);
 }
-void launch_pip_alias(hipStream_t s, const uint16_t* lists, const uint32_t* offs, uint32_t m, uint32_t n,
-                      uint16_t* alias) {
-    hipLaunchKernelGGL(k_pip_alias, dim3(m), dim3(1024), 0, s, lists, offs, n, alias);
+void launch_pip_gens(hipStream_t s, const uint32_t* gens, uint32_t n, uint32_t* tab, PipPlan* plan) {
+    hipLaunchKernelGGL(k_pip_gens, dim3((n + 3) / 4), dim3(256), 0, s, gens, n, tab, plan);
 }
-void launch_pip_bucket(hipStream_t s, const uint32_t* gens, const uint16_t* lists, const uint32_t* offs,
-                       const uint16_t* alias, uint32_t m, uint32_t n, uint32_t* buckets) {
-    // a chain is long from n/8 additions on: twice the mean of a window whose digits are
-    // spread evenly, so evenly spread scalars never take the quad path
-    const uint32_t long_min = n / 8 > 32 ? n / 8 : 32;
-    const uint32_t nq = (m + 15) / 16 * 960, ns = (m + 63) / 64 * 960;
-    hipLaunchKernelGGL(k_pip_bucket, dim3(nq + ns), dim3(64), 0, s, gens, lists, offs, alias, m, n, long_min, nq,
-                       buckets);
+void launch_pip_alias(hipStream_t s, const uint16_t* lists, const uint32_t* offs, uint32_t m, uint32_t n,
+                      uint16_t* alias, uint16_t* walias, PipPlan* plan, uint32_t* wins) {
+    hipLaunchKernelGGL(k_pip_alias, dim3(m), dim3(1024), 0, s, lists, offs, n, alias, walias, plan, wins);
+}
+void launch_pip_bucket(hipStream_t s, const uint32_t* tab, const uint16_t* lists, const uint32_t* offs,
+                       const uint16_t* alias, uint32_t m, uint32_t n, PipPlan* plan, uint32_t* items,
+                       uint32_t* buckets) {
+    hipLaunchKernelGGL(k_pip_plan, dim3(1), dim3(512), 0, s, plan);
+    hipLaunchKernelGGL(k_pip_scatter, dim3(m), dim3(1024), 0, s, offs, alias, plan, items);
+    hipLaunchKernelGGL(k_pip_bucket, dim3(2048), dim3(64), 0, s, tab, lists, offs, items, n, plan, buckets);
 }
 void launch_pip_window(hipStream_t s, const uint32_t* buckets, const uint32_t* offs, const uint16_t* alias,
-                       uint32_t m, uint32_t* partials) {
-    hipLaunchKernelGGL(k_pip_window, dim3(64 * m), dim3(64), 0, s, buckets, offs, alias, partials);
+                       uint32_t m, const PipPlan* plan, const uint32_t* wins, uint32_t* partials) {
+    const uint32_t most = m * 64;
+    hipLaunchKernelGGL(k_pip_window_rows, dim3(most < 8192 ? most : 8192), dim3(64), 0, s, buckets, offs, alias, plan,
+                       wins, partials);
+    if (most > PIP_WIN_LANES)
+        hipLaunchKernelGGL(k_pip_window_lanes, dim3(2048), dim3(64), 0, s, buckets, offs, alias, plan, wins, partials);
 }
-void launch_pip_combine(hipStream_t s, const uint32_t* partials, uint32_t m, uint32_t* out) {
-    hipLaunchKernelGGL(k_pip_combine, dim3(m), dim3(64), 0, s, partials, out);
+void launch_pip_combine(hipStream_t s, const uint32_t* partials, const uint16_t* walias, uint32_t m, uint32_t* out) {
+    hipLaunchKernelGGL(k_pip_combine, dim3(m), dim3(64), 0, s, partials, walias, out);
 }

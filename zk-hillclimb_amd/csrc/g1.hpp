@@ -8,21 +8,19 @@
 // The reference runs one thread per (row, window) that walks all n generators adding
 // each into one of 16 buckets.  Here the work is split where the Jacobian result allows
 // it -- each bucket's additions form an independent chain (its generators in ascending
-// index order), so one lane runs one (row, window, digit) chain with its bucket in
-// registers, after a sort pass has listed each chain's generator indices:
-//   pip_sort    one wave per row, lane w = window w: per-digit counts, then the index
-//               lists (uint16, generators in ascending order) and their offsets;
-//   pip_alias   one wave per row: chains whose index lists are equal (the usual case for
+// index order) -- after the chains' generator indices have been listed:
+//   pip_gens    generators in row form with Z^2, Z^3; the plan's counters cleared
+//   pip_sort    a block per row, lane w = window w: per-digit counts, then the index
+//               lists (uint16, generators in ascending order) and their offsets
+//   pip_alias   a block per row: chains whose index lists are equal (the usual case for
 //               small signed scalars, where every window above the witness width holds
 //               the list of negative entries) are computed once; lists are matched by a
-//               fingerprint and confirmed entry by entry;
-//   pip_bucket  each distinct nonempty (row, window, digit) chain once: a long chain on a
-//               quad of lanes that share every point addition (latency-bound), a short
-//               one on one lane (throughput-bound);
-//   pip_window  one quad per (row, window): the running sum over digits 15..1;
-//   pip_combine one quad per row: Horner over windows 63..0 (four doublings, one add).
-// Quads share each point operation (g1_add_quad, g1_dbl_quad): the window and Horner
-// chains are short in total work but sequential, so their latency is what counts.
+//               fingerprint and confirmed entry by entry.  Windows whose digits share
+//               their buckets are summed once
+//   pip_bucket  plan and sort of the distinct nonempty chains by length, then each once: the
+//               long ones on a wave each (latency), the others on a lane each (throughput)
+//   pip_window  each distinct window once: the running sum over digits 15..1
+//   pip_combine one wave per row: Horner over windows 63..0 (four doublings, one add)
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -32,20 +30,32 @@
 // scalars: FR limb planes (lo: limbs 0-3, hi: limbs 4-7 as uint4 per element), m*n entries
 void launch_pip_sort(hipStream_t s, const uint32_t* lo, const uint32_t* hi, uint32_t m, uint32_t n,
                      uint16_t* lists, uint32_t* offs);
+#define ZKH_ROW_WORDS 48       // a point in row form (fp_row.hpp)
+#define PIP_GEN_WORDS 80       // and with Z^2 and Z^3 behind it
+#define PIP_BINS 288           // chain length classes
+struct PipPlan {
+    uint32_t total[PIP_BINS];   // distinct chains per length class
+    uint32_t cursor[PIP_BINS];  // the class's next place in the sorted list
+    uint32_t items, waves;      // chains, and how many of the longest go to waves
+    uint32_t nwin;              // distinct windows
+    uint32_t taken[2];          // queues of the bucket launch: wave chains, lane groups
+    uint32_t pad[3];
+};
+void launch_pip_gens(hipStream_t s, const uint32_t* gens, uint32_t n, uint32_t* tab, PipPlan* plan);
 void launch_pip_alias(hipStream_t s, const uint16_t* lists, const uint32_t* offs, uint32_t m, uint32_t n,
-                      uint16_t* alias);
-void launch_pip_bucket(hipStream_t s, const uint32_t* gens, const uint16_t* lists, const uint32_t* offs,
-                       const uint16_t* alias, uint32_t m, uint32_t n, uint32_t* buckets);
+                      uint16_t* alias, uint16_t* walias, PipPlan* plan, uint32_t* wins);
+void launch_pip_bucket(hipStream_t s, const uint32_t* tab, const uint16_t* lists, const uint32_t* offs,
+                       const uint16_t* alias, uint32_t m, uint32_t n, PipPlan* plan, uint32_t* items,
+                       uint32_t* buckets);
 void launch_pip_window(hipStream_t s, const uint32_t* buckets, const uint32_t* offs, const uint16_t* alias,
-                       uint32_t m, uint32_t* partials);
-void launch_pip_combine(hipStream_t s, const uint32_t* partials, uint32_t m, uint32_t* out);
+                       uint32_t m, const PipPlan* plan, const uint32_t* wins, uint32_t* partials);
+void launch_pip_combine(hipStream_t s, const uint32_t* partials, const uint16_t* walias, uint32_t m, uint32_t* out);
 // inner-product argument rounds (ipa_prove) of up to ZKH_IPA_MAX_JOBS openings per launch
 // (blockIdx.y = job); a, b plain Fr 8 words per entry.  g, g2, Qr, P: points in row form
 // (fp_row.hpp, ZKH_ROW_WORDS each); g_in, Q: 144-byte points; LR: two 144-byte points (host).
 // A job with h = 0 has finished its rounds and is skipped.  x, xi plain; xm, xim in
 // Montgomery form.
 #define ZKH_IPA_MAX_JOBS 8
-#define ZKH_ROW_WORDS 48
 struct IpaJobDev {
     const uint32_t *g_in, *Q, *g, *a, *b, *Qr;
     uint32_t *g0, *P, *LR, *g2, *a2, *b2;

@@ -3822,37 +3822,42 @@ extern "C" int zkh_commit(zkh_ctx* c, const zkh_g1* gens, const zkh_tensor* t, z
     if ((rc = g1_alloc(c, m, &o))) return rc;
     if (m) {
         DevPlanes p;
-        uint16_t* lists = nullptr;
-        uint32_t *offs = nullptr, *buckets = nullptr, *partials = nullptr;
+        uint16_t *lists = nullptr, *alias = nullptr;
+        uint32_t *offs = nullptr, *buckets = nullptr, *partials = nullptr, *tab = nullptr;
+        const size_t nt = (size_t)n * PIP_GEN_WORDS, np = sizeof(PipPlan) / 4, ni = (size_t)m * 1024, nw = (size_t)m * 64;
         if (!(rc = as_planes(c, t, SL_TMP0, &p))) lists = (uint16_t*)scratch_slot(c, SL_TMP1, (size_t)m * 64 * n * 2, &rc);
         if (!rc) offs = (uint32_t*)scratch_slot(c, SL_TMP2, (size_t)m * 64 * 16 * 4, &rc);
-        if (!rc) buckets = (uint32_t*)scratch_slot(c, SL_TMP3, (size_t)m * 64 * 16 * 144, &rc);
+        if (!rc) buckets = (uint32_t*)scratch_slot(c, SL_TMP3, (size_t)m * 64 * 16 * ZKH_ROW_WORDS * 4, &rc);
         if (!rc) partials = (uint32_t*)scratch_slot(c, SL_TMP6, (size_t)m * 64 * ZKH_ROW_WORDS * 4, &rc);
-        uint16_t* alias = nullptr;
-        if (!rc) alias = (uint16_t*)scratch_slot(c, SL_TMP4, (size_t)m * 64 * 16 * 2, &rc);
+        if (!rc) alias = (uint16_t*)scratch_slot(c, SL_TMP4, (size_t)m * 64 * (16 + 1) * 2, &rc);
+        if (!rc) tab = (uint32_t*)scratch_slot(c, SL_TMP5, (nt + np + ni + nw) * 4, &rc);
         if (rc) {
             zkh_g1_free(o);
             return rc;
         }
+        uint16_t* walias = alias + (size_t)m * 1024;
+        PipPlan* plan = (PipPlan*)(tab + nt);
+        uint32_t *items = tab + nt + np, *wins = items + ni;
         {
             ProfScope ps(c, "pip_sort", (double)m * n * 32);
+            launch_pip_gens(c->stream, (const uint32_t*)gens->d, n, tab, plan);
             launch_pip_sort(c->stream, p.lo(), p.hi(), m, n, lists, offs);
         }
         {
             ProfScope ps(c, "pip_alias", (double)m * 64 * 64);
-            launch_pip_alias(c->stream, lists, offs, m, n, alias);
+            launch_pip_alias(c->stream, lists, offs, m, n, alias, walias, plan, wins);
         }
         {
             ProfScope ps(c, "pip_bucket", (double)m * n * 32 + (double)n * 144);
-            launch_pip_bucket(c->stream, (const uint32_t*)gens->d, lists, offs, alias, m, n, buckets);
+            launch_pip_bucket(c->stream, tab, lists, offs, alias, m, n, plan, items, buckets);
         }
         {
             ProfScope ps(c, "pip_window", (double)m * 64 * 144);
-            launch_pip_window(c->stream, buckets, offs, alias, m, partials);
+            launch_pip_window(c->stream, buckets, offs, alias, m, plan, wins, partials);
         }
         {
             ProfScope ps(c, "pip_combine", (double)m * 144);
-            launch_pip_combine(c->stream, partials, m, (uint32_t*)o->d);
+            launch_pip_combine(c->stream, partials, walias, m, (uint32_t*)o->d);
         }
         hipError_t e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
