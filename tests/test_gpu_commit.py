@@ -274,6 +274,64 @@ def test_ipa_special_points_vs_oracle(zkh, ctx, ns):
         assert bytes(st) == st_o
 
 
+@pytest.mark.parametrize("nj,n", [(5, 1024), (5, 8192)])
+def test_ipa_quad_rounds(zkh, ctx, nj, n):
+    """Batches of more points than the row form takes (their first rounds run on lane quads;
+    40960 points need two table slices), with infinity, equal and opposite generators: each
+    job equals its own zkh_ipa_prove (fewer points: row form, or one slice), and at n = 1024
+    the first equals the oracle's."""
+    rng = np.random.default_rng(n)
+    base = gens_for(120, 64)
+    sc = np.frombuffer(rng.bytes(32 * (n + 1)), np.uint32).reshape(-1, 8).copy()
+    sc[:, 7] %= 0x73EDA753
+    pts = ctx.g1_mul(ctx.g1_from_host(base), ctx.from_fr(sc)).to_host()
+    for i in (0, 63, n):
+        assert np.array_equal(pts[i], C.g1_mul(base[i % 64], sc[i]))
+    pts[1] = G.g1_zero()
+    pts[n // 2] = pts[0]
+    pts[n // 2 + 1] = C.g1_mul(pts[2], np.array(P.to_limbs(P.R - 1), np.uint32))
+    jobs, alone = [], []
+    for t in range(nj):
+        a = np.frombuffer(rng.bytes(32 * n), np.uint32).reshape(n, 8).copy()
+        a[:, 7] %= 0x73EDA753
+        a[0], a[3], a[n // 2], a[n - 1] = P.to_limbs(1), 0, P.to_limbs(1), P.to_limbs(P.R - 1)
+        b = np.roll(a, 7, axis=0)
+        g = np.roll(pts[:n], t, axis=0)
+        args = (ctx.from_fr(a), ctx.from_fr(b), ctx.g1_from_host(g), pts[n])
+        st = zkh.transcript("ipaq-%d" % t)
+        alone.append((ctx.ipa_prove(st, *args), bytes(st)))
+        jobs.append((zkh.transcript("ipaq-%d" % t),) + args)
+        if t == 0 and n == 1024:
+            st_o = C.tr_init("ipaq-0")
+            rc, L, R, af = C.ipa_prove(st_o, a, b, g, pts[n], n)
+            assert rc == 0 and np.array_equal(alone[0][0]["L"], L) and np.array_equal(alone[0][0]["R"], R)
+            assert np.array_equal(alone[0][0]["a_final"], af) and alone[0][1] == bytes(st_o)
+    got = ctx.ipa_prove_batch(jobs)
+    for (st, *_), g, (want, want_st) in zip(jobs, got, alone):
+        for k in ("L", "R", "a_final"):
+            assert np.array_equal(g[k], want[k]), k
+        assert bytes(st) == want_st
+
+
+@pytest.mark.parametrize("nb,n", [(1, 40), (7, 5003), (5100, 5100), (5001, 12000)])
+def test_g1_mul_tables_vs_oracle(zkh, ctx, nb, n):
+    """zkh_g1_mul through tables of few and many bases, on waves and on quads: sampled products
+    against the oracle, the group element of the others against their neighbours' path."""
+    rng = np.random.default_rng(nb + n)
+    src = gens_for(130, 5)
+    k = np.frombuffer(rng.bytes(32 * nb), np.uint32).reshape(nb, 8).copy()
+    k[:, 7] %= 0x73EDA753
+    base = ctx.g1_mul(ctx.g1_from_host(src), ctx.from_fr(k)).to_host()
+    if nb > 1:
+        base[1] = G.g1_zero()
+    sc = np.frombuffer(rng.bytes(32 * n), np.uint32).reshape(n, 8).copy()
+    sc[:, 7] %= 0x73EDA753
+    sc[0], sc[2], sc[n - 1], sc[n // 2] = 0, P.to_limbs(1), P.to_limbs(P.R - 1), P.to_limbs(2**254)
+    got = ctx.g1_mul(ctx.g1_from_host(base), ctx.from_fr(sc)).to_host()
+    for i in [0, 1, 2, 3, 15, 16, n // 2, n - 2, n - 1] + [int(x) for x in rng.integers(0, n, 12)]:
+        assert np.array_equal(got[i], C.g1_mul(base[i % nb], sc[i])), i
+
+
 def test_ipa_prove_int_witness_and_errors(zkh, ctx):
     """a from an int32 tensor (a folded weight row is small until it is folded); sizes that
     are not a power of two or disagree are ZKH_EARG."""

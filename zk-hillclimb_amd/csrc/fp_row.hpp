@@ -1,23 +1,34 @@
 // fp_row.hpp -- BLS12-381 Fp and G1 with every element spread over the 16 lanes of a DPP row.
 //
+// A G1 point in memory is {x, y, z} Jacobian, 144 bytes, the reference's G1Jacobian_t: each
+// coordinate 12 x 32-bit limbs, little-endian, canonical in [0, p), in Montgomery form with R =
+// 2^384 (bls12-381.cuh:220-229, g1-tensor.cuh:26-63); {0, ONE, 0} is the point at infinity
+// (bls12-381.cuh:422).  The representative of a group operation depends on the formula, and
+// the bytes of a commitment are absorbed by the transcript: doubling is dbl-2009-l and addition
+// add-2007-bl with the reference's infinity and equal-point branches (bls12-381.cu:1359-1465).
+// Any computation of the same field elements gives the same bytes.
+//
 // A scalar multiply (G1Jacobian_mul, g1-tensor.cu:445-454) is one chain of dependent point
 // operations, and its length is the latency of a field product times the chain's depth.  With
-// a whole element per lane (fp_dev.hpp) a product is ~750 instructions in sequence; here lane
-// k of a row holds limb k (14 limbs of 28 bits), a product is ~107 instructions, and the four
-// rows of a wave run the up to four independent products of a point operation's level side by
-// side: one wave per point, a doubling is three levels and an addition five.  On an idle SIMD
-// a doubling takes 0.77 us and an addition 1.28 (a lane quad per point: 6.9 and 13.5); with the
-// SIMD full, 0.64 and 1.06 us of its time per point (a quad: 0.30 and 0.59), so this form is
-// for chains whose latency counts.
+// a whole element of 32-bit limbs per lane a product is ~750 instructions in sequence; here
+// lane k of a row holds limb k (14 limbs of 28 bits), a product is ~107 instructions, and the
+// four rows of a wave run the up to four independent products of a point operation's level
+// side by side: one wave per point, a doubling is three levels and an addition five.  On an
+// idle SIMD a doubling takes 0.77 us and an addition 1.28 (32-bit limbs on a lane quad per
+// point: 6.9 and 13.5); with the SIMD full, 0.64 and 1.06 us of its time per point (0.30 and
+// 0.59), so this form is for chains whose latency counts.
 //
 // Form: Montgomery with R' = 2^392, residues not canonical: a product is below 3 p with limbs
 // below 2^28 + 16, sums are taken limb by limb and renormalised by one carry pass where the next
 // use needs it.  The bound on every value is written beside it; canonical values exist only at
-// g1r_store and in the exact tests.  The group formulas are those of fp_dev.hpp (dbl-2009-l,
-// add-2007-bl, the reference's branches, bls12-381.cu:1359-1465) on equal field elements, so
-// the stored points are the same bytes.
+// g1r_store and in the exact tests.
 #pragma once
-#include "fp_dev.hpp"
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#ifndef FDEV
+#define FDEV __device__ __forceinline__
+#endif
 #include "fp_row_consts.inc"
 
 #define FPR_MASK 0x0fffffffu
@@ -179,20 +190,29 @@ FDEV uint32_t fpr_unpack(const uint32_t* w, const fpr_k& c) {
 }
 // a point in memory or LDS in row form: 16 words each for x, y, z (14 limbs), word 14 the flag
 #define G1R_WORDS 48
+FDEV uint32_t g1r_word(const g1r_t& a, const fpr_k& c) {  // this lane's word (row 3: unused)
+    return c.row == 0 && c.lane == 14 ? (a.inf ? 1u : 0u) : row_sel(c, a.x, a.y, a.z, a.z);
+}
 FDEV void g1r_put(uint32_t* p, const g1r_t& a, const fpr_k& c) {
-    const uint32_t v = c.row == 0 && c.lane == 14 ? (a.inf ? 1u : 0u) : row_sel(c, a.x, a.y, a.z, a.z);
+    const uint32_t v = g1r_word(a, c);
     if (c.row < 3) p[threadIdx.x & 63] = v;
 }
-FDEV g1r_t g1r_get(const uint32_t* p, const fpr_k& c) {
+// the words of a point as loaded: taken apart only where the point is used, so that a load made
+// ahead does not wait
+struct g1r_raw {
+    uint32_t x, y, z;
+};
+FDEV g1r_raw g1r_fetch(const uint32_t* p, const fpr_k& c) { return {p[c.lane], p[16 + c.lane], p[32 + c.lane]}; }
+FDEV g1r_t g1r_take(const g1r_raw& w, const fpr_k& c) {
     g1r_t o;
-    const uint32_t x = p[c.lane];
-    o.x = c.lane < 14 ? x : 0;
-    o.y = p[16 + c.lane];
-    o.z = p[32 + c.lane];
-    o.inf = __builtin_amdgcn_readfirstlane((int)row_bcast<14>(x)) != 0;
+    o.x = c.lane < 14 ? w.x : 0;
+    o.y = w.y;
+    o.z = w.z;
+    o.inf = __builtin_amdgcn_readfirstlane((int)row_bcast<14>(w.x)) != 0;
     return o;
 }
-// 144-byte point (fp_dev.hpp form): row r converts coordinate r
+FDEV g1r_t g1r_get(const uint32_t* p, const fpr_k& c) { return g1r_take(g1r_fetch(p, c), c); }
+// 144-byte point: row r converts coordinate r
 FDEV g1r_t g1r_load(const uint32_t* p, const fpr_k& c) {
     const uint32_t raw = fpr_unpack(p + 12 * (c.row < 3 ? c.row : 2), c);
     const uint32_t v = fpr_mul(raw, k_fpr_tab[4][c.lane], c);
@@ -244,7 +264,9 @@ FDEV g1r_t g1r_dbl(const g1r_t& a, const fpr_k& c) {
     return o;
 }
 
-// add-2007-bl with Z3 = 2 Z1 Z2 H, branches as g1_add (fp_dev.hpp)
+// add-2007-bl with Z3 = 2 Z1 Z2 H for ((Z1 + Z2)^2 - Z1Z1 - Z2Z2) H: an operand at infinity returns
+// the other unchanged, U1 = U2 and S1 = S2 doubles the first operand, and U1 = U2 with S1 != S2
+// runs the general formula (Z3 = 0)
 FDEV g1r_t g1r_add(const g1r_t& a, const g1r_t& b, const fpr_k& c) {
     if (a.inf) return b;
     if (b.inf) return a;

@@ -1,5 +1,4 @@
 // g1.hip -- G1 Pedersen commitment kernels (bucket method, commitment.cu:47-103).
-#include "fp_dev.hpp"
 #include "fp_lane28.hpp"
 #include "fp_row.hpp"
 #include "fr_dev.hpp"
@@ -293,16 +292,19 @@ __global__ __launch_bounds__(64, 2) void k_pip_bucket(const uint32_t* __restrict
                 const uint32_t item = items[task];
                 uint32_t len;
                 const uint16_t* L = pip_list(item, lists, offs, n, len);
-                g1r_t acc = g1r_get(tab + PIP_GEN_WORDS * (size_t)L[0], c), nxt = acc;
-                // the next generator is loaded one addition ahead, its index two
-                uint32_t idx = len > 1 ? L[1] : 0;
-                if (len > 1) nxt = g1r_get(tab + PIP_GEN_WORDS * (size_t)idx, c);
-                if (len > 2) idx = L[2];
+                const uint32_t last = len - 1;
+                auto fetch = [&](uint32_t i) { return g1r_fetch(tab + PIP_GEN_WORDS * (size_t)i, c); };
+                auto index = [&](uint32_t k) { return (uint32_t)L[k < last ? k : last]; };
+                g1r_t acc = g1r_take(fetch(L[0]), c);
+                // the next generator is loaded one addition ahead, its index two (past the end:
+                // the last one again)
+                g1r_raw nxt = fetch(index(1));
+                uint32_t idx = index(2);
                 for (uint32_t k = 1; k < len; k++) {
-                    const g1r_t g = nxt;
-                    if (k + 1 < len) nxt = g1r_get(tab + PIP_GEN_WORDS * (size_t)idx, c);
-                    if (k + 2 < len) idx = L[k + 2];
-                    acc = g1r_add(acc, g, c);
+                    const g1r_raw g = nxt;
+                    nxt = fetch(idx);
+                    idx = index(k + 2);
+                    acc = g1r_add(acc, g1r_take(g, c), c);
                 }
                 g1r_put(buckets + (size_t)item * G1R_WORDS, acc, c);
             } else {
@@ -403,54 +405,110 @@ __global__ __launch_bounds__(64) void k_pip_combine(const uint32_t* __restrict__
     g1r_store(out + (size_t)row * 36, acc, c);
 }
 
-// G1Jacobian_mul (g1-tensor.cu:445-454) on a quad: double-and-add over the scalar's raw
-// bits, low bit first.  The doublings after the highest set bit do not reach the result
-// and are skipped.
+// ---- G1Jacobian_mul (g1-tensor.cu:445-454): double-and-add over the scalar's raw bits, low bit
+// first.  The doubling chain a, 2a, 4a, ... does not depend on the scalar, so a product is a
+// doubling chain and a chain of the ones whose bit is set; the operations and their order are
+// those of the one loop, so the representative is the same.  A base's chain is kept as a table
+// (2^i a for i < 255 in row form, 48 KiB) where more than one scalar multiplies it.
+#define G1_BITS 255u  // scalars are below 2^255
 __device__ __forceinline__ uint32_t limb8(const uint32_t s[8], uint32_t l) {
     return l == 0 ? s[0] : l == 1 ? s[1] : l == 2 ? s[2] : l == 3 ? s[3]
          : l == 4 ? s[4] : l == 5 ? s[5] : l == 6 ? s[6] : s[7];
 }
-__device__ __forceinline__ g1_t g1_mul_quad(g1_t a, const uint32_t s[8], int q) {
+__device__ __forceinline__ int top_bit(const uint32_t s[8]) {
     int top = -1;
     for (int l = 7; l >= 0 && top < 0; l--)
         if (s[l]) top = 32 * l + 31 - __builtin_clz(s[l]);
-    g1_t acc = g1_zero();
-    uint32_t w = 0;
-    for (int i = 0; i <= top; i++) {
-        if ((i & 31) == 0) w = limb8(s, (uint32_t)i >> 5);
-        if ((w >> (i & 31)) & 1u) acc = g1_add_quad(acc, a, q);
-        if (i < top) a = g1_dbl_quad(a, q);
+    return top;
+}
+// the set bits of a scalar in ascending order, -1 after the last
+struct SetBits {
+    uint32_t w, l;
+    __device__ __forceinline__ explicit SetBits(const uint32_t s[8]) : w(s[0]), l(0) {}
+    __device__ __forceinline__ int next(const uint32_t s[8]) {
+        while (!w && l < 7) w = limb8(s, ++l);
+        if (!w) return -1;
+        const int b = __builtin_ctz(w);
+        w &= w - 1;
+        return (int)(32 * l) + b;
+    }
+};
+// one product from its base's table, one wave in row form: 1.3 us per set bit
+__device__ __forceinline__ g1r_t g1r_tab_mul(const uint32_t* tab, const uint32_t s[8], const fpr_k& c) {
+    g1r_t acc = g1r_zero(c);
+    SetBits bits(s);
+    // two points are loaded ahead of the addition (past the last bit: entry 0)
+    int b0 = bits.next(s), b1 = b0 < 0 ? -1 : bits.next(s);
+    auto fetch = [&](int b) { return g1r_fetch(tab + G1R_WORDS * (b < 0 ? 0 : b), c); };
+    g1r_raw p0 = fetch(b0), p1 = fetch(b1);
+    while (b0 >= 0) {
+        const g1r_raw p = p0;
+        p0 = p1;
+        b0 = b1;
+        if (b1 >= 0) b1 = bits.next(s);
+        p1 = fetch(b1);
+        acc = g1r_add(acc, g1r_take(p, c), c);
     }
     return acc;
 }
-
-// G1Jacobian_mul (g1-tensor.cu:445-454) on two waves of the row form (fp_row.hpp): wave 0 of
-// the pair runs the doubling chain a, 2a, 4a, ... and hands each 2^i a to wave 1 through LDS,
-// G1P_B doublings per block barrier; wave 1 adds the ones whose bit is set into acc one barrier
-// later.  The additions and doublings are those of the one-chain form in the same order (the
-// same Jacobian representative), and the doublings after the highest set bit are skipped.  The
-// chain is latency-bound: 0.77 us per doubling and 1.28 us per addition on an idle SIMD (a
-// lane quad per point took 6.9 and 13.5 us), so 255 doublings and 127 additions side by side
-// take 0.2 ms.  At 16 doublings per barrier the additions of a chunk (10 +- 2.6 us) rarely
-// outlast its doublings (12.3 us).  Every wave of the block calls it (dbl: its part), with one
-// scalar per pair; the product is in the adding wave, which does not read `a`.
+// the same on a lane quad
+__device__ __forceinline__ g28_t g28q_tab_mul(const uint32_t* tab, const uint32_t s[8], int q, bool& inf) {
+    g28_t acc = g28_zero();
+    inf = true;
+    SetBits bits(s);
+    int b = bits.next(s);
+    // the next point is loaded one addition ahead (past the last bit: entry 0)
+    auto fetch = [&](int i) { return g28_fetch(tab + G1R_WORDS * (i < 0 ? 0 : i)); };
+    g28_raw nxt = fetch(b);
+    while (b >= 0) {
+        bool pinf;
+        const g28_t p = g28_take(nxt, pinf);
+        b = bits.next(s);
+        nxt = fetch(b);
+        if (!pinf) g28q_add(acc, inf, p, q);
+    }
+    return acc;
+}
+// a base's table on a lane quad
+__device__ __forceinline__ void g28q_table(g28_t a, bool inf, uint32_t* tab, int q) {
+    for (uint32_t i = 0; i < G1_BITS; i++) {
+        // lane q stores coordinate q; signed limbs as they are: the tables of quads are read by quads
+        const f28_t v = f28_sel(q == 0, a.x, f28_sel(q == 1, a.y, a.z));
+        if (q < 3) f28_put(tab + G1R_WORDS * i + 16 * q, v, inf ? 1u : 0u);
+        if (!inf && i + 1 < G1_BITS) {
+            inf = f28_zero(a.y);  // Z3 = 2 Y Z
+            a = g28q_dbl(a, q);
+        }
+    }
+}
+// One product on two waves in row form: wave 0 of the pair runs the doubling chain and hands
+// each 2^i a to wave 1 through LDS, G1P_B doublings per block barrier; wave 1 adds the ones
+// whose bit is set one barrier later.  The chain is latency-bound (0.77 us per doubling, 1.28
+// per addition on an idle SIMD): 255 doublings and 127 additions side by side take 0.25 ms.
+// At 16 doublings per barrier the additions of a chunk (10 +- 2.6 us) rarely outlast its
+// doublings (12.3 us).  Every wave of the block calls it (dbl: its part), with one scalar per
+// pair; the product is in the adding wave, which does not read `a`.  tab: where the base's
+// table is wanted too (all 255 doublings then), else null and the doublings after the highest
+// set bit are skipped.
 #define G1P_B 16
 typedef uint32_t g1_pipe_buf[2][G1P_B][G1R_WORDS];
 __device__ __forceinline__ g1r_t g1r_mul_pipe(g1r_t a, const uint32_t s[8], bool dbl, g1_pipe_buf& buf,
-                                              const fpr_k& c) {
+                                              uint32_t* tab, const fpr_k& c) {
     static_assert(32 % G1P_B == 0, "a chunk's bits lie in one scalar limb");
-    int top = -1;
-    for (int l = 7; l >= 0 && top < 0; l--)
-        if (s[l]) top = 32 * l + 31 - __builtin_clz(s[l]);
+    const int top = top_bit(s), last = tab ? (int)G1_BITS - 1 : top;
     g1r_t acc = g1r_zero(c);
     constexpr int NC = 256 / G1P_B;
     for (int k = 0; k <= NC; k++) {
         if (dbl) {
             for (int j = 0; j < G1P_B; j++) {
                 const int i = k * G1P_B + j;
-                if (i > top) break;
-                g1r_put(buf[k & 1][j], a, c);
-                if (i < top) a = g1r_dbl(a, c);
+                if (i > last) break;
+                const uint32_t v = g1r_word(a, c);
+                if (c.row < 3) {
+                    buf[k & 1][j][threadIdx.x & 63] = v;
+                    if (tab) tab[G1R_WORDS * i + (threadIdx.x & 63)] = v;
+                }
+                if (i < last) a = g1r_dbl(a, c);
             }
         } else if (k > 0) {
             const uint32_t w = limb8(s, (uint32_t)((k - 1) * G1P_B) >> 5);
@@ -465,30 +523,94 @@ __device__ __forceinline__ g1r_t g1r_mul_pipe(g1r_t a, const uint32_t s[8], bool
 }
 
 // elementwise with a broadcast base (G1_jacobian_elementwise_mul_broadcast,
-// g1-tensor.cu:463-468): out[i] = base[i % nb] * s[i], one quad per element
-__global__ __launch_bounds__(64) void k_g1_mul(const uint32_t* __restrict__ base, uint32_t nb,
-                                               const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
-                                               uint32_t n, uint32_t* __restrict__ out) {
-    const uint32_t i = blockIdx.x * 16 + threadIdx.x / 4;
-    const int q = threadIdx.x & 3;
-    if (i >= n) return;
+// g1-tensor.cu:463-468): out[i] = base[i % nb] * s[i].
+// The tables of bases [b0, b0 + nt): one wave each in row form (0.2 ms a chain) or, from
+// G1_QUADS on, where the SIMDs are full that way, one quad each (0.75 ms; a third of the work)
+#define G1_QUADS 5000u
+__global__ __launch_bounds__(64) void k_g1_tables(const uint32_t* __restrict__ base, uint32_t b0,
+                                                  uint32_t* __restrict__ tab) {
+    const uint32_t i = blockIdx.x;
+    const fpr_k c = fpr_consts();
+    g1r_t a = g1r_load(base + 36 * (size_t)(b0 + i), c);
+    uint32_t* t = tab + (size_t)i * G1_BITS * G1R_WORDS;
+    for (uint32_t k = 0; k < G1_BITS; k++) {
+        g1r_put(t + G1R_WORDS * k, a, c);
+        if (k + 1 < G1_BITS) a = g1r_dbl(a, c);
+    }
+}
+// out[i] = base[i] * s[i], two waves per product, no table
+__global__ __launch_bounds__(128) void k_g1_mul(const uint32_t* __restrict__ base, const uint32_t* __restrict__ lo,
+                                                const uint32_t* __restrict__ hi, uint32_t* __restrict__ out) {
+    __shared__ g1_pipe_buf buf;
+    const uint32_t i = blockIdx.x;
+    const fpr_k c = fpr_consts();
+    const bool dbl = __builtin_amdgcn_readfirstlane(threadIdx.x / 64) == 0;
     const uint4 s0 = ((const uint4*)lo)[i], s1 = ((const uint4*)hi)[i];
     const uint32_t sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-    const g1_t r = g1_mul_quad(g1_load(base + 36 * (size_t)(i % nb)), sc, q);
-    if (q == 0) g1_store(out + 36 * (size_t)i, r);
+    g1r_t p = g1r_zero(c);
+    if (dbl) p = g1r_load(base + 36 * (size_t)i, c);
+    const g1r_t m = g1r_mul_pipe(p, sc, dbl, buf, nullptr, c);
+    if (!dbl) g1r_store(out + 36 * (size_t)i, m, c);
 }
-
-// out[i] = b[i] + a[i] * s: one scalar for every row, the sum with b[i] as first operand
-// (hb_addmul with mul_first = false, zkob_fastg1.cuh:56-88: k_g1_mul then k_g1_addsub)
-__global__ __launch_bounds__(64) void k_g1_addmul(const uint32_t* __restrict__ a, G1Scalar sc,
-                                                  const uint32_t* __restrict__ b, uint32_t n,
-                                                  uint32_t* __restrict__ out) {
-    const uint32_t i = blockIdx.x * 16 + threadIdx.x / 4;
-    const int q = threadIdx.x & 3;
+// row forms of n points, one wave each
+__global__ __launch_bounds__(256) void k_g1_rows(const uint32_t* __restrict__ base, uint32_t n,
+                                                 uint32_t* __restrict__ out) {
+    const uint32_t i = blockIdx.x * 4 + threadIdx.x / 64;
     if (i >= n) return;
-    const g1_t m = g1_mul_quad(g1_load(a + 36 * (size_t)i), sc.v, q);
-    const g1_t r = g1_add_quad(g1_load(b + 36 * (size_t)i), m, q);
-    if (q == 0) g1_store(out + 36 * (size_t)i, r);
+    const fpr_k c = fpr_consts();
+    g1r_put(out + G1R_WORDS * (size_t)i, g1r_load(base + 36 * (size_t)i, c), c);
+}
+__global__ __launch_bounds__(64) void k_g1_tables4(const uint32_t* __restrict__ rows, uint32_t nt,
+                                                   uint32_t* __restrict__ tab) {
+    const uint32_t i = blockIdx.x * 16 + threadIdx.x / 4;
+    if (i >= nt) return;
+    bool inf;
+    const g28_t a = g28_load(rows + G1R_WORDS * (size_t)i, inf);
+    g28q_table(a, inf, tab + (size_t)i * G1_BITS * G1R_WORDS, threadIdx.x & 3);
+}
+// products i0 + k (k < count) of the bases at hand (base (i0 + k) % nb - b0): one wave each
+__global__ __launch_bounds__(64) void k_g1_tab_mul(const uint32_t* __restrict__ tab, uint32_t nb, uint32_t b0,
+                                                   const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
+                                                   uint32_t i0, uint32_t* __restrict__ out) {
+    const uint32_t i = i0 + blockIdx.x;
+    const fpr_k c = fpr_consts();
+    const uint4 s0 = ((const uint4*)lo)[i], s1 = ((const uint4*)hi)[i];
+    const uint32_t sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+    g1r_store(out + 36 * (size_t)i, g1r_tab_mul(tab + (size_t)(i % nb - b0) * G1_BITS * G1R_WORDS, sc, c), c);
+}
+// one quad each, products in row form to rows[k]
+__global__ __launch_bounds__(64) void k_g1_tab_mul4(const uint32_t* __restrict__ tab, uint32_t nb, uint32_t b0,
+                                                    const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
+                                                    uint32_t i0, uint32_t count, uint32_t* __restrict__ rows) {
+    const uint32_t k = blockIdx.x * 16 + threadIdx.x / 4, i = i0 + k;
+    if (k >= count) return;
+    const uint4 s0 = ((const uint4*)lo)[i], s1 = ((const uint4*)hi)[i];
+    const uint32_t sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+    const int q = threadIdx.x & 3;
+    bool inf;
+    const g28_t r = g28q_tab_mul(tab + (size_t)(i % nb - b0) * G1_BITS * G1R_WORDS, sc, q, inf);
+    if (q == 0) g28_store(rows + G1R_WORDS * (size_t)k, r, inf);
+}
+__global__ __launch_bounds__(256) void k_g1_points(const uint32_t* __restrict__ rows, uint32_t n,
+                                                   uint32_t* __restrict__ out) {
+    const uint32_t i = blockIdx.x * 4 + threadIdx.x / 64;
+    if (i >= n) return;
+    const fpr_k c = fpr_consts();
+    g1r_store(out + 36 * (size_t)i, g1r_get(rows + G1R_WORDS * (size_t)i, c), c);
+}
+// out[i] = b[i] + a[i] * s: one scalar for every row, the sum with b[i] as first operand
+// (hb_addmul with mul_first = false, zkob_fastg1.cuh:56-88: k_g1_mul then k_g1_addsub); two
+// waves per row
+__global__ __launch_bounds__(128) void k_g1_addmul(const uint32_t* __restrict__ a, G1Scalar sc,
+                                                   const uint32_t* __restrict__ b, uint32_t* __restrict__ out) {
+    __shared__ g1_pipe_buf buf;
+    const uint32_t i = blockIdx.x;
+    const fpr_k c = fpr_consts();
+    const bool dbl = __builtin_amdgcn_readfirstlane(threadIdx.x / 64) == 0;
+    g1r_t p = g1r_zero(c);
+    if (dbl) p = g1r_load(a + 36 * (size_t)i, c);
+    const g1r_t m = g1r_mul_pipe(p, sc.v, dbl, buf, nullptr, c);
+    if (!dbl) g1r_store(out + 36 * (size_t)i, g1r_add(g1r_load(b + 36 * (size_t)i, c), m, c), c);
 }
 
 // ---- inner-product argument rounds (ipa_prove, vrf_common.cuh:302-336) ----
@@ -545,28 +667,79 @@ __device__ __forceinline__ void ipa_inner(const IpaJobDev& J, uint32_t side, con
     __syncthreads();
 }
 // L and R terms (vrf_common.cuh:316-319): P[j] = g[h + j] a[j], P[h + j] = g[j] a[h + j],
-// P[2h], P[2h + 1] = Q <a_lo, b_hi>, Q <a_hi, b_lo>; one product per block.  Blocks 0 and 1
-// take the Q products and their inner products (first, since they are the longest).
-__global__ __launch_bounds__(128) void k_ipa_scale(IpaBatchDev B, uint32_t nj, fr_t r2) {
-    const IpaJobDev& J = B.j[ipa_job(B, nj, blockIdx.x, true)];
-    const uint32_t h = J.h, blk = blockIdx.x - J.scale0;
-    if (blk >= 2 * h + 2) return;  // whole block
-    __shared__ g1_pipe_buf buf;
-    __shared__ fr_t red[128];
-    __shared__ uint32_t ip[8];
+// P[2h], P[2h + 1] = Q <a_lo, b_hi>, Q <a_hi, b_lo>.  The fold multiplies the same generators,
+// so their tables are kept for it: point id 2 i + hi of a job is g[i + hi h], its table at
+// D + pt0 + id.
+__device__ __forceinline__ uint32_t* ipa_table(const IpaBatchDev& B, const IpaJobDev& J, uint32_t id) {
+    return B.D + (size_t)(J.pt0 + id - B.slice0) * G1_BITS * G1R_WORDS;
+}
+// one product by waves 0 and 1 of the block (more only take its barriers): blk 0, 1 the Q products with their inner products (first,
+// since they are the longest), then P[blk - 2] with its generator's table
+__device__ __forceinline__ void ipa_product(const IpaBatchDev& B, const IpaJobDev& J, uint32_t blk, const fr_t& r2,
+                                            g1_pipe_buf& buf, fr_t* red, uint32_t* ip) {
+    const uint32_t h = J.h;
     const fpr_k c = fpr_consts();
     const uint32_t j = blk < 2 ? 2 * h + blk : blk - 2;
-    const bool dbl = __builtin_amdgcn_readfirstlane(threadIdx.x / 64) == 0;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const bool dbl = wave == 0;
     if (blk < 2) ipa_inner(J, blk, r2, red, ip);
     const uint32_t* sp = blk < 2 ? ip : J.a + 8 * (size_t)j;
     uint32_t sc[8];
 #pragma unroll
-    for (int k = 0; k < 8; k++) sc[k] = __builtin_amdgcn_readfirstlane(sp[k]);
+    for (int k = 0; k < 8; k++) sc[k] = wave < 2 ? __builtin_amdgcn_readfirstlane(sp[k]) : 0;
     const uint32_t* bp = j < h ? J.g + G1R_WORDS * (size_t)(h + j) : j < 2 * h ? J.g + G1R_WORDS * (size_t)(j - h) : J.Qr;
     g1r_t base = g1r_zero(c);
     if (dbl) base = g1r_get(bp, c);
-    const g1r_t r = g1r_mul_pipe(base, sc, dbl, buf, c);
-    if (!dbl) g1r_put(J.P + G1R_WORDS * (size_t)j, r, c);
+    uint32_t* tab = blk < 2 ? nullptr : ipa_table(B, J, j < h ? 2 * j + 1 : 2 * (j - h));
+    const g1r_t r = g1r_mul_pipe(base, sc, dbl, buf, tab, c);
+    if (wave == 1) g1r_put(J.P + G1R_WORDS * (size_t)j, r, c);
+}
+// few points: one product per block
+__global__ __launch_bounds__(128) void k_ipa_scale(IpaBatchDev B, uint32_t nj, fr_t r2) {
+    __shared__ g1_pipe_buf buf;
+    __shared__ fr_t red[128];
+    __shared__ uint32_t ip[8];
+    const IpaJobDev& J = B.j[ipa_job(B, nj, blockIdx.x, true)];
+    const uint32_t blk = blockIdx.x - J.scale0;
+    if (blk >= 2 * J.h + 2) return;  // whole block
+    ipa_product(B, J, blk, r2, buf, red, ip);
+}
+// many points (G1_QUADS): the Q products on two waves each (blocks below 2 nj, where asked),
+// the tables of points [slice0, slice0 + count) on quads; then every product on a quad
+__device__ __forceinline__ uint32_t ipa_point(const IpaBatchDev& B, uint32_t nj, uint32_t pt) {
+    uint32_t job = 0;
+    for (uint32_t j = 1; j < nj; j++)
+        if (B.j[j].h && pt >= B.j[j].pt0) job = j;
+    return job;
+}
+__global__ __launch_bounds__(256) void k_ipa_tables4(IpaBatchDev B, uint32_t nj, uint32_t nq, uint32_t count, fr_t r2) {
+    __shared__ g1_pipe_buf buf;
+    __shared__ fr_t red[256];
+    __shared__ uint32_t ip[8];
+    if (blockIdx.x < nq) {
+        const IpaJobDev& J = B.j[blockIdx.x / 2];
+        if (J.h) ipa_product(B, J, blockIdx.x & 1, r2, buf, red, ip);
+        return;
+    }
+    const uint32_t k = (blockIdx.x - nq) * 64 + threadIdx.x / 4;
+    if (k >= count) return;
+    const IpaJobDev& J = B.j[ipa_point(B, nj, B.slice0 + k)];
+    const uint32_t id = B.slice0 + k - J.pt0;
+    bool inf;
+    const g28_t a = g28_load(J.g + G1R_WORDS * (size_t)(id / 2 + (id & 1) * J.h), inf);
+    g28q_table(a, inf, ipa_table(B, J, id), threadIdx.x & 3);
+}
+__global__ __launch_bounds__(64) void k_ipa_scale4(IpaBatchDev B, uint32_t nj, uint32_t count) {
+    const uint32_t k = blockIdx.x * 16 + threadIdx.x / 4;
+    if (k >= count) return;
+    const IpaJobDev& J = B.j[ipa_point(B, nj, B.slice0 + k)];
+    const uint32_t id = B.slice0 + k - J.pt0, j = id / 2 + (id & 1 ? 0 : J.h);
+    uint32_t sc[8];
+#pragma unroll
+    for (int l = 0; l < 8; l++) sc[l] = J.a[8 * (size_t)j + l];
+    bool inf;
+    const g28_t r = g28q_tab_mul(ipa_table(B, J, id), sc, threadIdx.x & 3, inf);
+    if ((threadIdx.x & 3) == 0) g28_store(J.P + G1R_WORDS * (size_t)j, r, inf);
 }
 // pairwise trees over P[0, h) and P[h, 2h): of a side's m = h >> shift remaining points a block
 // takes the K = min(m, 64) at distance m / K (six levels of the tree: level by level the halves
@@ -600,44 +773,91 @@ __global__ __launch_bounds__(1024) void k_ipa_tree(IpaBatchDev B, uint32_t shift
     if (dist > 1) g1r_put(P, r, c);
     else g1r_store(J.LR + 36 * side, g1r_add(r, g1r_get(J.P + G1R_WORDS * (size_t)(2 * h + side), c), c), c);
 }
-// one folded generator per block: waves 0 and 1 compute x^-1 g_lo[i], waves 2 and 3 x g_hi[i]
-// (k_g1_fold2's two products, vrf_common.cuh:71-76), then wave 1 adds them in that order; two
-// lanes of wave 1 fold a and b while its first doublings are under way
-__global__ __launch_bounds__(256) void k_ipa_fold(IpaBatchDev B, uint32_t nj) {
+// a' and b' of entry i, on lane 0 (a) and 1 (b) of a pair
+__device__ __forceinline__ void ipa_fold_ab(const IpaJobDev& J, uint32_t i, uint32_t sel) {
+    const uint32_t h = J.h;
+    fr_t xm, xim;
+#pragma unroll
+    for (int k = 0; k < 8; k++) xm.v[k] = J.xm[k], xim.v[k] = J.xim[k];
+    const uint32_t* src = sel ? J.b : J.a;
+    st_aos(sel ? J.b2 : J.a2, i,
+           fr_add(mont_mul(sel ? xim : xm, ld_aos(src, i)), mont_mul(sel ? xm : xim, ld_aos(src, i + h))));
+}
+// one folded generator per block, from the tables: wave 0 computes x^-1 g_lo[i], wave 1
+// x g_hi[i] (k_g1_fold2's two products, vrf_common.cuh:71-76), then wave 0 adds them in that
+// order; two lanes of wave 1 fold a and b first
+__global__ __launch_bounds__(128) void k_ipa_fold(IpaBatchDev B, uint32_t nj) {
     const IpaJobDev& J = B.j[ipa_job(B, nj, blockIdx.x, false)];
-    const uint32_t h = J.h, i = blockIdx.x - J.fold0;
-    if (i >= h) return;  // whole block
-    __shared__ g1_pipe_buf buf[2];
+    const uint32_t i = blockIdx.x - J.fold0;
+    if (i >= J.h) return;  // whole block
+    __shared__ uint32_t other[G1R_WORDS];
     const fpr_k c = fpr_consts();
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), hi = wave >> 1;
-    const bool dbl = !(wave & 1);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     uint32_t sc[8];
 #pragma unroll
     for (int k = 0; k < 8; k++) sc[k] = hi ? J.x[k] : J.xi[k];
-    g1r_t base = g1r_zero(c);
-    if (dbl) base = g1r_get(J.g + G1R_WORDS * (size_t)(i + hi * h), c);
-    if (wave == 1 && c.lane == 0 && c.row < 2) {
-        fr_t xm, xim;
-#pragma unroll
-        for (int k = 0; k < 8; k++) xm.v[k] = J.xm[k], xim.v[k] = J.xim[k];
-        const uint32_t* src = c.row ? J.b : J.a;
-        uint32_t* dst = c.row ? J.b2 : J.a2;
-        st_aos(dst, i, fr_add(mont_mul(c.row ? xim : xm, ld_aos(src, i)), mont_mul(c.row ? xm : xim, ld_aos(src, i + h))));
-    }
-    g1r_t r = g1r_mul_pipe(base, sc, dbl, buf[hi], c);
-    if (wave == 3) g1r_put(buf[0][0][0], r, c);
+    if (hi && c.lane == 0 && c.row < 2) ipa_fold_ab(J, i, c.row);
+    const g1r_t r = g1r_tab_mul(ipa_table(B, J, 2 * i + hi), sc, c);
+    if (hi) g1r_put(other, r, c);
     __syncthreads();
-    if (wave == 1) g1r_put(J.g2 + G1R_WORDS * (size_t)i, g1r_add(r, g1r_get(buf[0][0][0], c), c), c);
+    if (!hi) g1r_put(J.g2 + G1R_WORDS * (size_t)i, g1r_add(r, g1r_get(other, c), c), c);
+}
+// many points: the same on two quads per generator
+__global__ __launch_bounds__(64) void k_ipa_fold4(IpaBatchDev B, uint32_t nj, uint32_t count) {
+    const uint32_t k = blockIdx.x * 16 + threadIdx.x / 4;
+    if (k >= count) return;  // count is even: both quads of a generator or neither
+    const IpaJobDev& J = B.j[ipa_point(B, nj, B.slice0 + k)];
+    const uint32_t id = B.slice0 + k - J.pt0, i = id / 2, hi = id & 1;
+    const int q = threadIdx.x & 3;
+    uint32_t sc[8];
+#pragma unroll
+    for (int l = 0; l < 8; l++) sc[l] = hi ? J.x[l] : J.xi[l];
+    if (hi && q < 2) ipa_fold_ab(J, i, q);
+    bool inf;
+    g28_t r = g28q_tab_mul(ipa_table(B, J, id), sc, q, inf);
+    // the upper quad's product to the lower one
+    g28_t o;
+#pragma unroll
+    for (int l = 0; l < 14; l++) {
+        o.x.v[l] = __shfl_xor(r.x.v[l], 4);
+        o.y.v[l] = __shfl_xor(r.y.v[l], 4);
+        o.z.v[l] = __shfl_xor(r.z.v[l], 4);
+    }
+    const bool oinf = __shfl_xor((int)inf, 4) != 0;
+    if (hi) return;
+    if (!oinf) g28q_add(r, inf, o, q);
+    if (q == 0) g28_store(J.g2 + G1R_WORDS * (size_t)i, r, inf);
 }
 void launch_ipa_points(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax) {
     hipLaunchKernelGGL(k_ipa_points, dim3((2 * hmax + 1 + 3) / 4, nj), dim3(256), 0, s, B);
 }
-void launch_ipa_scale(hipStream_t s, const IpaBatchDev& B, uint32_t nj, const uint32_t r2[8]) {
+// blocks of four waves, one per SIMD (of two, the dispatcher put three waves on one SIMD: 2.6 ms
+// for 20480 tables)
+static void launch_ipa_tables(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t nq, uint32_t count, fr_t r2) {
+    const uint32_t blocks = nq + (count + 63) / 64;
+    hipLaunchKernelGGL(k_ipa_tables4, dim3(blocks), dim3(256), lds_share(blocks, 1, sizeof(g1_pipe_buf) + 257 * 32), s, B,
+                       nj, nq, count, r2);
+}
+void launch_ipa_scale(hipStream_t s, IpaBatchDev& B, uint32_t nj, const uint32_t r2[8]) {
     fr_t R2;
     for (int k = 0; k < 8; k++) R2.v[k] = r2[k];
-    uint32_t blocks = 0;
-    for (uint32_t j = 0; j < nj; j++) blocks += B.j[j].h ? 2 * B.j[j].h + 2 : 0;
-    hipLaunchKernelGGL(k_ipa_scale, dim3(blocks), dim3(128), lds_share(blocks, 2, sizeof(g1_pipe_buf) + 129 * 32), s, B, nj, R2);
+    uint32_t blocks = 0, points = 0;
+    for (uint32_t j = 0; j < nj; j++) {
+        blocks += B.j[j].h ? 2 * B.j[j].h + 2 : 0;
+        points += 2 * B.j[j].h;
+    }
+    B.slice0 = 0;
+    if (points < G1_QUADS) {
+        hipLaunchKernelGGL(k_ipa_scale, dim3(blocks), dim3(128), lds_share(blocks, 2, sizeof(g1_pipe_buf) + 129 * 32), s,
+                           B, nj, R2);
+        return;
+    }
+    for (; B.slice0 < points; B.slice0 += ZKH_IPA_TABLES) {
+        const uint32_t count = points - B.slice0 < ZKH_IPA_TABLES ? points - B.slice0 : ZKH_IPA_TABLES;
+        const uint32_t nq = B.slice0 ? 0 : 2 * nj;
+        launch_ipa_tables(s, B, nj, nq, count, R2);
+        hipLaunchKernelGGL(k_ipa_scale4, dim3((count + 15) / 16), dim3(64), lds_share((count + 15) / 16, 4, 0), s, B, nj, count);
+    }
 }
 void launch_ipa_tree(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax) {
     for (uint32_t shift = 0; shift == 0 || (hmax >> (shift - 6)) > 64; shift += 6) {
@@ -645,10 +865,22 @@ void launch_ipa_tree(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t 
         hipLaunchKernelGGL(k_ipa_tree, dim3(m > 64 ? m / 64 : 1, nj, 2), dim3(1024), 0, s, B, shift);
     }
 }
-void launch_ipa_fold(hipStream_t s, const IpaBatchDev& B, uint32_t nj) {
+void launch_ipa_fold(hipStream_t s, IpaBatchDev& B, uint32_t nj) {
     uint32_t blocks = 0;
     for (uint32_t j = 0; j < nj; j++) blocks += B.j[j].h;
-    hipLaunchKernelGGL(k_ipa_fold, dim3(blocks), dim3(256), lds_share(blocks, 1, sizeof(g1_pipe_buf) * 2), s, B, nj);
+    const uint32_t points = 2 * blocks;
+    B.slice0 = 0;
+    if (points < G1_QUADS) {
+        hipLaunchKernelGGL(k_ipa_fold, dim3(blocks), dim3(128), lds_share(blocks, 2, G1R_WORDS * 4), s, B, nj);
+        return;
+    }
+    fr_t none = {};
+    for (; B.slice0 < points; B.slice0 += ZKH_IPA_TABLES) {
+        const uint32_t count = points - B.slice0 < ZKH_IPA_TABLES ? points - B.slice0 : ZKH_IPA_TABLES;
+        if (points > ZKH_IPA_TABLES)  // more than the tables hold: this slice's again
+            launch_ipa_tables(s, B, nj, 0, count, none);
+        hipLaunchKernelGGL(k_ipa_fold4, dim3((count + 15) / 16), dim3(64), lds_share((count + 15) / 16, 4, 0), s, B, nj, count);
+    }
 }
 // planes -> 8-word entries
 __global__ __launch_bounds__(256) void k_planes_to_aos(const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
@@ -662,11 +894,48 @@ void launch_planes_to_aos(hipStream_t s, const uint32_t* lo, const uint32_t* hi,
 }
 void launch_g1_addmul(hipStream_t s, const uint32_t* a, const G1Scalar& sc, const uint32_t* b, uint32_t n,
                       uint32_t* out) {
-    hipLaunchKernelGGL(k_g1_addmul, dim3((n + 15) / 16), dim3(64), 0, s, a, sc, b, n, out);
+    hipLaunchKernelGGL(k_g1_addmul, dim3(n), dim3(128), lds_share(n, 2, sizeof(g1_pipe_buf)), s, a, sc, b, out);
+}
+// bases whose tables are held at once, and the words of scratch for them
+static uint32_t g1_mul_tables(uint32_t nb, uint32_t n) {
+    const uint32_t used = nb < n ? nb : n;
+    if (used == n && n < G1_QUADS) return 0;  // each base once: no table
+    return used < ZKH_IPA_TABLES ? used : ZKH_IPA_TABLES;
+}
+size_t g1_mul_words(uint32_t nb, uint32_t n) {
+    const uint32_t nt = g1_mul_tables(nb, n);
+    return nt ? (size_t)nt * G1_BITS * G1R_WORDS + (size_t)(n > nt ? n : nt) * G1R_WORDS : 0;
 }
 void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint32_t* lo, const uint32_t* hi,
-                   uint32_t n, uint32_t* out) {
-    hipLaunchKernelGGL(k_g1_mul, dim3((n + 15) / 16), dim3(64), 0, s, base, nb, lo, hi, n, out);
+                   uint32_t n, uint32_t* out, uint32_t* work) {
+    const uint32_t nt = g1_mul_tables(nb, n), used = nb < n ? nb : n;
+    if (!nt) {
+        hipLaunchKernelGGL(k_g1_mul, dim3(n), dim3(128), lds_share(n, 2, sizeof(g1_pipe_buf)), s, base, lo, hi, out);
+        return;
+    }
+    uint32_t* rows = work + (size_t)nt * G1_BITS * G1R_WORDS;
+    for (uint32_t b0 = 0; b0 < used; b0 += nt) {
+        const uint32_t bases = used - b0 < nt ? used - b0 : nt;
+        if (bases < G1_QUADS) {
+            hipLaunchKernelGGL(k_g1_tables, dim3(bases), dim3(64), 0, s, base, b0, work);
+        } else {
+            hipLaunchKernelGGL(k_g1_rows, dim3((bases + 3) / 4), dim3(256), 0, s, base + 36 * (size_t)b0, bases, rows);
+            hipLaunchKernelGGL(k_g1_tables4, dim3((bases + 15) / 16), dim3(64), 0, s, rows, bases, work);
+        }
+        // the products of these bases: all at once if they are all the bases, else pass by pass
+        const bool all = bases == nb;
+        for (uint64_t i0 = b0; i0 < n; i0 += nb) {
+            const uint32_t count = all ? n : (uint32_t)(n - i0 < bases ? n - i0 : bases);
+            if (count < G1_QUADS && bases < G1_QUADS) {  // quads leave signed limbs: read by quads
+                hipLaunchKernelGGL(k_g1_tab_mul, dim3(count), dim3(64), 0, s, work, nb, b0, lo, hi, (uint32_t)i0, out);
+            } else {
+                hipLaunchKernelGGL(k_g1_tab_mul4, dim3((count + 15) / 16), dim3(64), 0, s, work, nb, b0, lo, hi,
+                                   (uint32_t)i0, count, rows);
+                hipLaunchKernelGGL(k_g1_points, dim3((count + 3) / 4), dim3(256), 0, s, rows, count, out + 36 * i0);
+            }
+            if (all) break;
+        }
+    }
 }
 void launch_pip_sort(hipStream_t s, const uint32_t* lo, const uint32_t* hi, uint32_t m, uint32_t n,
                      uint16_t* lists, uint32_t* offs) {

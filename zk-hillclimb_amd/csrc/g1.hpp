@@ -59,18 +59,24 @@ void launch_pip_combine(hipStream_t s, const uint32_t* partials, const uint16_t*
 struct IpaJobDev {
     const uint32_t *g_in, *Q, *g, *a, *b, *Qr;
     uint32_t *g0, *P, *LR, *g2, *a2, *b2;
-    uint32_t h, scale0, fold0, pad;  // scale0, fold0: the job's first block of the launch
+    uint32_t h, scale0, fold0, pt0;  // the job's first block of a scale and fold launch, first point
     uint32_t x[8], xi[8], xm[8], xim[8];
 };
+// D: the points' tables (2^i g, i < 255), of points [slice0, slice0 + ZKH_IPA_TABLES) where
+// there are more (the points of all jobs in order, ipa_table)
+#define ZKH_IPA_TABLES 32768u
+#define ZKH_TABLE_WORDS (255u * ZKH_ROW_WORDS)
 struct IpaBatchDev {
     IpaJobDev j[ZKH_IPA_MAX_JOBS];
+    uint32_t* D;
+    uint32_t slice0;
 };
 // g0[0, 2h] = row forms of g_in[0, 2h) and Q
 void launch_ipa_points(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax);
-void launch_ipa_scale(hipStream_t s, const IpaBatchDev& B, uint32_t nj, const uint32_t r2[8]);
+void launch_ipa_scale(hipStream_t s, IpaBatchDev& B, uint32_t nj, const uint32_t r2[8]);
 // every tree level and L, R (hmax the largest h)
 void launch_ipa_tree(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax);
-void launch_ipa_fold(hipStream_t s, const IpaBatchDev& B, uint32_t nj);
+void launch_ipa_fold(hipStream_t s, IpaBatchDev& B, uint32_t nj);
 void launch_planes_to_aos(hipStream_t s, const uint32_t* lo, const uint32_t* hi, uint32_t n, uint32_t* out);
 // out[i] = base[i % nb] * s[i] (G1Jacobian_mul, raw scalar bits)
 // a scalar passed by value to a kernel: 8 plain little-endian words
@@ -81,4 +87,6 @@ struct G1Scalar {
 void launch_g1_addmul(hipStream_t s, const uint32_t* a, const G1Scalar& sc, const uint32_t* b, uint32_t n,
                       uint32_t* out);
 void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint32_t* lo, const uint32_t* hi,
-                   uint32_t n, uint32_t* out);
+                   uint32_t n, uint32_t* out, uint32_t* work);
+// words of launch_g1_mul's scratch `work`
+size_t g1_mul_words(uint32_t nb, uint32_t n);

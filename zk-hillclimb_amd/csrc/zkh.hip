@@ -3776,7 +3776,12 @@ extern "C" int zkh_g1_mul(zkh_ctx* c, const zkh_g1* base, const zkh_tensor* t, z
             zkh_g1_free(o);
             return rc;
         }
-        launch_g1_mul(c->stream, (const uint32_t*)base->d, base->n, p.lo(), p.hi(), t->n, (uint32_t*)o->d);
+        uint32_t* work = (uint32_t*)scratch_slot(c, SL_TMP3, g1_mul_words(base->n, t->n) * 4, &rc);
+        if (rc) {
+            zkh_g1_free(o);
+            return rc;
+        }
+        launch_g1_mul(c->stream, (const uint32_t*)base->d, base->n, p.lo(), p.hi(), t->n, (uint32_t*)o->d, work);
         hipError_t e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) {
@@ -3879,7 +3884,7 @@ extern "C" int zkh_ipa_prove_batch(zkh_ctx* c, uint32_t nj, uint8_t* const* tran
                                    uint32_t* const* L_out, uint32_t* const* R_out, uint32_t* const* a_final) {
     if (!c || !transcripts || !a || !b || !g || !Q || !a_final || !L_out || !R_out) return fail(c, ZKH_EARG, "null argument");
     if (!nj || nj > ZKH_IPA_MAX_JOBS) return fail(c, ZKH_EARG, "ipa_prove_batch: 1 to %d jobs", ZKH_IPA_MAX_JOBS);
-    size_t fr_words = 0, g_words = 0, p_words = 0;
+    size_t fr_words = 0, g_words = 0, p_words = 0, points = 0;
     uint32_t nmax = 0;
     for (uint32_t j = 0; j < nj; j++) {
         if (!transcripts[j] || !a[j] || !b[j] || !g[j] || !Q[j] || !a_final[j]) return fail(c, ZKH_EARG, "null argument");
@@ -3890,6 +3895,7 @@ extern "C" int zkh_ipa_prove_batch(zkh_ctx* c, uint32_t nj, uint8_t* const* tran
         fr_words += (size_t)n * 32;
         g_words += (size_t)(n + n / 2 + 1) * ZKH_ROW_WORDS;
         p_words += (size_t)(n + 2) * ZKH_ROW_WORDS;
+        points += n;
         nmax = std::max(nmax, n);
     }
     HIPCHK(c, hipSetDevice(c->device));
@@ -3900,10 +3906,11 @@ extern "C" int zkh_ipa_prove_batch(zkh_ctx* c, uint32_t nj, uint8_t* const* tran
     uint32_t* fr_w = (uint32_t*)scratch_slot(c, SL_TMP1, fr_words * 4, &rc);
     uint32_t* g_w = rc ? nullptr : (uint32_t*)scratch_slot(c, SL_TMP2, g_words * 4, &rc);
     uint32_t* p_w = rc ? nullptr : (uint32_t*)scratch_slot(c, SL_TMP3, (p_words + 36 * (size_t)nj) * 4, &rc);
+    IpaBatchDev B{};
+    if (!rc) B.D = (uint32_t*)scratch_slot(c, SL_TMP4, std::min(points, (size_t)ZKH_IPA_TABLES) * ZKH_TABLE_WORDS * 4, &rc);
     if (rc) return rc;
     static_assert(72 * ZKH_IPA_MAX_JOBS <= ZKH_MAX_BATCH * 11 * 8, "L and R of a round fit the published sums");
     uint32_t* lr = c->pub_host;
-    IpaBatchDev B{};
     uint32_t sz[ZKH_IPA_MAX_JOBS];
     uint32_t *A0[ZKH_IPA_MAX_JOBS], *B0[ZKH_IPA_MAX_JOBS], *G0[ZKH_IPA_MAX_JOBS];
     uint32_t *A1[ZKH_IPA_MAX_JOBS], *B1[ZKH_IPA_MAX_JOBS], *G1[ZKH_IPA_MAX_JOBS];
@@ -3947,6 +3954,7 @@ extern "C" int zkh_ipa_prove_batch(zkh_ctx* c, uint32_t nj, uint8_t* const* tran
             const uint32_t h = B.j[j].h = sz[j] > 1 ? sz[j] / 2 : 0;
             B.j[j].scale0 = scale0;
             B.j[j].fold0 = fold0;
+            B.j[j].pt0 = 2 * fold0;
             scale0 += h ? 2 * h + 2 : 0;
             fold0 += h;
             hmax = std::max(hmax, h);
