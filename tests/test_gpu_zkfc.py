@@ -58,6 +58,27 @@ def test_pad(zkh, ctx, shape):
         ctx.pad(ctx.from_fr(x), shape + [2])
 
 
+@pytest.mark.parametrize("O,C_,W", [(1, 1, 1), (3, 1, 1), (1, 1, 70), (2, 3, 65), (1, 100003, 1), (3, 4097, 2),
+                                    (70001, 3, 1), (5, 257, 64), (1, 1025, 300), (2, 129, 1000)])
+@pytest.mark.parametrize("kind", ["fr", "i32", "i64"])
+def test_partial_me_splits(zkh, ctx, O, C_, W, kind):
+    """The weighted sum over the middle dimension at the edges of its split: one term, remainders
+    of the lanes along each dimension, and sums split over chunks of blocks."""
+    rng = np.random.default_rng(O + C_ + W)
+    n, k = O * C_ * W, P.ceil_log2(C_)
+    vals = rng.integers(-2**31, 2**31, size=n)
+    if kind == "fr":
+        t = np.frombuffer(rng.bytes(32 * n), np.uint32).reshape(n, 8).copy()
+        t[:, 7] %= 0x73EDA753
+    else:
+        t = zkh.ints_to_fr(vals)
+    u = rand_fr(rng, k)
+    rc, want = C.partial_me(t, u, C_, W)
+    assert rc == 0
+    tg = ctx.from_fr(t) if kind == "fr" else ctx.from_i32(vals) if kind == "i32" else ctx.from_i64(vals)
+    assert fr_eq(ctx.partial_me(tg, u, C_, W).to_fr(), want)
+
+
 @pytest.mark.parametrize("low,length,N", [(-8, 16, 16), (-32768, 65536, 65536), (5, 3, 8), (-(1 << 21), 1 << 22, 1 << 22),
                                            (2**31 - 4, 8, 8), (-2**31, 4, 8)])
 def test_range_table(zkh, ctx, low, length, N):

@@ -1357,24 +1357,51 @@ extern "C" int zkh_me_static(zkh_ctx* c, const zkh_tensor* t, const uint32_t* u,
     fr_store(s, out);
     return ZKH_OK;
 }
-// eq table (Montgomery AoS) of u over n entries into a scratch slot
+// eq table (Montgomery AoS) of u over n entries into a scratch slot; the factors go with the
+// launch where they and the table fit its small form, else by an upload ahead of it
 static int eq_table_mont(zkh_ctx* c, const std::vector<Fr>& u, uint32_t n, int slot, uint32_t** out) {
     int rc = 0;
     std::vector<uint32_t> fac;
     make_fac(u, 0, fac);
+    uint32_t* e = (uint32_t*)scratch_slot(c, slot, (size_t)std::max<uint32_t>(n, 1) * 32, &rc);
+    if (rc) return rc;
+    *out = e;
+    if (fac.size() <= sizeof(FacArg) / 4) {
+        FacArg fa;
+        memcpy(fa.w, fac.data(), fac.size() * 4);
+        if (launch_eq_mont2_ka(c->stream, fa, (uint32_t)u.size(), n, e, 0, 0, e)) return 0;
+    }
     uint32_t* fac_d = (uint32_t*)scratch_slot(c, SL_FAC, std::max<size_t>(fac.size() * 4, 32), &rc);
     if (rc) return rc;
     if (!fac.empty() && (rc = upload(c, fac_d, fac.data(), fac.size() * 4))) return rc;
-    uint32_t* e = (uint32_t*)scratch_slot(c, slot, (size_t)std::max<uint32_t>(n, 1) * 32, &rc);
-    if (rc) return rc;
     launch_eq_mont(c->stream, fac_d, (uint32_t)u.size(), n, e);
-    *out = e;
     return 0;
 }
+// the weighted sum over the middle dimension of a [O, C, W] view of t into o (queued)
+static int partial_me_queue(zkh_ctx* c, const zkh_tensor* t, uint32_t O, uint32_t C, uint32_t W, const uint32_t* E,
+                            DevPlanes o) {
+    int rc = 0;
+    const void* src = t->d;
+    int kind = t->kind == ZKH_KIND_FR ? 0 : t->kind == ZKH_KIND_I32 ? 1 : 2;
+    uint32_t cap = t->cap;
+    if (t->weights) {  // logical (row-major) W from the OUT-major copy
+        DevPlanes p;
+        if ((rc = as_planes(c, t, SL_TMP0, &p))) return rc;
+        src = p.base;
+        cap = p.cap;
+        kind = 0;
+    }
+    uint32_t* work = (uint32_t*)scratch_slot(c, SL_PARTIAL, partial_me_words(O, C, W) * 4, &rc);
+    if (rc) return rc;
+    launch_partial_me(c->stream, kind, src, cap, t->n, O, C, W, E, o, work);
+    return 0;
+}
+// FrTensor::partial_me(u, cur_dim, window)'s checks and its work, queued: the result is ready
+// for later work on the stream
 static int partial_me_impl(zkh_ctx* c, const zkh_tensor* t, const std::vector<Fr>& u,
                            uint32_t cur_dim, uint32_t window, zkh_tensor** out) {
     uint32_t k = (uint32_t)u.size();
-    // FrTensor::partial_me(u, cur_dim, window) checks (fr-tensor.cu:554-560)
+    // (fr-tensor.cu:554-560)
     if (k >= 32 || cur_dim <= ((1u << k) >> 1) || cur_dim > (1u << k))
         return fail(c, ZKH_EARG, "partial_me: incompatible dimensions");
     if (!window || t->n % ((uint64_t)cur_dim * window) != 0)
@@ -1385,35 +1412,63 @@ static int partial_me_impl(zkh_ctx* c, const zkh_tensor* t, const std::vector<Fr
     if ((rc = eq_table_mont(c, u, cur_dim, SL_EB, &E))) return rc;
     zkh_tensor* o;
     if ((rc = tensor_alloc(c, ZKH_KIND_FR, O * window, &o))) return rc;
-    if (t->kind == ZKH_KIND_FR) launch_partial_me_planes(c->stream, t->planes(), O, cur_dim, window, E, o->planes());
-    else if (t->kind == ZKH_KIND_I64)
-        launch_partial_me_i64(c->stream, (const int64_t*)t->d, O, cur_dim, window, E, o->planes());
-    else {
-        DevPlanes p;
-        if (t->weights) {
-            if ((rc = as_planes(c, t, SL_TMP0, &p))) {
-                zkh_tensor_free(o);
-                return rc;
-            }
-            launch_partial_me_planes(c->stream, p, O, cur_dim, window, E, o->planes());
-        } else {
-            launch_partial_me_i32(c->stream, (const int32_t*)t->d, O, cur_dim, window, E, o->planes());
-        }
-    }
-    hipError_t e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) {
+    if ((rc = partial_me_queue(c, t, O, cur_dim, window, E, o->planes()))) {
         zkh_tensor_free(o);
-        return fail(c, ZKH_EDEV, "partial_me: %s", hipGetErrorString(e));
+        return rc;
     }
     *out = o;
     return 0;
+}
+// the end of an entry point that leaves `o`: waits for it, or frees it after an error
+static int finish_tensor(zkh_ctx* c, zkh_tensor* o, zkh_tensor** out) {
+    const hipError_t e = hipGetLastError();
+    int rc = e == hipSuccess ? settle(c) : fail(c, ZKH_EDEV, "launch failed: %s", hipGetErrorString(e));
+    if (rc) {
+        zkh_tensor_free(o);
+        return rc;
+    }
+    *out = o;
+    return ZKH_OK;
 }
 extern "C" int zkh_partial_me(zkh_ctx* c, const zkh_tensor* t, const uint32_t* u, uint32_t k,
                               uint32_t cur_dim, uint32_t window, zkh_tensor** out) {
     if (!c || !t || !out || (!u && k)) return fail(c, ZKH_EARG, "null argument");
     if (!all_canonical(u, k)) return fail(c, ZKH_EARG, "non-canonical challenge");
     HIPCHK(c, hipSetDevice(c->device));
-    return partial_me_impl(c, t, load_frs(u, k), cur_dim, window, out);
+    zkh_tensor* o;
+    const int rc = partial_me_impl(c, t, load_frs(u, k), cur_dim, window, &o);
+    return rc ? rc : finish_tensor(c, o, out);
+}
+// FrTensor::multi_dim_me's value left on the device (one-entry tensor, queued): the dimensions
+// bound last first (fr-tensor.cu:643-652)
+static int multi_dim_me_queue(zkh_ctx* c, const zkh_tensor* t, const std::vector<Fr>* uv, const uint32_t* shape,
+                              uint32_t ndim, zkh_tensor** out) {
+    const zkh_tensor* cur = t;
+    zkh_tensor* owned = nullptr;
+    for (uint32_t d = ndim; d-- > 0;) {
+        const uint32_t k = (uint32_t)uv[d].size();
+        // the first dimension takes all that is left (FrTensor::operator(), fr-tensor.cu:437-442)
+        const uint32_t n = d ? shape[d] : cur->n;
+        zkh_tensor* nxt;
+        int rc;
+        if (!d && (k >= 32 || n <= ((1u << k) / 2) || n > (1u << k))) rc = fail(c, ZKH_EARG, "Incompatible dimensions");
+        else rc = partial_me_impl(c, cur, uv[d], n, 1, &nxt);
+        if (owned) zkh_tensor_free(owned);  // its buffer serves later work on this stream only
+        if (rc) return rc;
+        cur = owned = nxt;
+    }
+    *out = owned;
+    return 0;
+}
+// the value of a queued one-entry tensor, which is freed
+static int read_entry(zkh_ctx* c, zkh_tensor* t, uint32_t out[8]) {
+    uint32_t w[8];
+    const hipError_t e = hipGetLastError();
+    int rc = e == hipSuccess ? settle(c, (const uint32_t*)t->d, w, 8)
+                             : fail(c, ZKH_EDEV, "launch failed: %s", hipGetErrorString(e));
+    zkh_tensor_free(t);
+    if (!rc) memcpy(out, w, 32);
+    return rc;
 }
 extern "C" int zkh_multi_dim_me(zkh_ctx* c, const zkh_tensor* t, const uint32_t* us,
                                 const uint32_t* ks, const uint32_t* shape, uint32_t ndim,
@@ -1432,24 +1487,10 @@ extern "C" int zkh_multi_dim_me(zkh_ctx* c, const zkh_tensor* t, const uint32_t*
         uv[d] = load_frs(us + 8 * off, ks[d]);
         off += ks[d];
     }
-    // bind the last dimension first (fr-tensor.cu:643-652)
-    const zkh_tensor* cur = t;
-    zkh_tensor* owned = nullptr;
-    int rc = 0;
-    for (uint32_t d = ndim - 1; d >= 1; d--) {
-        zkh_tensor* nxt;
-        rc = partial_me_impl(c, cur, uv[d], shape[d], 1, &nxt);
-        if (owned) zkh_tensor_free(owned);
-        if (rc) return rc;
-        owned = nxt;
-        cur = nxt;
-    }
-    uint32_t k0 = ks[0];
-    std::vector<uint32_t> u0(8 * (size_t)k0);
-    for (uint32_t i = 0; i < k0; i++) fr_store(uv[0][i], &u0[8 * (size_t)i]);
-    rc = zkh_me(c, cur, u0.data(), k0, out);
-    if (owned) zkh_tensor_free(owned);
-    return rc;
+    if (ndim == 1) return zkh_me(c, t, us, ks[0], out);
+    zkh_tensor* v;
+    const int rc = multi_dim_me_queue(c, t, uv.data(), shape, ndim, &v);
+    return rc ? rc : read_entry(c, v, out);
 }
 extern "C" int zkh_eq_table(zkh_ctx* c, const uint32_t* u, uint32_t k, zkh_tensor** out) {
     if (!c || !out || (!u && k) || k > 30) return fail(c, ZKH_EARG, "bad arguments");
@@ -4668,26 +4709,11 @@ extern "C" int zkh_partial_me_window(zkh_ctx* c, const zkh_tensor* t, const uint
     if ((rc = eq_table_mont(c, load_frs(u, k), (uint32_t)C, SL_EB, &E))) return rc;
     zkh_tensor* o;
     if ((rc = tensor_alloc(c, ZKH_KIND_FR, (uint32_t)(orows * window), &o))) return rc;
-    const void* src = t->d;
-    int kind = t->kind == ZKH_KIND_FR ? 0 : t->kind == ZKH_KIND_I32 ? 1 : 2;
-    DevPlanes p{(uint32_t*)t->d, t->cap};
-    if (t->weights) {  // logical (row-major) W from the OUT-major copy
-        if ((rc = as_planes(c, t, SL_TMP0, &p))) {
-            zkh_tensor_free(o);
-            return rc;
-        }
-        src = p.base;
-        kind = 0;
-    }
-    launch_partial_me_window(c->stream, kind, src, p.cap, t->n, (uint32_t)orows, (uint32_t)C, window, E,
-                             o->planes());
-    hipError_t e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) {
+    if ((rc = partial_me_queue(c, t, (uint32_t)orows, (uint32_t)C, window, E, o->planes()))) {
         zkh_tensor_free(o);
-        return fail(c, ZKH_EDEV, "partial_me: %s", hipGetErrorString(e));
+        return rc;
     }
-    *out = o;
-    return ZKH_OK;
+    return finish_tensor(c, o, out);
 }
 
 // ---------------------------------------------------------------------------------------
