@@ -114,7 +114,9 @@ def _stacked_claim(A, B, uN, N, D):
     return np.array(P.to_limbs(s), np.uint32)
 
 
-@pytest.mark.parametrize("N,D", [(1, 4), (2, 3), (3, 5), (4, 8), (7, 6), (8, 1), (16, 100), (7, 2048)])
+@pytest.mark.parametrize("N,D", [(1, 4), (2, 3), (3, 5), (4, 8), (7, 6), (8, 1), (16, 100), (7, 2048),
+                                 (1, 1024), (1, 1025), (4, 256), (5, 205), (33, 31), (700, 1), (1025, 1), (1500, 3),
+                                 (3, 700), (64, 64), (2, 2047)])
 def test_zkip_stacked(zkh, ctx, N, D):
     rng = np.random.default_rng(N * 1000 + D)
     A, B = rand_fr(rng, N * D), rand_fr(rng, N * D)
@@ -131,7 +133,8 @@ def test_zkip_stacked(zkh, ctx, N, D):
 
 
 @pytest.mark.parametrize("num,B,IN,OUT,bias", [(2, 4, 8, 4, False), (3, 5, 6, 3, True), (1, 2, 3, 2, True),
-                                               (4, 1, 4, 5, False), (7, 64, 256, 96, True)])
+                                               (4, 1, 4, 5, False), (7, 64, 256, 96, True), (1, 3, 2, 1, False),
+                                               (1, 1, 1, 1, True), (12, 17, 100, 9, False), (70, 5, 33, 65, True)])
 def test_fc_stacked_prove(zkh, ctx, num, B, IN, OUT, bias):
     rng = np.random.default_rng(num * 100 + B + IN)
     X = rng.integers(-300, 300, size=(num, B, IN)).astype(np.int64)

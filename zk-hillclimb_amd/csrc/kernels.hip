@@ -355,6 +355,18 @@ bool launch_eq_mont2_ka(hipStream_t s, const FacArg& f, uint32_t K0, uint32_t n0
     k_eq_mont_quad_ka<<<g0 + g1, NT, 0, s>>>(f, K0, n0, out0, K1, n1, out1, g0, plain1 ? 1u : 0u);
     return true;
 }
+// several tables in one launch, one after the other in out (table j of EqSet entries from at[j])
+__global__ __launch_bounds__(NT) void k_eq_mont_set(FacArg f, EqSet T, uint32_t* out) {
+    const uint32_t i = blockIdx.x * NT + threadIdx.x, b = i >> 2, q = i & 3;
+    uint32_t j = 0, k0 = 0;
+    while (j + 1 < T.count && b >= T.at[j + 1]) k0 += T.K[j++];
+    const bool in = b < T.at[T.count];
+    const fr_t e = eq_prod_quad(f.w + 16 * k0, T.K[j], in ? b - T.at[j] : 0, q);
+    if (q == 0 && in) st_aos(out, b, e);
+}
+void launch_eq_mont_set(hipStream_t s, const FacArg& f, const EqSet& T, uint32_t* out) {
+    k_eq_mont_set<<<(4 * T.at[T.count] + NT - 1) / NT, NT, 0, s>>>(f, T, out);
+}
 void launch_eq_mont2(hipStream_t s, const uint32_t* fac0, uint32_t K0, uint32_t n0, uint32_t* out0,
                      const uint32_t* fac1, uint32_t K1, uint32_t n1, uint32_t* out1) {
     if (n0 > EQ_QUAD_MAX || n1 > EQ_QUAD_MAX) {
@@ -584,56 +596,147 @@ void launch_range_table_i32(hipStream_t s, int32_t low, uint32_t len, uint32_t N
 }
 
 // ------------------------------------------------------------------------------------
-// plain and stacked inner-product sumcheck rounds over a [N, D] row layout: row n < Nh
-// pairs with row n + Nh (Nh = 2^ceil(log2 N) / 2; rows >= N read as zero) and carries the
-// weight E[n] (Montgomery form, AoS) or 1 when E is null.  Sums, each x 2^-256:
-// c0 = sum w a0 b0, c1 = sum w (a0 db + b0 da), c2 = sum w da db.
+// plain and stacked inner-product sumcheck rounds (zkfc.cu:94-246).  A round takes a table pair
+// of M entries: entry i < h pairs with entry i + h (zero past M), weighted by E[i / D]
+// (Montgomery form, AoS) or 1 when E is null, and leaves h entries bound to its challenge.
+// Sums, each x 2^-256: S0 = sum w a0 b0, S1 = sum w a1 b1, S2 = sum w da db, from which the
+// round's coefficients are c0 = S0, c1 = S1 - S0 - S2, c2 = S2 (three products a pair
+// instead of four).
+//
+// The challenges are the caller's, all known before the first round, so no round waits for
+// the host: the rounds of large tables are a launch each (the previous round's fold and this
+// one's sums), and from 1024 entries on one block runs all that are left in LDS.  One launch,
+// fold, eq upload and host round trip per round took 45 us a round; the block takes 6.
 // ------------------------------------------------------------------------------------
-__global__ __launch_bounds__(NT) void k_stk_round(const uint4* alo, const uint4* ahi, const uint4* blo,
-                                                  const uint4* bhi, uint32_t N, uint32_t D, uint32_t Nh,
-                                                  const uint32_t* __restrict__ E, Publish pub) {
+ZDEV fr_t stk_entry(const uint4* lo, const uint4* hi, uint32_t i, uint32_t n) {
+    return i < n ? ld_fr(lo, hi, i) : fr_zero();
+}
+// the table's entry i after the pending fold of a table of `full` entries to M (v: its
+// challenge), or as it is
+ZDEV fr_t stk_folded(const uint4* lo, const uint4* hi, uint32_t i, uint32_t M, uint32_t full, bool fold,
+                     const fr_t& v) {
+    const fr_t x = stk_entry(lo, hi, i, fold ? full : M);
+    return fold ? fr_add(x, mont_mul(v, fr_sub(stk_entry(lo, hi, i + M, full), x))) : x;
+}
+__global__ __launch_bounds__(NT) void k_stk_step(const uint4* alo, const uint4* ahi, const uint4* blo,
+                                                 const uint4* bhi, uint4* oalo, uint4* oahi, uint4* oblo,
+                                                 uint4* obhi, uint32_t full, uint32_t fold, fr_t v, uint32_t M,
+                                                 uint32_t h, uint32_t D, const uint32_t* __restrict__ E,
+                                                 Publish pub) {
     fr_t acc[3] = {fr_zero(), fr_zero(), fr_zero()};
-    const uint32_t tot = Nh * D, hiD = Nh * D, full = N * D;
-    for (uint32_t idx = blockIdx.x * NT + threadIdx.x; idx < tot; idx += gridDim.x * NT) {
-        fr_t a0 = ld_fr(alo, ahi, idx), b0 = ld_fr(blo, bhi, idx);
-        const bool up = idx + hiD < full;
-        fr_t da = fr_sub(up ? ld_fr(alo, ahi, idx + hiD) : fr_zero(), a0);
-        fr_t db = fr_sub(up ? ld_fr(blo, bhi, idx + hiD) : fr_zero(), b0);
+    for (uint32_t i = blockIdx.x * NT + threadIdx.x; i < h; i += gridDim.x * NT) {
+        const bool up = i + h < M;
+        fr_t a0 = stk_folded(alo, ahi, i, M, full, fold, v), b0 = stk_folded(blo, bhi, i, M, full, fold, v);
+        fr_t a1 = up ? stk_folded(alo, ahi, i + h, M, full, fold, v) : fr_zero();
+        fr_t b1 = up ? stk_folded(blo, bhi, i + h, M, full, fold, v) : fr_zero();
+        if (fold) {
+            st_fr(oalo, oahi, i, a0);
+            st_fr(oblo, obhi, i, b0);
+            if (up) {
+                st_fr(oalo, oahi, i + h, a1);
+                st_fr(oblo, obhi, i + h, b1);
+            }
+        }
+        fr_t da = fr_sub(a1, a0);
+        const fr_t db = fr_sub(b1, b0);
         if (E) {
-            const fr_t wm = ld_aos(E, idx / D);
-            a0 = mont_mul(wm, a0);  // w * a0 (plain)
-            da = mont_mul(wm, da);
+            const fr_t w = ld_aos(E, i / D);
+            a0 = mont_mul(w, a0);  // w a0 (plain)
+            a1 = mont_mul(w, a1);
+            da = fr_sub(a1, a0);
         }
         acc[0] = fr_add(acc[0], mont_mul(a0, b0));
-        acc[1] = fr_add(acc[1], fr_add(mont_mul(a0, db), mont_mul(da, b0)));
+        acc[1] = fr_add(acc[1], mont_mul(a1, b1));
         acc[2] = fr_add(acc[2], mont_mul(da, db));
     }
     reduce_publish<3>(acc, pub, 0, 0, gridDim.x, blockIdx.x);
 }
-// in-place bind of the top row bit: t[idx] = t0 + v (t1 - t0) for idx < Nh*D (t1 = 0 past N)
-__global__ void k_stk_fold(uint4* alo, uint4* ahi, uint4* blo, uint4* bhi, uint32_t N, uint32_t D,
-                           uint32_t Nh, fr_t vm) {
-    const uint32_t tot = Nh * D, hiD = Nh * D, full = N * D;
-    for (uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x; idx < tot; idx += gridDim.x * blockDim.x) {
-        const bool up = idx + hiD < full;
-        const fr_t a0 = ld_fr(alo, ahi, idx), b0 = ld_fr(blo, bhi, idx);
-        const fr_t a1 = up ? ld_fr(alo, ahi, idx + hiD) : fr_zero();
-        const fr_t b1 = up ? ld_fr(blo, bhi, idx + hiD) : fr_zero();
-        st_fr(alo, ahi, idx, fr_add(a0, mont_mul(vm, fr_sub(a1, a0))));
-        st_fr(blo, bhi, idx, fr_add(b0, mont_mul(vm, fr_sub(b1, b0))));
+// All rounds left, one block: five waves take each sum's products; then the last wave adds
+// their sums and writes them to the host while the others fold the tables (and the weights:
+// the eq table without its top variable is the sum of its halves).
+__global__ __launch_bounds__(1024) void k_stk_tail(const uint4* alo, const uint4* ahi, const uint4* blo,
+                                                   const uint4* bhi, uint32_t full, uint32_t fold, fr_t v,
+                                                   StkTail T, const uint32_t* __restrict__ E, uint32_t* host_out,
+                                                   uint32_t* host_flag, uint32_t seq) {
+    __shared__ fr_t A[ZKH_STK_TAIL], B[ZKH_STK_TAIL], W[ZKH_STK_TAIL / 2], red[3][5];
+    const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    uint32_t M = T.M;
+    for (uint32_t i = t; i < M; i += 1024) {
+        A[i] = stk_folded(alo, ahi, i, M, full, fold, v);
+        B[i] = stk_folded(blo, bhi, i, M, full, fold, v);
+    }
+    if (E)
+        for (uint32_t i = t; i < T.h[0] / T.D; i += 1024) W[i] = ld_aos(E, i);
+    __syncthreads();
+    for (uint32_t r = 0; r < T.rounds; r++) {
+        const uint32_t h = T.h[r];
+        const bool weighted = r < T.weighted;
+        if (wave < 15) {
+            const uint32_t k = wave / 5;
+            fr_t s = fr_zero();
+            for (uint32_t i = (wave % 5) * 64 + lane; i < h; i += 320) {
+                const bool up = i + h < M;
+                fr_t a = k == 1 ? fr_zero() : A[i], b = k == 1 ? fr_zero() : B[i];
+                if (k && up) {
+                    a = k == 2 ? fr_sub(A[i + h], a) : A[i + h];
+                    b = k == 2 ? fr_sub(B[i + h], b) : B[i + h];
+                } else if (k == 2) {  // the partner is zero: da = -a0, db = -b0
+                    a = fr_sub(fr_zero(), a);
+                    b = fr_sub(fr_zero(), b);
+                }
+                if (weighted) a = mont_mul(W[i / T.D], a);
+                s = fr_add(s, mont_mul(a, b));
+            }
+            if (h > (wave % 5) * 64) s = fr_wave_sum(s);
+            if (lane == 0) red[k][wave % 5] = s;
+        }
+        __syncthreads();
+        if (wave == 15) {
+            if (lane < 3) {
+                fr_t s = red[lane][0];
+                for (uint32_t j = 1; j < 5 && j * 64 < h; j++) s = fr_add(s, red[lane][j]);
+                st_aos(host_out, 3 * r + lane, s);
+            }
+        } else if (r + 1 < T.rounds) {
+            const fr_t x = to_fr(T.v[r]);
+            for (uint32_t i = t; i < 2 * h; i += 960) {
+                fr_t* tab = i < h ? A : B;
+                const uint32_t j = i < h ? i : i - h;
+                const fr_t e = tab[j], p = j + h < M ? tab[j + h] : fr_zero();
+                tab[j] = fr_add(e, mont_mul(x, fr_sub(p, e)));
+            }
+            const uint32_t half = h / T.D / 2;
+            if (r + 1 < T.weighted && t < half) W[t] = fr_add(W[t], W[t + half]);
+        }
+        M = h;
+        __syncthreads();
+    }
+    if (t == 0) {
+        __threadfence_system();
+        __hip_atomic_store(host_flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
-uint32_t launch_stk_round(hipStream_t s, DevPlanes a, DevPlanes b, uint32_t N, uint32_t D, uint32_t Nh,
-                          const uint32_t* E, Publish pub) {
-    const uint32_t g = grid_for(Nh * D, NT, 1024);
-    k_stk_round<<<g, NT, 0, s>>>(PL_LO(a), PL_HI(a), PL_LO(b), PL_HI(b), N, D, Nh, E, pub);
+void launch_stk_step(hipStream_t s, DevPlanes a, DevPlanes b, DevPlanes oa, DevPlanes ob, uint32_t full,
+                     const uint32_t* v_m, uint32_t M, uint32_t h, uint32_t D, const uint32_t* E, Publish pub) {
+    fr_t v = {};
+    if (v_m) v = to_fr(v_m);
+    k_stk_step<<<grid_for(h, NT, 1024), NT, 0, s>>>(PL_LO(a), PL_HI(a), PL_LO(b), PL_HI(b), PL_LO(oa), PL_HI(oa),
+                                                    PL_LO(ob), PL_HI(ob), full, v_m ? 1u : 0u, v, M, h, D, E, pub);
     launch_publish(s, pub);
-    return g;
 }
-void launch_stk_fold(hipStream_t s, DevPlanes a, DevPlanes b, uint32_t N, uint32_t D, uint32_t Nh,
-                     const uint32_t* v_m_host) {
-    k_stk_fold<<<grid_for(Nh * D, NT, 8192), NT, 0, s>>>(PL_LO(a), PL_HI(a), PL_LO(b), PL_HI(b), N, D, Nh,
-                                                        to_fr(v_m_host));
+void launch_stk_tail(hipStream_t s, DevPlanes a, DevPlanes b, uint32_t full, const uint32_t* v_m, const StkTail& T,
+                     const uint32_t* E, uint32_t* host_out, uint32_t* host_flag, uint32_t seq) {
+    fr_t v = {};
+    if (v_m) v = to_fr(v_m);
+    k_stk_tail<<<1, 1024, 0, s>>>(PL_LO(a), PL_HI(a), PL_LO(b), PL_HI(b), full, v_m ? 1u : 0u, v, T, E, host_out,
+                                  host_flag, seq);
+}
+// 8-word entries p[0 .. n) to host_out, one after the other
+__global__ void k_entries(EntryPtrs p, uint32_t n, uint32_t* host_out) {
+    if (threadIdx.x < 8 * n) host_out[threadIdx.x] = p.p[threadIdx.x / 8][threadIdx.x % 8];
+}
+void launch_entries(hipStream_t s, const EntryPtrs& p, uint32_t n, uint32_t* host_out) {
+    k_entries<<<1, 64, 0, s>>>(p, n, host_out);
 }
 
 // ------------------------------------------------------------------------------------

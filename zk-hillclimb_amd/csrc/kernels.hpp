@@ -82,6 +82,13 @@ struct FacArg {
 };
 bool launch_eq_mont2_ka(hipStream_t s, const FacArg& f, uint32_t K0, uint32_t n0, uint32_t* out0, uint32_t K1,
                         uint32_t n1, uint32_t* out1, bool plain1 = false);
+// up to ZKH_EQ_SET tables of at most 2^14 entries in all, their factors (ZKH_FAC_ARG_VARS in all)
+// as launch arguments: table j has K[j] variables and entries at[j] .. at[j + 1] of out
+#define ZKH_EQ_SET 8
+struct EqSet {
+    uint32_t count, K[ZKH_EQ_SET], at[ZKH_EQ_SET + 1];
+};
+void launch_eq_mont_set(hipStream_t s, const FacArg& f, const EqSet& T, uint32_t* out);
 
 // ---- dot products / sums (block partials, AoS, summed on the host) ----
 // partial[b] = sum montmul(a_i, b_i) over the block's range (carries 2^-256)
@@ -108,13 +115,27 @@ void launch_pad(hipStream_t s, DevPlanes src, const PadDims& pd, uint32_t total,
 // tLookupRange table of N entries: low + min(i, len - 1)
 void launch_range_table(hipStream_t s, int32_t low, uint32_t len, uint32_t N, DevPlanes out);
 void launch_range_table_i32(hipStream_t s, int32_t low, uint32_t len, uint32_t N, int32_t* out);
-// zkip / zkip_stacked round over a [N, D] layout (rows n, n + Nh paired, rows >= N zero,
-// weights E[n] Montgomery AoS of Nh entries, or 1 when E is null): publishes c0, c1, c2
-// (x 2^-256) as job 0 of pub; the fold binds the top row bit in place with v (Montgomery)
-uint32_t launch_stk_round(hipStream_t s, DevPlanes a, DevPlanes b, uint32_t N, uint32_t D, uint32_t Nh,
-                          const uint32_t* E, Publish pub);
-void launch_stk_fold(hipStream_t s, DevPlanes a, DevPlanes b, uint32_t N, uint32_t D, uint32_t Nh,
-                     const uint32_t* v_m_host);
+// zkip / zkip_stacked rounds (see kernels.hip).  One round: the tables a, b of `full` entries
+// folded to M by v_m (Montgomery; written to oa, ob, which may be a, b) or, v_m null, of M
+// entries as they are; pairs (i, i + h), weights E[i / D]; publishes S0, S1, S2 as job 0 of pub
+void launch_stk_step(hipStream_t s, DevPlanes a, DevPlanes b, DevPlanes oa, DevPlanes ob, uint32_t full,
+                     const uint32_t* v_m, uint32_t M, uint32_t h, uint32_t D, const uint32_t* E, Publish pub);
+// the last rounds of a table of M <= ZKH_STK_TAIL entries (after the pending fold): distances
+// h, challenges v (Montgomery), the first `weighted` of them weighted by E; S0, S1, S2 of round
+// r to host_out + 24 r, then seq to the flag
+#define ZKH_STK_TAIL 1024u
+struct StkTail {
+    uint32_t M, D, rounds, weighted;
+    uint32_t h[16];
+    uint32_t v[16][8];
+};
+void launch_stk_tail(hipStream_t s, DevPlanes a, DevPlanes b, uint32_t full, const uint32_t* v_m, const StkTail& T,
+                     const uint32_t* E, uint32_t* host_out, uint32_t* host_flag, uint32_t seq);
+// 8-word entries p[0 .. n) (n <= 8) to host_out, one after the other
+struct EntryPtrs {
+    const uint32_t* p[8];
+};
+void launch_entries(hipStream_t s, const EntryPtrs& p, uint32_t n, uint32_t* host_out);
 // rescaling witness: q = (x - rem) / sf, rem = ((x + sf/2) mod sf) - sf/2 for x of the given
 // kind (0: FR planes read through scalar_to_long, 1: int32, 2: int64)
 void launch_rescale(hipStream_t s, int kind, const void* x, uint32_t cap, uint32_t n, int64_t sf,

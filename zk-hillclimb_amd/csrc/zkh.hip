@@ -1377,6 +1377,49 @@ static int eq_table_mont(zkh_ctx* c, const std::vector<Fr>& u, uint32_t n, int s
     launch_eq_mont(c->stream, fac_d, (uint32_t)u.size(), n, e);
     return 0;
 }
+// several eq tables into one slot: tables[j].n entries of the eq table of tables[j].u at
+// tables[j].E; one launch where they and their factors fit its arguments
+struct EqWant {
+    const std::vector<Fr>* u;
+    uint32_t n;
+    uint32_t* E;
+};
+static int eq_tables_mont(zkh_ctx* c, EqWant* tables, uint32_t count, int slot) {
+    int rc = 0;
+    size_t n = 0, vars = 0;
+    for (uint32_t j = 0; j < count; j++) n += tables[j].n, vars += tables[j].u->size();
+    uint32_t* out = (uint32_t*)scratch_slot(c, slot, std::max<size_t>(n, 1) * 32, &rc);
+    if (rc) return rc;
+    EqSet T{};
+    FacArg fa;
+    const bool one = count <= ZKH_EQ_SET && vars <= ZKH_FAC_ARG_VARS && n <= (1u << 14);
+    size_t at = 0, k0 = 0;
+    for (uint32_t j = 0; j < count; j++) {
+        const EqWant& t = tables[j];
+        std::vector<uint32_t> fac;
+        make_fac(*t.u, 0, fac);
+        tables[j].E = out + 8 * at;
+        if (one) {
+            memcpy(fa.w + 16 * k0, fac.data(), fac.size() * 4);
+            T.K[j] = (uint32_t)t.u->size();
+            T.at[j] = (uint32_t)at;
+        } else if (t.n) {
+            // the factors in a slot region of their own: the launches run one after the other
+            uint32_t* fac_d = (uint32_t*)scratch_slot(c, SL_FAC, (vars * 16 + 16) * 4, &rc);
+            if (rc) return rc;
+            if (!fac.empty() && (rc = upload(c, fac_d + 16 * k0, fac.data(), fac.size() * 4))) return rc;
+            launch_eq_mont(c->stream, fac_d + 16 * k0, (uint32_t)t.u->size(), t.n, tables[j].E);
+        }
+        at += t.n;
+        k0 += t.u->size();
+    }
+    if (one && at) {
+        T.count = count;
+        T.at[count] = (uint32_t)at;
+        launch_eq_mont_set(c->stream, fa, T, out);
+    }
+    return 0;
+}
 // the weighted sum over the middle dimension of a [O, C, W] view of t into o (queued)
 static int partial_me_queue(zkh_ctx* c, const zkh_tensor* t, uint32_t O, uint32_t C, uint32_t W, const uint32_t* E,
                             DevPlanes o) {
@@ -1396,22 +1439,22 @@ static int partial_me_queue(zkh_ctx* c, const zkh_tensor* t, uint32_t O, uint32_
     launch_partial_me(c->stream, kind, src, cap, t->n, O, C, W, E, o, work);
     return 0;
 }
-// FrTensor::partial_me(u, cur_dim, window)'s checks and its work, queued: the result is ready
-// for later work on the stream
-static int partial_me_impl(zkh_ctx* c, const zkh_tensor* t, const std::vector<Fr>& u,
-                           uint32_t cur_dim, uint32_t window, zkh_tensor** out) {
-    uint32_t k = (uint32_t)u.size();
-    // (fr-tensor.cu:554-560)
+// FrTensor::partial_me(u, cur_dim, window)'s checks (fr-tensor.cu:554-560), for |u| = k
+static int partial_me_check(zkh_ctx* c, const zkh_tensor* t, uint32_t k, uint32_t cur_dim, uint32_t window) {
     if (k >= 32 || cur_dim <= ((1u << k) >> 1) || cur_dim > (1u << k))
         return fail(c, ZKH_EARG, "partial_me: incompatible dimensions");
     if (!window || t->n % ((uint64_t)cur_dim * window) != 0)
         return fail(c, ZKH_EARG, "t.size %% (cur_dim * window) != 0");
-    uint32_t O = t->n / (cur_dim * window);
-    int rc = 0;
-    uint32_t* E;
-    if ((rc = eq_table_mont(c, u, cur_dim, SL_EB, &E))) return rc;
+    return 0;
+}
+// and its work with the eq table at hand, queued: the result is ready for later work on the
+// stream
+static int partial_me_bind(zkh_ctx* c, const zkh_tensor* t, const uint32_t* E, uint32_t cur_dim, uint32_t window,
+                           zkh_tensor** out) {
+    const uint32_t O = t->n / (cur_dim * window);
     zkh_tensor* o;
-    if ((rc = tensor_alloc(c, ZKH_KIND_FR, O * window, &o))) return rc;
+    int rc = tensor_alloc(c, ZKH_KIND_FR, O * window, &o);
+    if (rc) return rc;
     if ((rc = partial_me_queue(c, t, O, cur_dim, window, E, o->planes()))) {
         zkh_tensor_free(o);
         return rc;
@@ -1435,24 +1478,28 @@ extern "C" int zkh_partial_me(zkh_ctx* c, const zkh_tensor* t, const uint32_t* u
     if (!c || !t || !out || (!u && k)) return fail(c, ZKH_EARG, "null argument");
     if (!all_canonical(u, k)) return fail(c, ZKH_EARG, "non-canonical challenge");
     HIPCHK(c, hipSetDevice(c->device));
+    int rc;
+    uint32_t* E;
     zkh_tensor* o;
-    const int rc = partial_me_impl(c, t, load_frs(u, k), cur_dim, window, &o);
-    return rc ? rc : finish_tensor(c, o, out);
+    if ((rc = partial_me_check(c, t, k, cur_dim, window)) || (rc = eq_table_mont(c, load_frs(u, k), cur_dim, SL_EB, &E)) ||
+        (rc = partial_me_bind(c, t, E, cur_dim, window, &o)))
+        return rc;
+    return finish_tensor(c, o, out);
 }
-// FrTensor::multi_dim_me's value left on the device (one-entry tensor, queued): the dimensions
-// bound last first (fr-tensor.cu:643-652)
-static int multi_dim_me_queue(zkh_ctx* c, const zkh_tensor* t, const std::vector<Fr>* uv, const uint32_t* shape,
-                              uint32_t ndim, zkh_tensor** out) {
+// FrTensor::multi_dim_me's value left on the device (one-entry tensor, queued) with the
+// dimensions' eq tables at hand: the last dimension is bound first (fr-tensor.cu:643-652)
+static int multi_dim_me_queue(zkh_ctx* c, const zkh_tensor* t, const EqWant* const* tab, uint32_t ndim,
+                              zkh_tensor** out) {
     const zkh_tensor* cur = t;
     zkh_tensor* owned = nullptr;
     for (uint32_t d = ndim; d-- > 0;) {
-        const uint32_t k = (uint32_t)uv[d].size();
-        // the first dimension takes all that is left (FrTensor::operator(), fr-tensor.cu:437-442)
-        const uint32_t n = d ? shape[d] : cur->n;
+        const uint32_t k = (uint32_t)tab[d]->u->size(), n = tab[d]->n;
         zkh_tensor* nxt;
-        int rc;
-        if (!d && (k >= 32 || n <= ((1u << k) / 2) || n > (1u << k))) rc = fail(c, ZKH_EARG, "Incompatible dimensions");
-        else rc = partial_me_impl(c, cur, uv[d], n, 1, &nxt);
+        int rc = 0;
+        // the first dimension takes all that is left (FrTensor::operator(), fr-tensor.cu:437-442)
+        if (!d && cur->n != n) rc = fail(c, ZKH_EARG, "Incompatible dimensions");
+        if (!rc) rc = partial_me_check(c, cur, k, n, 1);
+        if (!rc) rc = partial_me_bind(c, cur, tab[d]->E, n, 1, &nxt);
         if (owned) zkh_tensor_free(owned);  // its buffer serves later work on this stream only
         if (rc) return rc;
         cur = owned = nxt;
@@ -1488,9 +1535,26 @@ extern "C" int zkh_multi_dim_me(zkh_ctx* c, const zkh_tensor* t, const uint32_t*
         off += ks[d];
     }
     if (ndim == 1) return zkh_me(c, t, us, ks[0], out);
+    std::vector<EqWant> tab(ndim);
+    std::vector<const EqWant*> dims(ndim);
+    uint64_t inner = 1;
+    for (uint32_t d = ndim; d-- > 0;) {
+        // as the checks along the way: every dimension within its challenges, the first one
+        // whatever the others leave
+        const uint32_t k = ks[d];
+        if (d && !shape[d]) return fail(c, ZKH_EARG, "partial_me: incompatible dimensions");
+        const uint64_t n = d ? shape[d] : t->n / inner;
+        if (d && t->n % (inner * shape[d]) != 0) return fail(c, ZKH_EARG, "t.size %% (cur_dim * window) != 0");
+        if (k >= 32 || n <= ((1u << k) >> 1) || n > (1u << k)) return fail(c, ZKH_EARG, "partial_me: incompatible dimensions");
+        inner *= n;
+        tab[d] = {&uv[d], (uint32_t)n, nullptr};
+        dims[d] = &tab[d];
+    }
     zkh_tensor* v;
-    const int rc = multi_dim_me_queue(c, t, uv.data(), shape, ndim, &v);
-    return rc ? rc : read_entry(c, v, out);
+    int rc;
+    if ((rc = eq_tables_mont(c, tab.data(), ndim, SL_EB)) || (rc = multi_dim_me_queue(c, t, dims.data(), ndim, &v)))
+        return rc;
+    return read_entry(c, v, out);
 }
 extern "C" int zkh_eq_table(zkh_ctx* c, const uint32_t* u, uint32_t k, zkh_tensor** out) {
     if (!c || !out || (!u && k) || k > 30) return fail(c, ZKH_EARG, "bad arguments");
@@ -4719,86 +4783,122 @@ extern "C" int zkh_partial_me_window(zkh_ctx* c, const zkh_tensor* t, const uint
 // ---------------------------------------------------------------------------------------
 // zkip and zkip_stacked (zkfc.cu:94-246) and zkFCStacked::prove (zkfc.cu:288-307)
 // ---------------------------------------------------------------------------------------
-// one round over the [N, D] working tables: p = (c0, c1, c2) with the weights of E
-static int stk_round(zkh_ctx* c, DevPlanes a, DevPlanes b, uint32_t N, uint32_t D, uint32_t Nh,
-                     const uint32_t* E, Fr p[3]) {
-    Publish pb = make_pub(c, 1);
-    {
-        ProfScope ps(c, "stk_round", (double)N * D * 64);
-        launch_stk_round(c->stream, a, b, N, D, Nh, E, pb);
-    }
-    int rc = wait_pub(c, pb.seq);
-    if (rc) return rc;
-    pub_read(c, 0, 3, p);
-    for (int i = 0; i < 3; i++) p[i] = fix1(p[i]);
-    return 0;
-}
-// working copies of two tensors of n entries (read by the rounds, folded in place)
-static int stk_copies(zkh_ctx* c, const zkh_tensor* A, const zkh_tensor* B, DevPlanes* a, DevPlanes* b) {
+// The rounds of zkip_stacked (zkfc.cu:153-246): |uN| rounds over the N rows of [N, D] tables, row
+// n paired with row n + 2^ceil(log2 N) / 2 and weighted by eq(u_, row) of the remaining uN
+// prefix, bound to vN.back() first, then zkip's (zkfc.cu:129-151) over the D entries left,
+// bound to uD.back() first.  Every challenge is the caller's, so all rounds are queued at once;
+// stk_finish waits for their sums and runs the claims through them.
+struct StkRound {
+    uint32_t M, h;  // entries before the round, pair distance
+    Fr v;           // its challenge
+};
+struct StkRun {
+    std::vector<StkRound> r;
+    uint32_t rows = 0;  // rounds over the rows
+    uint32_t seq = 0;   // published by the last launch
+};
+static int stk_queue(zkh_ctx* c, DevPlanes a, DevPlanes b, uint32_t N, uint32_t D, const std::vector<Fr>& uN,
+                     const std::vector<Fr>& uD, const std::vector<Fr>& vN, StkRun& run) {
     int rc = 0;
-    DevPlanes sa, sb;
-    if ((rc = as_planes(c, A, SL_TMP0, &sa)) || (rc = as_planes(c, B, SL_TMP1, &sb))) return rc;
-    *a = scratch_planes(c, SL_TMP2, A->n, &rc);
-    if (rc) return rc;
-    *b = scratch_planes(c, SL_TMP3, B->n, &rc);
-    if (rc) return rc;
-    const size_t q = (size_t)A->n * 16;
-    HIPCHK(c, hipMemcpyAsync(a->lo(), sa.lo(), q, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(a->hi(), sa.hi(), q, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(b->lo(), sb.lo(), q, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(b->hi(), sb.hi(), q, hipMemcpyDeviceToDevice, c->stream));
-    return 0;
-}
-// zkip (zkfc.cu:129-151) over the working tables of n entries: |u| rounds, u.back() first
-static int zkip_rounds(zkh_ctx* c, Fr& claim, DevPlanes a, DevPlanes b, uint32_t n,
-                       const std::vector<Fr>& u, std::vector<Fr>& proof) {
-    uint32_t N = n;
-    for (size_t r = 0; r < u.size(); r++) {
-        const uint32_t Nh = (1u << ceil_log2(N)) >> 1;
-        Fr p[3];
-        int rc = stk_round(c, a, b, N, 1, Nh, nullptr, p);
+    for (uint32_t n = N, k = 0; k < uN.size(); k++) {
+        const uint32_t nh = (1u << ceil_log2(n)) >> 1;
+        run.r.push_back({n * D, nh * D, vN[vN.size() - 1 - k]});
+        n = nh;
+    }
+    run.rows = (uint32_t)run.r.size();
+    for (uint32_t n = D, k = 0; k < uD.size(); k++) {
+        const uint32_t nh = (1u << ceil_log2(n)) >> 1;
+        run.r.push_back({n, nh, uD[uD.size() - 1 - k]});
+        n = nh;
+    }
+    const uint32_t R = (uint32_t)run.r.size(), weighted = run.rows ? run.rows - 1 : 0;
+    if (!R) return 0;
+    static_assert(64 * 24 <= ZKH_MAX_BATCH * 11 * 8, "the sums of all rounds fit the published sums");
+    // the round's weights: the eq table over the uN prefix that stays
+    auto weights = [&](uint32_t r, uint32_t** E) {
+        *E = nullptr;
+        if (r >= weighted) return 0;
+        return eq_table_mont(c, std::vector<Fr>(uN.begin(), uN.end() - 1 - r), run.r[r].h / D, SL_EB, E);
+    };
+    DevPlanes oa = a, ob = b;  // the folded tables: scratch, in place from the second fold on
+    if (R > 1 && run.r[0].M > ZKH_STK_TAIL) {
+        oa = scratch_planes(c, SL_TMP2, run.r[0].h, &rc);
         if (rc) return rc;
-        proof.insert(proof.end(), p, p + 3);
-        // claim != p(0) + p(1) (zkfc.cu:145)
-        if (!fr_eq(claim, fr_add(p[0], fr_add(p[0], fr_add(p[1], p[2])))))
-            return fail(c, ZKH_EROUND, "zkip: claim != p(0) + p(1) at round %zu", r);
-        const Fr x = u[u.size() - 1 - r];
-        claim = fr_poly_eval(p, 2, x);
-        uint32_t xm[8];
-        fr_store(fr_to_mont(x), xm);
-        launch_stk_fold(c->stream, a, b, N, 1, Nh, xm);
-        N = Nh;
+        ob = scratch_planes(c, SL_TMP3, run.r[0].h, &rc);
+        if (rc) return rc;
+    }
+    uint32_t* E;
+    uint32_t r = 0, vm[8];
+    for (; r < R && run.r[r].M > ZKH_STK_TAIL; r++) {
+        if ((rc = weights(r, &E))) return rc;
+        if (r) fr_store(fr_to_mont(run.r[r - 1].v), vm);
+        Publish pb = make_pub(c, 1);
+        pb.host_out = c->pub_host + 24 * r;
+        run.seq = pb.seq;
+        ProfScope ps(c, "stk_round", (double)run.r[r].M * (r ? 192 : 64));
+        launch_stk_step(c->stream, a, b, oa, ob, r ? run.r[r - 1].M : 0, r ? vm : nullptr, run.r[r].M, run.r[r].h, D, E,
+                        pb);
+        if (r) a = oa, b = ob;
+    }
+    if (r < R) {
+        StkTail T{};
+        T.M = run.r[r].M;
+        T.D = D;
+        T.rounds = R - r;
+        if (T.rounds > 16) return fail(c, ZKH_EARG, "zkip: more rounds than variables");
+        T.weighted = weighted > r ? weighted - r : 0;
+        for (uint32_t k = 0; k < T.rounds; k++) {
+            T.h[k] = run.r[r + k].h;
+            fr_store(fr_to_mont(run.r[r + k].v), T.v[k]);
+        }
+        if ((rc = weights(r, &E))) return rc;
+        if (r) fr_store(fr_to_mont(run.r[r - 1].v), vm);
+        const Publish pb = make_pub(c, 1);
+        run.seq = pb.seq;
+        ProfScope ps(c, "stk_tail", (double)T.M * 64);
+        launch_stk_tail(c->stream, a, b, r ? run.r[r - 1].M : 0, r ? vm : nullptr, T, E, c->pub_host + 24 * r,
+                        pb.host_flag, pb.seq);
     }
     return 0;
 }
-// zkip_stacked (zkfc.cu:230-246): |uN| rounds over the N rows of [N, D] tables, each
-// weighted by eq(u_, row) of the remaining uN prefix, then zkip over D with uD
-static int zkip_stacked_rounds(zkh_ctx* c, Fr& claim, DevPlanes a, DevPlanes b, uint32_t N, uint32_t D,
-                               const std::vector<Fr>& uN, const std::vector<Fr>& uD,
-                               const std::vector<Fr>& vN, std::vector<Fr>& proof) {
-    int rc = 0;
-    std::vector<Fr> u_ = uN;
-    for (size_t r = 0; r < uN.size(); r++) {
-        const uint32_t Nh = (1u << ceil_log2(N)) >> 1;
-        const Fr ul = u_.back();
-        u_.pop_back();
-        uint32_t* E = nullptr;
-        if (!u_.empty() && (rc = eq_table_mont(c, u_, Nh, SL_EB, &E))) return rc;
-        Fr p[3];
-        if ((rc = stk_round(c, a, b, N, D, Nh, E, p))) return rc;
+// the rounds' claims (ZKH_EROUND at the first that does not follow), after their sums arrived
+static int stk_finish(zkh_ctx* c, const StkRun& run, const std::vector<Fr>& uN, Fr& claim, std::vector<Fr>& proof) {
+    for (uint32_t r = 0; r < run.r.size(); r++) {
+        Fr s[3], p[3];
+        for (int i = 0; i < 3; i++) s[i] = fix1(fr_load(c->pub_host + 24 * r + 8 * i));
+        p[0] = s[0];
+        p[1] = fr_sub(fr_sub(s[1], s[0]), s[2]);
+        p[2] = s[2];
         proof.insert(proof.end(), p, p + 3);
-        // q = eq(u_last, X) * p: claim != q(0) + q(1) (zkfc.cu:236-237)
-        const Fr p1 = fr_add(p[0], fr_add(p[1], p[2]));
-        if (!fr_eq(claim, fr_add(fr_mul(fr_sub(kOne, ul), p[0]), fr_mul(ul, p1))))
-            return fail(c, ZKH_EROUND, "zkip_stacked: claim != q(0) + q(1) at round %zu", r);
-        const Fr v = vN[vN.size() - 1 - r];
-        claim = fr_poly_eval(p, 2, v);
-        uint32_t vm[8];
-        fr_store(fr_to_mont(v), vm);
-        launch_stk_fold(c->stream, a, b, N, D, Nh, vm);
-        N = Nh;
+        if (r < run.rows) {  // q = eq(u_last, X) * p: claim != q(0) + q(1) (zkfc.cu:236-237)
+            const Fr ul = uN[uN.size() - 1 - r];
+            if (!fr_eq(claim, fr_add(fr_mul(fr_sub(kOne, ul), p[0]), fr_mul(ul, s[1]))))
+                return fail(c, ZKH_EROUND, "zkip_stacked: claim != q(0) + q(1) at round %u", r);
+        } else if (!fr_eq(claim, fr_add(p[0], s[1]))) {  // claim != p(0) + p(1) (zkfc.cu:145)
+            return fail(c, ZKH_EROUND, "zkip: claim != p(0) + p(1) at round %u", r - run.rows);
+        }
+        claim = fr_poly_eval(p, 2, run.r[r].v);
     }
-    return zkip_rounds(c, claim, a, b, D, uD, proof);
+    return 0;
+}
+// both, over two tensors of N x D entries: the proof so far goes out with an error too
+static int stk_prove(zkh_ctx* c, const uint32_t claim_l[8], const zkh_tensor* A, const zkh_tensor* B, uint32_t N,
+                     uint32_t D, const std::vector<Fr>& uN, const std::vector<Fr>& uD, const std::vector<Fr>& vN,
+                     uint32_t* proof_out, uint32_t final_out[8]) {
+    int rc;
+    DevPlanes a, b;
+    if ((rc = as_planes(c, A, SL_TMP0, &a)) || (rc = as_planes(c, B, SL_TMP1, &b))) return rc;
+    StkRun run;
+    if ((rc = stk_queue(c, a, b, N, D, uN, uD, vN, run))) return rc;
+    HIPCHK(c, hipGetLastError());
+    if (!run.r.empty() && (rc = wait_pub(c, run.seq))) return rc;
+    Fr claim = fr_load(claim_l);
+    std::vector<Fr> proof;
+    rc = stk_finish(c, run, uN, claim, proof);
+    if (proof_out)
+        for (size_t i = 0; i < proof.size(); i++) fr_store(proof[i], proof_out + 8 * i);
+    if (!rc) fr_store(claim, final_out);
+    return rc;
 }
 extern "C" int zkh_zkip(zkh_ctx* c, const uint32_t claim_l[8], const zkh_tensor* A, const zkh_tensor* B,
                         const uint32_t* u, uint32_t k, uint32_t* proof_out, uint32_t final_out[8]) {
@@ -4807,18 +4907,7 @@ extern "C" int zkh_zkip(zkh_ctx* c, const uint32_t claim_l[8], const zkh_tensor*
     if (!A->n || k > ceil_log2(A->n)) return fail(c, ZKH_EARG, "zkip: more challenges than variables");
     if (!fr_is_canonical(claim_l) || !all_canonical(u, k)) return fail(c, ZKH_EARG, "non-canonical input");
     HIPCHK(c, hipSetDevice(c->device));
-    DevPlanes a, b;
-    int rc = stk_copies(c, A, B, &a, &b);
-    if (rc) return rc;
-    Fr claim = fr_load(claim_l);
-    std::vector<Fr> proof;
-    rc = zkip_rounds(c, claim, a, b, A->n, load_frs(u, k), proof);
-    if (proof_out)
-        for (size_t i = 0; i < proof.size(); i++) fr_store(proof[i], proof_out + 8 * i);
-    if (rc) return rc;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    fr_store(claim, final_out);
-    return ZKH_OK;
+    return stk_prove(c, claim_l, A, B, 1, A->n, {}, load_frs(u, k), {}, proof_out, final_out);
 }
 static int stacked_args(zkh_ctx* c, const zkh_tensor* A, const zkh_tensor* B, uint32_t N, uint32_t D,
                         uint32_t kN, uint32_t kD) {
@@ -4839,35 +4928,7 @@ extern "C" int zkh_zkip_stacked(zkh_ctx* c, const uint32_t claim_l[8], const zkh
     if (!fr_is_canonical(claim_l) || !all_canonical(uN, kN) || !all_canonical(vN, kN) || !all_canonical(uD, kD))
         return fail(c, ZKH_EARG, "non-canonical input");
     HIPCHK(c, hipSetDevice(c->device));
-    DevPlanes a, b;
-    if ((rc = stk_copies(c, A, B, &a, &b))) return rc;
-    Fr claim = fr_load(claim_l);
-    std::vector<Fr> proof;
-    rc = zkip_stacked_rounds(c, claim, a, b, N, D, load_frs(uN, kN), load_frs(uD, kD), load_frs(vN, kN), proof);
-    if (proof_out)
-        for (size_t i = 0; i < proof.size(); i++) fr_store(proof[i], proof_out + 8 * i);
-    if (rc) return rc;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    fr_store(claim, final_out);
-    return ZKH_OK;
-}
-static int mdm(zkh_ctx* c, const zkh_tensor* t, std::initializer_list<const std::vector<Fr>*> us,
-               std::initializer_list<uint32_t> shape, Fr* out) {
-    std::vector<uint32_t> cat, ks;
-    for (auto* u : us) {
-        ks.push_back((uint32_t)u->size());
-        for (const Fr& x : *u) {
-            uint32_t l[8];
-            fr_store(x, l);
-            cat.insert(cat.end(), l, l + 8);
-        }
-    }
-    cat.resize(cat.size() + 8);
-    std::vector<uint32_t> shp(shape);
-    uint32_t o[8];
-    int rc = zkh_multi_dim_me(c, t, cat.data(), ks.data(), shp.data(), (uint32_t)shp.size(), o);
-    if (!rc) *out = fr_load(o);
-    return rc;
+    return stk_prove(c, claim_l, A, B, N, D, load_frs(uN, kN), load_frs(uD, kD), load_frs(vN, kN), proof_out, final_out);
 }
 extern "C" int zkh_fc_stacked_prove(zkh_ctx* c, const zkh_tensor* X, const zkh_tensor* W,
                                     const zkh_tensor* Y, const zkh_tensor* bias, uint32_t num,
@@ -4891,41 +4952,58 @@ extern "C" int zkh_fc_stacked_prove(zkh_ctx* c, const zkh_tensor* X, const zkh_t
     HIPCHK(c, hipSetDevice(c->device));
     const std::vector<Fr> un = load_frs(u_num, kn), vn = load_frs(v_num, kn), ub = load_frs(u_batch, kb),
                           ui = load_frs(u_input, ki), uo = load_frs(u_output, ko);
-    int rc = 0;
+    // Everything is queued before the first wait; one-entry values are read at the end.
     // claim = Y(u_num, u_batch, u_output) - ones_B(u_batch) * b(u_num, u_output) (zkfc.cu:292-302)
-    Fr claim;
-    if ((rc = mdm(c, Y, {&un, &ub, &uo}, {num, B, OUT}, &claim))) return rc;
-    if (bias) {
-        Fr bb;
-        if ((rc = mdm(c, bias, {&un, &uo}, {num, OUT}, &bb))) return rc;
-        claim = fr_sub(claim, fr_mul(eq_prefix_sum(ub, B), bb));
-    }
     // X_reduced = X.partial_me(u_batch, B, IN), W_reduced = W.partial_me(u_output, OUT, 1)
-    zkh_tensor *Xr = nullptr, *Wr = nullptr;
-    if ((rc = partial_me_impl(c, X, ub, B, IN, &Xr))) return rc;
-    if ((rc = partial_me_impl(c, W, uo, OUT, 1, &Wr))) {
-        zkh_tensor_free(Xr);
-        return rc;
-    }
+    // opening = X(v_num, u_batch, u_input) * W(v_num, u_input, u_output) (zkfc.cu:305-306), the
+    // second from W_reduced (u_output is bound first)
+    enum { tY, tB, tXr, tWr, tX, tW, tCount };
+    struct Owned {
+        zkh_tensor* t[tCount] = {};
+        ~Owned() {
+            for (zkh_tensor* x : t)
+                if (x) zkh_tensor_free(x);
+        }
+    } o;
+    auto mdm = [&](const zkh_tensor* t, std::initializer_list<const EqWant*> dims, int to) {
+        return multi_dim_me_queue(c, t, dims.begin(), (uint32_t)dims.size(), &o.t[to]);
+    };
+    enum { eN, eV, eB, eI, eO, eCount };
+    EqWant e[eCount] = {{&un, num, nullptr}, {&vn, num, nullptr}, {&ub, B, nullptr}, {&ui, IN, nullptr}, {&uo, OUT, nullptr}};
+    int rc = 0;
+    StkRun run;
     DevPlanes a, b;
+    // (SL_EO: the rounds' own weights use SL_EB)
+    if ((rc = eq_tables_mont(c, e, eCount, SL_EO))) return rc;
+    if ((rc = mdm(Y, {&e[eN], &e[eB], &e[eO]}, tY))) return rc;
+    if (bias && (rc = mdm(bias, {&e[eN], &e[eO]}, tB))) return rc;
+    if ((rc = partial_me_check(c, X, kb, B, IN)) || (rc = partial_me_bind(c, X, e[eB].E, B, IN, &o.t[tXr])) ||
+        (rc = partial_me_check(c, W, ko, OUT, 1)) || (rc = partial_me_bind(c, W, e[eO].E, OUT, 1, &o.t[tWr])))
+        return rc;
+    if ((rc = stacked_args(c, o.t[tXr], o.t[tWr], num, IN, kn, ki))) return rc;
+    if ((rc = as_planes(c, o.t[tXr], SL_TMP0, &a)) || (rc = as_planes(c, o.t[tWr], SL_TMP1, &b))) return rc;
+    if ((rc = stk_queue(c, a, b, num, IN, un, ui, vn, run))) return rc;
+    if ((rc = mdm(X, {&e[eV], &e[eB], &e[eI]}, tX)) || (rc = mdm(o.t[tWr], {&e[eV], &e[eI]}, tW))) return rc;
+    EntryPtrs ep{};
+    const int vals[4] = {tY, tX, tW, tB};
+    for (int i = 0; i < (bias ? 4 : 3); i++) ep.p[i] = (const uint32_t*)o.t[vals[i]]->d;
+    static_assert(64 * 24 + 32 <= ZKH_MAX_BATCH * 11 * 8, "rounds and values fit the published sums");
+    const uint32_t* ev = c->pub_host + 64 * 24;
+    launch_entries(c->stream, ep, bias ? 4 : 3, c->pub_host + 64 * 24);
+    HIPCHK(c, hipGetLastError());
+    if ((rc = settle(c))) return rc;
+    Fr claim = fr_load(ev);
+    if (bias) claim = fr_sub(claim, fr_mul(eq_prefix_sum(ub, B), fr_load(ev + 24)));
+    const Fr opening = fr_mul(fr_load(ev + 8), fr_load(ev + 16));
     Fr cur = claim;
     std::vector<Fr> proof;
-    rc = stacked_args(c, Xr, Wr, num, IN, kn, ki);
-    if (!rc) rc = stk_copies(c, Xr, Wr, &a, &b);
-    if (!rc) rc = zkip_stacked_rounds(c, cur, a, b, num, IN, un, ui, vn, proof);
-    if (!rc) rc = hipStreamSynchronize(c->stream) == hipSuccess ? 0 : fail(c, ZKH_EDEV, "zkip_stacked sync");
-    zkh_tensor_free(Xr);
-    zkh_tensor_free(Wr);
+    rc = stk_finish(c, run, un, cur, proof);
     if (proof_out)
         for (size_t i = 0; i < proof.size(); i++) fr_store(proof[i], proof_out + 8 * i);
     if (rc) return rc;
-    // opening = X(v_num, u_batch, u_input) * W(v_num, u_input, u_output) (zkfc.cu:305-306)
-    Fr ox, ow;
-    if ((rc = mdm(c, X, {&vn, &ub, &ui}, {num, B, IN}, &ox))) return rc;
-    if ((rc = mdm(c, W, {&vn, &ui, &uo}, {num, IN, OUT}, &ow))) return rc;
     fr_store(claim, claims_out);
     fr_store(cur, claims_out + 8);
-    if (!fr_eq(cur, fr_mul(ox, ow))) return fail(c, ZKH_EROUND, "final claim != opening");
+    if (!fr_eq(cur, opening)) return fail(c, ZKH_EROUND, "final claim != opening");
     return ZKH_OK;
 }
 
