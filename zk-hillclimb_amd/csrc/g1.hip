@@ -437,19 +437,23 @@ struct SetBits {
 __device__ __forceinline__ g1r_t g1r_tab_mul(const uint32_t* tab, const uint32_t s[8], const fpr_k& c) {
     g1r_t acc = g1r_zero(c);
     SetBits bits(s);
-    // two points are loaded ahead of the addition (past the last bit: entry 0)
+    // two points are loaded ahead of the addition, each into its own registers (moving one to
+    // the other's would wait for it); past the last bit: entry 0
     int b0 = bits.next(s), b1 = b0 < 0 ? -1 : bits.next(s);
     auto fetch = [&](int b) { return g1r_fetch(tab + G1R_WORDS * (b < 0 ? 0 : b), c); };
     g1r_raw p0 = fetch(b0), p1 = fetch(b1);
-    while (b0 >= 0) {
-        const g1r_raw p = p0;
-        p0 = p1;
-        b0 = b1;
-        if (b1 >= 0) b1 = bits.next(s);
+    for (;;) {
+        if (b0 < 0) return acc;
+        g1r_t p = g1r_take(p0, c);
+        b0 = b1 < 0 ? -1 : bits.next(s);
+        p0 = fetch(b0);
+        acc = g1r_add(acc, p, c);
+        if (b1 < 0) return acc;
+        p = g1r_take(p1, c);
+        b1 = b0 < 0 ? -1 : bits.next(s);
         p1 = fetch(b1);
-        acc = g1r_add(acc, g1r_take(p, c), c);
+        acc = g1r_add(acc, p, c);
     }
-    return acc;
 }
 // the same on a lane quad
 __device__ __forceinline__ g28_t g28q_tab_mul(const uint32_t* tab, const uint32_t s[8], int q, bool& inf) {
