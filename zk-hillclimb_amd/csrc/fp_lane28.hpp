@@ -239,16 +239,20 @@ FDEV void g28_add(g28_t& a, bool& inf, const g28_t& b, const f28_t& zz2, const f
 }
 
 // ---- a point on a lane quad: the four lanes hold the same point and share each operation, one
-// product per lane and level (three levels a doubling, five an addition, fp_row.hpp's
+// product per lane and level (three levels a doubling, four an addition, fp_row.hpp's
 // schedules), results moving by DPP quad permutations.  Between the row form (a wave per point)
 // and the lane form in latency and in work: on an idle SIMD a doubling takes 3.5 us and an
 // addition 6.5, for sixteen points at once.
+// (the empty asm keeps the permutation a move of its own: folded into a reversed subtraction,
+// v_subrev_u32_dpp, the lane's own value was read instead of the permuted one)
 template <int P0, int P1, int P2, int P3>
 FDEV f28_t f28_perm(const f28_t& x) {
     f28_t r;
 #pragma unroll
-    for (int i = 0; i < 14; i++)
+    for (int i = 0; i < 14; i++) {
         r.v[i] = __builtin_amdgcn_update_dpp(0, x.v[i], P0 | P1 << 2 | P2 << 4 | P3 << 6, 0xf, 0xf, true);
+        asm("" : "+v"(r.v[i]));
+    }
     return r;
 }
 template <int K>
@@ -261,19 +265,24 @@ FDEV f28_t f28_sel(bool c, const f28_t& a, const f28_t& b) {
     for (int i = 0; i < 14; i++) r.v[i] = c ? a.v[i] : b.v[i];
     return r;
 }
-// q: the lane in its quad; a not at infinity
-FDEV g28_t g28q_dbl(const g28_t& a, int q) {
-    // X X, Y Y, Y Z, Y Z
-    f28_t t = f28_mul(f28_sel(q == 0, a.x, a.y), f28_sel(q == 0, a.x, f28_sel(q == 1, a.y, a.z)));
+FDEV f28_t f28_sel4(int q, const f28_t& a, const f28_t& b, const f28_t& c, const f28_t& d) {
+    return f28_sel(q == 0, a, f28_sel(q == 1, b, f28_sel(q == 2, c, d)));
+}
+// q: the lane in its quad; a not at infinity.  zz, zzz: lane 3's are a's Z^2 and Z^3
+FDEV g28_t g28q_dbl(const g28_t& a, int q, f28_t& zz, f28_t& zzz) {
+    // X X, Y Y, Y Z, Z Z
+    f28_t t = f28_mul(f28_sel4(q, a.x, a.y, a.y, a.z), f28_sel4(q, a.x, a.y, a.z, a.z));
     const f28_t A = f28_quad<0>(t), B = f28_quad<1>(t);
     g28_t o;
     o.z = f28_twice(f28_quad<2>(t));
+    zz = t;
     f28_t E, u;
 #pragma unroll
     for (int i = 0; i < 14; i++) E.v[i] = 3 * A.v[i];
     E = f28_carry(E);
-    // B B, X B, E E, E E
-    t = f28_mul(f28_sel(q == 0, B, f28_sel(q == 1, a.x, E)), f28_sel(q < 2, B, E));
+    // B B, X B, E E, Z^2 Z
+    t = f28_mul(f28_sel4(q, B, a.x, E, t), f28_sel4(q, B, B, E, a.z));
+    zzz = t;
     const f28_t C = f28_quad<0>(t), XB = f28_quad<1>(t), F = f28_quad<2>(t);
 #pragma unroll
     for (int i = 0; i < 14; i++) u.v[i] = F.v[i] - 8 * XB.v[i];
@@ -286,45 +295,44 @@ FDEV g28_t g28q_dbl(const g28_t& a, int q) {
     o.y = f28_carry(u);
     return o;
 }
-// a += b (b not at infinity); inf: a's flag
-FDEV void g28q_add(g28_t& a, bool& inf, const g28_t& b, int q) {
+// a += b (b not at infinity) in g1z_add's four levels; inf: a's flag.  next() is called once b
+// has been read (its registers are free for what is loaded ahead)
+template <typename Next>
+FDEV void g28q_add(g28_t& a, bool& inf, const g28_t& b, const f28_t& zz2, const f28_t& zzz2, int q, Next next) {
     if (inf) {
         a = b;
         inf = false;
+        next();
         return;
     }
-    const bool odd = q & 1, low = q < 2;
-    // Z2^2, Z1^2, Y1 Z2, Y2 Z1
-    f28_t t = f28_mul(f28_sel(low, f28_sel(odd, a.z, b.z), f28_sel(odd, b.y, a.y)), f28_sel(odd, a.z, b.z));
-    // U1 = X1 Z2Z2, U2 = X2 Z1Z1, S1 = Y1 Z2 Z2Z2, S2 = Y2 Z1 Z1Z1
-    t = f28_mul(f28_sel(low, f28_sel(odd, b.x, a.x), t), f28_perm<0, 1, 0, 1>(t));
-    const f28_t ev = f28_perm<0, 0, 2, 2>(t);                // U1, U1, S1, S1
-    const f28_t d = f28_sub(f28_perm<1, 1, 3, 3>(t), ev);  // H, H, S2 - S1, S2 - S1
-    bool hz = false;
-    int m = f28_maybe_zero(d);  // of any lane of the quad
-    m |= __builtin_amdgcn_update_dpp(0, m, 0xb1, 0xf, 0xf, true);
-    m |= __builtin_amdgcn_update_dpp(0, m, 0x4e, 0xf, 0xf, true);
-    if (m) {
-        const int z = f28_zero(d);
-        hz = __builtin_amdgcn_update_dpp(0, z, 0x00, 0xf, 0xf, true) != 0;
-        const bool rz = __builtin_amdgcn_update_dpp(0, z, 0xaa, 0xf, 0xf, true) != 0;
-        if (hz && rz) {
-            inf = f28_zero(a.y);  // Z3 = 2 Y Z
-            a = g28q_dbl(a, q);
-            return;
-        }
+    // Z1^2, S1 = Y1 Z2^3, Y2 Z1, Z1 Z2
+    f28_t t = f28_mul(f28_sel4(q, a.z, a.y, b.y, a.z), f28_sel4(q, a.z, zzz2, a.z, b.z));
+    const f28_t S1 = f28_quad<1>(t), ZZ = f28_quad<3>(t);
+    // U2 = X2 Z1^2, U1 = X1 Z2^2, S2 = Y2 Z1 Z1^2
+    t = f28_mul(f28_sel(q == 0, b.x, f28_sel(q == 1, a.x, t)), f28_sel(q == 1, zz2, f28_quad<0>(t)));
+    next();
+    const f28_t U1 = f28_quad<1>(t);
+    const f28_t H = f28_sub(f28_quad<0>(t), U1), R = f28_sub(f28_quad<2>(t), S1);
+    const bool hz = f28_zero(H);
+    if (hz && f28_zero(R)) {
+        f28_t zz, zzz;
+        inf = f28_zero(a.y);  // Z3 = 2 Y Z
+        a = g28q_dbl(a, q, zz, zzz);
+        return;
     }
-    const f28_t H = f28_quad<0>(d), d2 = f28_twice(d);
-    // I = (2 H)^2, Z1 Z2, r^2, r^2
-    t = f28_mul(f28_sel(q == 1, a.z, d2), f28_sel(q == 1, b.z, d2));
-    const f28_t rr = f28_quad<2>(t);
-    // J = H I, V = U1 I, Z1 Z2 H, Z1 Z2 H
-    t = f28_mul(f28_sel(q == 1, ev, H), f28_perm<0, 0, 1, 1>(t));
-    const f28_t J = f28_quad<0>(t), V = f28_quad<1>(t);
-    a.z = f28_twice(f28_quad<2>(t));
-    a.x = f28_carry(f28_sub(f28_sub(rr, J), f28_twice(V)));
-    // r (V - X3) twice, S1 J twice
-    t = f28_mul(f28_sel(low, f28_quad<2>(d2), ev), f28_sel(low, f28_sub(V, a.x), J));
-    a.y = f28_carry(f28_sub(f28_quad<0>(t), f28_twice(f28_quad<2>(t))));
     inf = hz;
+    f28_t u;
+#pragma unroll
+    for (int i = 0; i < 14; i++) u.v[i] = 3 * U1.v[i] + H.v[i];
+    // H H, R (3 U1 + H), R R, S1 H: limbs 1 x 4 at most
+    t = f28_mul(f28_sel(q == 1 || q == 2, R, H), f28_sel4(q, H, u, R, S1));
+    const f28_t HH2 = f28_twice(f28_quad<0>(t)), RR2 = f28_twice(f28_quad<2>(t));
+    const f28_t P2 = f28_twice(f28_sub(f28_quad<1>(t), f28_quad<3>(t)));
+#pragma unroll
+    for (int i = 0; i < 14; i++) u.v[i] = H.v[i] + 2 * U1.v[i];
+    // (H + 2 U1) 2 HH, Z1 Z2 2 H, 2 P 2 HH, 2 R 2 RR: limbs 3 x 2 at most
+    t = f28_mul(f28_sel4(q, u, ZZ, P2, f28_twice(R)), f28_sel(q == 1, f28_twice(H), f28_sel(q == 3, RR2, HH2)));
+    a.x = f28_carry(f28_twice(f28_sub(RR2, f28_quad<0>(t))));
+    a.z = f28_quad<1>(t);
+    a.y = f28_carry(f28_twice(f28_sub(f28_quad<2>(t), f28_quad<3>(t))));
 }

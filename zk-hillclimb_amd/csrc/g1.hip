@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256) void k_pip_gens(const uint32_t* __restrict__ g
     if (i >= n) return;
     const fpr_k c = fpr_consts();
     const g1r_t g = g1r_load(gens + 36 * (size_t)i, c);
-    uint32_t* o = tab + PIP_GEN_WORDS * (size_t)i;
+    uint32_t* o = tab + G1Z_WORDS * (size_t)i;
     g1r_put(o, g, c);
     const uint32_t zz = fpr_mul(g.z, g.z, c), zzz = fpr_mul(zz, g.z, c);
     if (c.row < 2) o[G1R_WORDS + 16 * c.row + c.lane] = c.row ? zzz : zz;
@@ -293,18 +293,18 @@ __global__ __launch_bounds__(64, 2) void k_pip_bucket(const uint32_t* __restrict
                 uint32_t len;
                 const uint16_t* L = pip_list(item, lists, offs, n, len);
                 const uint32_t last = len - 1;
-                auto fetch = [&](uint32_t i) { return g1r_fetch(tab + PIP_GEN_WORDS * (size_t)i, c); };
+                auto fetch = [&](uint32_t i) { return g1z_fetch(tab + G1Z_WORDS * (size_t)i, c); };
                 auto index = [&](uint32_t k) { return (uint32_t)L[k < last ? k : last]; };
-                g1r_t acc = g1r_take(fetch(L[0]), c);
+                g1r_t acc = g1z_take(fetch(L[0]), c).p;
                 // the next generator is loaded one addition ahead, its index two (past the end:
                 // the last one again)
-                g1r_raw nxt = fetch(index(1));
+                g1z_raw nxt = fetch(index(1));
                 uint32_t idx = index(2);
                 for (uint32_t k = 1; k < len; k++) {
-                    const g1r_raw g = nxt;
+                    const g1z_raw g = nxt;
                     nxt = fetch(idx);
                     idx = index(k + 2);
-                    acc = g1r_add(acc, g1r_take(g, c), c);
+                    acc = g1z_add(acc, g1z_take(g, c), c);
                 }
                 g1r_put(buckets + (size_t)item * G1R_WORDS, acc, c);
             } else {
@@ -314,10 +314,10 @@ __global__ __launch_bounds__(64, 2) void k_pip_bucket(const uint32_t* __restrict
                 uint32_t len;
                 const uint16_t* L = pip_list(item, lists, offs, n, len);
                 bool inf;
-                g28_t acc = g28_load(tab + PIP_GEN_WORDS * (size_t)L[0], inf);
+                g28_t acc = g28_load(tab + G1Z_WORDS * (size_t)L[0], inf);
                 uint32_t idx = len > 1 ? L[1] : 0;
                 for (uint32_t k = 1; k < len; k++) {
-                    const uint32_t* p = tab + PIP_GEN_WORDS * (size_t)idx;
+                    const uint32_t* p = tab + G1Z_WORDS * (size_t)idx;
                     if (k + 1 < len) idx = L[k + 1];
                     bool binf;
                     const g28_t b = g28_load(p, binf);
@@ -409,7 +409,9 @@ __global__ __launch_bounds__(64) void k_pip_combine(const uint32_t* __restrict__
 // first.  The doubling chain a, 2a, 4a, ... does not depend on the scalar, so a product is a
 // doubling chain and a chain of the ones whose bit is set; the operations and their order are
 // those of the one loop, so the representative is the same.  A base's chain is kept as a table
-// (2^i a for i < 255 in row form, 48 KiB) where more than one scalar multiplies it.
+// (2^i a with its Z^2 and Z^3 for i < 255, 80 KiB) where more than one scalar multiplies it.
+// The tables of a launch's bases lie entry by entry (entry i of every base, then entry i + 1):
+// its waves run through the bits side by side, so they write and read neighbouring entries.
 #define G1_BITS 255u  // scalars are below 2^255
 __device__ __forceinline__ uint32_t limb8(const uint32_t s[8], uint32_t l) {
     return l == 0 ? s[0] : l == 1 ? s[1] : l == 2 ? s[2] : l == 3 ? s[3]
@@ -433,56 +435,81 @@ struct SetBits {
         return (int)(32 * l) + b;
     }
 };
-// one product from its base's table, one wave in row form: 1.3 us per set bit
-__device__ __forceinline__ g1r_t g1r_tab_mul(const uint32_t* tab, const uint32_t s[8], const fpr_k& c) {
+// a base's table: entry i at p + i * step
+struct G1Tab {
+    uint32_t* p;
+    size_t step;
+    __device__ __forceinline__ uint32_t* at(uint32_t i) const { return p + i * step; }
+};
+// that of the k-th of n bases
+__device__ __forceinline__ G1Tab g1_tab(uint32_t* tab, uint32_t k, uint32_t n) {
+    return {tab + (size_t)k * G1Z_WORDS, (size_t)n * G1Z_WORDS};
+}
+// one product from its base's table, one wave in row form: 1.1 us per set bit
+__device__ __forceinline__ g1r_t g1r_tab_mul(const G1Tab& tab, const uint32_t s[8], const fpr_k& c) {
     g1r_t acc = g1r_zero(c);
     SetBits bits(s);
     // two points are loaded ahead of the addition, each into its own registers (moving one to
     // the other's would wait for it); past the last bit: entry 0
     int b0 = bits.next(s), b1 = b0 < 0 ? -1 : bits.next(s);
-    auto fetch = [&](int b) { return g1r_fetch(tab + G1R_WORDS * (b < 0 ? 0 : b), c); };
-    g1r_raw p0 = fetch(b0), p1 = fetch(b1);
+    auto fetch = [&](int b) { return g1z_fetch(tab.at(b < 0 ? 0 : b), c); };
+    g1z_raw p0 = fetch(b0), p1 = fetch(b1);
     for (;;) {
         if (b0 < 0) return acc;
-        g1r_t p = g1r_take(p0, c);
+        g1z_t p = g1z_take(p0, c);
         b0 = b1 < 0 ? -1 : bits.next(s);
         p0 = fetch(b0);
-        acc = g1r_add(acc, p, c);
+        acc = g1z_add(acc, p, c);
         if (b1 < 0) return acc;
-        p = g1r_take(p1, c);
+        p = g1z_take(p1, c);
         b1 = b0 < 0 ? -1 : bits.next(s);
         p1 = fetch(b1);
-        acc = g1r_add(acc, p, c);
+        acc = g1z_add(acc, p, c);
     }
 }
 // the same on a lane quad
-__device__ __forceinline__ g28_t g28q_tab_mul(const uint32_t* tab, const uint32_t s[8], int q, bool& inf) {
+__device__ __forceinline__ g28_t g28q_tab_mul(const G1Tab& tab, const uint32_t s[8], int q, bool& inf) {
     g28_t acc = g28_zero();
     inf = true;
     SetBits bits(s);
     int b = bits.next(s);
-    // the next point is loaded one addition ahead (past the last bit: entry 0)
-    auto fetch = [&](int i) { return g28_fetch(tab + G1R_WORDS * (i < 0 ? 0 : i)); };
-    g28_raw nxt = fetch(b);
+    // the next point is loaded during the addition (past the last bit: entry 0), as soon as the
+    // addition has read its own
+    g28_raw p;
+    f28_t zz, zzz;
+    auto fetch = [&] {
+        const uint32_t* e = tab.at(b < 0 ? 0 : b);
+        p = g28_fetch(e);
+        zz = f28_load(e + G1R_WORDS);
+        zzz = f28_load(e + G1R_WORDS + 16);
+    };
+    fetch();
     while (b >= 0) {
         bool pinf;
-        const g28_t p = g28_take(nxt, pinf);
+        const g28_t x = g28_take(p, pinf);
+        const f28_t xz = zz, xzz = zzz;
         b = bits.next(s);
-        nxt = fetch(b);
-        if (!pinf) g28q_add(acc, inf, p, q);
+        if (pinf) fetch();
+        else g28q_add(acc, inf, x, xz, xzz, q, fetch);
     }
     return acc;
 }
-// a base's table on a lane quad
-__device__ __forceinline__ void g28q_table(g28_t a, bool inf, uint32_t* tab, int q) {
+// a base's table on a lane quad: lane q < 3 stores coordinate q, lane 3 Z^2 and Z^3; signed limbs
+// as they are (the tables of quads are read by quads)
+__device__ __forceinline__ void g28q_table(g28_t a, bool inf, const G1Tab& tab, int q) {
     for (uint32_t i = 0; i < G1_BITS; i++) {
-        // lane q stores coordinate q; signed limbs as they are: the tables of quads are read by quads
-        const f28_t v = f28_sel(q == 0, a.x, f28_sel(q == 1, a.y, a.z));
-        if (q < 3) f28_put(tab + G1R_WORDS * i + 16 * q, v, inf ? 1u : 0u);
-        if (!inf && i + 1 < G1_BITS) {
-            inf = f28_zero(a.y);  // Z3 = 2 Y Z
-            a = g28q_dbl(a, q);
+        f28_t zz = {}, zzz = {};
+        g28_t d = a;
+        bool dinf = inf;
+        if (!inf) {
+            dinf = f28_zero(a.y);  // Z3 = 2 Y Z
+            d = g28q_dbl(a, q, zz, zzz);
         }
+        uint32_t* e = tab.at(i);
+        f28_put(e + 16 * q, f28_sel4(q, a.x, a.y, a.z, zz), q == 0 && inf ? 1u : 0u);
+        if (q == 3) f28_put(e + 64, zzz, 0);
+        a = d;
+        inf = dinf;
     }
 }
 // One product on two waves in row form: wave 0 of the pair runs the doubling chain and hands
@@ -495,11 +522,11 @@ __device__ __forceinline__ void g28q_table(g28_t a, bool inf, uint32_t* tab, int
 // table is wanted too (all 255 doublings then), else null and the doublings after the highest
 // set bit are skipped.
 #define G1P_B 16
-typedef uint32_t g1_pipe_buf[2][G1P_B][G1R_WORDS];
+typedef uint32_t g1_pipe_buf[2][G1P_B][G1Z_WORDS];
 __device__ __forceinline__ g1r_t g1r_mul_pipe(g1r_t a, const uint32_t s[8], bool dbl, g1_pipe_buf& buf,
-                                              uint32_t* tab, const fpr_k& c) {
+                                              const G1Tab& tab, const fpr_k& c) {
     static_assert(32 % G1P_B == 0, "a chunk's bits lie in one scalar limb");
-    const int top = top_bit(s), last = tab ? (int)G1_BITS - 1 : top;
+    const int top = top_bit(s), last = tab.p ? (int)G1_BITS - 1 : top;
     g1r_t acc = g1r_zero(c);
     constexpr int NC = 256 / G1P_B;
     for (int k = 0; k <= NC; k++) {
@@ -507,18 +534,18 @@ __device__ __forceinline__ g1r_t g1r_mul_pipe(g1r_t a, const uint32_t s[8], bool
             for (int j = 0; j < G1P_B; j++) {
                 const int i = k * G1P_B + j;
                 if (i > last) break;
-                const uint32_t v = g1r_word(a, c);
-                if (c.row < 3) {
-                    buf[k & 1][j][threadIdx.x & 63] = v;
-                    if (tab) tab[G1R_WORDS * i + (threadIdx.x & 63)] = v;
-                }
-                if (i < last) a = g1r_dbl(a, c);
+                g1z_t z{a, 0, 0};
+                a = g1z_dbl(z, c);
+                const uint32_t v = g1z_word(z, c);
+                g1z_put(buf[k & 1][j], v, z, c);
+                if (tab.p) g1z_put(tab.at(i), v, z, c);
             }
         } else if (k > 0) {
             const uint32_t w = limb8(s, (uint32_t)((k - 1) * G1P_B) >> 5);
             for (int j = 0; j < G1P_B; j++) {
                 const int i = (k - 1) * G1P_B + j;
-                if (i <= top && ((w >> (i & 31)) & 1u)) acc = g1r_add(acc, g1r_get(buf[(k - 1) & 1][j], c), c);
+                if (i <= top && ((w >> (i & 31)) & 1u))
+                    acc = g1z_add(acc, g1z_take(g1z_fetch(buf[(k - 1) & 1][j], c), c), c);
             }
         }
         __syncthreads();
@@ -536,10 +563,11 @@ __global__ __launch_bounds__(64) void k_g1_tables(const uint32_t* __restrict__ b
     const uint32_t i = blockIdx.x;
     const fpr_k c = fpr_consts();
     g1r_t a = g1r_load(base + 36 * (size_t)(b0 + i), c);
-    uint32_t* t = tab + (size_t)i * G1_BITS * G1R_WORDS;
+    const G1Tab t = g1_tab(tab, i, gridDim.x);
     for (uint32_t k = 0; k < G1_BITS; k++) {
-        g1r_put(t + G1R_WORDS * k, a, c);
-        if (k + 1 < G1_BITS) a = g1r_dbl(a, c);
+        g1z_t z{a, 0, 0};
+        a = g1z_dbl(z, c);
+        g1z_put(t.at(k), g1z_word(z, c), z, c);
     }
 }
 // out[i] = base[i] * s[i], two waves per product, no table
@@ -553,7 +581,7 @@ __global__ __launch_bounds__(128) void k_g1_mul(const uint32_t* __restrict__ bas
     const uint32_t sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
     g1r_t p = g1r_zero(c);
     if (dbl) p = g1r_load(base + 36 * (size_t)i, c);
-    const g1r_t m = g1r_mul_pipe(p, sc, dbl, buf, nullptr, c);
+    const g1r_t m = g1r_mul_pipe(p, sc, dbl, buf, G1Tab{}, c);
     if (!dbl) g1r_store(out + 36 * (size_t)i, m, c);
 }
 // row forms of n points, one wave each
@@ -570,20 +598,20 @@ __global__ __launch_bounds__(64) void k_g1_tables4(const uint32_t* __restrict__ 
     if (i >= nt) return;
     bool inf;
     const g28_t a = g28_load(rows + G1R_WORDS * (size_t)i, inf);
-    g28q_table(a, inf, tab + (size_t)i * G1_BITS * G1R_WORDS, threadIdx.x & 3);
+    g28q_table(a, inf, g1_tab(tab, i, nt), threadIdx.x & 3);
 }
 // products i0 + k (k < count) of the bases at hand (base (i0 + k) % nb - b0): one wave each
-__global__ __launch_bounds__(64) void k_g1_tab_mul(const uint32_t* __restrict__ tab, uint32_t nb, uint32_t b0,
+__global__ __launch_bounds__(64) void k_g1_tab_mul(uint32_t* __restrict__ tab, uint32_t nt, uint32_t nb, uint32_t b0,
                                                    const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
                                                    uint32_t i0, uint32_t* __restrict__ out) {
     const uint32_t i = i0 + blockIdx.x;
     const fpr_k c = fpr_consts();
     const uint4 s0 = ((const uint4*)lo)[i], s1 = ((const uint4*)hi)[i];
     const uint32_t sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-    g1r_store(out + 36 * (size_t)i, g1r_tab_mul(tab + (size_t)(i % nb - b0) * G1_BITS * G1R_WORDS, sc, c), c);
+    g1r_store(out + 36 * (size_t)i, g1r_tab_mul(g1_tab(tab, i % nb - b0, nt), sc, c), c);
 }
 // one quad each, products in row form to rows[k]
-__global__ __launch_bounds__(64) void k_g1_tab_mul4(const uint32_t* __restrict__ tab, uint32_t nb, uint32_t b0,
+__global__ __launch_bounds__(64, 2) void k_g1_tab_mul4(uint32_t* __restrict__ tab, uint32_t nt, uint32_t nb, uint32_t b0,
                                                     const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
                                                     uint32_t i0, uint32_t count, uint32_t* __restrict__ rows) {
     const uint32_t k = blockIdx.x * 16 + threadIdx.x / 4, i = i0 + k;
@@ -592,7 +620,7 @@ __global__ __launch_bounds__(64) void k_g1_tab_mul4(const uint32_t* __restrict__
     const uint32_t sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
     const int q = threadIdx.x & 3;
     bool inf;
-    const g28_t r = g28q_tab_mul(tab + (size_t)(i % nb - b0) * G1_BITS * G1R_WORDS, sc, q, inf);
+    const g28_t r = g28q_tab_mul(g1_tab(tab, i % nb - b0, nt), sc, q, inf);
     if (q == 0) g28_store(rows + G1R_WORDS * (size_t)k, r, inf);
 }
 __global__ __launch_bounds__(256) void k_g1_points(const uint32_t* __restrict__ rows, uint32_t n,
@@ -613,7 +641,7 @@ __global__ __launch_bounds__(128) void k_g1_addmul(const uint32_t* __restrict__ 
     const bool dbl = __builtin_amdgcn_readfirstlane(threadIdx.x / 64) == 0;
     g1r_t p = g1r_zero(c);
     if (dbl) p = g1r_load(a + 36 * (size_t)i, c);
-    const g1r_t m = g1r_mul_pipe(p, sc.v, dbl, buf, nullptr, c);
+    const g1r_t m = g1r_mul_pipe(p, sc.v, dbl, buf, G1Tab{}, c);
     if (!dbl) g1r_store(out + 36 * (size_t)i, g1r_add(g1r_load(b + 36 * (size_t)i, c), m, c), c);
 }
 
@@ -672,10 +700,10 @@ __device__ __forceinline__ void ipa_inner(const IpaJobDev& J, uint32_t side, con
 }
 // L and R terms (vrf_common.cuh:316-319): P[j] = g[h + j] a[j], P[h + j] = g[j] a[h + j],
 // P[2h], P[2h + 1] = Q <a_lo, b_hi>, Q <a_hi, b_lo>.  The fold multiplies the same generators,
-// so their tables are kept for it: point id 2 i + hi of a job is g[i + hi h], its table at
-// D + pt0 + id.
-__device__ __forceinline__ uint32_t* ipa_table(const IpaBatchDev& B, const IpaJobDev& J, uint32_t id) {
-    return B.D + (size_t)(J.pt0 + id - B.slice0) * G1_BITS * G1R_WORDS;
+// so their tables are kept for it: point id 2 i + hi of a job is g[i + hi h], its table the
+// (pt0 + id - slice0)-th.
+__device__ __forceinline__ G1Tab ipa_table(const IpaBatchDev& B, const IpaJobDev& J, uint32_t id) {
+    return g1_tab(B.D, J.pt0 + id - B.slice0, B.slice);
 }
 // one product by waves 0 and 1 of the block (more only take its barriers): blk 0, 1 the Q products with their inner products (first,
 // since they are the longest), then P[blk - 2] with its generator's table
@@ -694,7 +722,7 @@ __device__ __forceinline__ void ipa_product(const IpaBatchDev& B, const IpaJobDe
     const uint32_t* bp = j < h ? J.g + G1R_WORDS * (size_t)(h + j) : j < 2 * h ? J.g + G1R_WORDS * (size_t)(j - h) : J.Qr;
     g1r_t base = g1r_zero(c);
     if (dbl) base = g1r_get(bp, c);
-    uint32_t* tab = blk < 2 ? nullptr : ipa_table(B, J, j < h ? 2 * j + 1 : 2 * (j - h));
+    const G1Tab tab = blk < 2 ? G1Tab{} : ipa_table(B, J, j < h ? 2 * j + 1 : 2 * (j - h));
     const g1r_t r = g1r_mul_pipe(base, sc, dbl, buf, tab, c);
     if (wave == 1) g1r_put(J.P + G1R_WORDS * (size_t)j, r, c);
 }
@@ -733,7 +761,7 @@ __global__ __launch_bounds__(256) void k_ipa_tables4(IpaBatchDev B, uint32_t nj,
     const g28_t a = g28_load(J.g + G1R_WORDS * (size_t)(id / 2 + (id & 1) * J.h), inf);
     g28q_table(a, inf, ipa_table(B, J, id), threadIdx.x & 3);
 }
-__global__ __launch_bounds__(64) void k_ipa_scale4(IpaBatchDev B, uint32_t nj, uint32_t count) {
+__global__ __launch_bounds__(64, 2) void k_ipa_scale4(IpaBatchDev B, uint32_t nj, uint32_t count) {
     const uint32_t k = blockIdx.x * 16 + threadIdx.x / 4;
     if (k >= count) return;
     const IpaJobDev& J = B.j[ipa_point(B, nj, B.slice0 + k)];
@@ -750,7 +778,7 @@ __global__ __launch_bounds__(64) void k_ipa_scale4(IpaBatchDev B, uint32_t nj, u
 // are added, as dev_msm does) and leaves their sum in the first; the block that takes the last
 // ones adds the side's Q term and writes L or R, canonical, to the host.  Sixteen waves, one
 // addition each per level; partial sums stay in LDS.
-static_assert(ZKH_ROW_WORDS == G1R_WORDS, "point size");
+static_assert(ZKH_ROW_WORDS == G1R_WORDS && ZKH_POINTZ_WORDS == G1Z_WORDS, "point sizes");
 __global__ __launch_bounds__(1024) void k_ipa_tree(IpaBatchDev B, uint32_t shift) {
     const IpaJobDev& J = B.j[blockIdx.y];
     const uint32_t h = J.h, side = blockIdx.z, m = h >> shift;
@@ -807,7 +835,7 @@ __global__ __launch_bounds__(128) void k_ipa_fold(IpaBatchDev B, uint32_t nj) {
     if (!hi) g1r_put(J.g2 + G1R_WORDS * (size_t)i, g1r_add(r, g1r_get(other, c), c), c);
 }
 // many points: the same on two quads per generator
-__global__ __launch_bounds__(64) void k_ipa_fold4(IpaBatchDev B, uint32_t nj, uint32_t count) {
+__global__ __launch_bounds__(64, 2) void k_ipa_fold4(IpaBatchDev B, uint32_t nj, uint32_t count) {
     const uint32_t k = blockIdx.x * 16 + threadIdx.x / 4;
     if (k >= count) return;  // count is even: both quads of a generator or neither
     const IpaJobDev& J = B.j[ipa_point(B, nj, B.slice0 + k)];
@@ -829,7 +857,10 @@ __global__ __launch_bounds__(64) void k_ipa_fold4(IpaBatchDev B, uint32_t nj, ui
     }
     const bool oinf = __shfl_xor((int)inf, 4) != 0;
     if (hi) return;
-    if (!oinf) g28q_add(r, inf, o, q);
+    if (!oinf) {
+        const f28_t zz = f28_sqr(o.z);
+        g28q_add(r, inf, o, zz, f28_mul(zz, o.z), q, [] {});
+    }
     if (q == 0) g28_store(J.g2 + G1R_WORDS * (size_t)i, r, inf);
 }
 void launch_ipa_points(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax) {
@@ -851,6 +882,7 @@ void launch_ipa_scale(hipStream_t s, IpaBatchDev& B, uint32_t nj, const uint32_t
         points += 2 * B.j[j].h;
     }
     B.slice0 = 0;
+    B.slice = points < ZKH_IPA_TABLES ? points : ZKH_IPA_TABLES;
     if (points < G1_QUADS) {
         hipLaunchKernelGGL(k_ipa_scale, dim3(blocks), dim3(128), lds_share(blocks, 2, sizeof(g1_pipe_buf) + 129 * 32), s,
                            B, nj, R2);
@@ -874,6 +906,7 @@ void launch_ipa_fold(hipStream_t s, IpaBatchDev& B, uint32_t nj) {
     for (uint32_t j = 0; j < nj; j++) blocks += B.j[j].h;
     const uint32_t points = 2 * blocks;
     B.slice0 = 0;
+    B.slice = points < ZKH_IPA_TABLES ? points : ZKH_IPA_TABLES;
     if (points < G1_QUADS) {
         hipLaunchKernelGGL(k_ipa_fold, dim3(blocks), dim3(128), lds_share(blocks, 2, G1R_WORDS * 4), s, B, nj);
         return;
@@ -908,7 +941,7 @@ static uint32_t g1_mul_tables(uint32_t nb, uint32_t n) {
 }
 size_t g1_mul_words(uint32_t nb, uint32_t n) {
     const uint32_t nt = g1_mul_tables(nb, n);
-    return nt ? (size_t)nt * G1_BITS * G1R_WORDS + (size_t)(n > nt ? n : nt) * G1R_WORDS : 0;
+    return nt ? (size_t)nt * G1_BITS * G1Z_WORDS + (size_t)(n > nt ? n : nt) * G1R_WORDS : 0;
 }
 void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint32_t* lo, const uint32_t* hi,
                    uint32_t n, uint32_t* out, uint32_t* work) {
@@ -917,7 +950,7 @@ void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint3
         hipLaunchKernelGGL(k_g1_mul, dim3(n), dim3(128), lds_share(n, 2, sizeof(g1_pipe_buf)), s, base, lo, hi, out);
         return;
     }
-    uint32_t* rows = work + (size_t)nt * G1_BITS * G1R_WORDS;
+    uint32_t* rows = work + (size_t)nt * G1_BITS * G1Z_WORDS;
     for (uint32_t b0 = 0; b0 < used; b0 += nt) {
         const uint32_t bases = used - b0 < nt ? used - b0 : nt;
         if (bases < G1_QUADS) {
@@ -931,9 +964,9 @@ void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint3
         for (uint64_t i0 = b0; i0 < n; i0 += nb) {
             const uint32_t count = all ? n : (uint32_t)(n - i0 < bases ? n - i0 : bases);
             if (count < G1_QUADS && bases < G1_QUADS) {  // quads leave signed limbs: read by quads
-                hipLaunchKernelGGL(k_g1_tab_mul, dim3(count), dim3(64), 0, s, work, nb, b0, lo, hi, (uint32_t)i0, out);
+                hipLaunchKernelGGL(k_g1_tab_mul, dim3(count), dim3(64), 0, s, work, bases, nb, b0, lo, hi, (uint32_t)i0, out);
             } else {
-                hipLaunchKernelGGL(k_g1_tab_mul4, dim3((count + 15) / 16), dim3(64), 0, s, work, nb, b0, lo, hi,
+                hipLaunchKernelGGL(k_g1_tab_mul4, dim3((count + 15) / 16), dim3(64), 0, s, work, bases, nb, b0, lo, hi,
                                    (uint32_t)i0, count, rows);
                 hipLaunchKernelGGL(k_g1_points, dim3((count + 3) / 4), dim3(256), 0, s, rows, count, out + 36 * i0);
             }

@@ -31,7 +31,7 @@
 void launch_pip_sort(hipStream_t s, const uint32_t* lo, const uint32_t* hi, uint32_t m, uint32_t n,
                      uint16_t* lists, uint32_t* offs);
 #define ZKH_ROW_WORDS 48       // a point in row form (fp_row.hpp)
-#define PIP_GEN_WORDS 80       // and with Z^2 and Z^3 behind it
+#define ZKH_POINTZ_WORDS 80    // and with Z^2 and Z^3 behind it
 #define PIP_BINS 288           // chain length classes
 struct PipPlan {
     uint32_t total[PIP_BINS];   // distinct chains per length class
@@ -64,12 +64,12 @@ struct IpaJobDev {
 };
 // D: the points' tables (2^i g, i < 255), of points [slice0, slice0 + ZKH_IPA_TABLES) where
 // there are more (the points of all jobs in order, ipa_table)
-#define ZKH_IPA_TABLES 32768u
-#define ZKH_TABLE_WORDS (255u * ZKH_ROW_WORDS)
+#define ZKH_IPA_TABLES 24576u
+#define ZKH_TABLE_WORDS (255u * ZKH_POINTZ_WORDS)
 struct IpaBatchDev {
     IpaJobDev j[ZKH_IPA_MAX_JOBS];
     uint32_t* D;
-    uint32_t slice0;
+    uint32_t slice0, slice;  // the first point whose table is at hand, and how many are
 };
 // g0[0, 2h] = row forms of g_in[0, 2h) and Q
 void launch_ipa_points(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax);

@@ -3934,7 +3934,7 @@ extern "C" int zkh_commit(zkh_ctx* c, const zkh_g1* gens, const zkh_tensor* t, z
         DevPlanes p;
         uint16_t *lists = nullptr, *alias = nullptr;
         uint32_t *offs = nullptr, *buckets = nullptr, *partials = nullptr, *tab = nullptr;
-        const size_t nt = (size_t)n * PIP_GEN_WORDS, np = sizeof(PipPlan) / 4, ni = (size_t)m * 1024, nw = (size_t)m * 64;
+        const size_t nt = (size_t)n * ZKH_POINTZ_WORDS, np = sizeof(PipPlan) / 4, ni = (size_t)m * 1024, nw = (size_t)m * 64;
         if (!(rc = as_planes(c, t, SL_TMP0, &p))) lists = (uint16_t*)scratch_slot(c, SL_TMP1, (size_t)m * 64 * n * 2, &rc);
         if (!rc) offs = (uint32_t*)scratch_slot(c, SL_TMP2, (size_t)m * 64 * 16 * 4, &rc);
         if (!rc) buckets = (uint32_t*)scratch_slot(c, SL_TMP3, (size_t)m * 64 * 16 * ZKH_ROW_WORDS * 4, &rc);
