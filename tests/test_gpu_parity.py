@@ -1045,6 +1045,65 @@ def test_lu_hp_per_round_launch_path(zkh, ctx, mode, monkeypatch):
         assert bytes(st_g) == bytes(st_o)
 
 
+# the entries that a persistent loop leaves to the host: all of a table (k <= 5), one message
+# before it (6, 7), both parities of the rounds before, and several blocks (from 10)
+@pytest.mark.parametrize("k", [0, 1, 2, 4, 5, 6, 7, 8, 9, 10, 11, 12])
+def test_persistent_loops_host_tail(zkh, ctx, k):
+    rng = np.random.default_rng(4100 + k)
+    n = 1 << k
+    # matmul
+    B, IN, OUT = 3, n, 2
+    X, W, Y = _mm_inputs((B, IN, OUT), 4200 + k)
+    st_g, st_o = seed_transcript(zkh, "tail:mm:%d" % k)
+    rc, want = C.mm_prove(st_o, X, W, Y, B, IN, OUT)
+    assert rc == 0
+    got = ctx.mm_prove(st_g, ctx.from_i32(X), ctx.from_i32(W), ctx.from_i64(Y), B, IN, OUT)
+    for key in ("ev", "claims", "u_batch", "u_output", "u_input"):
+        assert fr_eq(got[key], want[key]), key
+    assert bytes(st_g) == bytes(st_o)
+    # lookup: the loop from the start (D = N) and after two rounds (D = 4 N)
+    for D in (n, 4 * n):
+        low = -(n // 2)
+        vals = rng.integers(low, low + n, size=D).astype(np.int32)
+        S, T = C.ints_to_fr(vals), C.range_table(low, n, n)
+        rc, m = C.lu_prep(S, low, n)
+        assert rc == 0
+        beta, alpha = rand_fr_full(rng, 2)
+        u = rand_fr_full(rng, P.ceil_log2(D))
+        st_g, st_o = seed_transcript(zkh, "tail:lu:%d:%d" % (D, n))
+        rc, want = C.lu_prove(st_o, C.lu_inverse(S, beta), S, T, m, alpha, beta, u)
+        assert rc == 0
+        Sg = ctx.from_i32(vals)
+        got = ctx.lu_prove(st_g, ctx.lu_inverse(Sg, beta), Sg, ctx.range_table(low, n, n), ctx.from_fr(m), alpha,
+                           beta, u)
+        for key in ("ev", "term", "ws"):
+            assert fr_eq(got[key], want[key]), (D, key)
+        assert bytes(st_g) == bytes(st_o)
+    # Hadamard: explicit E (one round per message), eq form and U all ones (two)
+    u = rand_fr_full(rng, k)
+    E = C.build_eq(u)
+    Sv = rng.integers(-2**31, 2**31, size=n)
+    S, U = C.ints_to_fr(Sv), rand_fr_full(rng, n)
+    one = C.ints_to_fr(np.ones(n, np.int64))
+    for form in ("E", "eq", "ones"):
+        Uf = one if form == "ones" else U
+        claim = C.ints_to_fr([sum(a * b % P.R * c for a, b, c in
+                                  zip(C.fr_to_ints(E), C.fr_to_ints(S), C.fr_to_ints(Uf))) % P.R])[0]
+        st_g, st_o = seed_transcript(zkh, "tail:hp:%d:%s" % (k, form))
+        rc, want = C.hp_prove(st_o, claim, E, S, Uf)
+        assert rc == 0
+        if form == "ones":
+            got = ctx.hp_prove(st_g, claim, ctx.from_fr(E), ctx.from_i32(Sv.astype(np.int32)),
+                               ctx.from_i32(np.ones(n, np.int32)))
+        elif form == "eq":
+            got = ctx.hp_prove_eq(st_g, claim, u, ctx.from_fr(S), ctx.from_fr(U))
+        else:
+            got = ctx.hp_prove(st_g, claim, ctx.from_fr(E), ctx.from_fr(S), ctx.from_fr(U))
+        for key in ("ev", "term", "ws"):
+            assert fr_eq(got[key], want[key]), (form, key)
+        assert bytes(st_g) == bytes(st_o)
+
+
 def test_calib_fr_mul(zkh, ctx):
     """The multiply-rate probe runs and reports a plausible device-wide rate; zero
     iterations are refused."""

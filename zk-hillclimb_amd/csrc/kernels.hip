@@ -3237,6 +3237,24 @@ ZDEV void persist_publish(uint32_t* slot, const uint32_t* pub, uint32_t nw, uint
         st_quad_sys(slot + 4 * qd, make_uint4(seq, pub[b], b + 1 < nw ? pub[b + 1] : 0u, b + 2 < nw ? pub[b + 2] : 0u));
     }
 }
+// all threads: a block's final message, the m entries of each of its tables (planes lo[i],
+// hi[i] in LDS), table by table, as quads with seq into fin (ZKH_FIN_WORDS(tables, m) words)
+template <int NTAB>
+ZDEV void persist_final(uint32_t* fin, const uint4* const (&lo)[NTAB], const uint4* const (&hi)[NTAB], uint32_t tables,
+                        uint32_t m, uint32_t seq) {
+    const uint32_t nw = 8 * tables * m;
+    auto word = [&](uint32_t w) {
+        const uint32_t i = w / (8 * m), k = w / 8 - i * m;
+        if (w >= nw) return 0u;
+        const uint4 *l = lo[0], *h = hi[0];
+#pragma unroll
+        for (int t = 1; t < NTAB; t++)
+            if (i == (uint32_t)t) l = lo[t], h = hi[t];
+        return reinterpret_cast<const uint32_t*>((w & 4) ? h + k : l + k)[w & 3];
+    };
+    for (uint32_t qd = threadIdx.x; qd * 3 < nw; qd += blockDim.x)
+        st_quad_sys(fin + 4 * qd, make_uint4(seq, word(3 * qd), word(3 * qd + 1), word(3 * qd + 2)));
+}
 // completion flag of a stream (the host's settle): the value of *word (when given) to
 // host_word, then seq to the host flag
 __global__ void k_fence(uint32_t* flag, uint32_t seq, const uint32_t* word, uint32_t nwords, uint32_t* host_word) {
@@ -3355,6 +3373,12 @@ __global__ __launch_bounds__(NTP) void k_zkip_persist(ZkipPersist P) {
     uint64_t t_cmd = 0;
     for (uint32_t seq = 1;; seq++) {
         uint32_t nw;
+        if (m == q.me) {  // the block's folded entries
+            const uint4 *const lo[2] = {alo, blo}, *const hi[2] = {ahi, bhi};
+            if (threadIdx.x == 0) persist_stamp(slot, seq, t_cmd);
+            persist_final(q.out + ((size_t)ZKH_PSLOT << q.lgnb) + lb * ZKH_FIN_WORDS(2, m), lo, hi, 2, m, seq);
+            return;
+        }
         if (m >= 4) {
             const uint32_t q4 = m >> 2, h = m >> 1;
             // S = min(q4, 64) lanes per type and k = min(4, 64 / S) types per wave, the
@@ -3399,18 +3423,11 @@ __global__ __launch_bounds__(NTP) void k_zkip_persist(ZkipPersist P) {
 #pragma unroll
                 for (int i = 0; i < 8; i++) pubw[8 * lane + i] = red[lane].v[i];
             }
-        } else if (m == 2) {
+        } else {  // m == 2
             nw = ZKH_MSG_ONE;
             if (wv == 0 && lane < 3) {
                 const fr_t x = half_opnd(alo, ahi, lane, 0, 1), y = half_opnd(blo, bhi, lane, 0, 1);
                 const fr_t t = mont_mul_ol(x, y);
-#pragma unroll
-                for (int i = 0; i < 8; i++) pubw[8 * lane + i] = t.v[i];
-            }
-        } else {  // the block's folded entries a[0], b[0]
-            nw = ZKH_MSG_FINAL;
-            if (wv == 0 && lane < 2) {
-                const fr_t t = lane ? ld_fr(blo, bhi, 0) : ld_fr(alo, ahi, 0);
 #pragma unroll
                 for (int i = 0; i < 8; i++) pubw[8 * lane + i] = t.v[i];
             }
@@ -3420,7 +3437,6 @@ __global__ __launch_bounds__(NTP) void k_zkip_persist(ZkipPersist P) {
             if (lane == 0) persist_stamp(slot, seq, t_cmd);
             persist_publish(slot, pubw, nw, seq);
         }
-        if (m == 1) return;
         if (wv == 0) {
             uint4 qd;
             const uint32_t nq = zkh_quad_count(m >= 4 ? 32 : 8);
@@ -3534,8 +3550,14 @@ __global__ __launch_bounds__(NTP) void k_hp_persist(HpPersist P) {
     uint32_t m = ls;
     uint64_t t_cmd = 0;
     for (uint32_t seq = 1;; seq++) {
+        if (m == P.me) {  // the block's folded entries of S, U (, E)
+            const uint4 *const lo[3] = {tlo[0], tlo[1], tlo[2]}, *const hi[3] = {thi[0], thi[1], thi[2]};
+            if (threadIdx.x == 0) persist_stamp(slot, seq, t_cmd);
+            persist_final(P.out + ((size_t)ZKH_PSLOT << P.lgnb) + lb * ZKH_FIN_WORDS(ntab, m), lo, hi, ntab, m, seq);
+            return;
+        }
         uint32_t nw;
-        const bool dbl = P.two && m >= 4;
+        const bool dbl = P.two && m >= 4 * P.me;
         if (dbl) {  // two rounds: the nine point sums over the cells c < q
             const uint32_t q = m >> 2;
             uint4* xlo = rlo + (em ? 0 : hs);  // 9 rows of q after the W row (eq mode)
@@ -3558,7 +3580,7 @@ __global__ __launch_bounds__(NTP) void k_hp_persist(HpPersist P) {
                     for (int i = 0; i < 8; i++) pubw[8 * wv + i] = acc.v[i];
             }
             nw = ZKH_HP_MSG2;
-        } else if (m >= 2) {
+        } else {
             const uint32_t h = m >> 1;
             if (!em) {
                 for (uint32_t t = threadIdx.x; t < 2 * h; t += NTP) {  // level 1
@@ -3606,20 +3628,12 @@ __global__ __launch_bounds__(NTP) void k_hp_persist(HpPersist P) {
                     for (int i = 0; i < 8; i++) pubw[8 * wv + i] = acc.v[i];
             }
             nw = ZKH_HP_MSG;
-        } else {  // the block's folded entries S[0], U[0] (, E[0])
-            nw = 8 * ntab;
-            if (wv == 0 && lane < ntab) {
-                const fr_t t = ld_fr(tlo[lane], thi[lane], 0);
-#pragma unroll
-                for (int i = 0; i < 8; i++) pubw[8 * lane + i] = t.v[i];
-            }
         }
         __syncthreads();
         if (wv == 0) {
             if (lane == 0) persist_stamp(slot, seq, t_cmd);
             persist_publish(slot, pubw, nw, seq);
         }
-        if (m == 1) return;
         if (wv == 0) {
             uint4 qd;
             const uint32_t nq = dbl ? zkh_quad_count(32) : 3;
@@ -3718,8 +3732,15 @@ __global__ __launch_bounds__(NTP) void k_lu_persist(LuPersist P) {
     uint32_t m = ls;
     uint64_t t_cmd = 0;
     for (uint32_t seq = 1;; seq++) {
+        if (m == P.me) {  // the block's folded entries of A, S, B, T, m
+            const uint4 *const lo[5] = {tlo[0], tlo[1], tlo[2], tlo[3], tlo[4]};
+            const uint4 *const hi[5] = {thi[0], thi[1], thi[2], thi[3], thi[4]};
+            if (threadIdx.x == 0) persist_stamp(slot, seq, t_cmd, ZKH_LU_PSTAMP);
+            persist_final(P.out + ((size_t)ZKH_LU_PSLOT << P.lgnb) + lb * ZKH_FIN_WORDS(5, m), lo, hi, 5, m, seq);
+            return;
+        }
         uint32_t nw;
-        const bool dbl = P.two && m >= 4;
+        const bool dbl = P.two && m >= 4 * P.me;
         if (dbl) {  // two rounds: the point sums over the cells c < q
             const uint32_t q = m >> 2;
             uint4* wlo = rlo + hs;  // W A, then W B, at the corners (2 rows of m after the W row)
@@ -3756,7 +3777,7 @@ __global__ __launch_bounds__(NTP) void k_lu_persist(LuPersist P) {
                     for (int i = 0; i < 8; i++) pubw[8 * ty + i] = acc.v[i];
             }
             nw = ZKH_LU_MSG2;
-        } else if (m >= 2) {
+        } else {
             const uint32_t h = m >> 1;
             for (uint32_t q = threadIdx.x; q < 4 * h; q += NTP) {  // level 1: row 1 + j, j = q / h
                 const uint32_t j = q / h, k = q - j * h;
@@ -3804,20 +3825,12 @@ __global__ __launch_bounds__(NTP) void k_lu_persist(LuPersist P) {
                     for (int i = 0; i < 8; i++) pubw[8 * ty + i] = acc.v[i];
             }
             nw = ZKH_LU_MSG;
-        } else {  // the block's folded entries A[0], S[0], B[0], T[0], m[0]
-            nw = 40;
-            if (wv == 0 && lane < 5) {
-                const fr_t t = ld_fr(tlo[lane], thi[lane], 0);
-#pragma unroll
-                for (int i = 0; i < 8; i++) pubw[8 * lane + i] = t.v[i];
-            }
         }
         __syncthreads();
         if (wv == 0) {
             if (lane == 0) persist_stamp(slot, seq, t_cmd, ZKH_LU_PSTAMP);
             persist_publish(slot, pubw, nw, seq);
         }
-        if (m == 1) return;
         if (wv == 0) {
             uint4 qd;
             const uint32_t nq = dbl ? zkh_quad_count(32) : 3;

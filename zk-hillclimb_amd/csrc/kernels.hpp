@@ -402,8 +402,10 @@ void launch_to_long(hipStream_t s, DevPlanes p, uint32_t n, int64_t* out);
 // both challenges and answers with the four weights (1-x)(1-y), x(1-y), (1-x)y, xy
 // (Montgomery form, 32 words) of the double fold T[k] <- w00 T[k] + w01 T[k + m/2] +
 // w10 T[k + m/4] + w11 T[k + 3m/4].  With m = 2 the block publishes one round's sums
-// (a0b0, a1b1, da*db: ZKH_MSG_ONE words) and receives the challenge (8 words); with m = 1
-// its folded entries a[0], b[0] (ZKH_MSG_FINAL words), then exits.  Message s carries seq
+// (a0b0, a1b1, da*db: ZKH_MSG_ONE words) and receives the challenge (8 words); with m = me
+// left it writes its folded entries a[0, me), b[0, me) behind the slots (block after block,
+// ZKH_FIN_WORDS(2, me) words each) and exits: the host does the rounds of the last nb me
+// entries, which take it less than the messages would.  Message s carries seq
 // s (1, 2, ...) both ways.  A command quad with seq ZKH_QUIT makes the job's blocks exit;
 // a block that waits longer than `deadline` ticks of the 100 MHz clock sets *err and
 // exits.  Slot words 128..131 hold the block's clock at its last message (publication, and
@@ -414,10 +416,11 @@ void launch_to_long(hipStream_t s, DevPlanes p, uint32_t n, int64_t* out);
 #define ZKH_PSTAMP 128  // first clock-stamp word of a slot
 #define ZKH_MSG_PAIR 72
 #define ZKH_MSG_ONE 24
-#define ZKH_MSG_FINAL 16
 // quad messages: data word i lives at 4*(i/3) + 1 + i%3, quad q's seq at 4*q
 __host__ __device__ inline uint32_t zkh_quad_word(uint32_t i) { return 4 * (i / 3) + 1 + i % 3; }
 __host__ __device__ inline uint32_t zkh_quad_count(uint32_t nwords) { return (nwords + 2) / 3; }
+// words of a block's final message: the m entries of each of its tables as quads
+#define ZKH_FIN_WORDS(tables, m) ((size_t)4 * zkh_quad_count(8 * (tables) * (m)))
 #define ZKH_PLS_MAX 512u  // entries per block and table (32 KiB of LDS for both tables)
 
 // ---- persistent Hadamard rounds (the small rounds of zkh_hp_prove / zkh_hp_prove_eq) ----
@@ -427,11 +430,11 @@ __host__ __device__ inline uint32_t zkh_quad_count(uint32_t nwords) { return (nw
 // (k, k + m/2), sum_k eq_w(g) S_t[k] U_t[k] for t = 0..3 (g = block + nb*k the global pair
 // index, eq_w the device eq weight of the per-round kernels; x 2^-256) or, with E,
 // sum_k E_t[k] S_t[k] U_t[k] (x 2^-512): 32 words, 11 quads.  It then waits for the
-// challenge (Montgomery form, 3 quads) and folds the tables; with m = 1 it publishes S[0],
-// U[0] (and E[0]) (16 or 24 words) and exits.  Message s carries seq s.  Slot layout,
+// challenge (Montgomery form, 3 quads) and folds the tables; with m = me it writes the me
+// entries of S, U (and E) behind the slots and exits.  Message s carries seq s.  Slot layout,
 // ZKH_QUIT and the deadline as in ZkipPersist.
 // With `two` set (eq mode, or an E table with U all ones) a message covers two rounds while
-// m >= 4: over its cells c < m/4 (entries c + j m/4, j = 2 y1 + y2, y1 the first round's
+// m >= 4 me: over its cells c < m/4 (entries c + j m/4, j = 2 y1 + y2, y1 the first round's
 // variable) each block publishes sum_c eq_w(g_c) S_c(y) U_c(y) (eq mode, x 2^-256) or
 // sum_c E_c(y) S_c(y) (x 2^-256) at the nine points y of {0, 1, inf}^2, point 3 a + b
 // (inf: the difference along that axis), ZKH_HP_MSG2 words, and receives the four weights
@@ -445,13 +448,14 @@ struct HpPersist {
     const uint32_t* e_hi;
     const uint32_t* elo;  // eq factor tables (EqW)
     const uint32_t* ehi;
-    uint32_t* out;  // pinned host, nb slots
+    uint32_t* out;  // pinned host, nb slots, then the nb final messages
     uint32_t* cmd;  // pinned host, one command area
     uint32_t* err;
     unsigned long long deadline;
     fr_arg vm;        // the owed fold's challenge (Montgomery form) when fold != 0
     const uint32_t* vmp;  // or, when given, device words from a relay (vmp[8] != 0: return at once)
     uint32_t n, lgnb, fold, two;  // fold: entries g and g + n of the sources fold into g
+    uint32_t me, pad_;
 };
 #define ZKH_HP_MSG 32
 #define ZKH_HP_MSG2 72
@@ -464,10 +468,10 @@ struct HpPersist {
 // w a1 (s1 + beta), w da ds, sum a0, sum a1, sum w b0 (t0 + beta), w b1 (t1 + beta),
 // w db dt, m0 b0, m1 b1, dm db (products x 2^-256; w = eq_w(g) of the global pair index;
 // 88 words, 30 quads), waits for the challenge (3 quads) and folds all five tables; with
-// m = 1 it publishes A[0], S[0], B[0], T[0], m[0] (40 words) and exits.  Slots of
+// m = me it writes the me entries of A, S, B, T, m behind the slots and exits.  Slots of
 // ZKH_LU_PSLOT words (clock stamps from word ZKH_LU_PSTAMP); ZKH_QUIT and the deadline as in
 // ZkipPersist.
-// With `two` set a message covers two rounds while m >= 4: over its cells c < m/4 (entries
+// With `two` set a message covers two rounds while m >= 4 me: over its cells c < m/4 (entries
 // c + j m/4, j = 2 y1 + y2, y1 the first round's variable) each block publishes, at the
 // nine points y of {0, 1, inf}^2 (point 3 a + b, inf: the difference along that axis),
 // sum_c W_c A(y) (S(y) + beta'), sum_c W_c B(y) (T(y) + beta'), sum_c m(y) B(y) (x 2^-256;
@@ -479,7 +483,7 @@ struct LuPersist {
     const uint32_t* hi[5];
     const uint32_t* elo;  // eq factor tables (EqW)
     const uint32_t* ehi;
-    uint32_t* out;  // pinned host, nb slots
+    uint32_t* out;  // pinned host, nb slots, then the nb final messages
     uint32_t* cmd;  // pinned host, one command area
     uint32_t* err;
     unsigned long long deadline;
@@ -487,7 +491,7 @@ struct LuPersist {
     const uint32_t* vmp;  // or, when given, device words from a relay (vmp[8] != 0: return at once)
     fr_arg beta;  // plain
     uint32_t n, lgnb, fold_as, fold_btm;  // fold_*: that group's sources hold 2n entries
-    uint32_t two, pad_[3];
+    uint32_t two, me, pad_[2];
 };
 #define ZKH_LU_MSG 88
 #define ZKH_LU_MSG2 248
@@ -511,9 +515,9 @@ struct ZkipPJob {
     const uint32_t* a_hi;
     const uint32_t* b_lo;
     const uint32_t* b_hi;
-    uint32_t* out;  // pinned host, nb slots
+    uint32_t* out;  // pinned host, nb slots, then the nb final messages
     uint32_t* cmd;  // pinned host, one command area
-    uint32_t n, lgnb, blk_begin, pad_;
+    uint32_t n, lgnb, blk_begin, me;
 };
 struct ZkipPersist {  // passed by value as the kernel argument
     ZkipPJob d[ZKH_MAX_BATCH];

@@ -662,6 +662,22 @@ static uint32_t ceil_log2(uint32_t n) {
     }
     return r;
 }
+// Entries per block that a persistent round loop of nb blocks of ls entries hands over to the
+// host (a power of two).  A message of two rounds costs 12 to 22 us (device sums and fold 4 to
+// 13, host round trip 5 to 8, host work 1 to 5); the host's products take 24 ns, so the rounds
+// of 32 entries left in all take it 4 us (matmul, 5 products a pair), 9 (Hadamard) or 18
+// (logUp, 23): one message fewer, two to four where a single block would go on alone, while 64
+// cost twice the time for no further message.  With two rounds per message their number stays
+// even unless a block goes down to one entry.  Down to one entry per block in every case -> so:
+// matmul 64 x 128 x 64 66.9 -> 51.6 us, 512 lookups in a table of 64 371 -> 348 (a block alone);
+// matmul of 7 jobs of 2048 to 8192 180 -> 176, 2^20 lookups 599 -> 593, RoPE 574 -> 566.
+#define ZKH_HOST_TAIL 32u
+static uint32_t persist_tail(uint32_t ls, uint32_t nb, bool two) {
+    uint32_t me = 1;
+    while (2 * me * nb <= ZKH_HOST_TAIL && 2 * me <= ls) me *= 2;
+    if (two && me > 1 && ceil_log2(ls / me) % 2) me /= 2;
+    return me;
+}
 static uint32_t bits_for(uint64_t absmax) {
     uint32_t b = 0;
     while (b < 63 && ((uint64_t)1 << b) <= absmax) b++;
@@ -2166,7 +2182,7 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
     uint32_t max_inp = 0;
     for (auto& q : J) max_inp = std::max(max_inp, q.INp);
     if (max_inp <= ZKH_PLS_MAX * 128 && !getenv("ZKH_NO_PERSIST")) {
-        std::vector<uint32_t> lgnb(nj), slot_off(nj), cmd_off(nj), grp_of(nj);
+        std::vector<uint32_t> lgnb(nj), slot_off(nj), cmd_off(nj), grp_of(nj), me(nj);
         std::vector<ZkipPersist> groups_p;
         std::vector<uint32_t> grp_blocks;
         size_t words = ZKH_PSLOT;  // word 0: error flag
@@ -2175,8 +2191,9 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
             // ZKH_PLS_MAX entries per block (up to 128 blocks)
             lgnb[j] = INp > ZKH_PLS_MAX ? ceil_log2(INp / ZKH_PLS_MAX) : 0;
             const uint32_t nb = 1u << lgnb[j];
+            me[j] = persist_tail(INp >> lgnb[j], nb, true);
             slot_off[j] = (uint32_t)words;
-            words += (size_t)nb * ZKH_PSLOT;
+            words += nb * (ZKH_PSLOT + ZKH_FIN_WORDS(2, me[j]));
             cmd_off[j] = (uint32_t)words;
             words += ZKH_PSLOT;
             if (groups_p.empty() || grp_blocks.back() + nb > 256 || groups_p.back().nd == ZKH_MAX_BATCH) {
@@ -2190,7 +2207,7 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
         uint32_t* ps = c->ps_host;
         for (uint32_t j = 0; j < nj; j++) {
             const uint32_t nb = 1u << lgnb[j];
-            for (uint32_t b = 0; b < nb; b++) memset(ps + slot_off[j] + b * ZKH_PSLOT, 0, ZKH_PSLOT * 4);
+            memset(ps + slot_off[j], 0, nb * (ZKH_PSLOT + ZKH_FIN_WORDS(2, me[j])) * 4);
             memset(ps + cmd_off[j], 0, ZKH_PSLOT * 4);
         }
         ps[0] = 0;
@@ -2206,6 +2223,7 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
             d.cmd = ps + cmd_off[j];
             d.n = J[j].INp;
             d.lgnb = lgnb[j];
+            d.me = me[j];
             d.blk_begin = grp_blocks[grp_of[j]];
             grp_blocks[grp_of[j]] += 1u << lgnb[j];
             P.err = ps;
@@ -2241,22 +2259,24 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
         // host side: each worker thread advances its jobs (j = t mod T) whenever all of a
         // job's blocks have published
         std::vector<uint32_t> R(nj);
-        for (uint32_t j = 0; j < nj; j++) R[j] = J[j].L - lgnb[j];
+        for (uint32_t j = 0; j < nj; j++) R[j] = J[j].L - lgnb[j] - ceil_log2(me[j]);
         const double t_start = now_us();
         // words of the message that follows `done` local rounds: two rounds' sums, one
         // round's sums, or the folded entries after the last local round
         auto msg_words = [&](uint32_t j, uint32_t done) {
             const uint32_t rem = R[j] - done;
-            return rem >= 2 ? (uint32_t)ZKH_MSG_PAIR : rem == 1 ? (uint32_t)ZKH_MSG_ONE : (uint32_t)ZKH_MSG_FINAL;
+            return rem >= 2 ? (uint32_t)ZKH_MSG_PAIR : rem == 1 ? (uint32_t)ZKH_MSG_ONE : 16 * me[j];
         };
-        // all blocks of job j have published message seq of nw words
-        auto ready = [&](uint32_t j, uint32_t seq, uint32_t nw) {
+        // all blocks of job j have published message seq, which follows `done` rounds
+        auto ready = [&](uint32_t j, uint32_t seq, uint32_t done) {
             const uint32_t nb = 1u << lgnb[j];
-            const uint32_t nq = zkh_quad_count(nw);
+            const uint32_t nq = zkh_quad_count(msg_words(j, done));
+            const bool last = done == R[j];
+            const uint32_t* at = ps + slot_off[j] + (last ? nb * ZKH_PSLOT : 0);
+            const size_t step = last ? ZKH_FIN_WORDS(2, me[j]) : ZKH_PSLOT;
             for (uint32_t b = 0; b < nb; b++)
                 for (uint32_t qd = 0; qd < nq; qd++)
-                    if (__atomic_load_n(ps + slot_off[j] + b * ZKH_PSLOT + 4 * qd, __ATOMIC_ACQUIRE) != seq)
-                        return false;
+                    if (__atomic_load_n(at + b * step + 4 * qd, __ATOMIC_ACQUIRE) != seq) return false;
             return true;
         };
         auto slot_fr = [&](const uint32_t* sl, uint32_t k) {  // Fr k of a block's message
@@ -2295,8 +2315,7 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
         auto serve = [&](uint32_t j, std::vector<Fr>& ta, std::vector<Fr>& tb) -> bool {
             const uint32_t nb = 1u << lgnb[j];
             const uint32_t* sl = ps + slot_off[j];
-            const uint32_t nw = msg_words(j, rnd[j]);
-            if (!ready(j, msg[j] + 1, nw)) return false;
+            if (!ready(j, msg[j] + 1, rnd[j])) return false;
             if (tracing) tr_host[j].push_back(now_us());
             // a block has run, so every earlier launch (the claim partials) has completed
             if (msg[j] == 0) absorb_claim(j);
@@ -2306,7 +2325,7 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
                 lp->fin[j] = 1;
                 lp->open_jobs.fetch_sub(1, std::memory_order_acq_rel);
             };
-            if (nw == ZKH_MSG_PAIR) {  // rounds r and r + 1
+            if (R[j] - r >= 2) {  // rounds r and r + 1
                 Fr sm[9];
                 for (int k = 0; k < 9; k++) sm[k] = kZero;
                 for (uint32_t b = 0; b < nb; b++)
@@ -2343,7 +2362,7 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
                 if (tracing) tr_host[j].push_back(now_us());
                 return true;
             }
-            if (nw == ZKH_MSG_ONE) {
+            if (R[j] - r == 1) {
                 Fr s3[3] = {kZero, kZero, kZero};
                 for (uint32_t b = 0; b < nb; b++)
                     for (int k = 0; k < 3; k++) s3[k] = fr_add(s3[k], slot_fr(sl + b * ZKH_PSLOT, k));
@@ -2366,15 +2385,18 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
                     tr_gpu[j].push_back(m2 <= msg[j] ? st[5 + 2 * m2] - st[4 + 2 * m2] : 0);
                 }
             }
-            // the blocks' folded entries: the remaining lgnb rounds on the host
-            ta.resize(nb);
-            tb.resize(nb);
-            for (uint32_t b = 0; b < nb; b++) {
-                ta[b] = slot_fr(sl + b * ZKH_PSLOT, 0);
-                tb[b] = slot_fr(sl + b * ZKH_PSLOT, 1);
+            // the blocks' folded entries (entry k of block b is index b + nb k): the remaining
+            // rounds on the host
+            const uint32_t left = nb * me[j];
+            ta.resize(left);
+            tb.resize(left);
+            for (uint32_t i = 0; i < left; i++) {
+                const uint32_t* fin = sl + nb * ZKH_PSLOT + (i % nb) * ZKH_FIN_WORDS(2, me[j]);
+                ta[i] = slot_fr(fin, i / nb);
+                tb[i] = slot_fr(fin, me[j] + i / nb);
             }
             bool ok = true;
-            for (uint32_t rr = R[j], m = nb; m > 1 && ok; rr++, m >>= 1) {
+            for (uint32_t rr = R[j], m = left; m > 1 && ok; rr++, m >>= 1) {
                 const uint32_t h = m >> 1;
                 Fr c0 = kZero, q1 = kZero, c2 = kZero;  // each x 2^-256
                 for (uint32_t i = 0; i < h; i++) {
@@ -2395,7 +2417,7 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
             return true;
         };
         // captures by value but for what is used under a job's lock
-        auto worker = [lp, c, ps, nj, tracing, &serve, &ready, &msg_words, &msg, &rnd](int t) {
+        auto worker = [lp, c, ps, nj, tracing, &serve, &ready, &msg, &rnd](int t) {
             Loop& L = *lp;
             struct Stamp {
                 double* at;
@@ -2436,7 +2458,7 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
                         bool all = true;
                         for (uint32_t j = 0; j < nj; j++) {
                             if (L.busy[j].exchange(1, std::memory_order_acquire)) continue;  // being served
-                            all = all && (L.fin[j] || ready(j, msg[j] + 1, msg_words(j, rnd[j])));
+                            all = all && (L.fin[j] || ready(j, msg[j] + 1, rnd[j]));
                             L.busy[j].store(0, std::memory_order_release);
                         }
                         if (!all) why = 4;
@@ -3105,13 +3127,17 @@ static int lu_persist_rounds(zkh_ctx* c, uint8_t tr[32], LuState& L, uint32_t r0
                              bool fold_as, bool fold_btm, const uint32_t vm[8], RelayGuard* rg,
                              const uint32_t beta_l[8], uint32_t* ev_out, uint32_t* ws_out, Fr fin[5], int mode) {
     const uint32_t lgnb = n > ZKH_LH_PLS ? ceil_log2(n / ZKH_LH_PLS) : 0, nb = 1u << lgnb;
-    const uint32_t R = ceil_log2(n) - lgnb;  // local rounds
+    const bool two = !getenv("ZKH_PERSIST_ONE");  // two rounds per message while a block holds >= 4 me entries
+    const uint32_t me = persist_tail(n >> lgnb, nb, two), left = nb * me;
+    const uint32_t R = ceil_log2(n) - ceil_log2(left);  // rounds in the loop
+    const size_t fin_words = ZKH_FIN_WORDS(5, me), words = ZKH_LU_PSLOT * (size_t)(nb + 2) + nb * fin_words;
     int rc;
-    if ((rc = ensure_ps(c, (size_t)ZKH_LU_PSLOT * (nb + 2)))) return rc;
+    if ((rc = ensure_ps(c, words))) return rc;
     uint32_t* ps = c->ps_host;
     uint32_t* slots = ps + ZKH_LU_PSLOT;
-    uint32_t* cmd = ps + (size_t)ZKH_LU_PSLOT * (nb + 1);
-    if (mode != 2) memset(ps, 0, (size_t)ZKH_LU_PSLOT * (nb + 2) * 4);
+    uint32_t* fin_msg = slots + (size_t)ZKH_LU_PSLOT * nb;  // the blocks' final messages
+    uint32_t* cmd = fin_msg + nb * fin_words;
+    if (mode != 2) memset(ps, 0, words * 4);
     LuPersist P{};
     for (int i = 0; i < 5; i++) {
         P.lo[i] = src[i].lo();
@@ -3133,7 +3159,8 @@ static int lu_persist_rounds(zkh_ctx* c, uint8_t tr[32], LuState& L, uint32_t r0
     P.lgnb = lgnb;
     P.fold_as = fold_as;
     P.fold_btm = fold_btm;
-    P.two = getenv("ZKH_PERSIST_ONE") ? 0 : 1;  // two rounds per message while a block holds >= 4 entries
+    P.two = two;
+    P.me = me;
     auto send = [&](uint32_t seq, const uint32_t* xm, uint32_t nw) {
         for (uint32_t i = 0; i < nw && xm; i++) __atomic_store_n(cmd + zkh_quad_word(i), xm[i], __ATOMIC_RELAXED);
         for (uint32_t qd = 0; qd < zkh_quad_count(nw); qd++) __atomic_store_n(cmd + 4 * qd, seq, __ATOMIC_RELEASE);
@@ -3152,19 +3179,22 @@ static int lu_persist_rounds(zkh_ctx* c, uint8_t tr[32], LuState& L, uint32_t r0
         if (mode == 1) return 0;
     }
     const double t_launch = now_us();
-    auto slot_fr = [&](uint32_t b, uint32_t i) {
+    auto quad_fr = [](const uint32_t* msg, uint32_t i) {
         uint32_t v[8];
-        for (uint32_t j = 0; j < 8; j++) v[j] = slots[(size_t)b * ZKH_LU_PSLOT + zkh_quad_word(8 * i + j)];
+        for (uint32_t j = 0; j < 8; j++) v[j] = msg[zkh_quad_word(8 * i + j)];
         return fr_load(v);
     };
-    auto wait_msg = [&](uint32_t seq, uint32_t nw) -> int {
+    auto slot_fr = [&](uint32_t b, uint32_t i) { return quad_fr(slots + (size_t)b * ZKH_LU_PSLOT, i); };
+    auto wait_msg = [&](uint32_t seq, uint32_t nw, bool last) -> int {
         const uint32_t nq = zkh_quad_count(nw);
+        const uint32_t* at = last ? fin_msg : slots;
+        const size_t step = last ? fin_words : (size_t)ZKH_LU_PSLOT;
         const double t0 = now_us();
         for (uint64_t spins = 1;; spins++) {
             bool all = true;
             for (uint32_t b = 0; b < nb && all; b++)
                 for (uint32_t qd = 0; qd < nq; qd++)
-                    if (__atomic_load_n(slots + (size_t)b * ZKH_LU_PSLOT + 4 * qd, __ATOMIC_ACQUIRE) != seq) {
+                    if (__atomic_load_n(at + b * step + 4 * qd, __ATOMIC_ACQUIRE) != seq) {
                         all = false;
                         break;
                     }
@@ -3190,7 +3220,7 @@ static int lu_persist_rounds(zkh_ctx* c, uint8_t tr[32], LuState& L, uint32_t r0
     for (uint32_t lr = 0; lr < R; seq++) {
         const uint32_t r1 = r0 + lr;
         if (!P.two || R - lr < 2) {  // one round
-            if ((rc = wait_msg(seq, ZKH_LU_MSG))) return rc;
+            if ((rc = wait_msg(seq, ZKH_LU_MSG, false))) return rc;
             if (tracing) tr_h.push_back(now_us());
             Fr sm[11];
             for (int t = 0; t < 11; t++) sm[t] = kZero;
@@ -3214,7 +3244,7 @@ static int lu_persist_rounds(zkh_ctx* c, uint8_t tr[32], LuState& L, uint32_t r0
         // 2 y1 + y2 = G[27 + j].  Round r1's sums over the pairs (c + y2 q, c + y2 q + 2q):
         // the eq-weighted pieces as X(t, 0) + rho X(t, 1) (rho = u/(1 - u) of y2 relative to
         // the cell weight), the others X(t, 0) + X(t, 1); round r1 + 1's: X(v1, t)
-        if ((rc = wait_msg(seq, ZKH_LU_MSG2))) return rc;
+        if ((rc = wait_msg(seq, ZKH_LU_MSG2, false))) return rc;
         if (tracing) tr_h.push_back(now_us());
         Fr G[31];
         for (int p = 0; p < 31; p++) G[p] = kZero;
@@ -3256,18 +3286,18 @@ static int lu_persist_rounds(zkh_ctx* c, uint8_t tr[32], LuState& L, uint32_t r0
         if (tracing) tr_h.push_back(now_us());
         lr += 2;
     }
-    if ((rc = wait_msg(seq, 40))) return rc;
+    if ((rc = wait_msg(seq, 40 * me, true))) return rc;
     std::vector<Fr> t[5];
-    for (int i = 0; i < 5; i++) {
-        t[i].resize(nb);
-        for (uint32_t b = 0; b < nb; b++) t[i][b] = slot_fr(b, i);
+    for (uint32_t i = 0; i < 5; i++) {
+        t[i].resize(left);
+        for (uint32_t k = 0; k < left; k++) t[i][k] = quad_fr(fin_msg + (k % nb) * fin_words, i * me + k / nb);
     }
     // (no wait for the blocks to exit: none touches the slots after its last message, and
     // later work on the stream is ordered behind the kernel; tracing reads the clock stamps)
     if (tracing) HIPCHK(c, hipStreamSynchronize(c->stream));
     const Fr beta = fr_load(beta_l);
-    // the last lgnb rounds over the blocks' entries (entry b is global index b)
-    for (uint32_t r = r0 + R, m = nb; m > 1; r++, m >>= 1) {
+    // the last rounds, over the blocks' entries (entry k of block b is index b + nb k)
+    for (uint32_t r = r0 + R, m = left; m > 1; r++, m >>= 1) {
         const uint32_t h = m >> 1, K = L.logD - r - 1;
         Fr sm[11];
         for (int q = 0; q < 11; q++) sm[q] = kZero;
@@ -3298,7 +3328,7 @@ static int lu_persist_rounds(zkh_ctx* c, uint8_t tr[32], LuState& L, uint32_t r0
     for (int i = 0; i < 5; i++) fin[i] = t[i][0];
     if (tracing) {
         fprintf(stderr, "[zkh] lu persistent loop: n=%u, %u blocks, %u device + %u host rounds in %.1f us\n", n, nb, R,
-                lgnb, now_us() - t_launch);
+                ceil_log2(left), now_us() - t_launch);
         trace_persist(c, "lu", slots, seq, tr_h, ZKH_LU_PSTAMP);
     }
     return 0;
@@ -4148,13 +4178,19 @@ static int hp_persist_rounds(zkh_ctx* c, uint8_t tr[32], const std::vector<Fr>* 
     const bool em = u == nullptr;  // explicit E table
     static const char* lab[4] = {"hp0", "hp1", "hp2", "hp3"};
     const uint32_t lgnb = sz > ZKH_LH_PLS ? ceil_log2(sz / ZKH_LH_PLS) : 0, nb = 1u << lgnb;
-    const uint32_t R = ceil_log2(sz) - lgnb;  // local rounds
+    // two rounds per message while a block holds >= 4 me entries: the product is then of degree
+    // 2 in each variable (eq mode, or an E table with U all ones)
+    const bool two = (!em || u_ones) && !getenv("ZKH_PERSIST_ONE");
+    const uint32_t me = persist_tail(sz >> lgnb, nb, two), left = nb * me;
+    const uint32_t R = ceil_log2(sz) - ceil_log2(left);  // rounds in the loop
+    const size_t fin_words = ZKH_FIN_WORDS(em ? 3 : 2, me), words = ZKH_PSLOT * (size_t)(nb + 2) + nb * fin_words;
     int rc;
-    if ((rc = ensure_ps(c, (size_t)ZKH_PSLOT * (nb + 2)))) return rc;
+    if ((rc = ensure_ps(c, words))) return rc;
     uint32_t* ps = c->ps_host;
     uint32_t* slots = ps + ZKH_PSLOT;
-    uint32_t* cmd = ps + (size_t)ZKH_PSLOT * (nb + 1);
-    if (mode != 2) memset(ps, 0, (size_t)ZKH_PSLOT * (nb + 2) * 4);
+    uint32_t* fin_msg = slots + (size_t)ZKH_PSLOT * nb;  // the blocks' final messages
+    uint32_t* cmd = fin_msg + nb * fin_words;
+    if (mode != 2) memset(ps, 0, words * 4);
     HpPersist P{};
     P.s_lo = s_src.lo();
     P.s_hi = s_src.hi();
@@ -4176,9 +4212,8 @@ static int hp_persist_rounds(zkh_ctx* c, uint8_t tr[32], const std::vector<Fr>* 
     P.n = sz;
     P.lgnb = lgnb;
     P.fold = fold ? 1 : 0;
-    // two rounds per message while a block holds >= 4 entries: the product is then of degree
-    // 2 in each variable (eq mode, or an E table with U all ones)
-    P.two = (!em || u_ones) && !getenv("ZKH_PERSIST_ONE") ? 1 : 0;
+    P.two = two;
+    P.me = me;
     auto send = [&](uint32_t seq, const uint32_t* xm, uint32_t nw) {
         for (uint32_t i = 0; i < nw && xm; i++) __atomic_store_n(cmd + zkh_quad_word(i), xm[i], __ATOMIC_RELAXED);
         for (uint32_t qd = 0; qd < zkh_quad_count(nw); qd++) __atomic_store_n(cmd + 4 * qd, seq, __ATOMIC_RELEASE);
@@ -4197,21 +4232,24 @@ static int hp_persist_rounds(zkh_ctx* c, uint8_t tr[32], const std::vector<Fr>* 
         if (mode == 1) return 0;
     }
     const double t_launch = now_us();
-    auto slot_fr = [&](uint32_t b, uint32_t i) {
+    auto quad_fr = [](const uint32_t* msg, uint32_t i) {
         uint32_t v[8];
-        for (uint32_t j = 0; j < 8; j++) v[j] = slots[(size_t)b * ZKH_PSLOT + zkh_quad_word(8 * i + j)];
+        for (uint32_t j = 0; j < 8; j++) v[j] = msg[zkh_quad_word(8 * i + j)];
         return fr_load(v);
     };
+    auto slot_fr = [&](uint32_t b, uint32_t i) { return quad_fr(slots + (size_t)b * ZKH_PSLOT, i); };
     // every block has published message seq (nw words); device errors, a block's
     // deadline and an ended kernel stop the wait
-    auto wait_msg = [&](uint32_t seq, uint32_t nw) -> int {
+    auto wait_msg = [&](uint32_t seq, uint32_t nw, bool last) -> int {
         const uint32_t nq = zkh_quad_count(nw);
+        const uint32_t* at = last ? fin_msg : slots;
+        const size_t step = last ? fin_words : (size_t)ZKH_PSLOT;
         const double t0 = now_us();
         for (uint64_t spins = 1;; spins++) {
             bool all = true;
             for (uint32_t b = 0; b < nb && all; b++)
                 for (uint32_t qd = 0; qd < nq; qd++)
-                    if (__atomic_load_n(slots + (size_t)b * ZKH_PSLOT + 4 * qd, __ATOMIC_ACQUIRE) != seq) {
+                    if (__atomic_load_n(at + b * step + 4 * qd, __ATOMIC_ACQUIRE) != seq) {
                         all = false;
                         break;
                     }
@@ -4271,7 +4309,7 @@ static int hp_persist_rounds(zkh_ctx* c, uint8_t tr[32], const std::vector<Fr>* 
     for (uint32_t lr = 0; lr < R; seq++) {
         const uint32_t r1 = r0 + lr;
         if (!P.two || R - lr < 2) {  // one round
-            if ((rc = wait_msg(seq, ZKH_HP_MSG))) return rc;
+            if ((rc = wait_msg(seq, ZKH_HP_MSG, false))) return rc;
             if (tracing) tr_h.push_back(now_us());
             Fr sums[4] = {kZero, kZero, kZero, kZero};
             for (uint32_t b = 0; b < nb; b++)
@@ -4292,7 +4330,7 @@ static int hp_persist_rounds(zkh_ctx* c, uint8_t tr[32], const std::vector<Fr>* 
         // second y2; 0, 1, inf): round r1's sums at t, over the pairs (c + y2 q, c + y2 q +
         // 2q) of its table, are G(t, 0) + rho G(t, 1), rho = u/(1 - u) of y2 relative to the
         // cell weight (eq mode; 1 with E); round r1 + 1's are G(w1, t)
-        if ((rc = wait_msg(seq, ZKH_HP_MSG2))) return rc;
+        if ((rc = wait_msg(seq, ZKH_HP_MSG2, false))) return rc;
         if (tracing) tr_h.push_back(now_us());
         Fr G[9];
         for (int p = 0; p < 9; p++) G[p] = kZero;
@@ -4335,18 +4373,19 @@ static int hp_persist_rounds(zkh_ctx* c, uint8_t tr[32], const std::vector<Fr>* 
         if (tracing) tr_h.push_back(now_us());
         lr += 2;
     }
-    if ((rc = wait_msg(seq, em ? 24 : 16))) return rc;
-    std::vector<Fr> ta(nb), tb(nb), te(em ? nb : 0);
-    for (uint32_t b = 0; b < nb; b++) {
-        ta[b] = slot_fr(b, 0);
-        tb[b] = slot_fr(b, 1);
-        if (em) te[b] = slot_fr(b, 2);
+    if ((rc = wait_msg(seq, (em ? 24 : 16) * me, true))) return rc;
+    std::vector<Fr> ta(left), tb(left), te(em ? left : 0);
+    for (uint32_t i = 0; i < left; i++) {
+        const uint32_t* msg = fin_msg + (i % nb) * fin_words;
+        ta[i] = quad_fr(msg, i / nb);
+        tb[i] = quad_fr(msg, me + i / nb);
+        if (em) te[i] = quad_fr(msg, 2 * me + i / nb);
     }
     // (no wait for the blocks to exit: none touches the slots after its last message, and
     // later work on the stream is ordered behind the kernel; tracing reads the clock stamps)
     if (tracing) HIPCHK(c, hipStreamSynchronize(c->stream));
-    // the last lgnb rounds over the blocks' entries (entry b is global index b)
-    for (uint32_t r = r0 + R, m = nb; m > 1; r++, m >>= 1) {
+    // the last rounds, over the blocks' entries (entry k of block b is index b + nb k)
+    for (uint32_t r = r0 + R, m = left; m > 1; r++, m >>= 1) {
         const uint32_t h = m >> 1, K = k - r - 1;
         Fr sums[4] = {kZero, kZero, kZero, kZero};
         std::vector<Fr> wl;
@@ -4378,7 +4417,7 @@ static int hp_persist_rounds(zkh_ctx* c, uint8_t tr[32], const std::vector<Fr>* 
     e_fin = em ? te[0] : cE;
     if (tracing) {
         fprintf(stderr, "[zkh] hp persistent loop: n=%u, %u blocks, %u device + %u host rounds in %.1f us\n", sz, nb, R,
-                lgnb, now_us() - t_launch);
+                ceil_log2(left), now_us() - t_launch);
         trace_persist(c, "hp", slots, seq, tr_h);
     }
     return 0;
