@@ -503,7 +503,8 @@ def test_lu_prove(zkh, ctx, shape):
 
 
 @pytest.mark.parametrize("D,N,zeros", [(1 << 16, 1 << 16, ()), (1 << 16, 1 << 12, ()),
-                                        (1 << 16, 1 << 16, (14, 13)), (1 << 16, 1 << 12, (15, 11, 3))])
+                                        (1 << 16, 1 << 16, (14, 13)), (1 << 16, 1 << 12, (15, 11, 3)),
+                                        (1 << 18, 1 << 5, ())])
 def test_lu_prove_derived_rounds(zkh, ctx, D, N, zeros):
     """Tables above the persistent loop's size: the folding rounds leave their sums at 1 to the
     pieces' claims (phase 1, the phase-1 -> 2 round, phase 2).  Coordinates of u set to 0 make

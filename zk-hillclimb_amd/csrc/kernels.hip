@@ -1935,19 +1935,6 @@ uint32_t launch_lu_first_nz(hipStream_t s, Tab A, Tab S, Tab B, Tab T, Tab m, ui
     launch_publish(s, partial);
     return ga + gb;
 }
-uint32_t launch_lu_phase1(hipStream_t s, Tab A, Tab S, uint32_t n, int fold,
-                          const uint32_t* v_m_host, const uint32_t* vmp, const uint32_t* beta_host, EqW eq,
-                          Publish partial, int inv, int derive) {
-    const uint32_t g = grid_for(n >> 1, NT, 1024);
-    fr_t vm = fold && !vmp ? to_fr(v_m_host) : fr_t{};
-    EqDev e{eq.elo, eq.ehi, eq.K};
-    const fr_t beta = to_fr(beta_host);
-    if (fold && derive) k_lu_phase1<1, 1><<<g, NT, 0, s>>>(tab_dev(A), tab_dev(S), n, vm, vmp, beta, e, partial, inv);
-    else if (fold) k_lu_phase1<1, 0><<<g, NT, 0, s>>>(tab_dev(A), tab_dev(S), n, vm, vmp, beta, e, partial, inv);
-    else k_lu_phase1<0, 0><<<g, NT, 0, s>>>(tab_dev(A), tab_dev(S), n, vm, vmp, beta, e, partial, inv);
-    launch_publish(s, partial);
-    return g;
-}
 // ------------------------------------------------------------------------------------
 // Small folding rounds, one pair's products spread over the block's lanes
 // ------------------------------------------------------------------------------------
@@ -2052,6 +2039,46 @@ __global__ __launch_bounds__(NTW) void k_lu_phase2_wide(TabDev A, TabDev S, TabD
     }
     wide_publish(bs, 7, 3, pub);
 }
+// logUp phase 1 likewise: its A and S, rows 0..3 the folded a0 a1 s0 s1, 4 W, 5 W a0, 6 W da,
+// 7 W a0 (s0 + beta), 8 W da ds; sums rows 7, 8, 0.  A round of 64 to 1024 pairs 14.7 us as
+// k_lu_phase1<1, 1> (nine products per pair, one after the other), 7.3 so.
+__global__ __launch_bounds__(NTW) void k_lu_phase1_wide(TabDev A, TabDev S, uint32_t n, fr_t vm, const uint32_t* vmp,
+                                                       fr_t beta, EqDev eq, Publish pub) {
+    if (!relayed_vm(vmp, vm)) return;
+    constexpr uint32_t P = LUW_P;
+    __shared__ uint4 rlo[9 * P], rhi[9 * P];
+    const Rows<P> R{rlo, rhi};
+    const uint32_t h = n >> 1, np = h < P ? h : P, base = blockIdx.x * P;
+    for (uint32_t q = threadIdx.x; q < 5 * np; q += NTW) {  // level 1
+        const uint32_t k = q / np, p = q - k * np, i = base + p;
+        if (k == 4) {
+            R.st(4, p, eq_w(eq, i));
+            continue;
+        }
+        const TabDev& t = k < 2 ? A : S;
+        const uint32_t e = i + (k & 1) * h;
+        const fr_t v = tab_fold_at(t, e, n, vm);
+        st_fr(t.dlo, t.dhi, e, v);
+        R.st(k, p, v);
+    }
+    __syncthreads();
+    for (uint32_t q = threadIdx.x; q < 2 * np; q += NTW) {  // level 2
+        const uint32_t k = q / np, p = q - k * np;
+        const fr_t a0 = R.ld(0, p);
+        R.st(5 + k, p, mont_mul_ol(R.ld(4, p), k ? fr_sub(R.ld(1, p), a0) : a0));
+    }
+    __syncthreads();
+    for (uint32_t q = threadIdx.x; q < 2 * np; q += NTW) {  // level 3
+        const uint32_t k = q / np, p = q - k * np;
+        const fr_t s0 = R.ld(2, p);
+        R.st(7 + k, p, mont_mul_ol(R.ld(5 + k, p), k ? fr_sub(R.ld(3, p), s0) : fr_add(s0, beta)));
+    }
+    __syncthreads();
+    const uint32_t wv = threadIdx.x >> 6;
+    fr_t bs = fr_zero();
+    if (wv < 3) bs = wide_row_sum<P>(R, wv < 2 ? 7 + wv : 0, np);
+    wide_publish(bs, 3, 3, pub);
+}
 #ifndef HPW_P
 #define HPW_P 128
 #endif
@@ -2144,6 +2171,25 @@ __global__ __launch_bounds__(NT) void k_lu_phase2(TabDev A, TabDev S, TabDev B, 
     __shared__ uint4 accl[K * NT], acch[K * NT];
     if (blockIdx.x < ga) lu_phase2_as<fold_as, derive && fold_as>(A, S, n, vm, beta, eq, pub, blockIdx.x, ga, accl, acch, inv_as);
     else lu_phase2_btm<fold_btm, derive && fold_btm>(B, T, m, n, vm, beta, eq, pub, blockIdx.x - ga, gb, ga, accl, acch, inv_btm);
+}
+uint32_t launch_lu_phase1(hipStream_t s, Tab A, Tab S, uint32_t n, int fold,
+                          const uint32_t* v_m_host, const uint32_t* vmp, const uint32_t* beta_host, EqW eq,
+                          Publish partial, int inv, int derive) {
+    const uint32_t g = grid_for(n >> 1, NT, 1024);
+    fr_t vm = fold && !vmp ? to_fr(v_m_host) : fr_t{};
+    EqDev e{eq.elo, eq.ehi, eq.K};
+    const fr_t beta = to_fr(beta_host);
+    if (fold && derive && wide_round(n)) {
+        const uint32_t gw = ((n >> 1) + LUW_P - 1) / LUW_P;
+        k_lu_phase1_wide<<<gw, NTW, 0, s>>>(tab_dev(A), tab_dev(S), n, vm, vmp, beta, e, partial);
+        launch_publish(s, partial);
+        return gw;
+    }
+    if (fold && derive) k_lu_phase1<1, 1><<<g, NT, 0, s>>>(tab_dev(A), tab_dev(S), n, vm, vmp, beta, e, partial, inv);
+    else if (fold) k_lu_phase1<1, 0><<<g, NT, 0, s>>>(tab_dev(A), tab_dev(S), n, vm, vmp, beta, e, partial, inv);
+    else k_lu_phase1<0, 0><<<g, NT, 0, s>>>(tab_dev(A), tab_dev(S), n, vm, vmp, beta, e, partial, inv);
+    launch_publish(s, partial);
+    return g;
 }
 uint32_t launch_lu_phase2(hipStream_t s, Tab A, Tab S, Tab B, Tab T, Tab m, uint32_t n, int fold_as,
                           int fold_btm, const uint32_t* v_m_host, const uint32_t* vmp, const uint32_t* beta_host,

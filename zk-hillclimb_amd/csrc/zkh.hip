@@ -669,7 +669,7 @@ static uint32_t ceil_log2(uint32_t n) {
 // (logUp, 23): one message fewer, two to four where a single block would go on alone, while 64
 // cost twice the time for no further message.  With two rounds per message their number stays
 // even unless a block goes down to one entry.  Down to one entry per block in every case -> so:
-// matmul 64 x 128 x 64 66.9 -> 51.6 us, 512 lookups in a table of 64 371 -> 348 (a block alone);
+// matmul 64 x 128 x 64 66.9 -> 51.6 us, 4096 lookups in a table of 64 371 -> 348 (a block alone);
 // matmul of 7 jobs of 2048 to 8192 180 -> 176, 2^20 lookups 599 -> 593, RoPE 574 -> 566.
 #define ZKH_HOST_TAIL 32u
 static uint32_t persist_tail(uint32_t ls, uint32_t nb, bool two) {
