@@ -3796,12 +3796,16 @@ __global__ __launch_bounds__(NTP) void k_lu_persist(LuPersist P) {
                 st_fr(wlo, whi, t, mont_mul_ol(ld_fr(rlo, rhi, r & (q - 1)), ld_fr(tlo[2 * g2], thi[2 * g2], r)));
             }
             __syncthreads();
-            // wave wv: sum types wv, wv + 16: 0..8 W A(y) (S(y) + beta'), 9..17 W B(y) (T(y) +
-            // beta'), 18..26 m(y) B(y), 27..30 A at corner j
-            for (uint32_t ty = wv; ty < 31; ty += NTP / 64) {
+            // sum types: 0..8 W A(y) (S(y) + beta'), 9..17 W B(y) (T(y) + beta'), 18..26 m(y)
+            // B(y), 27..30 A at corner j.  A type takes as many lanes as there are cells, 8 to
+            // 64, so that few cells leave few waves: each takes its products' time on its SIMD
+            // however many lanes it has (one type per wave at every q: 12 to 13 us a message of at
+            // most 32 cells and 18.6 of 128, instead of 7 to 8 and 15.5)
+            const uint32_t S = q < 8 ? 8 : q < 64 ? q : 64, k = 64 / S, sub = lane % S;
+            for (uint32_t ty = wv * k + lane / S; ty - lane / S < 31; ty += NTP / 64 * k) {
                 fr_t acc = fr_zero();
                 const uint32_t grp = ty / 9, pt = ty - 9 * grp;
-                for (uint32_t cc = lane; cc < q; cc += 64) {
+                for (uint32_t cc = sub; cc < q && ty < 31; cc += S) {
                     if (ty >= 27) {
                         acc = fr_add(acc, ld_fr(tlo[0], thi[0], cc + (ty - 27) * q));
                         continue;
@@ -3809,7 +3813,7 @@ __global__ __launch_bounds__(NTP) void k_lu_persist(LuPersist P) {
                     fr_t x, y;
                     if (grp < 2) {
                         x = pt_val(wlo + grp * m, whi + grp * m, cc, q, pt);
-                        y = pt_val(tlo[1 + 2 * grp], thi[1 + 2 * grp], cc, q, pt);
+                        y = pt_val(grp ? tlo[3] : tlo[1], grp ? thi[3] : thi[1], cc, q, pt);
                         if (pt / 3 < 2 && pt % 3 < 2) y = fr_add(y, beta);
                     } else {
                         x = pt_val(tlo[4], thi[4], cc, q, pt);
@@ -3817,8 +3821,10 @@ __global__ __launch_bounds__(NTP) void k_lu_persist(LuPersist P) {
                     }
                     acc = fr_add(acc, mont_mul_ol(x, y));
                 }
-                acc = fr_wave_sum(acc);
-                if (lane == 0)
+                if (S == 64) acc = fr_wave_sum(acc);
+                else
+                    for (uint32_t z = S >> 1; z >= 1; z >>= 1) acc = fr_add(acc, fr_shfl_xor(acc, z));
+                if (sub == 0 && ty < 31)
 #pragma unroll
                     for (int i = 0; i < 8; i++) pubw[8 * ty + i] = acc.v[i];
             }
