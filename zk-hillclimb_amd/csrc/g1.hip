@@ -176,14 +176,14 @@ __global__ __launch_bounds__(1024) void k_pip_alias(const uint16_t* __restrict__
 
 // ---- bucket chains.  A chain starts from the point at infinity, so its first addition returns
 // the generator itself (bls12-381.cu:1432), as the reference's bucket does.  Two ways to run
-// one: in row form a wave takes one chain, 1.3 us per addition and 1.06 us of a SIMD's time; a
-// lane takes one chain (fp_lane28.hpp), 13 us per addition and 0.2 us of a SIMD's time.  With
+// one: in row form a wave takes one chain, 1.1 us per addition and 0.9 us of a SIMD's time; a
+// lane takes one chain (fp_lane28.hpp), 15 us per addition and 0.2 us of a SIMD's time.  With
 // small signed scalars the row's shared list of negative entries is a chain of n/2 additions,
 // with full-size scalars every chain has about n/16: so the chains are sorted by length, the
 // ones from a length on go to waves and the others, 64 of about one length together, to lanes.
 // 512 rows of 2048 int16: 17.7 ms with long chains on lane quads and short ones on lanes of
-// 32-bit limbs, 2.7 so; 512 rows of 1000 field elements 15.3 and 6.7 (0.2 us x 31M additions
-// over 1024 SIMDs = 6.0).
+// 32-bit limbs, 2.5 so; 512 rows of 1000 field elements 15.3 and 6.0 (0.2 us x 31M additions
+// over 1024 SIMDs).
 
 // the generators in row form with Z^2 and Z^3 behind them (they enter every addition), one
 // wave per point; the plan's counters start at zero
@@ -226,8 +226,8 @@ __global__ __launch_bounds__(512) void k_pip_plan(PipPlan* __restrict__ plan) {
         __syncthreads();
     }
     // the choice b: classes from b on to waves
-    const float rows = work[b], lanes = work[0] - rows, sum = (rows * 1.06f + lanes * 0.2f) / 1024;
-    const float lane_t = b ? 13.0f * lmax[b - 1] : 0, wave_t = rows > 0 ? 1.3f * lmax[511] : 0;
+    const float rows = work[b], lanes = work[0] - rows, sum = (rows * 0.9f + lanes * 0.2f) / 1024;
+    const float lane_t = b ? 15.0f * lmax[b - 1] : 0, wave_t = rows > 0 ? 1.1f * lmax[511] : 0;
     best[b] = fmaxf(sum, fmaxf(lane_t, wave_t)) + 0.1f * sum;
     arg[b] = b;
     __syncthreads();
@@ -653,8 +653,10 @@ __global__ __launch_bounds__(128) void k_g1_addmul(const uint32_t* __restrict__ 
 //   pairwise trees over P[0, h) and P[h, 2h)                  (dev_msm's order)
 //   L = P[0] + P[2h], R = P[h] + P[2h+1]
 //   fold: a' = x a_lo + x^-1 a_hi, b' = x^-1 b_lo + x b_hi, g' = x^-1 g_lo + x g_hi
-// A round of few points is the latency of its two scalar-multiply chains (scale and fold) and
-// one of many points the instruction rate; both are taken on two waves per product.
+// A round of few points is the latency of its two scalar-multiply chains (scale and fold): one
+// product per block, doublings and additions on a wave each.  One of many points is the
+// instruction rate: the points' doubling tables once on lane quads, then the additions of both
+// products of a point from them.
 
 // the working copies of g and Q in row form, one wave per point (point n of a job is Q)
 __global__ __launch_bounds__(256) void k_ipa_points(IpaBatchDev B) {
@@ -705,8 +707,8 @@ __device__ __forceinline__ void ipa_inner(const IpaJobDev& J, uint32_t side, con
 __device__ __forceinline__ G1Tab ipa_table(const IpaBatchDev& B, const IpaJobDev& J, uint32_t id) {
     return g1_tab(B.D, J.pt0 + id - B.slice0, B.slice);
 }
-// one product by waves 0 and 1 of the block (more only take its barriers): blk 0, 1 the Q products with their inner products (first,
-// since they are the longest), then P[blk - 2] with its generator's table
+// one product by waves 0 and 1 of the block (more only take its barriers): blk 0, 1 the Q
+// products with their inner products (first, since they are the longest), then P[blk - 2] with its generator's table
 __device__ __forceinline__ void ipa_product(const IpaBatchDev& B, const IpaJobDev& J, uint32_t blk, const fr_t& r2,
                                             g1_pipe_buf& buf, fr_t* red, uint32_t* ip) {
     const uint32_t h = J.h;
