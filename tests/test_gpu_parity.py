@@ -659,6 +659,19 @@ def test_lu_inverse_sizes(zkh, ctx, n):
     assert not np.asarray(A).reshape(-1, 8)[5].any()
 
 
+@pytest.mark.parametrize("blocks", [1, 2, 4, 5, 16, 17, 64, 65, 256, 257])
+def test_lu_inverse_block_counts(zkh, ctx, blocks):
+    """Batched inversion of tables of that many blocks of 1024 entries, the last one partial:
+    both sides of each leaf count of the stage that joins the blocks."""
+    n = 1024 * blocks - 3
+    rng = np.random.default_rng(blocks)
+    S = rng.integers(0, 2**32, size=(n, 8), dtype=np.uint64).astype(np.uint32)
+    S[:, 7] %= 0x73EDA753  # below r
+    beta = rand_fr_full(rng, 1)[0]
+    A = ctx.lu_inverse(ctx.from_fr(S), beta).to_fr()
+    assert C.check_inverse(S, A, beta) == 0
+
+
 def tuple_case(D, N, ln, seed):
     """A SwiGLU-style tuple lookup: witness G in the table's domain with zero padding in its
     last eighth, a mapped table with int32 extremes, and where the table is padded (ln < N)
