@@ -108,6 +108,26 @@ def test_zkip(zkh, ctx, n, k):
         assert e.value.code == zkh.EROUND
 
 
+@pytest.mark.parametrize("n", [2, 16, 1024, 1500])
+def test_zkip_calls_follow_each_other(zkh, ctx, n):
+    """Calls in sequence whose last rounds lie in the same place of the published sums: each
+    returns its own sums of every round, the last one's coefficients included (its claim check
+    does not see the quadratic one), never the call's before it."""
+    rng = np.random.default_rng(n)
+    k = P.ceil_log2(n)
+    calls = []
+    for _ in range(4):
+        a, b, u = rand_fr(rng, n), rand_fr(rng, n), rand_fr(rng, k)
+        claim = P.to_limbs(sum(x * y for x, y in zip(C.fr_to_ints(a), C.fr_to_ints(b))) % P.R)
+        rc, pw, fw = C.zkip(claim, a, b, u)
+        assert rc == 0
+        calls.append((claim, ctx.from_fr(a), ctx.from_fr(b), u, pw, fw))
+    for i in range(100):
+        claim, a, b, u, pw, fw = calls[i % len(calls)]
+        pg, fg = ctx.zkip(claim, a, b, u)
+        assert fr_eq(pg, pw) and fr_eq(fg, fw), i
+
+
 def _stacked_claim(A, B, uN, N, D):
     Ai, Bi, ui = C.fr_to_ints(A), C.fr_to_ints(B), C.fr_to_ints(uN)
     s = sum(P.eq_weight(n, ui) * Ai[n * D + d] * Bi[n * D + d] for n in range(N) for d in range(D)) % P.R

@@ -711,7 +711,9 @@ __global__ __launch_bounds__(1024) void k_stk_tail(const uint4* alo, const uint4
         M = h;
         __syncthreads();
     }
-    if (t == 0) {
+    // by the wave that wrote the sums: a fence waits for its own wave's stores only, and the
+    // barrier for none
+    if (t == 15 * 64) {
         __threadfence_system();
         __hip_atomic_store(host_flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
