@@ -124,6 +124,19 @@ def test_commit_lane_chains_special_generators(ctx, m, n):
     check(ctx, gens, ctx.from_fr(sc), sc, n, rows=[0, 1, 2, 3, 4, 5, 6, 7, m // 2, m - 2, m - 1])
 
 
+def test_commit_copied_points(ctx):
+    """Every window of a row holds one generator under digit 1, and there are enough chains and
+    windows for lanes to take both: the generator goes from store to store without an addition."""
+    m, n = 420, 64
+    gens = gens_for(14, n)
+    sc = np.zeros((m, n, 8), np.uint32)
+    for r in range(m):
+        for w in range(64):
+            sc[r, (w + r) % n, w // 8] = 1 << (4 * (w % 8))
+    sc = sc.reshape(-1, 8)
+    check(ctx, gens, ctx.from_fr(sc), sc, n, rows=[0, 1, 63, m // 2, m - 1])
+
+
 def test_commit_dimension_errors(zkh, ctx):
     gens = ctx.g1_from_host(gens_for(6, 4))
     with pytest.raises(zkh.ZkhError) as e:

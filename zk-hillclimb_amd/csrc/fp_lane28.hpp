@@ -90,16 +90,16 @@ FDEV f28_t f28_dot(const f28_t& a0, const f28_t& b0, const f28_t& a1, const f28_
 FDEV f28_t f28_mul(const f28_t& a, const f28_t& b) { return f28_dot<1, false>(a, b, a, b); }
 FDEV f28_t f28_sqr(const f28_t& a) { return f28_dot<1, true>(a, a, a, a); }
 
-// whether x (within 32 p of zero) is a multiple of p: a multiple j p has limb 0 = j p_0 mod 2^28,
-// so all but 2^-22 of the other values stop at the first test
-FDEV bool f28_maybe_zero(const f28_t& x) { return (((uint32_t)x.v[0] * FPR_PINV + 32) & FPR_MASK) <= 64; }
+// whether x (in (-32 p, 64 p)) is a multiple of p: a multiple j p has limb 0 = j p_0 mod 2^28, so
+// all but 2^-21 of the other values stop at the first test
+FDEV bool f28_maybe_zero(const f28_t& x) { return (((uint32_t)x.v[0] * FPR_PINV + 32) & FPR_MASK) <= 96; }
 FDEV bool f28_zero(const f28_t& x) {
     if (!f28_maybe_zero(x)) return false;
     f28_t t = x;
 #pragma unroll
     for (int i = 0; i < 14; i++) t.v[i] += k_f28_kb[i];
 #pragma unroll 1
-    for (int j = 0; j <= 64; j++) {
+    for (int j = 0; j <= 96; j++) {
         t = f28_carry(t);
         int32_t o = 0;
 #pragma unroll
@@ -142,11 +142,13 @@ FDEV void f28_put(uint32_t* p, const f28_t& t, uint32_t extra) {  // limbs as th
         q[k] = make_uint4((uint32_t)t.v[4 * k], (uint32_t)t.v[4 * k + 1], (uint32_t)t.v[4 * k + 2], (uint32_t)t.v[4 * k + 3]);
     q[3] = make_uint4((uint32_t)t.v[12], (uint32_t)t.v[13], extra, 0);
 }
-// as a nonnegative value with carried limbs (x within 32 p of zero, stored plus 32 p)
+// as a nonnegative value with carried limbs: a negative x (above -32 p; its top limb is negative)
+// plus 32 p, any other as it is, so that a value that was loaded and only copied stays within
+// its bound however often it is stored
 FDEV void f28_store(uint32_t* p, const f28_t& x, uint32_t extra) {
     f28_t t;
 #pragma unroll
-    for (int i = 0; i < 14; i++) t.v[i] = x.v[i] + k_f28_kb[i];
+    for (int i = 0; i < 14; i++) t.v[i] = x.v[i] + (x.v[13] < 0 ? k_f28_kb[i] : 0);
     f28_put(p, f28_carry(t), extra);
 }
 // a row-form point (fp_row.hpp; G1R_WORDS) as loaded, taken apart where it is used.  The words
@@ -183,8 +185,8 @@ FDEV void g28_store(uint32_t* p, const g28_t& a, bool inf) {
 }
 
 // dbl-2009-l as g1r_dbl, for a point not at infinity.  Coordinates between operations: limbs
-// [0, 1] (z from the row form: [0, 2]) with a signed top limb, x and y in (-17, 36), z in
-// (-1, 36).
+// [0, 1] (z from the row form: [0, 2]) with a signed top limb, x and y in (-17, 45), z in
+// (-1, 36): loaded ones up to the row form's bounds, computed ones below 9.
 FDEV g28_t g28_dbl(const g28_t& a) {
     const f28_t A = f28_sqr(a.x), B = f28_sqr(a.y), C = f28_sqr(B), XB = f28_mul(a.x, B);
     g28_t o;
