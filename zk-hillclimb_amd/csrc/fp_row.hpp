@@ -53,12 +53,12 @@ FDEV fpr_k fpr_consts() {
 }
 
 // ---- movement inside a row (DPP) and between rows (permlane swaps) ----
+// The compiler folds these moves into the additions that use them.  None feeds a subtraction:
+// folded into v_subrev_u32_dpp such a move gave wrong results in f28_perm (fp_lane28.hpp, whose
+// guard a subtraction here would need too).
 template <int I>
 FDEV uint32_t row_bcast(uint32_t x) {  // lane I of the row to all its lanes
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x150 + I, 0xf, 0xf, true);
-}
-FDEV uint32_t row_down(uint32_t x) {  // lane k takes lane k + 1's (lane 15: 0)
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x101, 0xf, 0xf, true);
 }
 FDEV uint32_t row_up(uint32_t x) {  // lane k takes lane k - 1's (lane 0: 0)
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);
@@ -83,8 +83,9 @@ FDEV uint32_t fpr_norm(uint32_t x) { return (x & FPR_MASK) + row_up(x >> 28); }
 
 // a b / R' mod p, below (alpha beta / 2520 + 2) p for operands below alpha p and beta p (p =
 // 2^392 / 2520): every use here keeps it below 2.96 p, or 4 p where that is written; limbs
-// below 2^28 + 16.  Limbs of a and b: their products below 2^59.9 (so that sums stay below
-// 2^60 and a step's carry below 2^32).
+// below 2^28 + 16.  Limbs of a and b: their products below 13 x 2^56 (the largest here are 9 x
+// 2^56), so that with m M's 2^56 and a carry the sum stays below 15 x 2^56 and its carry, plus the
+// 28-bit limb that moves in beside it, below 2^32.
 //
 // Lane k's v[4:5] holds the sum's limb k.  A step I drops the cleared limb 0 (its low 28 bits m
 // go to every lane), moves the limbs down one lane with their carries, and adds a_I b and the

@@ -238,7 +238,7 @@ __global__ __launch_bounds__(512) void k_pip_plan(PipPlan* __restrict__ plan) {
     if (b < PIP_BINS) plan->cursor[b] = cnt[b] - t;
     if (b == 0) {
         plan->items = cnt[0];
-        plan->waves = arg[0] < 512 ? cnt[arg[0]] : 0;
+        plan->waves = cnt[arg[0]];
     }
 }
 // the representative chains (row * 1024 + window * 16 + digit) into their classes' places
