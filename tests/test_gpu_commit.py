@@ -256,6 +256,27 @@ def test_ipa_prove_vs_oracle(zkh, ctx, n):
     assert bytes(st_g) == bytes(st_o)
 
 
+@pytest.mark.parametrize("n", [5999, 6000, 6013])
+@pytest.mark.parametrize("scalar", ["full", 0, 1, 40000])
+def test_g1_addmul_many_rows(ctx, n, scalar):
+    """Both sides of the switch from waves to lane quads: infinity on either side, a[i] s = b[i] and
+    a[i] s = -b[i], a partial last wave; sampled rows against the oracle."""
+    rng = np.random.default_rng(n)
+    k = np.frombuffer(rng.bytes(32 * n), np.uint32).reshape(n, 8).copy()
+    k[:, 7] %= 0x73EDA753
+    a = ctx.g1_mul(ctx.g1_from_host(gens_for(140, 3)), ctx.from_fr(k)).to_host()
+    s = int.from_bytes(rng.bytes(32), "little") % P.R if scalar == "full" else scalar
+    sl = np.array(P.to_limbs(s), np.uint32)
+    b = np.roll(a, 1, axis=0)
+    a[1] = b[2] = G.g1_zero()
+    b[3] = C.g1_mul(a[3], sl)
+    b[4] = C.g1_mul(a[4], np.array(P.to_limbs((-s) % P.R), np.uint32))
+    a[17] = b[17] = G.g1_zero()
+    got = ctx.g1_addmul(ctx.g1_from_host(a), sl, ctx.g1_from_host(b)).to_host()
+    for i in [0, 1, 2, 3, 4, 15, 16, 17, n - 14, n - 13, n - 1] + [int(x) for x in rng.integers(0, n, 8)]:
+        assert np.array_equal(got[i], C.g1_add(b[i], C.g1_mul(a[i], sl))), i
+
+
 @pytest.mark.parametrize("ns", [(16,), (128, 2, 512), (256, 1, 256, 256)])
 def test_ipa_special_points_vs_oracle(zkh, ctx, ns):
     """Batches whose generators hold the point at infinity, equal points and opposite ones, with

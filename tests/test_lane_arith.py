@@ -20,6 +20,13 @@ void store_point(uint32_t* w, const int32_t* x, const int32_t* y, const int32_t*
 }
 void copy_point(uint32_t* w) { bool inf; const g28_t a = g28_load(w, inf); g28_store(w, a, inf); }
 int is_zero(const int32_t* x) { return f28_zero(in(x)); }
+uint32_t from_words(int32_t* r, const uint32_t* w) {
+    uint32_t any;
+    const f28_t t = f28_from_words(w, any);
+    for (int i = 0; i < 14; i++) r[i] = t.v[i];
+    return any;
+}
+void to_words(uint32_t* w, const int32_t* x) { f28_to_words(w, in(x)); }
 }
 """
 
@@ -73,3 +80,20 @@ def test_zero_test_range(lib):
         assert lib.is_zero(ptr(limbs(j * G.P))), j
         for d in (-1, 1, 1 << 28, -(1 << 200)):
             assert not lib.is_zero(ptr(limbs(j * G.P + d))), (j, d)
+
+
+def test_words_of_a_coordinate(lib):
+    """Canonical words to R' = 2^392 residues below 3 p, and any value in (-45 p, 45 p) back to
+    canonical words: 0, 1, p - 1, single bits, multiples of p and random ones."""
+    rng = np.random.default_rng(144)
+    vals = [0, 1, G.P - 1, G.P - 2, 1 << 380] + [1 << i for i in range(0, 380, 7)]
+    vals += [int.from_bytes(rng.bytes(48), "little") % G.P for _ in range(100)]
+    for v in vals:
+        w, t = G.limbs12(v), np.zeros(14, np.int32)
+        assert (lib.from_words(ptr(t), ptr(w)) != 0) == (v != 0)
+        assert 0 <= value(t) < 3 * G.P and (value(t) - (v << 8)) % G.P == 0 and (t[:13] < 1 << 28).all()
+        for j in (-44, -17, -1, 0, 1, 36, 44):
+            x = v * (1 << 8) % G.P + j * G.P
+            back = np.zeros(12, np.uint32)
+            lib.to_words(ptr(back), ptr(limbs(x)))
+            assert np.array_equal(back, w), (v, j)

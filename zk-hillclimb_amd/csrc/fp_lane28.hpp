@@ -184,6 +184,57 @@ FDEV void g28_store(uint32_t* p, const g28_t& a, bool inf) {
     f28_store(p + 32, a.z, 0);
 }
 
+// a coordinate of a 144-byte point (fp_row.hpp) in R' form, below 3 p; any: its words or-ed
+FDEV f28_t f28_from_words(const uint32_t* p, uint32_t& any) {
+    constexpr int32_t in[16] = {FPR_IN_LIMBS};
+    uint32_t w[12];
+    f28_t r, k;
+    any = 0;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const uint4 t = ((const uint4*)p)[i];
+        w[4 * i] = t.x, w[4 * i + 1] = t.y, w[4 * i + 2] = t.z, w[4 * i + 3] = t.w;
+        any |= t.x | t.y | t.z | t.w;
+    }
+#pragma unroll
+    for (int i = 0; i < 14; i++) {
+        const int j = 28 * i / 32, off = 28 * i % 32;
+        uint32_t x = w[j] >> off;
+        if (off > 4 && j < 11) x |= w[j + 1] << (32 - off);
+        r.v[i] = (int32_t)(x & FPR_MASK);
+        k.v[i] = in[i];
+    }
+    return f28_mul(r, k);
+}
+// and back: canonical words of x (in (-45 p, 45 p))
+FDEV void f28_to_words(uint32_t* p, const f28_t& x) {
+    constexpr int32_t out[16] = {FPR_OUT_LIMBS};
+    f28_t k;
+#pragma unroll
+    for (int i = 0; i < 14; i++) k.v[i] = out[i];
+    f28_t t = f28_mul(x, k);  // in (-1, 3)
+#pragma unroll
+    for (int i = 0; i < 14; i++) t.v[i] += k_f28_p[i];
+    t = f28_carry(t);
+#pragma unroll 1
+    for (int n = 0; n < 3; n++) {  // less p where that is not negative
+        f28_t d;
+#pragma unroll
+        for (int i = 0; i < 14; i++) d.v[i] = t.v[i] - k_f28_p[i];
+        d = f28_carry(d);
+        if (d.v[13] >= 0) t = d;
+    }
+    uint32_t w[12];
+#pragma unroll
+    for (int j = 0; j < 12; j++) {
+        const int l = 32 * j / 28, off = 32 * j % 28;
+        w[j] = (uint32_t)t.v[l] >> off | (uint32_t)t.v[l + 1] << (28 - off);
+        if (off > 24) w[j] |= (uint32_t)t.v[l + 2] << (56 - off);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) ((uint4*)p)[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
+}
+
 // dbl-2009-l as g1r_dbl, for a point not at infinity.  Coordinates between operations: limbs
 // [0, 1] (z from the row form: [0, 2]) with a signed top limb, x and y in (-17, 45), z in
 // (-1, 36): loaded ones up to the row form's bounds, computed ones below 9.
@@ -269,6 +320,16 @@ FDEV f28_t f28_sel(bool c, const f28_t& a, const f28_t& b) {
 }
 FDEV f28_t f28_sel4(int q, const f28_t& a, const f28_t& b, const f28_t& c, const f28_t& d) {
     return f28_sel(q == 0, a, f28_sel(q == 1, b, f28_sel(q == 2, c, d)));
+}
+// a 144-byte point to and from a quad, lane q < 3 converting coordinate q
+FDEV g28_t g28q_load(const uint32_t* p, int q, bool& inf) {
+    uint32_t any;
+    const f28_t t = f28_from_words(p + 12 * (q < 3 ? q : 2), any);
+    inf = __builtin_amdgcn_update_dpp(0, (int)any, 0xaa, 0xf, 0xf, true) == 0;  // lane 2's: z = 0
+    return {f28_quad<0>(t), f28_quad<1>(t), f28_quad<2>(t)};
+}
+FDEV void g28q_store(uint32_t* p, const g28_t& a, int q) {
+    if (q < 3) f28_to_words(p + 12 * q, f28_sel4(q, a.x, a.y, a.z, a.z));
 }
 // q: the lane in its quad; a not at infinity.  zz, zzz: lane 3's are a's Z^2 and Z^3
 FDEV g28_t g28q_dbl(const g28_t& a, int q, f28_t& zz, f28_t& zzz) {
