@@ -366,6 +366,24 @@ def test_g1_mul_tables_vs_oracle(zkh, ctx, nb, n):
         assert np.array_equal(got[i], C.g1_mul(base[i % nb], sc[i])), i
 
 
+@pytest.mark.parametrize("nb,n", [(1, 40), (7, 5003), (300, 301), (5001, 5001), (5001, 12000)])
+@pytest.mark.parametrize("bits", [0, 1, 16, 33, 64, 65])
+def test_g1_mul_short_scalars(ctx, nb, n, bits):
+    """Tables that end at the longest scalar's highest bit: all scalars zero, one bit, either side
+    of a limb and of the last block's; sampled products against the oracle."""
+    rng = np.random.default_rng(nb + n + bits)
+    base = gens_for(150, min(nb, 6))
+    base = np.concatenate([base] * (nb // len(base) + 1))[:nb].copy()
+    base[nb // 2] = G.g1_zero()
+    sc = [int(x) & ((1 << bits) - 1) if bits < 64 else 0 for x in rng.integers(0, 2**62, size=n)]
+    sc[n - 1] = 1 << (bits - 1) if bits else 0
+    sc[n // 3] = (1 << bits) - 1
+    t = C.ints_to_fr(sc)
+    got = ctx.g1_mul(ctx.g1_from_host(base), ctx.from_fr(t)).to_host()
+    for i in [0, 1, 2, n // 3, n - 2, n - 1] + [int(x) for x in rng.integers(0, n, 8)]:
+        assert np.array_equal(got[i], C.g1_mul(base[i % nb], t[i])), i
+
+
 def test_ipa_prove_int_witness_and_errors(zkh, ctx):
     """a from an int32 tensor (a folded weight row is small until it is folded); sizes that
     are not a power of two or disagree are ZKH_EARG."""

@@ -495,9 +495,9 @@ __device__ __forceinline__ g28_t g28q_tab_mul(const G1Tab& tab, const uint32_t s
     return acc;
 }
 // a base's table on a lane quad: lane q < 3 stores coordinate q, lane 3 Z^2 and Z^3; signed limbs
-// as they are (the tables of quads are read by quads)
-__device__ __forceinline__ void g28q_table(g28_t a, bool inf, const G1Tab& tab, int q) {
-    for (uint32_t i = 0; i < G1_BITS; i++) {
+// as they are (the tables of quads are read by quads); entries below `bits`
+__device__ __forceinline__ void g28q_table(g28_t a, bool inf, const G1Tab& tab, int q, uint32_t bits) {
+    for (uint32_t i = 0; i < bits; i++) {
         f28_t zz = {}, zzz = {};
         g28_t d = a;
         bool dinf = inf;
@@ -556,15 +556,52 @@ __device__ __forceinline__ g1r_t g1r_mul_pipe(g1r_t a, const uint32_t s[8], bool
 // elementwise with a broadcast base (G1_jacobian_elementwise_mul_broadcast,
 // g1-tensor.cu:463-468): out[i] = base[i % nb] * s[i].
 // The tables of bases [b0, b0 + nt): one wave each in row form (0.2 ms a chain) or, from
-// G1_QUADS on, where the SIMDs are full that way, one quad each (0.75 ms; a third of the work)
+// G1_QUADS on, where the SIMDs are full that way, one quad each (0.75 ms; a third of the work).
+// They end at the highest bit of the launch's scalars, which a reduction ahead of them leaves
+// per block in tops: with 16-bit scalars whole tables took 1.1 ms at 5000 bases and 6.0 at 65536
+// (0.18 and 0.72 so).
 #define G1_QUADS 5000u
+#define G1_TOPS 256u
+// tops[block] = bits of the block's longest scalar
+__global__ __launch_bounds__(256) void k_g1_top(const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
+                                                uint32_t n, uint32_t* __restrict__ tops) {
+    __shared__ int red[4];
+    int top = -1;
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+        const uint4 s0 = ((const uint4*)lo)[i], s1 = ((const uint4*)hi)[i];
+        const uint32_t sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+        const int t = top_bit(sc);
+        top = t > top ? t : top;
+    }
+    for (int o = 32; o >= 1; o >>= 1) {
+        const int t = __shfl_xor(top, o);
+        top = t > top ? t : top;
+    }
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64] = top;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 0; w < 4; w++) top = red[w] > top ? red[w] : top;
+        tops[blockIdx.x] = (uint32_t)(top + 1);
+    }
+}
+// the longest of them all, at least 1 (entry 0 is read past a scalar's last bit); the whole wave
+__device__ __forceinline__ uint32_t g1_bits(const uint32_t* tops, uint32_t ntops) {
+    uint32_t b = 1;
+    for (uint32_t i = threadIdx.x & 63; i < ntops; i += 64) b = tops[i] > b ? tops[i] : b;
+    for (int o = 32; o >= 1; o >>= 1) {
+        const uint32_t t = (uint32_t)__shfl_xor((int)b, o);
+        b = t > b ? t : b;
+    }
+    return __builtin_amdgcn_readfirstlane(b);
+}
 __global__ __launch_bounds__(64) void k_g1_tables(const uint32_t* __restrict__ base, uint32_t b0,
+                                                  const uint32_t* __restrict__ tops, uint32_t ntops,
                                                   uint32_t* __restrict__ tab) {
-    const uint32_t i = blockIdx.x;
+    const uint32_t i = blockIdx.x, bits = g1_bits(tops, ntops);
     const fpr_k c = fpr_consts();
     g1r_t a = g1r_load(base + 36 * (size_t)(b0 + i), c);
     const G1Tab t = g1_tab(tab, i, gridDim.x);
-    for (uint32_t k = 0; k < G1_BITS; k++) {
+    for (uint32_t k = 0; k < bits; k++) {
         g1z_t z{a, 0, 0};
         a = g1z_dbl(z, c);
         g1z_put(t.at(k), g1z_word(z, c), z, c);
@@ -584,21 +621,14 @@ __global__ __launch_bounds__(128) void k_g1_mul(const uint32_t* __restrict__ bas
     const g1r_t m = g1r_mul_pipe(p, sc, dbl, buf, G1Tab{}, c);
     if (!dbl) g1r_store(out + 36 * (size_t)i, m, c);
 }
-// row forms of n points, one wave each
-__global__ __launch_bounds__(256) void k_g1_rows(const uint32_t* __restrict__ base, uint32_t n,
-                                                 uint32_t* __restrict__ out) {
-    const uint32_t i = blockIdx.x * 4 + threadIdx.x / 64;
-    if (i >= n) return;
-    const fpr_k c = fpr_consts();
-    g1r_put(out + G1R_WORDS * (size_t)i, g1r_load(base + 36 * (size_t)i, c), c);
-}
-__global__ __launch_bounds__(64) void k_g1_tables4(const uint32_t* __restrict__ rows, uint32_t nt,
+__global__ __launch_bounds__(64) void k_g1_tables4(const uint32_t* __restrict__ base, uint32_t b0, uint32_t nt,
+                                                   const uint32_t* __restrict__ tops, uint32_t ntops,
                                                    uint32_t* __restrict__ tab) {
-    const uint32_t i = blockIdx.x * 16 + threadIdx.x / 4;
+    const uint32_t i = blockIdx.x * 16 + threadIdx.x / 4, bits = g1_bits(tops, ntops);
     if (i >= nt) return;
     bool inf;
-    const g28_t a = g28_load(rows + G1R_WORDS * (size_t)i, inf);
-    g28q_table(a, inf, g1_tab(tab, i, nt), threadIdx.x & 3);
+    const g28_t a = g28q_load(base + 36 * (size_t)(b0 + i), threadIdx.x & 3, inf);
+    g28q_table(a, inf, g1_tab(tab, i, nt), threadIdx.x & 3, bits);
 }
 // products i0 + k (k < count) of the bases at hand (base (i0 + k) % nb - b0): one wave each
 __global__ __launch_bounds__(64) void k_g1_tab_mul(uint32_t* __restrict__ tab, uint32_t nt, uint32_t nb, uint32_t b0,
@@ -610,25 +640,17 @@ __global__ __launch_bounds__(64) void k_g1_tab_mul(uint32_t* __restrict__ tab, u
     const uint32_t sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
     g1r_store(out + 36 * (size_t)i, g1r_tab_mul(g1_tab(tab, i % nb - b0, nt), sc, c), c);
 }
-// one quad each, products in row form to rows[k]
+// one quad each
 __global__ __launch_bounds__(64, 2) void k_g1_tab_mul4(uint32_t* __restrict__ tab, uint32_t nt, uint32_t nb, uint32_t b0,
                                                     const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
-                                                    uint32_t i0, uint32_t count, uint32_t* __restrict__ rows) {
+                                                    uint32_t i0, uint32_t count, uint32_t* __restrict__ out) {
     const uint32_t k = blockIdx.x * 16 + threadIdx.x / 4, i = i0 + k;
     if (k >= count) return;
     const uint4 s0 = ((const uint4*)lo)[i], s1 = ((const uint4*)hi)[i];
     const uint32_t sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
     const int q = threadIdx.x & 3;
     bool inf;
-    const g28_t r = g28q_tab_mul(g1_tab(tab, i % nb - b0, nt), sc, q, inf);
-    if (q == 0) g28_store(rows + G1R_WORDS * (size_t)k, r, inf);
-}
-__global__ __launch_bounds__(256) void k_g1_points(const uint32_t* __restrict__ rows, uint32_t n,
-                                                   uint32_t* __restrict__ out) {
-    const uint32_t i = blockIdx.x * 4 + threadIdx.x / 64;
-    if (i >= n) return;
-    const fpr_k c = fpr_consts();
-    g1r_store(out + 36 * (size_t)i, g1r_get(rows + G1R_WORDS * (size_t)i, c), c);
+    g28q_store(out + 36 * (size_t)i, g28q_tab_mul(g1_tab(tab, i % nb - b0, nt), sc, q, inf), q);
 }
 // out[i] = b[i] + a[i] * s: one scalar for every row, the sum with b[i] as first operand
 // (hb_addmul with mul_first = false, zkob_fastg1.cuh:56-88: k_g1_mul then k_g1_addsub).  Two
@@ -790,7 +812,7 @@ __global__ __launch_bounds__(256) void k_ipa_tables4(IpaBatchDev B, uint32_t nj,
     const uint32_t id = B.slice0 + k - J.pt0;
     bool inf;
     const g28_t a = g28_load(J.g + G1R_WORDS * (size_t)(id / 2 + (id & 1) * J.h), inf);
-    g28q_table(a, inf, ipa_table(B, J, id), threadIdx.x & 3);
+    g28q_table(a, inf, ipa_table(B, J, id), threadIdx.x & 3, G1_BITS);
 }
 __global__ __launch_bounds__(64, 2) void k_ipa_scale4(IpaBatchDev B, uint32_t nj, uint32_t count) {
     const uint32_t k = blockIdx.x * 16 + threadIdx.x / 4;
@@ -975,7 +997,7 @@ static uint32_t g1_mul_tables(uint32_t nb, uint32_t n) {
 }
 size_t g1_mul_words(uint32_t nb, uint32_t n) {
     const uint32_t nt = g1_mul_tables(nb, n);
-    return nt ? (size_t)nt * G1_BITS * G1Z_WORDS + (size_t)(n > nt ? n : nt) * G1R_WORDS : 0;
+    return nt ? (size_t)nt * G1_BITS * G1Z_WORDS + G1_TOPS : 0;
 }
 void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint32_t* lo, const uint32_t* hi,
                    uint32_t n, uint32_t* out, uint32_t* work) {
@@ -984,15 +1006,15 @@ void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint3
         hipLaunchKernelGGL(k_g1_mul, dim3(n), dim3(128), lds_share(n, 2, sizeof(g1_pipe_buf)), s, base, lo, hi, out);
         return;
     }
-    uint32_t* rows = work + (size_t)nt * G1_BITS * G1Z_WORDS;
+    uint32_t* tops = work + (size_t)nt * G1_BITS * G1Z_WORDS;
+    const uint32_t ntops = n < 256 * G1_TOPS ? (n + 255) / 256 : G1_TOPS;
+    hipLaunchKernelGGL(k_g1_top, dim3(ntops), dim3(256), 0, s, lo, hi, n, tops);
     for (uint32_t b0 = 0; b0 < used; b0 += nt) {
         const uint32_t bases = used - b0 < nt ? used - b0 : nt;
-        if (bases < G1_QUADS) {
-            hipLaunchKernelGGL(k_g1_tables, dim3(bases), dim3(64), 0, s, base, b0, work);
-        } else {
-            hipLaunchKernelGGL(k_g1_rows, dim3((bases + 3) / 4), dim3(256), 0, s, base + 36 * (size_t)b0, bases, rows);
-            hipLaunchKernelGGL(k_g1_tables4, dim3((bases + 15) / 16), dim3(64), 0, s, rows, bases, work);
-        }
+        if (bases < G1_QUADS)
+            hipLaunchKernelGGL(k_g1_tables, dim3(bases), dim3(64), 0, s, base, b0, tops, ntops, work);
+        else
+            hipLaunchKernelGGL(k_g1_tables4, dim3((bases + 15) / 16), dim3(64), 0, s, base, b0, bases, tops, ntops, work);
         // the products of these bases: all at once if they are all the bases, else pass by pass
         const bool all = bases == nb;
         for (uint64_t i0 = b0; i0 < n; i0 += nb) {
@@ -1001,8 +1023,7 @@ void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint3
                 hipLaunchKernelGGL(k_g1_tab_mul, dim3(count), dim3(64), 0, s, work, bases, nb, b0, lo, hi, (uint32_t)i0, out);
             } else {
                 hipLaunchKernelGGL(k_g1_tab_mul4, dim3((count + 15) / 16), dim3(64), 0, s, work, bases, nb, b0, lo, hi,
-                                   (uint32_t)i0, count, rows);
-                hipLaunchKernelGGL(k_g1_points, dim3((count + 3) / 4), dim3(256), 0, s, rows, count, out + 36 * i0);
+                                   (uint32_t)i0, count, out);
             }
             if (all) break;
         }
