@@ -1503,12 +1503,13 @@ extern "C" int zkh_partial_me(zkh_ctx* c, const zkh_tensor* t, const uint32_t* u
     return finish_tensor(c, o, out);
 }
 // FrTensor::multi_dim_me's value left on the device (one-entry tensor, queued) with the
-// dimensions' eq tables at hand: the last dimension is bound first (fr-tensor.cu:643-652)
+// dimensions' eq tables at hand: the last dimension is bound first (fr-tensor.cu:643-652), the
+// ones before `first` not at all
 static int multi_dim_me_queue(zkh_ctx* c, const zkh_tensor* t, const EqWant* const* tab, uint32_t ndim,
-                              zkh_tensor** out) {
+                              zkh_tensor** out, uint32_t first = 0) {
     const zkh_tensor* cur = t;
     zkh_tensor* owned = nullptr;
-    for (uint32_t d = ndim; d-- > 0;) {
+    for (uint32_t d = ndim; d-- > first;) {
         const uint32_t k = (uint32_t)tab[d]->u->size(), n = tab[d]->n;
         zkh_tensor* nxt;
         int rc = 0;
@@ -1533,6 +1534,7 @@ static int read_entry(zkh_ctx* c, zkh_tensor* t, uint32_t out[8]) {
     if (!rc) memcpy(out, w, 32);
     return rc;
 }
+#define ZKH_MDM_TABLE 8192u
 extern "C" int zkh_multi_dim_me(zkh_ctx* c, const zkh_tensor* t, const uint32_t* us,
                                 const uint32_t* ks, const uint32_t* shape, uint32_t ndim,
                                 uint32_t out[8]) {
@@ -1566,11 +1568,18 @@ extern "C" int zkh_multi_dim_me(zkh_ctx* c, const zkh_tensor* t, const uint32_t*
         tab[d] = {&uv[d], (uint32_t)n, nullptr};
         dims[d] = &tab[d];
     }
+    // a long first dimension as zkh_me binds it, from two factor tables: a table of its own has
+    // as many entries as the tensor left
+    const uint32_t first = tab[0].n > ZKH_MDM_TABLE ? 1 : 0;
     zkh_tensor* v;
     int rc;
-    if ((rc = eq_tables_mont(c, tab.data(), ndim, SL_EB)) || (rc = multi_dim_me_queue(c, t, dims.data(), ndim, &v)))
+    if ((rc = eq_tables_mont(c, tab.data() + first, ndim - first, SL_EB)) ||
+        (rc = multi_dim_me_queue(c, t, dims.data(), ndim, &v, first)))
         return rc;
-    return read_entry(c, v, out);
+    if (!first) return read_entry(c, v, out);
+    rc = zkh_me(c, v, us, ks[0], out);
+    zkh_tensor_free(v);
+    return rc;
 }
 extern "C" int zkh_eq_table(zkh_ctx* c, const uint32_t* u, uint32_t k, zkh_tensor** out) {
     if (!c || !out || (!u && k) || k > 30) return fail(c, ZKH_EARG, "bad arguments");
