@@ -79,6 +79,41 @@ def test_partial_me_splits(zkh, ctx, O, C_, W, kind):
     assert fr_eq(ctx.partial_me(tg, u, C_, W).to_fr(), want)
 
 
+@pytest.mark.parametrize("O,C_,W", [(1 << 18, 2, 1), (1 << 18, 16, 1), (1 << 16, 65, 1), (70001, 3, 7), (1, 3, 300001),
+                                    (2, 5, 1 << 16), (3, 1, 1000)])
+@pytest.mark.parametrize("kind", ["fr", "i32"])
+def test_partial_me_many_outputs(zkh, ctx, O, C_, W, kind):
+    """Outputs enough to fill the chip: one or few lanes per sum, and rows so few that a block's
+    lanes all go along them."""
+    rng = np.random.default_rng(O + C_ + W)
+    n, k = O * C_ * W, P.ceil_log2(C_)
+    vals = rng.integers(-2**31, 2**31, size=n)
+    if kind == "fr":
+        t = np.frombuffer(rng.bytes(32 * n), np.uint32).reshape(n, 8).copy()
+        t[:, 7] %= 0x73EDA753
+    else:
+        t = zkh.ints_to_fr(vals)
+    u = rand_fr(rng, k)
+    rc, want = C.partial_me(t, u, C_, W)
+    assert rc == 0
+    tg = ctx.from_fr(t) if kind == "fr" else ctx.from_i32(vals)
+    assert fr_eq(ctx.partial_me(tg, u, C_, W).to_fr(), want)
+
+
+@pytest.mark.parametrize("shape", [(8192, 2), (8193, 3), (16385, 1), (9000, 5, 4), (3, 20000)])
+def test_multi_dim_me_long_dimensions(zkh, ctx, shape):
+    """A first dimension on either side of what one eq table binds, and tables too long for one
+    launch's set."""
+    rng = np.random.default_rng(shape[0])
+    vals = rng.integers(-2**31, 2**31, size=int(np.prod(shape)))
+    us = [rand_fr(rng, P.ceil_log2(d)) for d in shape]
+    t = zkh.ints_to_fr(vals)
+    rc, want = C.multi_dim_me(t, us, list(shape))
+    assert rc == 0
+    assert fr_eq(ctx.multi_dim_me(ctx.from_i32(vals), us, list(shape)), want)
+    assert fr_eq(ctx.multi_dim_me(ctx.from_fr(t), us, list(shape)), want)
+
+
 @pytest.mark.parametrize("low,length,N", [(-8, 16, 16), (-32768, 65536, 65536), (5, 3, 8), (-(1 << 21), 1 << 22, 1 << 22),
                                            (2**31 - 4, 8, 8), (-2**31, 4, 8)])
 def test_range_table(zkh, ctx, low, length, N):

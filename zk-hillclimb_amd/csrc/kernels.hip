@@ -442,11 +442,19 @@ struct PmPlan {
     uint32_t ltw, ltc, per, nch, tiles;  // tiles along w
     uint64_t tasks;
 };
-static PmPlan pm_plan(uint32_t O, uint32_t C, uint32_t W, bool split) {
+// Lanes along c: as many as fill the chip with a few waves per SIMD, more of them for long sums
+// (a thread's terms are a chain), and for outputs that lie C entries apart enough for neighbouring
+// lanes to read neighbouring entries (wide: 32-byte ones).  All that C gives, whatever the outputs,
+// took 2^22 x 4 x 1 int32 from 209 us (one lane) to 246, 100000 x 3 x 7 from 49 to 62, 2^18 x 64 x 1
+// from 256 to 303; one lane everywhere took 1000 x 1000 x 1 from 34 to 99.
+static PmPlan pm_plan(uint32_t O, uint32_t C, uint32_t W, bool split, bool wide) {
     PmPlan p;
     p.ltw = p.ltc = 0;
+    const uint64_t fill = (uint64_t)(C < 16 ? 1 : C < 64 ? 2 : 4) << 18, outs = (uint64_t)O * W;
+    const uint32_t near = W >= 4 ? 0 : C >= 16 ? 2 : C >= 4 && wide ? 1 : 0;
     while (p.ltw < 6 && (1u << p.ltw) < W) p.ltw++;
-    while (p.ltw + p.ltc < 8 && (1u << p.ltc) < C) p.ltc++;
+    while (p.ltw + p.ltc < 8 && (1u << p.ltc) < C && (p.ltc < near || outs << p.ltc < fill)) p.ltc++;
+    while (p.ltw + p.ltc < 8 && (256u >> (p.ltw + p.ltc)) > O && (1u << p.ltw) < W) p.ltw++;  // few rows
     const uint32_t tc = 1u << p.ltc, most = (C + tc - 1) / tc;  // terms per thread without a split
     const uint64_t per = split ? (uint64_t)O * C * W / 131072 : most;  // about two waves per SIMD
     p.per = per < 1 ? 1 : per > most ? most : (uint32_t)per;
@@ -516,18 +524,18 @@ struct LdBounded {
     size_t n;
     ZDEV fr_t operator()(size_t i) const { return i < n ? ld(i) : fr_zero(); }
 };
-size_t partial_me_words(uint32_t O, uint32_t C, uint32_t W) {
-    const PmPlan p = pm_plan(O, C, W, true);
+size_t partial_me_words(int kind, uint32_t O, uint32_t C, uint32_t W) {
+    const PmPlan p = pm_plan(O, C, W, true, kind == 0);
     return p.nch > 1 ? (size_t)p.nch * O * W * 8 : 0;
 }
 template <typename Ld>
-static void partial_me(hipStream_t s, Ld ld, uint32_t O, uint32_t C, uint32_t W, const uint32_t* E, DevPlanes out,
+static void partial_me(hipStream_t s, Ld ld, bool wide, uint32_t O, uint32_t C, uint32_t W, const uint32_t* E, DevPlanes out,
                        uint32_t* work) {
     auto grid = [](const PmPlan& p) { return (uint32_t)(p.tasks < 8192 ? (p.tasks ? p.tasks : 1) : 8192); };
-    const PmPlan p = pm_plan(O, C, W, true);
+    const PmPlan p = pm_plan(O, C, W, true, wide);
     k_partial_me<<<grid(p), 256, 0, s>>>(ld, O, C, W, p, E, PL_LO(out), PL_HI(out), p.nch > 1 ? work : nullptr);
     if (p.nch > 1) {
-        const PmPlan q = pm_plan(1, p.nch, O * W, false);
+        const PmPlan q = pm_plan(1, p.nch, O * W, false, true);
         k_partial_me<<<grid(q), 256, 0, s>>>(LdAos{work}, 1, p.nch, O * W, q, nullptr, PL_LO(out), PL_HI(out), nullptr);
     }
 }
@@ -537,16 +545,16 @@ void launch_partial_me(hipStream_t s, int kind, const void* t, uint32_t cap, siz
     if (kind == 0) {
         DevPlanes p{(uint32_t*)t, cap};
         const LdPlanes ld{PL_LO(p), PL_HI(p)};
-        if (whole) partial_me(s, ld, O, C, W, E, out, work);
-        else partial_me(s, LdBounded<LdPlanes>{ld, n}, O, C, W, E, out, work);
+        if (whole) partial_me(s, ld, true, O, C, W, E, out, work);
+        else partial_me(s, LdBounded<LdPlanes>{ld, n}, true, O, C, W, E, out, work);
     } else if (kind == 1) {
         const LdI32 ld{(const int32_t*)t};
-        if (whole) partial_me(s, ld, O, C, W, E, out, work);
-        else partial_me(s, LdBounded<LdI32>{ld, n}, O, C, W, E, out, work);
+        if (whole) partial_me(s, ld, false, O, C, W, E, out, work);
+        else partial_me(s, LdBounded<LdI32>{ld, n}, false, O, C, W, E, out, work);
     } else {
         const LdI64 ld{(const int64_t*)t};
-        if (whole) partial_me(s, ld, O, C, W, E, out, work);
-        else partial_me(s, LdBounded<LdI64>{ld, n}, O, C, W, E, out, work);
+        if (whole) partial_me(s, ld, false, O, C, W, E, out, work);
+        else partial_me(s, LdBounded<LdI64>{ld, n}, false, O, C, W, E, out, work);
     }
 }
 

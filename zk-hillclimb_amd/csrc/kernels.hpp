@@ -100,8 +100,8 @@ uint32_t launch_sum_planes(hipStream_t s, DevPlanes a, uint32_t n, Publish pub);
 // ---- generic MLE pieces ----
 // out[o*W + w] = sum_{c < C} montmul(E_m[c], t[(o*C + c)*W + w]) over a [O, C, W] view of a tensor
 // with n stored entries (entries at index >= n read as zero); kind 0: FR planes (t, cap), 1:
-// int32, 2: int64.  work: partial_me_words(O, C, W) words
-size_t partial_me_words(uint32_t O, uint32_t C, uint32_t W);
+// int32, 2: int64.  work: partial_me_words(kind, O, C, W) words
+size_t partial_me_words(int kind, uint32_t O, uint32_t C, uint32_t W);
 void launch_partial_me(hipStream_t s, int kind, const void* t, uint32_t cap, size_t n, uint32_t O, uint32_t C,
                        uint32_t W, const uint32_t* E, DevPlanes out, uint32_t* work);
 // padding (FrTensor::pad): dimension d of shape[d] entries padded to 2^lg[d]

@@ -1450,7 +1450,7 @@ static int partial_me_queue(zkh_ctx* c, const zkh_tensor* t, uint32_t O, uint32_
         cap = p.cap;
         kind = 0;
     }
-    uint32_t* work = (uint32_t*)scratch_slot(c, SL_PARTIAL, partial_me_words(O, C, W) * 4, &rc);
+    uint32_t* work = (uint32_t*)scratch_slot(c, SL_PARTIAL, partial_me_words(kind, O, C, W) * 4, &rc);
     if (rc) return rc;
     launch_partial_me(c->stream, kind, src, cap, t->n, O, C, W, E, o, work);
     return 0;
