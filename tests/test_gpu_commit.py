@@ -137,6 +137,36 @@ def test_commit_copied_points(ctx):
     check(ctx, gens, ctx.from_fr(sc), sc, n, rows=[0, 1, 63, m // 2, m - 1])
 
 
+def test_calls_after_a_failed_allocation(zkh):
+    """Scratch that no device has (2^21 rows: 412 GB of buckets) is ZKH_EDEV, and the calls after
+    it, which check their launches, are not taken for failed."""
+    c = zkh.Context(0)
+    try:
+        gens = gens_for(4, 16)
+        rng = np.random.default_rng(4)
+        big = c.from_i32(np.ones(1 << 21, np.int32))
+        a, b = (C.ints_to_fr([int.from_bytes(rng.bytes(32), "little") % P.R for _ in range(8)]) for _ in range(2))
+        u = C.ints_to_fr([5, 6, 7])
+        claim = P.to_limbs(sum(x * y for x, y in zip(C.fr_to_ints(a), C.fr_to_ints(b))) % P.R)
+        ta, tb, g = c.from_fr(a), c.from_fr(b), c.g1_from_host(gens[:8])
+        st_o = C.tr_init("oom")
+        want = C.ipa_prove(st_o, a, b, gens[:8], gens[8], 8)
+        calls = [
+            lambda: np.array_equal(c.partial_me(ta, u, 8, 1).to_fr(), C.partial_me(a, u, 8, 1)[1]),
+            lambda: np.array_equal(c.multi_dim_me(ta, [u[:1], u[1:]], [2, 4]), C.multi_dim_me(a, [u[:1], u[1:]], [2, 4])[1]),
+            lambda: np.array_equal(c.zkip(claim, ta, tb, u)[0], C.zkip(claim, a, b, u)[1]),
+            lambda: np.array_equal(c.ipa_prove(zkh.transcript("oom"), ta, tb, g, gens[8])["L"], want[1]),
+            lambda: np.array_equal(c.commit(g, ta).to_host()[0], C.g1_commit(gens[:8], a, 8)[1][0]),
+        ]
+        for call in calls:
+            with pytest.raises(zkh.ZkhError) as e:
+                c.commit(c.g1_from_host(gens[:1]), big)
+            assert e.value.code == zkh.EDEV
+            assert call()
+    finally:
+        c.close()
+
+
 def test_commit_dimension_errors(zkh, ctx):
     gens = ctx.g1_from_host(gens_for(6, 4))
     with pytest.raises(zkh.ZkhError) as e:

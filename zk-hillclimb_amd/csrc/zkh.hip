@@ -409,6 +409,21 @@ static int fail(zkh_ctx* c, int code, const char* fmt, ...) {
             return fail((ctx), ZKH_EDEV, "%s failed: %s", #x, hipGetErrorString(e_)); \
     } while (0)
 
+// hipMalloc and hipHostMalloc whose failure is the caller's to report: not left behind as the last
+// error, which the launch checks of later calls would take for their own
+static bool dev_alloc(void** p, size_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+}
+static bool host_alloc(void** p, size_t bytes, unsigned flags) {
+    if (hipHostMalloc(p, bytes, flags) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+}
+
 // named scratch slots, grown on demand (freed with the context)
 enum {
     SL_PARTIAL = 0,
@@ -439,7 +454,7 @@ static void* scratch_slot(zkh_ctx* c, int slot, size_t bytes, int* rc) {
         s.bytes = 0;
     }
     size_t want = bytes < 4096 ? 4096 : bytes;
-    if (hipMalloc(&s.p, want) != hipSuccess) {
+    if (!dev_alloc(&s.p, want)) {
         *rc = fail(c, ZKH_EDEV, "hipMalloc(%zu) failed", want);
         return nullptr;
     }
@@ -487,7 +502,7 @@ static int ensure_pinned(zkh_ctx* c, size_t bytes) {
     if (c->pinned) (void)hipHostFree(c->pinned);
     c->pinned = nullptr;
     size_t want = std::max(bytes, (size_t)1 << 20);
-    if (hipHostMalloc((void**)&c->pinned, want, hipHostMallocDefault) != hipSuccess)
+    if (!host_alloc((void**)&c->pinned, want, hipHostMallocDefault))
         return fail(c, ZKH_EDEV, "hipHostMalloc(%zu) failed", want);
     c->pinned_bytes = want;
     return 0;
@@ -501,7 +516,7 @@ static int ensure_ps(zkh_ctx* c, size_t words) {
     c->ps_host = nullptr;
     c->ps_words = 0;
     const size_t want = std::max(words, (size_t)1 << 16);
-    if (hipHostMalloc((void**)&c->ps_host, want * 4, hipHostMallocCoherent) != hipSuccess)
+    if (!host_alloc((void**)&c->ps_host, want * 4, hipHostMallocCoherent))
         return fail(c, ZKH_EDEV, "hipHostMalloc(coherent, %zu) failed", want * 4);
     memset(c->ps_host, 0, want * 4);
     c->ps_words = want;
@@ -636,7 +651,7 @@ static int upload(zkh_ctx* c, void* dst, const void* src, size_t bytes) {
         if (c->ring) (void)hipHostFree(c->ring);
         c->ring = nullptr;
         c->ring_bytes = std::max(need, (size_t)1 << 20);
-        if (hipHostMalloc((void**)&c->ring, c->ring_bytes, hipHostMallocDefault) != hipSuccess) {
+        if (!host_alloc((void**)&c->ring, c->ring_bytes, hipHostMallocDefault)) {
             c->ring_bytes = 0;
             return fail(c, ZKH_EDEV, "hipHostMalloc(ring) failed");
         }
@@ -851,12 +866,12 @@ extern "C" int zkh_ctx_create(int device, zkh_ctx** out) {
         return ZKH_EDEV;
     }
     c->slots.resize(SL_COUNT);
-    if (hipHostMalloc((void**)&c->pub_host, (ZKH_MAX_BATCH * 11 * 8 + 64) * 4, hipHostMallocCoherent) != hipSuccess ||
-        hipMalloc((void**)&c->pub_part, (size_t)4096 * 11 * 32) != hipSuccess ||
-        hipMalloc((void**)&c->pub_lay, ZKH_MAX_BATCH * 3 * 4) != hipSuccess ||
+    if (!host_alloc((void**)&c->pub_host, (ZKH_MAX_BATCH * 11 * 8 + 64) * 4, hipHostMallocCoherent) ||
+        !dev_alloc((void**)&c->pub_part, (size_t)4096 * 11 * 32) ||
+        !dev_alloc((void**)&c->pub_lay, ZKH_MAX_BATCH * 3 * 4) ||
         hipMemset(c->pub_lay, 0, ZKH_MAX_BATCH * 3 * 4) != hipSuccess ||
-        hipHostMalloc((void**)&c->relay_host, 64 * 4, hipHostMallocCoherent) != hipSuccess ||
-        hipMalloc((void**)&c->relay_vm, 16 * 4) != hipSuccess || hipMalloc((void**)&c->flag_d, 64 * 4) != hipSuccess ||
+        !host_alloc((void**)&c->relay_host, 64 * 4, hipHostMallocCoherent) ||
+        !dev_alloc((void**)&c->relay_vm, 16 * 4) || !dev_alloc((void**)&c->flag_d, 64 * 4) ||
         hipMemset(c->flag_d, 0, 64 * 4) != hipSuccess) {
         (void)hipStreamDestroy(c->stream);
         delete c;
@@ -967,7 +982,7 @@ static int tensor_alloc(zkh_ctx* c, int kind, uint32_t n, zkh_tensor** out) {
     t->pool = c->mem;
     t->cls = MemPool::size_class(bytes);
     t->d = c->mem->get(t->cls);
-    if (!t->d && hipMalloc(&t->d, t->cls) != hipSuccess) {
+    if (!t->d && !dev_alloc(&t->d, t->cls)) {
         delete t;
         return fail(c, ZKH_EDEV, "hipMalloc(%zu) failed", t->cls);
     }
@@ -2562,7 +2577,9 @@ static int mm_batch(zkh_ctx* c, zkh_mm_job* jobs, uint32_t nj) {
             HIPCHK(c, hipStreamSynchronize(c->stream));
             (void)hipFree(c->pub_part);
             c->pub_part = nullptr;
-            HIPCHK(c, hipMalloc((void**)&c->pub_part, (size_t)blocks * 3 * 32));
+            c->pub_part_cap = 0;
+            if (!dev_alloc((void**)&c->pub_part, (size_t)blocks * 3 * 32))
+                return fail(c, ZKH_EDEV, "hipMalloc(%zu) failed", (size_t)blocks * 3 * 32);
             c->pub_part_cap = (size_t)blocks * 3;
         }
         ZkipBatch bt;
@@ -3855,7 +3872,7 @@ static int g1_alloc(zkh_ctx* c, uint32_t n, zkh_g1** out) {
     g->pool = c->mem;
     g->cls = MemPool::size_class((size_t)(n ? n : 1) * 144);
     g->d = c->mem->get(g->cls);
-    if (!g->d && hipMalloc(&g->d, g->cls) != hipSuccess) {
+    if (!g->d && !dev_alloc(&g->d, g->cls)) {
         delete g;
         return fail(c, ZKH_EDEV, "hipMalloc(%zu) failed", (size_t)(n ? n : 1) * 144);
     }
