@@ -414,6 +414,51 @@ def test_g1_mul_short_scalars(ctx, nb, n, bits):
         assert np.array_equal(got[i], C.g1_mul(base[i % nb], t[i])), i
 
 
+@pytest.mark.parametrize("cap", [64, 66, 300])
+@pytest.mark.parametrize("ns", [(2, 1), (128, 2, 512), (256, 256, 64)])
+def test_ipa_few_tables(zkh, ctx, ns, cap, monkeypatch):
+    """Memory for fewer tables than a round has points: slices of them, in scale and fold, whose
+    edges lie inside jobs; byte-identical to the oracle."""
+    monkeypatch.setenv("ZKH_TABLE_POINTS", str(cap))
+    rng = np.random.default_rng(cap)
+    jobs, want = [], []
+    for t, n in enumerate(ns):
+        gens = gens_for(160 + t, n + 1)
+        if n > 2:
+            gens[1] = G.g1_zero()
+            gens[n // 2] = gens[0]
+        a, b = (C.ints_to_fr([int.from_bytes(rng.bytes(32), "little") % P.R for _ in range(n)]) for _ in range(2))
+        st_o = C.tr_init("ipaf-%d" % t)
+        rc, L, R, af = C.ipa_prove(st_o, a, b, gens[:n], gens[n], n)
+        assert rc == 0
+        want.append((L, R, af, bytes(st_o)))
+        jobs.append((zkh.transcript("ipaf-%d" % t), ctx.from_fr(a), ctx.from_fr(b), ctx.g1_from_host(gens[:n]), gens[n]))
+    got = ctx.ipa_prove_batch(jobs)
+    for (st, *_), g, (L, R, af, st_o) in zip(jobs, got, want):
+        assert np.array_equal(g["L"], L) and np.array_equal(g["R"], R)
+        assert np.array_equal(g["a_final"], af)
+        assert bytes(st) == st_o
+
+
+@pytest.mark.parametrize("nb,n,cap", [(7, 5003, None), (5001, 12000, 5000), (5001, 12000, 64), (5100, 5100, 5000),
+                                      (300, 301, 64), (25000, 25700, None), (30000, 25001, None)])
+def test_g1_mul_table_slices(ctx, nb, n, cap, monkeypatch):
+    """Tables for fewer bases than there are (more than 24576, or less memory) and for none at all:
+    products on both sides of each slice's edge and of the bases' wrap against the oracle."""
+    if cap:
+        monkeypatch.setenv("ZKH_TABLE_POINTS", str(cap))
+    rng = np.random.default_rng(nb + n)
+    src = gens_for(170, 5)
+    base = np.concatenate([src] * (nb // 5 + 1))[:nb].copy()
+    base[nb - 1] = G.g1_zero()
+    sc = np.frombuffer(rng.bytes(32 * n), np.uint32).reshape(n, 8).copy()
+    sc[:, 7] %= 0x73EDA753
+    got = ctx.g1_mul(ctx.g1_from_host(base), ctx.from_fr(sc)).to_host()
+    edges = [0, n - 1] + [i + d for i in (nb, cap or 24576, nb + (cap or 24576)) for d in (-1, 0, 1)]
+    for i in [i for i in edges if i < n] + [int(x) for x in rng.integers(0, n, 8)]:
+        assert np.array_equal(got[i], C.g1_mul(base[i % nb], sc[i])), i
+
+
 def test_ipa_prove_int_witness_and_errors(zkh, ctx):
     """a from an int32 tensor (a folded weight row is small until it is folded); sizes that
     are not a power of two or disagree are ZKH_EARG."""

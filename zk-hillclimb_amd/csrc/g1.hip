@@ -561,7 +561,6 @@ __device__ __forceinline__ g1r_t g1r_mul_pipe(g1r_t a, const uint32_t s[8], bool
 // per block in tops: with 16-bit scalars whole tables took 1.1 ms at 5000 bases and 6.0 at 65536
 // (0.18 and 0.72 so).
 #define G1_QUADS 5000u
-#define G1_TOPS 256u
 // tops[block] = bits of the block's longest scalar
 __global__ __launch_bounds__(256) void k_g1_top(const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
                                                 uint32_t n, uint32_t* __restrict__ tops) {
@@ -607,9 +606,10 @@ __global__ __launch_bounds__(64) void k_g1_tables(const uint32_t* __restrict__ b
         g1z_put(t.at(k), g1z_word(z, c), z, c);
     }
 }
-// out[i] = base[i] * s[i], two waves per product, no table
-__global__ __launch_bounds__(128) void k_g1_mul(const uint32_t* __restrict__ base, const uint32_t* __restrict__ lo,
-                                                const uint32_t* __restrict__ hi, uint32_t* __restrict__ out) {
+// out[i] = base[i % nb] * s[i], two waves per product, no table
+__global__ __launch_bounds__(128) void k_g1_mul(const uint32_t* __restrict__ base, uint32_t nb,
+                                                const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
+                                                uint32_t* __restrict__ out) {
     __shared__ g1_pipe_buf buf;
     const uint32_t i = blockIdx.x;
     const fpr_k c = fpr_consts();
@@ -617,7 +617,7 @@ __global__ __launch_bounds__(128) void k_g1_mul(const uint32_t* __restrict__ bas
     const uint4 s0 = ((const uint4*)lo)[i], s1 = ((const uint4*)hi)[i];
     const uint32_t sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
     g1r_t p = g1r_zero(c);
-    if (dbl) p = g1r_load(base + 36 * (size_t)i, c);
+    if (dbl) p = g1r_load(base + 36 * (size_t)(i % nb), c);
     const g1r_t m = g1r_mul_pipe(p, sc, dbl, buf, G1Tab{}, c);
     if (!dbl) g1r_store(out + 36 * (size_t)i, m, c);
 }
@@ -935,14 +935,14 @@ void launch_ipa_scale(hipStream_t s, IpaBatchDev& B, uint32_t nj, const uint32_t
         points += 2 * B.j[j].h;
     }
     B.slice0 = 0;
-    B.slice = points < ZKH_IPA_TABLES ? points : ZKH_IPA_TABLES;
-    if (points < G1_QUADS) {
+    B.slice = points < B.cap ? points : B.cap;
+    if (points < G1_QUADS && points <= B.cap) {
         hipLaunchKernelGGL(k_ipa_scale, dim3(blocks), dim3(128), lds_share(blocks, 2, sizeof(g1_pipe_buf) + 129 * 32), s,
                            B, nj, R2);
         return;
     }
-    for (; B.slice0 < points; B.slice0 += ZKH_IPA_TABLES) {
-        const uint32_t count = points - B.slice0 < ZKH_IPA_TABLES ? points - B.slice0 : ZKH_IPA_TABLES;
+    for (; B.slice0 < points; B.slice0 += B.cap) {
+        const uint32_t count = points - B.slice0 < B.cap ? points - B.slice0 : B.cap;
         const uint32_t nq = B.slice0 ? 0 : 2 * nj;
         launch_ipa_tables(s, B, nj, nq, count, R2);
         hipLaunchKernelGGL(k_ipa_scale4, dim3((count + 15) / 16), dim3(64), lds_share((count + 15) / 16, 4, 0), s, B, nj, count);
@@ -959,15 +959,15 @@ void launch_ipa_fold(hipStream_t s, IpaBatchDev& B, uint32_t nj) {
     for (uint32_t j = 0; j < nj; j++) blocks += B.j[j].h;
     const uint32_t points = 2 * blocks;
     B.slice0 = 0;
-    B.slice = points < ZKH_IPA_TABLES ? points : ZKH_IPA_TABLES;
-    if (points < G1_QUADS) {
+    B.slice = points < B.cap ? points : B.cap;
+    if (points < G1_QUADS && points <= B.cap) {
         hipLaunchKernelGGL(k_ipa_fold, dim3(blocks), dim3(128), lds_share(blocks, 2, G1R_WORDS * 4), s, B, nj);
         return;
     }
     fr_t none = {};
-    for (; B.slice0 < points; B.slice0 += ZKH_IPA_TABLES) {
-        const uint32_t count = points - B.slice0 < ZKH_IPA_TABLES ? points - B.slice0 : ZKH_IPA_TABLES;
-        if (points > ZKH_IPA_TABLES)  // more than the tables hold: this slice's again
+    for (; B.slice0 < points; B.slice0 += B.cap) {
+        const uint32_t count = points - B.slice0 < B.cap ? points - B.slice0 : B.cap;
+        if (points > B.cap)  // more than the tables hold: this slice's again
             launch_ipa_tables(s, B, nj, 0, count, none);
         hipLaunchKernelGGL(k_ipa_fold4, dim3((count + 15) / 16), dim3(64), lds_share((count + 15) / 16, 4, 0), s, B, nj, count);
     }
@@ -989,40 +989,36 @@ void launch_g1_addmul(hipStream_t s, const uint32_t* a, const G1Scalar& sc, cons
     else
         hipLaunchKernelGGL(k_g1_addmul4, dim3((n + 15) / 16), dim3(64), lds_share((n + 15) / 16, 4, 0), s, a, sc, b, n, out);
 }
-// bases whose tables are held at once, and the words of scratch for them
-static uint32_t g1_mul_tables(uint32_t nb, uint32_t n) {
+// Tables where bases are shared, or where there are enough products for quads; slices of fewer
+// bases down to G1_QUADS, below which every product runs its own doublings as without tables
+void g1_mul_tables(uint32_t nb, uint32_t n, uint32_t* want, uint32_t* least) {
     const uint32_t used = nb < n ? nb : n;
-    if (used == n && n < G1_QUADS) return 0;  // each base once: no table
-    return used < ZKH_IPA_TABLES ? used : ZKH_IPA_TABLES;
-}
-size_t g1_mul_words(uint32_t nb, uint32_t n) {
-    const uint32_t nt = g1_mul_tables(nb, n);
-    return nt ? (size_t)nt * G1_BITS * G1Z_WORDS + G1_TOPS : 0;
+    *want = used == n && n < G1_QUADS ? 0 : used < ZKH_IPA_TABLES ? used : ZKH_IPA_TABLES;
+    *least = *want < G1_QUADS ? *want : G1_QUADS;
 }
 void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint32_t* lo, const uint32_t* hi,
-                   uint32_t n, uint32_t* out, uint32_t* work) {
-    const uint32_t nt = g1_mul_tables(nb, n), used = nb < n ? nb : n;
+                   uint32_t n, uint32_t* out, uint32_t* tab, uint32_t nt, uint32_t* tops) {
+    const uint32_t used = nb < n ? nb : n;
     if (!nt) {
-        hipLaunchKernelGGL(k_g1_mul, dim3(n), dim3(128), lds_share(n, 2, sizeof(g1_pipe_buf)), s, base, lo, hi, out);
+        hipLaunchKernelGGL(k_g1_mul, dim3(n), dim3(128), lds_share(n, 2, sizeof(g1_pipe_buf)), s, base, nb, lo, hi, out);
         return;
     }
-    uint32_t* tops = work + (size_t)nt * G1_BITS * G1Z_WORDS;
-    const uint32_t ntops = n < 256 * G1_TOPS ? (n + 255) / 256 : G1_TOPS;
+    const uint32_t ntops = n < 256 * ZKH_G1_TOPS ? (n + 255) / 256 : ZKH_G1_TOPS;
     hipLaunchKernelGGL(k_g1_top, dim3(ntops), dim3(256), 0, s, lo, hi, n, tops);
     for (uint32_t b0 = 0; b0 < used; b0 += nt) {
         const uint32_t bases = used - b0 < nt ? used - b0 : nt;
         if (bases < G1_QUADS)
-            hipLaunchKernelGGL(k_g1_tables, dim3(bases), dim3(64), 0, s, base, b0, tops, ntops, work);
+            hipLaunchKernelGGL(k_g1_tables, dim3(bases), dim3(64), 0, s, base, b0, tops, ntops, tab);
         else
-            hipLaunchKernelGGL(k_g1_tables4, dim3((bases + 15) / 16), dim3(64), 0, s, base, b0, bases, tops, ntops, work);
+            hipLaunchKernelGGL(k_g1_tables4, dim3((bases + 15) / 16), dim3(64), 0, s, base, b0, bases, tops, ntops, tab);
         // the products of these bases: all at once if they are all the bases, else pass by pass
         const bool all = bases == nb;
         for (uint64_t i0 = b0; i0 < n; i0 += nb) {
             const uint32_t count = all ? n : (uint32_t)(n - i0 < bases ? n - i0 : bases);
             if (count < G1_QUADS && bases < G1_QUADS) {  // quads leave signed limbs: read by quads
-                hipLaunchKernelGGL(k_g1_tab_mul, dim3(count), dim3(64), 0, s, work, bases, nb, b0, lo, hi, (uint32_t)i0, out);
+                hipLaunchKernelGGL(k_g1_tab_mul, dim3(count), dim3(64), 0, s, tab, bases, nb, b0, lo, hi, (uint32_t)i0, out);
             } else {
-                hipLaunchKernelGGL(k_g1_tab_mul4, dim3((count + 15) / 16), dim3(64), 0, s, work, bases, nb, b0, lo, hi,
+                hipLaunchKernelGGL(k_g1_tab_mul4, dim3((count + 15) / 16), dim3(64), 0, s, tab, bases, nb, b0, lo, hi,
                                    (uint32_t)i0, count, out);
             }
             if (all) break;

@@ -62,14 +62,15 @@ struct IpaJobDev {
     uint32_t h, scale0, fold0, pt0;  // the job's first block of a scale and fold launch, first point
     uint32_t x[8], xi[8], xm[8], xim[8];
 };
-// D: the points' tables (2^i g, i < 255), of points [slice0, slice0 + ZKH_IPA_TABLES) where
-// there are more (the points of all jobs in order, ipa_table)
+// D: the points' tables (2^i g, i < 255), cap of them: of points [slice0, slice0 + cap) where
+// there are more (the points of all jobs in order, ipa_table; cap is even then)
 #define ZKH_IPA_TABLES 24576u
 #define ZKH_TABLE_WORDS (255u * ZKH_POINTZ_WORDS)
 struct IpaBatchDev {
     IpaJobDev j[ZKH_IPA_MAX_JOBS];
     uint32_t* D;
     uint32_t slice0, slice;  // the first point whose table is at hand, and how many are
+    uint32_t cap, pad_;
 };
 // g0[0, 2h] = row forms of g_in[0, 2h) and Q
 void launch_ipa_points(hipStream_t s, const IpaBatchDev& B, uint32_t nj, uint32_t hmax);
@@ -87,6 +88,8 @@ struct G1Scalar {
 void launch_g1_addmul(hipStream_t s, const uint32_t* a, const G1Scalar& sc, const uint32_t* b, uint32_t n,
                       uint32_t* out);
 void launch_g1_mul(hipStream_t s, const uint32_t* base, uint32_t nb, const uint32_t* lo, const uint32_t* hi,
-                   uint32_t n, uint32_t* out, uint32_t* work);
-// words of launch_g1_mul's scratch `work`
-size_t g1_mul_words(uint32_t nb, uint32_t n);
+                   uint32_t n, uint32_t* out, uint32_t* tab, uint32_t nt, uint32_t* tops);
+// its scratch: tab, tables of nt bases (ZKH_TABLE_WORDS each; want of them, fewer down to least,
+// or none), and tops, ZKH_G1_TOPS words beside tables
+#define ZKH_G1_TOPS 256u
+void g1_mul_tables(uint32_t nb, uint32_t n, uint32_t* want, uint32_t* least);

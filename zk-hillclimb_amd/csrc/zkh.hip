@@ -441,9 +441,10 @@ enum {
     SL_TMP5,
     SL_TMP6,
     SL_DESC,
+    SL_TABLES,
     SL_COUNT
 };
-static void* scratch_slot(zkh_ctx* c, int slot, size_t bytes, int* rc) {
+static void* scratch_try(zkh_ctx* c, int slot, size_t bytes) {
     if ((int)c->slots.size() < SL_COUNT) c->slots.resize(SL_COUNT);
     zkh_ctx::Slot& s = c->slots[slot];
     if (s.bytes >= bytes && s.p) return s.p;
@@ -454,12 +455,32 @@ static void* scratch_slot(zkh_ctx* c, int slot, size_t bytes, int* rc) {
         s.bytes = 0;
     }
     size_t want = bytes < 4096 ? 4096 : bytes;
-    if (!dev_alloc(&s.p, want)) {
-        *rc = fail(c, ZKH_EDEV, "hipMalloc(%zu) failed", want);
-        return nullptr;
-    }
+    if (!dev_alloc(&s.p, want)) return nullptr;
     s.bytes = want;
     return s.p;
+}
+static void* scratch_slot(zkh_ctx* c, int slot, size_t bytes, int* rc) {
+    void* p = scratch_try(c, slot, bytes);
+    if (!p) *rc = fail(c, ZKH_EDEV, "hipMalloc(%zu) failed", bytes < 4096 ? (size_t)4096 : bytes);
+    return p;
+}
+// Doubling tables of G1 points (2^i g, 80 KB a point) for `want` points, or for as many as can be
+// had, halved (even numbers) down to `least`; *count of them, or null and 0.  One slot for every
+// entry point that uses tables: at ZKH_IPA_TABLES points it is the 2 GB a context then holds.
+// ZKH_TABLE_POINTS caps their number (64 at least).
+static uint32_t* table_slot(zkh_ctx* c, uint32_t want, uint32_t least, uint32_t* count) {
+    if (const char* e = getenv("ZKH_TABLE_POINTS")) {
+        const long long most = std::max(atoll(e), 64ll) & ~1ll;
+        if (most < want) want = (uint32_t)most;
+    }
+    for (; want >= least && want; want = want / 2 & ~1u) {
+        if (void* p = scratch_try(c, SL_TABLES, (size_t)want * ZKH_TABLE_WORDS * 4)) {
+            *count = want;
+            return (uint32_t*)p;
+        }
+    }
+    *count = 0;
+    return nullptr;
 }
 // Device scratch of the allocation-free entry point zkh_me_static: its eq factor table, the
 // two eq tables (up to ZKH_STATIC_MAX_VARS variables), the block partials and job layout of
@@ -3937,12 +3958,15 @@ extern "C" int zkh_g1_mul(zkh_ctx* c, const zkh_g1* base, const zkh_tensor* t, z
             zkh_g1_free(o);
             return rc;
         }
-        uint32_t* work = (uint32_t*)scratch_slot(c, SL_TMP3, g1_mul_words(base->n, t->n) * 4, &rc);
+        uint32_t want, least, nt = 0, *tab = nullptr, *tops = nullptr;
+        g1_mul_tables(base->n, t->n, &want, &least);
+        if (want) tab = table_slot(c, want, least, &nt);
+        if (tab) tops = (uint32_t*)scratch_slot(c, SL_SMALL, ZKH_G1_TOPS * 4, &rc);
         if (rc) {
             zkh_g1_free(o);
             return rc;
         }
-        launch_g1_mul(c->stream, (const uint32_t*)base->d, base->n, p.lo(), p.hi(), t->n, (uint32_t*)o->d, work);
+        launch_g1_mul(c->stream, (const uint32_t*)base->d, base->n, p.lo(), p.hi(), t->n, (uint32_t*)o->d, tab, nt, tops);
         hipError_t e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) {
@@ -4068,8 +4092,10 @@ extern "C" int zkh_ipa_prove_batch(zkh_ctx* c, uint32_t nj, uint8_t* const* tran
     uint32_t* g_w = rc ? nullptr : (uint32_t*)scratch_slot(c, SL_TMP2, g_words * 4, &rc);
     uint32_t* p_w = rc ? nullptr : (uint32_t*)scratch_slot(c, SL_TMP3, (p_words + 36 * (size_t)nj) * 4, &rc);
     IpaBatchDev B{};
-    if (!rc) B.D = (uint32_t*)scratch_slot(c, SL_TMP4, std::min(points, (size_t)ZKH_IPA_TABLES) * ZKH_TABLE_WORDS * 4, &rc);
     if (rc) return rc;
+    const uint32_t want = (uint32_t)std::min(points, (size_t)ZKH_IPA_TABLES), least = std::min(want, 64u);
+    if (!(B.D = table_slot(c, want, least, &B.cap)))
+        return fail(c, ZKH_EDEV, "ipa_prove: no memory for the tables of %u points", least);
     static_assert(72 * ZKH_IPA_MAX_JOBS <= ZKH_MAX_BATCH * 11 * 8, "L and R of a round fit the published sums");
     uint32_t* lr = c->pub_host;
     uint32_t sz[ZKH_IPA_MAX_JOBS];
