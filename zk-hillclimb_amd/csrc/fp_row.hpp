@@ -95,7 +95,10 @@ FDEV uint32_t fpr_norm(uint32_t x) { return (x & FPR_MASK) + row_up(x >> 28); }
 // form brings below 2 p.  Straight-line code with its own registers, ordered so that two
 // instructions lie between a register's write and its DPP read; as separate statements the
 // compiler adds a 64-bit add and two wait states per step (0.90 against 0.77 us per
-// doubling).
+// doubling).  Nearly all of it is 8-byte instructions, aligned so by a no-op where the code
+// before it is not: four bytes off, a wave alone on its SIMD takes 3 to 6 % longer (a 16384-term
+// row's commitment 11.4 and 10.5 ms, an opening of 64 points 2.61 and 2.44), and which way it
+// lies changed with every edit of the file; on full SIMDs the no-ops cost 1 to 3 %.
 #define FPR_SHIFT                                                               \
     "v_and_b32_e32 v8, 0xfffffff, v4\n\t"                                     \
     "v_alignbit_b32 v9, v5, v4, 28\n\t"
@@ -108,7 +111,8 @@ FDEV uint32_t fpr_norm(uint32_t x) { return (x & FPR_MASK) + row_up(x >> 28); }
     "v_mad_u64_u32 v[4:5], vcc, v7, %3, v[4:5]\n\t"
 FDEV uint32_t fpr_mul(uint32_t a, uint32_t b, const fpr_k& c) {
     uint32_t r;
-    asm("v_mov_b32_e32 v3, 0\n\t"
+    asm(".p2align 3\n\t"
+        "v_mov_b32_e32 v3, 0\n\t"
         "s_nop 0\n\t"
         "v_mov_b32_dpp v6, %1 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
         "v_mad_u64_u32 v[4:5], vcc, v6, %2, 0\n\t"
