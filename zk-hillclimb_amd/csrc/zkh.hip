@@ -178,8 +178,11 @@ static int host_threads() {
 
 // Device buffers of a context's tensors.  A freed tensor's buffer goes back to the pool
 // and serves later allocations of the same size class: hipFree synchronises the device
-// and costs ~0.2 ms for a 128 MiB buffer, hipMalloc ~0.06 ms.  Every entry point returns
-// only after its device work has completed, so a buffer is idle when its tensor is freed.
+// and costs ~0.2 ms for a 128 MiB buffer, hipMalloc ~0.06 ms.  Entry points return only
+// after their device work has completed (zkh_axpy and zkh_hadamard: once it is queued, on
+// the context's own stream), so a buffer is idle when its tensor is freed, or is taken by
+// later work on that stream: tensors that an entry point makes and frees on the way are
+// read there only.
 // The pool is shared with the tensors: one freed after its context releases its buffer.
 struct MemPool {
     std::mutex mu;
@@ -1514,13 +1517,19 @@ static int partial_me_bind(zkh_ctx* c, const zkh_tensor* t, const uint32_t* E, u
     *out = o;
     return 0;
 }
+// An entry point's error return once work that reads the caller's tensors may be queued: the
+// caller may free them, and another context's stream take their buffers, as soon as it has it
+static int drained(zkh_ctx* c, int rc) {
+    if (rc) (void)hipStreamSynchronize(c->stream);
+    return rc;
+}
 // the end of an entry point that leaves `o`: waits for it, or frees it after an error
 static int finish_tensor(zkh_ctx* c, zkh_tensor* o, zkh_tensor** out) {
     const hipError_t e = hipGetLastError();
     int rc = e == hipSuccess ? settle(c) : fail(c, ZKH_EDEV, "launch failed: %s", hipGetErrorString(e));
     if (rc) {
         zkh_tensor_free(o);
-        return rc;
+        return drained(c, rc);
     }
     *out = o;
     return ZKH_OK;
@@ -1535,7 +1544,7 @@ extern "C" int zkh_partial_me(zkh_ctx* c, const zkh_tensor* t, const uint32_t* u
     zkh_tensor* o;
     if ((rc = partial_me_check(c, t, k, cur_dim, window)) || (rc = eq_table_mont(c, load_frs(u, k), cur_dim, SL_EB, &E)) ||
         (rc = partial_me_bind(c, t, E, cur_dim, window, &o)))
-        return rc;
+        return drained(c, rc);
     return finish_tensor(c, o, out);
 }
 // FrTensor::multi_dim_me's value left on the device (one-entry tensor, queued) with the
@@ -1611,11 +1620,11 @@ extern "C" int zkh_multi_dim_me(zkh_ctx* c, const zkh_tensor* t, const uint32_t*
     int rc;
     if ((rc = eq_tables_mont(c, tab.data() + first, ndim - first, SL_EB)) ||
         (rc = multi_dim_me_queue(c, t, dims.data(), ndim, &v, first)))
-        return rc;
-    if (!first) return read_entry(c, v, out);
+        return drained(c, rc);
+    if (!first) return drained(c, read_entry(c, v, out));
     rc = zkh_me(c, v, us, ks[0], out);
     zkh_tensor_free(v);
-    return rc;
+    return drained(c, rc);
 }
 extern "C" int zkh_eq_table(zkh_ctx* c, const uint32_t* u, uint32_t k, zkh_tensor** out) {
     if (!c || !out || (!u && k) || k > 30) return fail(c, ZKH_EARG, "bad arguments");
@@ -4866,7 +4875,7 @@ extern "C" int zkh_partial_me_window(zkh_ctx* c, const zkh_tensor* t, const uint
     if ((rc = tensor_alloc(c, ZKH_KIND_FR, (uint32_t)(orows * window), &o))) return rc;
     if ((rc = partial_me_queue(c, t, (uint32_t)orows, (uint32_t)C, window, E, o->planes()))) {
         zkh_tensor_free(o);
-        return rc;
+        return drained(c, rc);
     }
     return finish_tensor(c, o, out);
 }
@@ -4998,7 +5007,7 @@ extern "C" int zkh_zkip(zkh_ctx* c, const uint32_t claim_l[8], const zkh_tensor*
     if (!A->n || k > ceil_log2(A->n)) return fail(c, ZKH_EARG, "zkip: more challenges than variables");
     if (!fr_is_canonical(claim_l) || !all_canonical(u, k)) return fail(c, ZKH_EARG, "non-canonical input");
     HIPCHK(c, hipSetDevice(c->device));
-    return stk_prove(c, claim_l, A, B, 1, A->n, {}, load_frs(u, k), {}, proof_out, final_out);
+    return drained(c, stk_prove(c, claim_l, A, B, 1, A->n, {}, load_frs(u, k), {}, proof_out, final_out));
 }
 static int stacked_args(zkh_ctx* c, const zkh_tensor* A, const zkh_tensor* B, uint32_t N, uint32_t D,
                         uint32_t kN, uint32_t kD) {
@@ -5019,14 +5028,13 @@ extern "C" int zkh_zkip_stacked(zkh_ctx* c, const uint32_t claim_l[8], const zkh
     if (!fr_is_canonical(claim_l) || !all_canonical(uN, kN) || !all_canonical(vN, kN) || !all_canonical(uD, kD))
         return fail(c, ZKH_EARG, "non-canonical input");
     HIPCHK(c, hipSetDevice(c->device));
-    return stk_prove(c, claim_l, A, B, N, D, load_frs(uN, kN), load_frs(uD, kD), load_frs(vN, kN), proof_out, final_out);
+    return drained(c, stk_prove(c, claim_l, A, B, N, D, load_frs(uN, kN), load_frs(uD, kD), load_frs(vN, kN), proof_out,
+                                final_out));
 }
-extern "C" int zkh_fc_stacked_prove(zkh_ctx* c, const zkh_tensor* X, const zkh_tensor* W,
-                                    const zkh_tensor* Y, const zkh_tensor* bias, uint32_t num,
-                                    uint32_t B, uint32_t IN, uint32_t OUT, const uint32_t* u_num,
-                                    const uint32_t* v_num, const uint32_t* u_batch, const uint32_t* u_input,
-                                    const uint32_t* u_output, uint32_t* proof_out, uint32_t claims_out[16]) {
-    if (!c || !X || !W || !Y || !claims_out) return fail(c, ZKH_EARG, "null argument");
+static int fc_stacked(zkh_ctx* c, const zkh_tensor* X, const zkh_tensor* W, const zkh_tensor* Y,
+                      const zkh_tensor* bias, uint32_t num, uint32_t B, uint32_t IN, uint32_t OUT,
+                      const uint32_t* u_num, const uint32_t* v_num, const uint32_t* u_batch, const uint32_t* u_input,
+                      const uint32_t* u_output, uint32_t* proof_out, uint32_t claims_out[16]) {
     if (!num || !B || !IN || !OUT) return fail(c, ZKH_EARG, "zero dimension");
     // zkFCStacked constructor checks (zkfc.cu:266-269)
     if ((uint64_t)X->n != (uint64_t)num * B * IN) return fail(c, ZKH_EARG, "X size does not match");
@@ -5096,6 +5104,15 @@ extern "C" int zkh_fc_stacked_prove(zkh_ctx* c, const zkh_tensor* X, const zkh_t
     fr_store(cur, claims_out + 8);
     if (!fr_eq(cur, opening)) return fail(c, ZKH_EROUND, "final claim != opening");
     return ZKH_OK;
+}
+extern "C" int zkh_fc_stacked_prove(zkh_ctx* c, const zkh_tensor* X, const zkh_tensor* W,
+                                    const zkh_tensor* Y, const zkh_tensor* bias, uint32_t num,
+                                    uint32_t B, uint32_t IN, uint32_t OUT, const uint32_t* u_num,
+                                    const uint32_t* v_num, const uint32_t* u_batch, const uint32_t* u_input,
+                                    const uint32_t* u_output, uint32_t* proof_out, uint32_t claims_out[16]) {
+    if (!c || !X || !W || !Y || !claims_out) return fail(c, ZKH_EARG, "null argument");
+    return drained(c, fc_stacked(c, X, W, Y, bias, num, B, IN, OUT, u_num, v_num, u_batch, u_input, u_output, proof_out,
+                                 claims_out));
 }
 
 // ---------------------------------------------------------------------------------------
