@@ -137,6 +137,22 @@ def test_commit_copied_points(ctx):
     check(ctx, gens, ctx.from_fr(sc), sc, n, rows=[0, 1, 63, m // 2, m - 1])
 
 
+@pytest.mark.parametrize("n", [1025, 3000, 65535, 65536])
+def test_commit_long_chains(ctx, n):
+    """Chains in the classes of 16 lengths per factor of two, up to the longest there is: every
+    generator under one digit, an even spread over the digits of two windows, and (few
+    generators) signed values, whose upper windows share the list of negative ones."""
+    rng = np.random.default_rng(n)
+    k = np.frombuffer(rng.bytes(32 * n), np.uint32).reshape(n, 8).copy()
+    k[:, 7] %= 0x73EDA753
+    gens = ctx.g1_mul(ctx.g1_from_host(gens_for(180, 2)), ctx.from_fr(k)).to_host()
+    rows = [np.ones(n, np.int64), rng.integers(0, 256, size=n)]
+    if n < 5000:
+        rows += [-np.ones(n, np.int64), rng.integers(-2**15, 2**15, size=n), np.where(rng.random(n) < 0.3, -7, 9)]
+    v = np.concatenate(rows).astype(np.int32)
+    check(ctx, gens, ctx.from_i32(v), C.ints_to_fr(v), n)
+
+
 def test_calls_after_a_failed_allocation(zkh):
     """Scratch that no device has (2^21 rows: 412 GB of buckets) is ZKH_EDEV, and the calls after
     it, which check their launches, are not taken for failed."""

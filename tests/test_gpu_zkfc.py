@@ -215,6 +215,25 @@ def test_fc_stacked_prove(zkh, ctx, num, B, IN, OUT, bias):
     assert e.value.code == zkh.EROUND
 
 
+def test_fc_stacked_many_variables(zkh, ctx):
+    """33 variables in all: more than the eq tables' one launch takes, so each table has its own
+    with uploaded factors."""
+    num, B, IN, OUT = 17, 129, 65, 129
+    rng = np.random.default_rng(33)
+    X = rng.integers(-300, 300, size=(num, B, IN)).astype(np.int64)
+    W = rng.integers(-300, 300, size=(num, IN, OUT)).astype(np.int64)
+    bv = rng.integers(-99, 100, size=(num, OUT)).astype(np.int64)
+    Y = np.einsum("sbi,sio->sbo", X, W) + bv[:, None, :]
+    un, vn, ub, ui, uo = (rand_fr(rng, P.ceil_log2(x)) for x in (num, num, B, IN, OUT))
+    assert sum(len(x) for x in (un, vn, ub, ui, uo)) == 33
+    fr = [zkh.ints_to_fr(v.reshape(-1)) for v in (X, W, Y, bv)]
+    rc, pw, cw = C.fc_stacked_prove(*fr, num, B, IN, OUT, un, vn, ub, ui, uo)
+    assert rc == 0
+    pg, cg = ctx.fc_stacked_prove(ctx.from_i32(X), ctx.from_i32(W), ctx.from_i64(Y), ctx.from_i64(bv), num, B, IN, OUT,
+                                  un, vn, ub, ui, uo)
+    assert fr_eq(pg, pw) and fr_eq(cg, cw)
+
+
 # ---------------------------------------------------------------- rescaling witness
 @pytest.mark.parametrize("sf", [1, 2, 3, 256, 1 << 16])
 def test_rescale(zkh, ctx, sf):
