@@ -5,7 +5,7 @@
 // needs an add-with-carry beside it and every sum a canonical reduction; 28-bit limbs leave a
 // column of 28 products inside 64 bits, so a product is 392 multiply-adds and ~100 other
 // instructions, and sums and differences are taken limb by limb, signed, without carries: an
-// addition 0.19 us of a SIMD's time instead of 0.34 (12 us on an idle SIMD instead of 29).
+// addition 0.19 us of a SIMD's time instead of 0.34 (12 us with a SIMD to itself instead of 29).
 // Values lie within a few p of zero on either side.  Bounds (in units of 2^28 for limbs, of p for values) are written at each use: a
 // product's operands need (limb bound a) x (limb bound b), summed over the products it adds, of
 // at most 8 - 1 (14 x 2^56 x 8 < 2^63, the reduction adding one unit), and leaves limbs in [0, 1],

@@ -177,7 +177,8 @@ __global__ __launch_bounds__(1024) void k_pip_alias(const uint16_t* __restrict__
 // ---- bucket chains.  A chain starts from the point at infinity, so its first addition returns
 // the generator itself (bls12-381.cu:1432), as the reference's bucket does.  Two ways to run
 // one: in row form a wave takes one chain, 1.1 us per addition and 0.9 us of a SIMD's time; a
-// lane takes one chain (fp_lane28.hpp), 15 us per addition and 0.2 us of a SIMD's time.  With
+// lane takes one chain (fp_lane28.hpp), 15 us per addition here (two waves on a SIMD, operands
+// from the table) and 0.2 us of a SIMD's time.  With
 // small signed scalars the row's shared list of negative entries is a chain of n/2 additions,
 // with full-size scalars every chain has about n/16: so the chains are sorted by length, the
 // ones from a length on go to waves and the others, 64 of about one length together, to lanes.
@@ -514,9 +515,9 @@ __device__ __forceinline__ void g28q_table(g28_t a, bool inf, const G1Tab& tab, 
 }
 // One product on two waves in row form: wave 0 of the pair runs the doubling chain and hands
 // each 2^i a to wave 1 through LDS, G1P_B doublings per block barrier; wave 1 adds the ones
-// whose bit is set one barrier later.  The chain is latency-bound (0.77 us per doubling, 1.28
-// per addition on an idle SIMD): 255 doublings and 127 additions side by side take 0.25 ms.
-// At 16 doublings per barrier the additions of a chunk (10 +- 2.6 us) rarely outlast its
+// whose bit is set one barrier later.  The chain is latency-bound (0.77 us per doubling, 1.05
+// per addition on an idle SIMD): 255 doublings and 127 additions side by side take 0.23 ms.
+// At 16 doublings per barrier the additions of a chunk (8.4 +- 2.1 us) rarely outlast its
 // doublings (12.3 us).  Every wave of the block calls it (dbl: its part), with one scalar per
 // pair; the product is in the adding wave, which does not read `a`.  tab: where the base's
 // table is wanted too (all 255 doublings then), else null and the doublings after the highest
