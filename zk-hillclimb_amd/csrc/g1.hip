@@ -557,7 +557,7 @@ __device__ __forceinline__ g1r_t g1r_mul_pipe(g1r_t a, const uint32_t s[8], bool
 // elementwise with a broadcast base (G1_jacobian_elementwise_mul_broadcast,
 // g1-tensor.cu:463-468): out[i] = base[i % nb] * s[i].
 // The tables of bases [b0, b0 + nt): one wave each in row form (0.2 ms a chain) or, from
-// G1_QUADS on, where the SIMDs are full that way, one quad each (0.75 ms; a third of the work).
+// G1_QUADS on, where the SIMDs are full that way, one quad each (1.0 ms; a third of the work).
 // They end at the highest bit of the launch's scalars, which a reduction ahead of them leaves
 // per block in tops: with 16-bit scalars whole tables took 1.1 ms at 5000 bases and 6.0 at 65536
 // (0.18 and 0.72 so).
